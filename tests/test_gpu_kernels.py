@@ -1563,3 +1563,84 @@ def test_embed_suffix_and_euler_step(out_dtype):
     sync()
     v = orc.linear(got[:, n_lead:].reshape(-1, W), W_out, b_out).reshape(B, S - n_lead, A)
     assert rel_err(host(xd), x_t - 0.1 * v) < FP32_TOL
+
+
+# ---------------------------------------------- narrow tiles of few-row projections
+@pytest.mark.parametrize("plan", [1, 2, 3, 4])
+@pytest.mark.parametrize("M,N,K", [(1, 64, 64), (16, 48, 128), (17, 200, 720), (33, 1536, 1536), (64, 96, 1040), (65, 32, 4096),
+                                   (102, 720, 976), (300, 24, 336)])
+def test_narrow_tile_projection_has_the_tiled_kernels_bits(tune, plan, M, N, K):
+    """Every rows x columns split of the narrow-tile kernel (VLA_GEMM_ROWS_PLAN) at the edges of its
+    row blocks, column tiles (N not a multiple of 16) and 128-k stages (fewer stages than the ring,
+    partial last stage, half a 32-k product): the bits of the tiled kernel, plain, gated and with
+    the RMSNorm inside, and the oracle within fp32 rounding (1e-5)."""
+    r = np.random.default_rng(8800 + M + N)
+    x = orc.round_bf16(r.standard_normal((M, K)).astype(np.float32))
+    W = orc.round_bf16((0.05 * r.standard_normal((N, K))).astype(np.float32))
+    b = (0.1 * r.standard_normal(N)).astype(np.float32)
+    res = orc.round_bf16(r.standard_normal((M, N)).astype(np.float32))
+    xd, Wd, rd, bd = to_dev(x, BF16), to_dev(W, BF16), to_dev(res, BF16), dev(b)
+    gate = dev(r.standard_normal(N).astype(np.float32))
+    I = N // 2
+
+    def run():
+        y, yb, yg = torch.zeros((M, N), device="cuda"), empty((M, N), BF16), empty((M, N), BF16)
+        pkg.call("vla_linear", xd, Wd, None, None, y, BF16, F32, M, N, K)
+        pkg.call("vla_linear", xd, Wd, bd, rd, yb, BF16, BF16, M, N, K)
+        pkg.call("vla_linear_gated", xd, Wd, bd, gate, rd, yg, BF16, BF16, M, N, K)
+        out = [host(y), host(yb), host(yg)]
+        if I % 32 == 0:
+            for eps in (-1.0, 1e-5):
+                yu = torch.zeros((M, I), device="cuda")
+                pkg.call("vla_glu_linear", xd, Wd, bd, yu, BF16, F32, M, I, K, pkg.VLA_ACT_SILU, eps)
+                out.append(host(yu))
+        sync()
+        return out
+
+    tune.set("VLA_GEMM_ROWS_PLAN", plan)
+    got = run()
+    tune.set("VLA_GEMM_ROWS_MAX", 0)
+    tiled = run()
+    assert rel_err(got[0], orc.linear(x, W)) < FP32_TOL
+    assert bf16_close(orc.from_bf16(got[1].view(np.uint16)), orc.linear(x, W) + b + res)
+    for g, t in zip(got, tiled):
+        assert np.array_equal(g.view(np.uint8), t.view(np.uint8))
+
+
+@pytest.mark.parametrize("B,S,Hq,Hkv,D,K,rope", [(1, 50, 15, 5, 64, 720, True), (3, 51, 8, 1, 256, 1024, True), (1, 49, 32, 32, 48, 1536, False),
+                                                (2, 17, 4, 4, 48, 336, False)])
+def test_narrow_tile_qkv_projection_has_the_tiled_kernels_bits(tune, B, S, Hq, Hkv, D, K, rope):
+    """The fused Q | K | V launch on narrow tiles (rotation partners in lanes 32 apart, scatter into
+    Q and the caches, RMS and layer norms inside): the bits of the tiled kernel."""
+    r = np.random.default_rng(8900 + K)
+    M, N = B * S, (Hq + 2 * Hkv) * D
+    x = to_dev(r.standard_normal((M, K)).astype(np.float32), BF16)
+    W = to_dev((0.05 * r.standard_normal((N, K))).astype(np.float32), BF16)
+    b, cs = dev((0.1 * r.standard_normal(N)).astype(np.float32)), dev(r.standard_normal(N).astype(np.float32))
+    ang = r.uniform(0, 6.28, (S, D // 2)).astype(np.float32)
+    cos, sin = (dev(np.cos(ang)), dev(np.sin(ang))) if rope else (None, None)
+    t_max, tok = 128, 64
+
+    def run():
+        out = []
+        for norm in ("none", "rms", "layer"):
+            q, kc, vc = empty((M, Hq * D), BF16), empty((B, Hkv, t_max, D), BF16), empty((B, Hkv, D, t_max), BF16)
+            tail = (BF16, M, K, S, Hq, Hkv, 1, 1, D, cos, sin, q, kc, vc, t_max, tok)
+            if norm == "none":
+                pkg.call("vla_attn_qkv_rope", x, W, b, *tail)
+            elif norm == "rms":
+                pkg.call("vla_rmsnorm_attn_qkv_rope", x, W, b, *tail, 1e-5)
+            else:
+                pkg.call("vla_layernorm_attn_qkv_rope", x, W, cs, b, *tail, 1e-5)
+            out += [host(q), host(kc), host(vc)]
+        sync()
+        return out
+
+    outs = []
+    for rows_max, plan in ((0, 0), (512, 0), (512, 1), (512, 2), (512, 3), (512, 4)):
+        tune.set("VLA_GEMM_ROWS_MAX", rows_max)
+        tune.set("VLA_GEMM_ROWS_PLAN", plan)
+        outs.append(run())
+    for got in outs[1:]:
+        for g, t in zip(got, outs[0]):
+            assert np.array_equal(g, t)

@@ -47,10 +47,11 @@ def _check_no_spill(src, remarks):
             raise RuntimeError("no resource remarks for %s in %s" % (kernel, src))
 
 
-# Per-file compiler options.  dit_self.hip: accumulators of its MFMAs stay in the ordinary
-# vector registers; left to itself the compiler parks them in the accumulation registers and
-# copies them back and forth around every MFMA (1300 copies in the K loop).
-EXTRA_FLAGS = {"dit_self.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+# Per-file compiler options.  MFMA accumulators stay in the ordinary vector registers; left to
+# itself the compiler parks them in the accumulation registers and copies them back and forth
+# around the products (1300 copies in the K loop of dit_self.hip; every product of gemm.hip's
+# narrow-tile kernel).
+EXTRA_FLAGS = {"dit_self.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"], "gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 
 def _compile(src):

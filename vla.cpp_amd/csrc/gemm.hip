@@ -234,6 +234,16 @@ __device__ __forceinline__ float add_pair_bf16x2(uint32_t u, float acc) {
     return __builtin_amdgcn_fdot2_f32_bf16(v, ones, acc, false);
 }
 
+// Epilogue arithmetic that several kernels share to the bit: the fused multiply-adds are spelled
+// out, so that no kernel contracts the other product of a sum.
+__device__ __forceinline__ void rotate_pair(float& x0, float& x1, float c, float s) {  // NeoX rotation of (x0, x1)
+    const float a = x0, b = x1;
+    x0 = fmaf(a, c, -(b * s));
+    x1 = fmaf(b, c, a * s);
+}
+// rstd acc - (mean rstd) colsum: the projection of the centred and scaled row
+__device__ __forceinline__ float center_scale(float acc, float rstd, float mean_rstd, float colsum) { return fmaf(acc, rstd, -(mean_rstd * colsum)); }
+
 // Epilogue of one 64x64 sub-tile held in the LDS C tile: thread t owns row t/4 and
 // columns jg..jg+7 and 32+jg..32+jg+7 of the sub-tile.
 __device__ const float kNoBiasRegs[16] = {};
@@ -287,8 +297,8 @@ __device__ __forceinline__ void epilogue_64x64(const GemmArgs& a, const uint32_t
             const float ms = mean * f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                lo[e] = lo[e] * f - ms * a.colsum[tc.base0 + jg + e];
-                hi[e] = hi[e] * f - ms * a.colsum[tc.base1 + jg + e];
+                lo[e] = center_scale(lo[e], f, ms, a.colsum[tc.base0 + jg + e]);
+                hi[e] = center_scale(hi[e], f, ms, a.colsum[tc.base1 + jg + e]);
             }
         } else {
             const float f = rsqrtf(sq * inv_k + a.norm_eps);
@@ -434,9 +444,7 @@ __device__ __forceinline__ void epilogue_64x64(const GemmArgs& a, const uint32_t
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const float c = cr[e], sn = sr[e];
-            const float x0 = lo[e], x1 = hi[e];
-            lo[e] = x0 * c - x1 * sn;
-            hi[e] = x1 * c + x0 * sn;
+            rotate_pair(lo[e], hi[e], c, sn);
         }
     }
     const bool is_bf16 = (sizeof(T) == 2);
@@ -981,23 +989,25 @@ __global__ void __launch_bounds__(256) gemm_dl_kernel(GemmArgs a) {
     }
 }
 
-// ---- A few rows (M <= 64) of a bf16 projection: 16 columns per workgroup, K split over its wavefronts ----
-// One observation's suffix rows through a projection.  The weights are read once and from
+// ---- Few rows of a bf16 projection: narrow tiles over the whole chip ----
+// The suffix rows of one or a few observations through a projection.  The weights are read once and from
 // memory (a step touches every layer's weights once, more than the caches hold), and what a
-// CU gets out of memory is bounded by its own requests in flight, not by the chip: the tiled
-// kernels' 64-column tiles put such a launch on N / 64 CUs, a tenth of the chip, each walking
-// all of K tile by tile.  Here a workgroup owns 16 columns -- N / 16 workgroups -- and its
-// eight wavefronts each take an eighth of K and request all of it at once, straight into
-// MFMA operand registers: v_mfma_f32_16x16x32_bf16 with the weight rows as the left operand
-// (16 columns x 32 k) and 16 activation rows as the right one, so that lane (c, q) =
-// (lane % 16, lane / 16) reads 16 bytes (8 k) of weight row c and of activation row c, and
-// four lanes cover 64 consecutive bytes of a row.  The partial tiles meet in LDS and are
-// added in wavefront order; the epilogues (bias, fused-norm scaling, rotation, scatter into
-// the caches, residual) are the tiled kernels' arithmetic on a (row, column pair) per thread.
-// The 16 columns are 8 + 8: for rotated segments the columns d .. d + 7 of a head and their
-// partners d + D / 2, else 16 consecutive columns.  The sums are formed in another order than
-// by the tiled kernels: the two agree to fp32 rounding, not bit for bit.
-constexpr int SR_WAVES = 8, SR_MAX_ROWS = 64, SR_PSTR = 20, SR_MAX_K = 2048;
+// CU gets out of memory is bounded by its own requests in flight and by its path to the L2
+// (about 55 bytes per clock), not by the chip: the tiled kernels' 64-column tiles put such a
+// launch on N / 64 CUs, a tenth of the chip.  Here a workgroup owns 16 RB rows and 16 NB
+// columns, so that a CU moves 32 K (RB + NB) bytes; RB and NB are chosen per shape for the
+// fewest bytes per CU (launch_narrow).  As in gemm_dl_kernel the operands go straight into an
+// LDS ring (128 k per stage, 256-byte rows, pieces XOR-swizzled by the row, NS - 1 stages in
+// flight, one barrier per stage): a load instruction covers whole cache lines of four rows.
+// Fetching MFMA fragments from memory instead -- 16 rows x 16 bytes per quarter of a wavefront
+// -- is limited to about 16 bytes per clock and CU by the address unit, whatever is in flight.
+// A wavefront owns whole 16 x 16 blocks over all of K (v_mfma_f32_16x16x32_bf16, ascending k,
+// whose sums have the bits of the tiled kernels' 32x32x16: a row's result does not depend on
+// the batch it is in); W is the left operand, so that lane (c, q) = (lane % 16, lane / 16) ends
+// with columns 4 q .. 4 q + 3 of row c and the epilogue needs no LDS.  The 16 columns are 8 + 8:
+// for rotated segments the columns d .. d + 7 of a head and their partners d + D / 2, for gated
+// projections 8 gate columns and their up columns (the partner is lane ^ 32), else 16
+// consecutive columns.
 struct RowCols {
     int base_lo, base_hi;  // rows of W of tile columns [0, 8) and [8, 16)
     int seg;               // 0 Q, 1 K, 2 V (QKV mode)
@@ -1009,6 +1019,11 @@ __device__ __forceinline__ RowCols row_cols(const GemmArgs& a, int t) {
     RowCols rc;
     rc.seg = 0;
     rc.rope = false;
+    if (kEpi == EPI_GLU) {
+        rc.base_lo = rc.col_lo = t * 8;
+        rc.base_hi = rc.col_hi = a.N / 2 + t * 8;
+        return rc;
+    }
     if (kEpi != EPI_QKV) {
         rc.base_lo = rc.col_lo = t * 16;
         rc.base_hi = rc.col_hi = t * 16 + 8;
@@ -1040,195 +1055,243 @@ __device__ __forceinline__ RowCols row_cols(const GemmArgs& a, int t) {
     return rc;
 }
 
-template <int kEpi, int kNorm, int RB, int MAXC, int NB>  // RB: 16-row blocks; MAXC: 32-k chunks per wavefront held in registers, K <= 256 MAXC; NB: 16-column tiles per workgroup
-__global__ void __launch_bounds__(SR_WAVES * 64) gemm_rows_bf16_kernel(GemmArgs a) {
-    __shared__ __attribute__((aligned(16))) float part[SR_WAVES][NB][RB * 16][SR_PSTR];
-    __shared__ float stat_part[SR_WAVES][RB * 16][2];
+// The last min(nkt, LEFT) tiles of the ring: with LEFT tiles in flight, the oldest has landed
+// when at most (LEFT - 1) NLOAD loads are still due.
+template <int LEFT, int NLOAD, typename Body>
+__device__ __forceinline__ void narrow_tail(int nkt, Body body) {
+    if (LEFT <= nkt) {  // uniform
+        wait_vmcnt<(LEFT - 1) * NLOAD>();
+        body(LEFT == 1);
+    }
+    if constexpr (LEFT > 1) narrow_tail<LEFT - 1, NLOAD>(nkt, body);
+}
+
+template <int kEpi, int kNorm, int RB, int NB, int NS>  // RB: 16-row blocks, NB: 16-column tiles per workgroup
+__global__ void __launch_bounds__(256) gemm_narrow_kernel(GemmArgs a) {
+    constexpr int KB = 256, BK = 128, STAGE = (RB + NB) * 16 * KB, NLOAD = RB + NB;
+    constexpr int IN_FLIGHT = (NS - 2) * NLOAD;
+    constexpr int MY_NB = RB == 4 ? NB : 1;  // 16-column tiles per wavefront
+    static_assert(IN_FLIGHT <= 63, "ring depth exceeds the vector-memory counter");
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[NS * STAGE];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, q = lane >> 4;
     const int n_t16 = (a.N + 15) / 16;
+    // Workgroup -> (row group, columns).  The row groups of a column group sit eight apart, on
+    // one XCD: the second one finds the weight rows in the L2.
+    const int n_rg = (a.M + RB * 16 - 1) / (RB * 16);
+    const int rg = ((int)blockIdx.x >> 3) % n_rg, tg = (((int)blockIdx.x >> 3) / n_rg) * 8 + ((int)blockIdx.x & 7);
+    if (tg * NB >= n_t16) return;
+    const int m0 = rg * RB * 16;
     RowCols rc[NB];
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) rc[nb] = row_cols<kEpi>(a, min((int)blockIdx.x * NB + nb, n_t16 - 1));
-    const int nch = (a.K + 31) / 32, per = (nch + SR_WAVES - 1) / SR_WAVES, ch0 = wave * per;
+    for (int nb = 0; nb < NB; ++nb) rc[nb] = row_cols<kEpi>(a, min(tg * NB + nb, n_t16 - 1));
 
-    // rows past N or M and pieces past K are read from valid addresses; their products are dropped or zeroed
-    const unsigned char* wrow[NB];
+    // Loader: thread tid fills slot tid of each 4 KiB slab (16 rows of 256 bytes): position
+    // tid % 16 of row tid / 16, which holds logical piece (tid % 16) ^ row.  Rows past M or N and
+    // pieces past K are read from valid addresses; their products are dropped or zeroed.
+    const int lrow = tid >> 4, koff = ((tid & 15) ^ lrow) * 8;
+    const unsigned char* src[NLOAD];
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-        wrow[nb] = (const unsigned char*)a.W + (long)min(max(c < 8 ? rc[nb].base_lo + c : rc[nb].base_hi + c - 8, 0), a.N - 1) * a.K * 2;
-    const unsigned char* xrow[RB];
+    for (int i = 0; i < RB; ++i) src[i] = (const unsigned char*)a.A + (long)min(m0 + i * 16 + lrow, a.M - 1) * a.K * 2;
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) xrow[rb] = (const unsigned char*)a.A + (long)min(rb * 16 + c, a.M - 1) * a.K * 2;
-    u32x4_t wf[MAXC][NB], xf[MAXC][RB];
+    for (int i = 0; i < NB; ++i)
+        src[RB + i] = (const unsigned char*)a.W + (long)min(lrow < 8 ? rc[i].base_lo + lrow : rc[i].base_hi + lrow - 8, a.N - 1) * a.K * 2;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)lds + wave * 1024;  // low 32 bits of a shared-aperture address = LDS offset
+    const int nkt = (a.K + BK - 1) / BK;
+    auto issue = [&](int kt, int stage) __attribute__((always_inline)) {
+        const long kb = (long)min(kt * BK + koff, a.K - 8) * 2;
 #pragma unroll
-    for (int i = 0; i < MAXC; ++i) {
-        const int ch = min(ch0 + i, nch - 1);
-        const long off = (long)min(ch * 32 + 8 * q, a.K - 8) * 2;
+        for (int i = 0; i < NLOAD; ++i) load_to_lds16(src[i] + kb, lds0 + stage * STAGE + i * 4096);
+    };
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) wf[i][nb] = *reinterpret_cast<const u32x4_t*>(wrow[nb] + off);
+    for (int t = 0; t < NS - 1; ++t)
+        if (t < nkt) issue(t, t);  // uniform
+
+    // wavefront -> row block, first column tile
+    const bool active = RB * NB >= 4 || wave < RB * NB;
+    const int rb = RB == 4 ? wave : RB == 2 ? (NB == 2 ? wave >> 1 : wave & 1) : 0;
+    const int nb0 = RB == 4 ? 0 : NB == 2 ? wave & 1 : 0;
+    f32x4_t acc[MY_NB];
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb) xf[i][rb] = *reinterpret_cast<const u32x4_t*>(xrow[rb] + off);
-    }
-    // What the epilogue reads from memory is requested now, behind the operand loads.  Epilogue
-    // thread -> row tid / 8, tile columns i = tid % 8 and 8 + i.  No branch around the loads:
-    // addresses are clamped into the arrays and values that are not needed are dropped.
-    const int erow = tid >> 3, ei = tid & 7;
-    const int em = min(erow, a.M - 1);
-    int n_lo[NB], n_hi[NB];
-    float b_lo[NB], b_hi[NB], cs_lo[NB], cs_hi[NB], g_lo[NB], g_hi[NB], rot_c[NB], rot_s[NB], r_lo[NB], r_hi[NB];
+    for (int j = 0; j < MY_NB; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    // Row sums for the norm, in the tiled kernels' order: lane (c, q) sums its piece of every 32
+    // k with one accumulator per word; the pairs q, q ^ 1 are those kernels' two lane halves, the
+    // pairs q, q ^ 2 their two wavefronts.
+    float ssq[4] = {0.f, 0.f, 0.f, 0.f}, ssum[4] = {0.f, 0.f, 0.f, 0.f};
+    const int fx0 = (rb * 16 + c) * KB, fw0 = ((RB + nb0) * 16 + c) * KB;
+    auto multiply = [&](int stage, int k_left) __attribute__((always_inline)) {  // k_left: k of this tile inside K (the partial last tile), or BK
+        const unsigned char* base = lds + stage * STAGE;
+        u32x4_t fx[4], fw[4][MY_NB];
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-        n_lo[nb] = min(rc[nb].base_lo + ei, a.N - 1);
-        n_hi[nb] = min(rc[nb].base_hi + ei, a.N - 1);
-        b_lo[nb] = b_hi[nb] = cs_lo[nb] = cs_hi[nb] = r_lo[nb] = r_hi[nb] = rot_s[nb] = 0.f;
-        g_lo[nb] = g_hi[nb] = rot_c[nb] = 1.f;
-        if (a.bias) {
-            b_lo[nb] = a.bias[n_lo[nb]];
-            b_hi[nb] = a.bias[n_hi[nb]];
+        for (int ch = 0; ch < 4; ++ch) {
+            const int off = ((4 * ch + q) ^ c) * 16;
+            fx[ch] = *reinterpret_cast<const u32x4_t*>(base + fx0 + off);
+#pragma unroll
+            for (int j = 0; j < MY_NB; ++j) fw[ch][j] = *reinterpret_cast<const u32x4_t*>(base + fw0 + j * 16 * KB + off);
         }
-        if (kNorm == NORM_LAYER) {
-            cs_lo[nb] = a.colsum[n_lo[nb]];
-            cs_hi[nb] = a.colsum[n_hi[nb]];
+        if (k_left < BK) {  // K is a multiple of 8: a piece is inside or outside as a whole
+            const u32x4_t z = {0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int ch = 0; ch < 4; ++ch)
+                if (ch * 32 + 8 * q >= k_left) {
+                    fx[ch] = z;
+#pragma unroll
+                    for (int j = 0; j < MY_NB; ++j) fw[ch][j] = z;
+                }
         }
-        if (kEpi == EPI_PLAIN) {
-            if (a.col_gate) {
-                g_lo[nb] = a.col_gate[n_lo[nb]];
-                g_hi[nb] = a.col_gate[n_hi[nb]];
-            }
-            if (a.residual) {
-                if (a.out_bf16) {
-                    r_lo[nb] = bf2f(((const bf16_t*)a.residual)[(long)em * a.N + n_lo[nb]]);
-                    r_hi[nb] = bf2f(((const bf16_t*)a.residual)[(long)em * a.N + n_hi[nb]]);
-                } else {
-                    r_lo[nb] = ((const float*)a.residual)[(long)em * a.N + n_lo[nb]];
-                    r_hi[nb] = ((const float*)a.residual)[(long)em * a.N + n_hi[nb]];
+        __builtin_amdgcn_sched_barrier(0);  // all reads requested before the first product: left alone they are spread for fewer registers
+#pragma unroll
+        for (int ch = 0; ch < 4; ++ch) {
+#pragma unroll
+            for (int j = 0; j < MY_NB; ++j)
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, fw[ch][j]), __builtin_bit_cast(bf16x8_t, fx[ch]),
+                                                                 acc[j], 0, 0, 0);
+            if (kNorm) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    ssq[e] = add_squares_bf16x2(fx[ch][e], ssq[e]);
+                    if (kNorm == NORM_LAYER) ssum[e] = add_pair_bf16x2(fx[ch][e], ssum[e]);
                 }
             }
         }
-        if (kEpi == EPI_QKV && rc[nb].rope) {
-            const int half = a.D >> 1;
-            const long ri = (long)(em % a.S) * half + (rc[nb].col_lo % a.D) + ei;
-            rot_c[nb] = a.cos_t[ri];
-            rot_s[nb] = a.sin_t[ri];
-        }
+    };
+    // A wavefront without a block of its own multiplies along with another's (no branch in the
+    // loop) and drops the result.  The last NS - 1 tiles are multiplied without further loads:
+    // a ring that kept re-fetching past the end would double the traffic of a short K.
+    int cs = 0, ls = NS - 1, kt = 0;
+    for (; kt + NS - 1 < nkt; ++kt) {
+        wait_vmcnt<IN_FLIGHT>();
+        __syncthreads();  // this stage has landed for every wavefront; stage ls has been read by everyone
+        issue(kt + NS - 1, ls);
+        multiply(cs, BK);
+        cs = (cs + 1 == NS) ? 0 : cs + 1;
+        ls = (ls + 1 == NS) ? 0 : ls + 1;
     }
+    narrow_tail<NS - 1, NLOAD>(nkt, [&](bool last) __attribute__((always_inline)) {
+        __syncthreads();
+        multiply(cs, last ? a.K - (nkt - 1) * BK : BK);
+        cs = (cs + 1 == NS) ? 0 : cs + 1;
+    });
+    if (!active) return;
 
-    f32x4_t acc[NB][RB];
-    float ssq[RB], ssum[RB];
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) acc[nb][rb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        ssq[rb] = ssum[rb] = 0.f;
-    }
-#pragma unroll
-    for (int i = 0; i < MAXC; ++i) {
-        if (i < per && ch0 + i < nch) {  // uniform
-            const bool inside = (ch0 + i) * 32 + 8 * q < a.K;  // K is a multiple of 8: a piece is inside or outside as a whole
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb) {
-                u32x4_t xv = xf[i][rb];
-                if (!inside) xv = u32x4_t{0u, 0u, 0u, 0u};
-                if (kNorm) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        ssq[rb] = add_squares_bf16x2(xv[e], ssq[rb]);
-                        if (kNorm == NORM_LAYER) ssum[rb] = add_pair_bf16x2(xv[e], ssum[rb]);
-                    }
-                }
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb)
-                    acc[nb][rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf[i][nb]), __builtin_bit_cast(bf16x8_t, xv),
-                                                                          acc[nb][rb], 0, 0, 0);
-            }
-        }
-    }
-    // acc[nb][rb][e]: column 4 q + e of tile nb, row 16 rb + c
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) *reinterpret_cast<f32x4_t*>(&part[wave][nb][rb * 16 + c][4 * q]) = acc[nb][rb];
-        if (kNorm) {
-            const float s2 = rows_sum(ssq[rb]), s1 = rows_sum(ssum[rb]);
-            if (q == 0) {
-                stat_part[wave][rb * 16 + c][0] = s2;
-                stat_part[wave][rb * 16 + c][1] = s1;
-            }
-        }
-    }
-    __syncthreads();
-    if (erow >= RB * 16 || erow >= a.M) return;
-    const int m = erow;
-    float sq = 0.f, sm = 0.f;
+    float f = 1.f, ms = 0.f;
     if (kNorm) {
-#pragma unroll
-        for (int w = 0; w < SR_WAVES; ++w) {
-            sq += stat_part[w][erow][0];
-            sm += stat_part[w][erow][1];
+        const float inv_k = 1.0f / (float)a.K;
+        const float sq = rows_sum((ssq[0] + ssq[1]) + (ssq[2] + ssq[3]));
+        if (kNorm == NORM_LAYER) {
+            // sum_k (x - mean) rstd W[n][k] = rstd acc - (mean rstd) colsum[n]
+            const float mean = rows_sum((ssum[0] + ssum[1]) + (ssum[2] + ssum[3])) * inv_k;
+            f = rsqrtf(fmaxf(sq * inv_k - mean * mean, 0.f) + a.norm_eps);
+            ms = mean * f;
+        } else {
+            f = rsqrtf(sq * inv_k + a.norm_eps);
         }
     }
-    const int b = kEpi == EPI_QKV ? m / a.S : 0, s = kEpi == EPI_QKV ? m % a.S : 0;
+    const int m = m0 + rb * 16 + c;
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-        if ((int)blockIdx.x * NB + nb >= n_t16) break;  // uniform
-        float lo = 0.f, hi = 0.f;
+    for (int j = 0; j < MY_NB; ++j) {
+        const RowCols& t = rc[nb0 + j];
+        const bool live = m < a.M && tg * NB + nb0 + j < n_t16;
+        const int n0 = q < 2 ? t.base_lo + 4 * q : t.base_hi + 4 * q - 8;  // W row (= bias, column-sum index) of v[0]
+        float v[4];
 #pragma unroll
-        for (int w = 0; w < SR_WAVES; ++w) {
-            lo += part[w][nb][erow][ei];
-            hi += part[w][nb][erow][8 + ei];
+        for (int e = 0; e < 4; ++e) v[e] = acc[j][e];
+        if (kNorm == NORM_LAYER) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = center_scale(v[e], f, ms, a.colsum[min(n0 + e, a.N - 1)]);
+        } else if (kNorm) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] *= f;
         }
-        if (kNorm) {
-            const float inv_k = 1.0f / (float)a.K;
-            if (kNorm == NORM_LAYER) {
-                // sum_k (x - mean) rstd W[n][k] = rstd acc - (mean rstd) colsum[n]
-                const float mean = sm * inv_k;
-                const float f = rsqrtf(fmaxf(sq * inv_k - mean * mean, 0.f) + a.norm_eps);
-                const float ms = mean * f;
-                lo = lo * f - ms * cs_lo[nb];
-                hi = hi * f - ms * cs_hi[nb];
-            } else {
-                const float f = rsqrtf(sq * inv_k + a.norm_eps);
-                lo *= f;
-                hi *= f;
-            }
+        if (a.bias) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += a.bias[min(n0 + e, a.N - 1)];
         }
-        lo += b_lo[nb];
-        hi += b_hi[nb];
-        const bool ok_lo = rc[nb].base_lo + ei < a.N, ok_hi = rc[nb].base_hi + ei < a.N;
         if (kEpi == EPI_PLAIN) {
             if (a.act != VLA_ACT_NONE) {
-                lo = apply_act(lo, a.act);
-                hi = apply_act(hi, a.act);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = apply_act(v[e], a.act);
             }
-            lo = lo * g_lo[nb] + r_lo[nb];
-            hi = hi * g_hi[nb] + r_hi[nb];
-            const long o = (long)m * a.N;
-            if (a.out_bf16) {
-                if (ok_lo) ((bf16_t*)a.Y)[o + n_lo[nb]] = f2bf(lo);
-                if (ok_hi) ((bf16_t*)a.Y)[o + n_hi[nb]] = f2bf(hi);
-            } else {
-                if (ok_lo) ((float*)a.Y)[o + n_lo[nb]] = lo;
-                if (ok_hi) ((float*)a.Y)[o + n_hi[nb]] = hi;
+            if (a.col_gate) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] *= a.col_gate[min(n0 + e, a.N - 1)];
+            }
+            if (!live) continue;
+            const long o = (long)m * a.N + n0;
+            if (a.N % 4 == 0) {  // 4 consecutive columns are inside the row or outside as a whole
+                if (n0 >= a.N) continue;
+                if (a.out_bf16) {
+                    if (a.residual) {
+                        const u32x2_t rr = *reinterpret_cast<const u32x2_t*>((const bf16_t*)a.residual + o);
+#pragma unroll
+                        for (int e = 0; e < 2; ++e) {
+                            v[2 * e] += __uint_as_float(rr[e] << 16);
+                            v[2 * e + 1] += __uint_as_float(rr[e] & 0xffff0000u);
+                        }
+                    }
+                    *reinterpret_cast<u32x2_t*>((bf16_t*)a.Y + o) = u32x2_t{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+                } else {
+                    if (a.residual) {
+                        const f32x4_t rr = *reinterpret_cast<const f32x4_t*>((const float*)a.residual + o);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) v[e] += rr[e];
+                    }
+                    *reinterpret_cast<f32x4_t*>((float*)a.Y + o) = f32x4_t{v[0], v[1], v[2], v[3]};
+                }
+                continue;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (n0 + e >= a.N) continue;
+                float x = v[e];
+                if (a.out_bf16) {
+                    if (a.residual) x += bf2f(((const bf16_t*)a.residual)[o + e]);
+                    ((bf16_t*)a.Y)[o + e] = f2bf(x);
+                } else {
+                    if (a.residual) x += ((const float*)a.residual)[o + e];
+                    ((float*)a.Y)[o + e] = x;
+                }
             }
             continue;
         }
-        // QKV: rotation, scatter
-        if (rc[nb].rope) {
-            const float x0 = lo, x1 = hi;
-            lo = x0 * rot_c[nb] - x1 * rot_s[nb];
-            hi = x1 * rot_c[nb] + x0 * rot_s[nb];
-        }
+        float other[4];
 #pragma unroll
-        for (int hlf = 0; hlf < 2; ++hlf) {
-            const float v = hlf ? hi : lo;
-            const int col = (hlf ? rc[nb].col_hi : rc[nb].col_lo) + ei;
-            if (rc[nb].seg == 0) {
-                ((bf16_t*)a.q_out)[(long)m * (a.Hq * a.D) + col] = f2bf(v);
+        for (int e = 0; e < 4; ++e) other[e] = __shfl_xor(v[e], 32, 64);
+        if (kEpi == EPI_GLU) {  // I is a multiple of 32: no column of a tile lies past the row
+            if (q >= 2 || !live) continue;
+            float y[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] = apply_act(v[e], a.act) * other[e];
+            const long o = (long)m * (a.N / 2) + n0;
+            if (a.out_bf16) *reinterpret_cast<u32x2_t*>((bf16_t*)a.Y + o) = u32x2_t{pack_bf2(y[0], y[1]), pack_bf2(y[2], y[3])};
+            else *reinterpret_cast<f32x4_t*>((float*)a.Y + o) = f32x4_t{y[0], y[1], y[2], y[3]};
+            continue;
+        }
+        // QKV: rotation, scatter
+        const int b = min(m, a.M - 1) / a.S, s = min(m, a.M - 1) % a.S;
+        if (t.rope) {
+            const long ri = (long)s * (a.D >> 1) + (t.col_lo % a.D) + (q & 1) * 4;
+            const f32x4_t cr = *reinterpret_cast<const f32x4_t*>(a.cos_t + ri), sr = *reinterpret_cast<const f32x4_t*>(a.sin_t + ri);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float lo = q < 2 ? v[e] : other[e], hi = q < 2 ? other[e] : v[e];
+                rotate_pair(lo, hi, cr[e], sr[e]);
+                v[e] = q < 2 ? lo : hi;
+            }
+        }
+        if (!live) continue;
+        const int col = q < 2 ? t.col_lo + 4 * q : t.col_hi + 4 * q - 8;  // segment-local, 4 consecutive columns of one head
+        const u32x2_t pk = {pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+        if (t.seg == 0) {
+            *reinterpret_cast<u32x2_t*>((bf16_t*)a.q_out + (long)m * (a.Hq * a.D) + col) = pk;
+        } else {
+            const int head = col / a.D, d = col % a.D;
+            if (t.seg == 1) {
+                *reinterpret_cast<u32x2_t*>((bf16_t*)a.k_cache + (((long)b * a.Hkv + head) * a.t_max + a.tok_offset + s) * a.D + d) = pk;
             } else {
-                const int head = col / a.D, d = col % a.D;
-                if (rc[nb].seg == 1) ((bf16_t*)a.k_cache)[(((long)b * a.Hkv + head) * a.t_max + a.tok_offset + s) * a.D + d] = f2bf(v);
-                else ((bf16_t*)a.vt_cache)[(((long)b * a.Hkv + head) * a.D + d) * (long)a.t_max + a.tok_offset + s] = f2bf(v);
+                bf16_t* vt = (bf16_t*)a.vt_cache + (((long)b * a.Hkv + head) * a.D + d) * (long)a.t_max + a.tok_offset + s;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) vt[(long)e * a.t_max] = (bf16_t)(pk[e >> 1] >> (16 * (e & 1)));
             }
         }
     }
@@ -2153,6 +2216,53 @@ void launch_dl(GemmArgs a, hipStream_t st) {
     gemm_dl_kernel<kEpi, TM, TN, KB, NS, NORM_NONE><<<grid, 256, 0, st>>>(a);
 }
 
+// Row blocks and column tiles per workgroup of the narrow-tile kernel: the split with the least
+// operand traffic per CU among those whose workgroups are all on the chip at once.  A column
+// tile (weights, from memory) weighs 2.2 times a row block (activations, from the L2): the
+// ratio under which the rule picks the fastest split on the models' shapes at batch 1.  Without
+// such a split the tiled kernel is the faster one -- 98 rows through 4608 x 1536: 288 narrow
+// workgroups 14.0 us, tiled 11.0; 147 rows through 1536 x 6144: 144 workgroups 17.0, tiled 23.0 --
+// and -1 is returned.
+constexpr int NARROW_PLANS[4][2] = {{1, 1}, {2, 1}, {4, 1}, {4, 2}};
+inline long narrow_wgs(const GemmArgs& a, int p) {
+    const int rb = NARROW_PLANS[p][0], nb = NARROW_PLANS[p][1], n_t16 = (a.N + 15) / 16;
+    return (long)((n_t16 + nb - 1) / nb) * ((a.M + 16 * rb - 1) / (16 * rb));
+}
+int narrow_plan(const GemmArgs& a) {
+    const int force = tuning().gemm_rows_plan;
+    if (force > 0 && force <= 4) return force - 1;
+    int p = -1, best = 1 << 30;
+    for (int i = 0; i < 4; ++i) {
+        const int rb = NARROW_PLANS[i][0], nb = NARROW_PLANS[i][1];
+        if (rb > 1 && (rb / 2) * 16 >= a.M) continue;  // a smaller block holds every row
+        const int cost = 5 * rb + 11 * nb;
+        if (narrow_wgs(a, i) <= 256 && cost < best) {
+            best = cost;
+            p = i;
+        }
+    }
+    // more columns than one round holds: still this kernel where a single row block takes every row
+    return p < 0 && a.M <= 64 ? (a.M <= 16 ? 0 : a.M <= 32 ? 1 : 3) : p;
+}
+
+template <int kEpi, int kNorm>
+void launch_narrow(const GemmArgs& a, int p, hipStream_t st) {
+    const int rb = NARROW_PLANS[p][0], nb = NARROW_PLANS[p][1];
+    const int n_rg = (a.M + 16 * rb - 1) / (16 * rb), n_cg = ((a.N + 15) / 16 + nb - 1) / nb;
+    const unsigned grid = (unsigned)((n_cg + 7) / 8 * 8 * n_rg);
+    // Ring depths: more stages only delay the first one, fewer leave a CU short of requests; with
+    // more workgroups than CUs two of them share a CU's LDS and its requests.
+    switch (p) {
+        case 0: gemm_narrow_kernel<kEpi, kNorm, 1, 1, 6><<<grid, 256, 0, st>>>(a); break;
+        case 1:
+            if (narrow_wgs(a, 1) > 256) gemm_narrow_kernel<kEpi, kNorm, 2, 1, 4><<<grid, 256, 0, st>>>(a);
+            else gemm_narrow_kernel<kEpi, kNorm, 2, 1, 6><<<grid, 256, 0, st>>>(a);
+            break;
+        case 2: gemm_narrow_kernel<kEpi, kNorm, 4, 1, 4><<<grid, 256, 0, st>>>(a); break;
+        default: gemm_narrow_kernel<kEpi, kNorm, 4, 2, 4><<<grid, 256, 0, st>>>(a); break;
+    }
+}
+
 template <typename T, int kEpi>
 int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
     if (a.M == 0 || n_tiles == 0) return VLA_K_OK;
@@ -2166,43 +2276,21 @@ int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
             return hipGetLastError() == hipSuccess ? VLA_K_OK : VLA_K_ERR_LAUNCH;
         }
     }
-    if constexpr (std::is_same<T, bf16_t>::value && (kEpi == EPI_PLAIN || kEpi == EPI_QKV)) {
-        // a few bf16 rows (one observation's suffix through a projection): 16 columns per workgroup, K split over its wavefronts
-        bool rows_ok = a.M <= tuning().gemm_rows_max && a.M <= SR_MAX_ROWS && a.K % 8 == 0 && a.K >= 64 && a.K <= SR_MAX_K &&
-                       tuning().gemm_tile < 0 && (uintptr_t)a.A % 16 == 0 && (uintptr_t)a.W % 16 == 0 && !(a.colsum && a.norm_eps < 0.f) &&
-                       !a.stats_out && !a.stats_in;
-        if (kEpi == EPI_QKV) rows_ok = rows_ok && a.D % 16 == 0 && a.N % 16 == 0;
-        if (rows_ok) {
-            // more 16-column tiles than CUs: two per workgroup, so that no CU gets two workgroups' worth of requests while
-            // its neighbours get one (GR00T's fused Q | K | V: 288 tiles).  Up to 32 rows only (registers).
-            const int n_t16 = (a.N + 15) / 16, per = ((a.K + 31) / 32 + SR_WAVES - 1) / SR_WAVES, rb = (a.M + 15) / 16;
-            const bool two = n_t16 > 256 && rb <= 2 && per <= 6;
-            const unsigned grid = (unsigned)(two ? (n_t16 + 1) / 2 : n_t16);
-#define VLA_ROWS_K(NORM, RB, NB)                                                                                   \
-    do {                                                                                                           \
-        if (per <= 2) gemm_rows_bf16_kernel<kEpi, NORM, RB, 2, NB><<<grid, SR_WAVES * 64, 0, st>>>(a);              \
-        else if (per <= 4) gemm_rows_bf16_kernel<kEpi, NORM, RB, 4, NB><<<grid, SR_WAVES * 64, 0, st>>>(a);         \
-        else if (per <= 6) gemm_rows_bf16_kernel<kEpi, NORM, RB, 6, NB><<<grid, SR_WAVES * 64, 0, st>>>(a);         \
-        else if (NB == 1) gemm_rows_bf16_kernel<kEpi, NORM, RB, 8, 1><<<grid, SR_WAVES * 64, 0, st>>>(a);           \
-    } while (0)
-#define VLA_ROWS(NORM)                                \
-    do {                                              \
-        if (two && rb <= 1) VLA_ROWS_K(NORM, 1, 2);   \
-        else if (two) VLA_ROWS_K(NORM, 2, 2);         \
-        else if (rb <= 1) VLA_ROWS_K(NORM, 1, 1);     \
-        else if (rb == 2) VLA_ROWS_K(NORM, 2, 1);     \
-        else VLA_ROWS_K(NORM, 4, 1);                  \
-    } while (0)
-            if (a.norm_eps < 0.f) {
-                VLA_ROWS(NORM_NONE);
-            } else if constexpr (kEpi == EPI_QKV) {
-                if (a.colsum) VLA_ROWS(NORM_LAYER);
-                else VLA_ROWS(NORM_RMS);
-            } else {
-                return VLA_K_ERR_SHAPE;  // the row statistics belong to the fused QKV projections
+    if constexpr (std::is_same<T, bf16_t>::value && kEpi != EPI_TERNARY) {
+        // few bf16 rows (the suffix of one or a few observations through a projection): narrow tiles over the whole chip
+        bool rows_ok = a.M <= tuning().gemm_rows_max && a.K % 8 == 0 && a.K >= 64 && tuning().gemm_tile < 0 &&
+                       (uintptr_t)a.A % 16 == 0 && (uintptr_t)a.W % 16 == 0 && !(a.colsum && a.norm_eps < 0.f) && !a.stats_out && !a.stats_in;
+        if (kEpi == EPI_QKV) rows_ok = rows_ok && a.D % 16 == 0 && a.N % 16 == 0;  // 8 + 8 columns of one head
+        if (kEpi == EPI_PLAIN) rows_ok = rows_ok && a.norm_eps < 0.f;
+        const int plan = rows_ok ? narrow_plan(a) : -1;
+        if (plan >= 0) {
+            if (a.norm_eps < 0.f) launch_narrow<kEpi, NORM_NONE>(a, plan, st);
+            else if constexpr (kEpi == EPI_QKV) {
+                if (a.colsum) launch_narrow<kEpi, NORM_LAYER>(a, plan, st);
+                else launch_narrow<kEpi, NORM_RMS>(a, plan, st);
+            } else if constexpr (kEpi == EPI_GLU) {
+                launch_narrow<kEpi, NORM_RMS>(a, plan, st);
             }
-#undef VLA_ROWS
-#undef VLA_ROWS_K
             return hipGetLastError() == hipSuccess ? VLA_K_OK : VLA_K_ERR_LAUNCH;
         }
     }
