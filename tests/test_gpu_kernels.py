@@ -1644,3 +1644,34 @@ def test_narrow_tile_qkv_projection_has_the_tiled_kernels_bits(tune, B, S, Hq, H
     for got in outs[1:]:
         for g, t in zip(got, outs[0]):
             assert np.array_equal(g, t)
+
+
+@pytest.mark.parametrize("tile", [17, 18, 19, 20, 21])
+@pytest.mark.parametrize("M,N,K,ws_num", [(33, 96, 128, 1), (64, 640, 256, 1), (300, 288, 384, 3), (515, 352, 1152, 1)])
+def test_ternary_gemm_ring_tiles_bit_exact(tune, tile, M, N, K, ws_num):
+    """Every tile of the LDS-ring ternary kernel (VLA_TERNARY_TILE 17..21) on rows and columns that
+    end inside a tile and K from one stage to more than the ring holds: the oracle's int32
+    accumulators and bf16 epilogue, and with a residual the bits of GEMM followed by add."""
+    r = np.random.default_rng(tile + M)
+    A = r.integers(-127, 128, (M, K)).astype(np.int8)
+    t = r.integers(-1, 2, (N, K)).astype(np.int8)
+    s = (127.0 / np.abs(r.standard_normal(M) * 3 + 1e-3)).astype(np.float32)
+    if M > 400:
+        s[5], s[100], s[300] = 1e-25, 3e22, 7.5e-21  # the full-range division path
+    ws = (0.01 + 0.001 * r.integers(0, 50, ws_num)).astype(np.float32)
+    res = orc.to_bf16(r.standard_normal((M, N)).astype(np.float32))
+    dA, dW, ds, dws = dev(A), dev(_pack_plain(t)), dev(s), dev(ws)
+    rowsum = dev(A.astype(np.int32).sum(1).astype(np.int32))
+    acc = torch.zeros((M, N), dtype=torch.int32, device="cuda")
+    out = torch.zeros((M, N), dtype=torch.int16, device="cuda")
+    tune.set("VLA_TERNARY_TILE", str(tile))
+    pkg.call("vla_ternary_gemm", dA, dW, out, acc, ds, rowsum, dws, ws_num, M, N, K)
+    h = dev(res)
+    pkg.call("vla_ternary_gemm_add", dA, dW, h, h, ds, rowsum, dws, ws_num, M, N, K)
+    want_sum = torch.zeros_like(out)
+    pkg.call("bitvla_add_bf16", out, dev(res), want_sum, M * N)
+    sync()
+    want_acc = orc.ternary_gemm_i32(A, t)
+    assert np.array_equal(host(acc), want_acc)
+    assert np.array_equal(host(out, np.uint16), orc.ternary_epilogue(want_acc, s, ws))
+    assert np.array_equal(host(h), host(want_sum))

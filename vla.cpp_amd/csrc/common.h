@@ -34,7 +34,7 @@ struct Tuning {
     int gemm_panel = 0;          // VLA_GEMM_PANEL: N tiles per panel of an XCD's walk over its tiles; 0 = by size
     int gemm_dl = -1;            // VLA_GEMM_DL: 0 pins the register-staged GEMM
     int gemm_stages = 0;         // VLA_GEMM_STAGES: ring depth of the direct-to-LDS GEMM
-    int ternary_tile = 0;        // VLA_TERNARY_TILE: 64 | 128 | 256 (32x32x32 kernels) | 16 (16x16x64 kernel)
+    int ternary_tile = 0;        // VLA_TERNARY_TILE: 64 | 128 | 256 (32x32x32 kernels) | 16 (128 x 256) | 17 (128 x 128) | 18 (64 x 128) | 19 (64 x 64) | 20 (64 x 256) | 21 (32 x 64) (16x16x64 kernels)
 };
 const Tuning& tuning();
 

@@ -1594,12 +1594,9 @@ __global__ void __launch_bounds__(256, 2) ternary_gemm_x16_kernel(GemmArgs a) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
     const int q = lane >> 4, c = lane & 15;
-    // id % 8 (the XCD) = M tile % 8: workgroups sharing an L2 share their activation rows,
-    // the larger operand, and stream the whole (4x smaller) packed weight matrix.
-    const int m_tiles = (a.M + ROWS - 1) / ROWS, mt_pad = (m_tiles + 7) & ~7;
-    const int mt = blockIdx.x % mt_pad;
-    if (mt >= m_tiles) return;
-    const int m0 = mt * ROWS, n0 = (blockIdx.x / mt_pad) * COLS + wn * CW;
+    int mt, nt;
+    if (!xcd_tile(a, (a.N + COLS - 1) / COLS, (a.M + ROWS - 1) / ROWS, mt, nt)) return;
+    const int m0 = mt * ROWS, n0 = nt * COLS + wn * CW;
 
     // Row constants of the lane's four output rows m = m0 + 64 wm + 16 mb + c: requested
     // before everything else, valid after the first wait of the ring.
@@ -1806,6 +1803,229 @@ __global__ void __launch_bounds__(256, 2) ternary_gemm_x16_kernel(GemmArgs a) {
             const int row = p * 4 + (lane >> 4), c16 = lane & 15;
             u32x4_t v = *reinterpret_cast<const u32x4_t*>(tp + row * T_STRIDE + c16 * 16);
             const int m = m0 + wm * 64 + mb * 16 + row, n = n0 + c16 * 8;
+            if (m >= a.M || n + 8 > a.N) continue;
+            if (a.residual) {  // out = bf16(out + residual), both already bf16
+                const u32x4_t rr = res_v[p];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    v[e] = pack_bf2(__uint_as_float(v[e] << 16) + __uint_as_float(rr[e] << 16),
+                                    __uint_as_float(v[e] & 0xffff0000u) + __uint_as_float(rr[e] & 0xffff0000u));
+            }
+            // streaming store: the 2 M N bytes leave the L2 as they are produced instead of waiting, dirty, for the
+            // write-back at the end of the kernel (each XCD's L2 would hold its whole share until then)
+            __builtin_nontemporal_store(v, reinterpret_cast<u32x4_t*>((bf16_t*)a.Y + (long)m * a.N + n));
+        }
+    }
+}
+
+// ---- Ternary GEMM, both operands through an LDS ring ----------------------------------
+// 2 x 2 wavefronts, each 16 MB rows x 16 NB columns of 16 x 16 x 64 products (transposed, D = W .
+// A^T, as above): workgroup tile 32 MB x 32 NB.  A stage of the ring holds 128 k of the activation
+// rows (pieces XOR-swizzled by (row >> 1) & 7) and the packed words of the same 128 k, 1 KiB per
+// 32-column block, copied as they lie in the fragment-major layout; a lane's two words of a block
+// are one 8-byte read.  NS - 1 stages are in flight, one barrier per stage.  For a few hundred rows
+// (one observation's prefix) the 128 x 256 tiles above leave most of the chip idle -- 40 of 256
+// CUs at 512 x 2560 -- and a wavefront alone on its SIMD waits for every load it makes.  Bound by
+// the L2 -> CU fill (about 10 TB/s over the chip) below 128 x 128.  512 rows, M x N x K: 512 x 3840 x
+// 2560 19.0 -> 9.9 us, 512 x 2560 x 2560 20.5 -> 9.6, 512 x 13824 x 2560 34.2 -> 21.9, 512 x 2560 x
+// 6912 33.8 -> 17.1 (64 x 64 tiles with the words staged through registers before).
+template <int MB, int NB, int NS>
+__global__ void __launch_bounds__(256) ternary_gemm_ring_kernel(GemmArgs a) {
+    constexpr int ROWS = 32 * MB, CW = 16 * NB, COLS = 2 * CW, ABYTES = ROWS * 128, STAGE = ABYTES + NB * 1024;
+    constexpr int WL = NB >= 4 ? NB / 4 : 1, NLOAD = MB + WL;  // load instructions per wavefront and stage: activations, words
+    constexpr int T_STRIDE = 2 * CW + 16;                      // epilogue staging row: CW bf16 + 16 bytes
+    constexpr int LPR = CW / 8, RPP = 64 / LPR, PASSES = 16 / RPP;  // 16-byte pieces of a staging row, rows per store pass, passes
+    static_assert((NS - 2) * NLOAD <= 63, "ring depth exceeds the vector-memory counter");
+    static_assert(NS * STAGE >= 4 * 16 * T_STRIDE, "epilogue staging must fit in the ring");
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[NS * STAGE];
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 1, wn = wave & 1;
+    const int q = lane >> 4, c = lane & 15;
+    int mt, nt;
+    if (!xcd_tile(a, (a.N + COLS - 1) / COLS, (a.M + ROWS - 1) / ROWS, mt, nt)) return;
+    const int m0 = mt * ROWS, n0 = nt * COLS + wn * CW;
+
+    // Loader: wavefront w fills the activation slabs MB w + v (8 rows, 1 KiB each) and the word
+    // slabs WL w + v (one 32-column block each; with two blocks the wavefronts 2 and 3 repeat them).
+    const int kgroups = a.K / 32, nblocks = (a.N + 31) / 32, nkt = a.K / 128;
+    const unsigned char* src[NLOAD];
+#pragma unroll
+    for (int v = 0; v < MB; ++v) {
+        const int row = (wave * MB + v) * 8 + (lane >> 3), piece = (lane & 7) ^ ((row >> 1) & 7);
+        src[v] = (const unsigned char*)a.A + (long)min(m0 + row, a.M - 1) * a.K + piece * 16;  // rows past M: a valid row, result dropped
+    }
+#pragma unroll
+    for (int v = 0; v < WL; ++v)  // columns past N: any valid block, result dropped
+        src[MB + v] = (const unsigned char*)a.W + (long)min(nt * NB + (wave * WL + v) % NB, nblocks - 1) * kgroups * 256 + lane * 16;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)lds;  // low 32 bits of a shared-aperture address = LDS offset
+    auto issue = [&](int kt, int stage) __attribute__((always_inline)) {
+#pragma unroll
+        for (int v = 0; v < MB; ++v) load_to_lds16(src[v] + (long)kt * 128, lds0 + stage * STAGE + (wave * MB + v) * 1024);
+#pragma unroll
+        for (int v = 0; v < WL; ++v) load_to_lds16(src[MB + v] + (long)kt * 1024, lds0 + stage * STAGE + ABYTES + ((wave * WL + v) % NB) * 1024);
+    };
+#pragma unroll
+    for (int t = 0; t < NS - 1; ++t)
+        if (t < nkt) issue(t, t);  // uniform
+
+    i32x4_t acc[NB][MB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = i32x4_t{0, 0, 0, 0};
+    // Fragment reads: row 16 MB wm + 16 mb + c, logical piece 4 ch + q at position (4 ch + q) ^ ((c >> 1) & 7); words
+    // (k group 2 ch + q / 2, half q % 2, columns 2 c and 2 c + 1) of block wn NB / 2 + p.
+    const int fsw = (c >> 1) & 7;
+    const int fragA = (wm * MB * 16 + c) * 128, fragW = ABYTES + wn * (NB / 2) * 1024 + ((q >> 1) * 64 + (q & 1) * 32 + 2 * c) * 4;
+    auto multiply = [&](int stage) __attribute__((always_inline)) {
+        const unsigned char* cur = lds + stage * STAGE;
+        u32x4_t fa[2][MB];
+        u32x2_t w[2][NB / 2];
+#pragma unroll
+        for (int ch = 0; ch < 2; ++ch) {
+#pragma unroll
+            for (int p = 0; p < NB / 2; ++p) w[ch][p] = *reinterpret_cast<const u32x2_t*>(cur + fragW + p * 1024 + ch * 512);
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+                fa[ch][mb] = *reinterpret_cast<const u32x4_t*>(cur + fragA + mb * 16 * 128 + (((4 * ch + q) ^ fsw) * 16));
+        }
+        __builtin_amdgcn_sched_barrier(0);  // all reads requested before the first product
+#pragma unroll
+        for (int ch = 0; ch < 2; ++ch)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                const uint32_t x = w[ch][nb >> 1][nb & 1];
+                const u32x4_t fw = {x & 0x03030303u, (x >> 2) & 0x03030303u, (x >> 4) & 0x03030303u, (x >> 6) & 0x03030303u};
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb)
+                    acc[nb][mb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4_t, fw), __builtin_bit_cast(i32x4_t, fa[ch][mb]),
+                                                                        acc[nb][mb], 0, 0, 0);
+            }
+    };
+    int cs = 0, ls = NS - 1, kt = 0;
+    for (; kt + NS - 1 < nkt; ++kt) {
+        wait_vmcnt<(NS - 2) * NLOAD>();
+        __syncthreads();  // this stage has landed for every wavefront; stage ls has been read by everyone
+        issue(kt + NS - 1, ls);
+        multiply(cs);
+        cs = (cs + 1 == NS) ? 0 : cs + 1;
+        ls = (ls + 1 == NS) ? 0 : ls + 1;
+    }
+    // the row constants of the epilogue (rows m0 + 16 MB wm + 16 mb + c), under the last tiles
+    int rs_row[MB];
+    float sc_row[MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+        const int m = min(m0 + (wm * MB + mb) * 16 + c, a.M - 1);
+        rs_row[mb] = a.rowsum[m];
+        sc_row[mb] = a.s ? a.s[m] : 1.f;
+    }
+    narrow_tail<NS - 1, NLOAD>(nkt, [&](bool) __attribute__((always_inline)) {
+        __syncthreads();
+        multiply(cs);
+        cs = (cs + 1 == NS) ? 0 : cs + 1;
+    });
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)  // 2-bit codes are t + 2: sum_k q (t + 2) - 2 rowsum
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[nb][mb][i] -= 2 * rs_row[mb];
+    __syncthreads();  // the ring becomes the epilogue's staging area
+
+    // acc[nb][mb][i]: column n = n0 + 32 (nb / 2) + 2 (4 q + i) + nb % 2, row m = m0 + 16 MB wm + 16 mb + c
+    if (a.acc_out) {
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+            const int m = m0 + (wm * MB + mb) * 16 + c;
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int n = n0 + (nb >> 1) * 32 + 2 * (4 * q + i) + (nb & 1);
+                    if (m < a.M && n < a.N) a.acc_out[(long)m * a.N + n] = acc[nb][mb][i];
+                }
+        }
+    }
+    if (!a.Y) return;
+
+    // bf16 output: out = float(acc) / s[m] * ws[group], staged per wavefront as 16 rows x CW
+    // columns and written with 16-byte stores (LPR lanes per row), the residual added on the way.
+    // The quotient is the correctly rounded one.  For a positive scale away from the exponent
+    // limits it is computed with the scale's exponent taken out: y ~ 1 / mantissa by one Newton
+    // step on v_rcp_f32, q0 = a y, one residual correction; for |a| < 2^20 that sequence gives
+    // the IEEE quotient for every mantissa (checked exhaustively on the device), and the power
+    // of two goes back in exactly.  Larger accumulators take a second correction (the compiler's
+    // own sequence without its operand scaling); other scales take the division operator.
+    const int group = a.N / a.ws_num;
+    float wsc[NB / 2];  // one weight scale per 32-column block (the launcher checks that a scale group is a multiple of 32 columns)
+    bool ok = true;
+#pragma unroll
+    for (int p = 0; p < NB / 2; ++p) {
+        wsc[p] = a.ws[min(n0 + p * 32, a.N - 1) / group];
+        const float wa = fabsf(wsc[p]);
+        ok = ok && (wa == 0.f || (wa > 0x1p-60f && wa < 0x1p60f));  // 2^-e ws below is then exact
+    }
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+        const float sm = sc_row[mb];
+        ok = ok && sm > 0x1p-60f && sm < 0x1p60f;
+    }
+    const bool fast = __builtin_amdgcn_ballot_w64(ok) == ~0ull;
+    const bool one_step = a.K < 8192;  // |acc| <= 128 K < 2^20
+    unsigned char* tp = &lds[0] + wave * (16 * T_STRIDE);
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+        u32x4_t res_v[PASSES] = {};
+        if (a.residual) {  // this row block's residual vectors, requested ahead of the staging arithmetic
+#pragma unroll
+            for (int p = 0; p < PASSES; ++p) {
+                const int m = min(m0 + (wm * MB + mb) * 16 + p * RPP + lane / LPR, a.M - 1), n = min(n0 + (lane % LPR) * 8, a.N - 8);
+                res_v[p] = *reinterpret_cast<const u32x4_t*>((const bf16_t*)a.residual + (long)m * a.N + n);
+            }
+        }
+        const float sm = sc_row[mb];
+        if (fast) {
+            const uint32_t sb = __float_as_uint(sc_row[mb]);
+            const float mant = __uint_as_float((sb & 0x007fffffu) | 0x3f800000u);      // in [1, 2)
+            const float pw = __uint_as_float(0x7f000000u - (sb & 0x7f800000u));         // 2^-(exponent of sm), exact
+            const float y0 = __builtin_amdgcn_rcpf(mant);
+            const float y = __builtin_fmaf(__builtin_fmaf(-mant, y0, 1.0f), y0, y0);
+#pragma unroll
+            for (int p = 0; p < NB / 2; ++p) {
+                const float pws = pw * wsc[p];  // exact: (q 2^-e) ws and q (2^-e ws) round the same product once
+                u32x4_t o;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    float r2[2];
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const float av = (float)acc[2 * p + h][mb][i];
+                        const float q0 = av * y;
+                        float q1 = __builtin_fmaf(__builtin_fmaf(-mant, q0, av), y, q0);
+                        if (!one_step) q1 = __builtin_fmaf(__builtin_fmaf(-mant, q1, av), y, q1);
+                        r2[h] = q1 * pws;
+                    }
+                    o[i] = pack_bf2(r2[0], r2[1]);
+                }
+                *reinterpret_cast<u32x4_t*>(tp + c * T_STRIDE + (p * 32 + 8 * q) * 2) = o;
+            }
+        } else {
+#pragma unroll
+            for (int p = 0; p < NB / 2; ++p) {
+                u32x4_t o;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    o[i] = pack_bf2((float)acc[2 * p][mb][i] / sm * wsc[p], (float)acc[2 * p + 1][mb][i] / sm * wsc[p]);
+                *reinterpret_cast<u32x4_t*>(tp + c * T_STRIDE + (p * 32 + 8 * q) * 2) = o;
+            }
+        }
+#pragma unroll
+        for (int p = 0; p < PASSES; ++p) {
+            const int row = p * RPP + lane / LPR, c16 = lane % LPR;
+            u32x4_t v = *reinterpret_cast<const u32x4_t*>(tp + row * T_STRIDE + c16 * 16);
+            const int m = m0 + (wm * MB + mb) * 16 + row, n = n0 + c16 * 8;
             if (m >= a.M || n + 8 > a.N) continue;
             if (a.residual) {  // out = bf16(out + residual), both already bf16
                 const u32x4_t rr = res_v[p];
@@ -2148,6 +2368,24 @@ __global__ void __launch_bounds__(GEMV_WAVES * 64) ternary_gemv_norm_kernel(Gemm
     }
 }
 
+// The walk constants of xcd_tile for the XCD grid and panel width already in a; returns the grid size.
+unsigned xcd_walk(GemmArgs& a, int m_wg, int n_wg) {
+    auto magic = [](int d) { return d > 1 ? (unsigned)((1ull << 32) / (unsigned)d) + 1u : 0u; };
+    a.cn = (n_wg + a.xn - 1) / a.xn;
+    a.cm = (m_wg + a.xm - 1) / a.xm;
+    a.per_panel = a.pn * a.cm;
+    a.full = a.cn / a.pn;
+    a.w_last = a.cn - a.full * a.pn;
+    a.xn_shift = a.xn == 1 ? 0 : a.xn == 2 ? 1 : a.xn == 4 ? 2 : 3;
+    a.mg_cn = magic(a.cn);
+    a.mg_pp = magic(a.per_panel);
+    a.mg_pn = magic(a.pn);
+    a.mg_wl = magic(a.w_last);
+    const long wgs = (long)a.cm * a.cn;
+    if (wgs >= 65536) return 0;  // the tile walk's divisions are exact below 2^16 workgroups per XCD
+    return (unsigned)(wgs * 8);
+}
+
 // XCD grid xm x xn = 8 for a tile grid of m_wg x n_wg workgroup tiles of tile_cols columns:
 // every L2 reads its N tiles' rows of W once and its M tiles' rows of A once per panel of N
 // tiles (xcd_tile).  One panel while an XCD's rows of W fit in half of its 4 MiB L2 beside
@@ -2174,20 +2412,7 @@ unsigned xcd_split(GemmArgs& a, int m_wg, int n_wg, double w_bytes_per_elem, int
             a.pn = pn;
         }
     }
-    auto magic = [](int d) { return d > 1 ? (unsigned)((1ull << 32) / (unsigned)d) + 1u : 0u; };
-    a.cn = (n_wg + a.xn - 1) / a.xn;
-    a.cm = (m_wg + a.xm - 1) / a.xm;
-    a.per_panel = a.pn * a.cm;
-    a.full = a.cn / a.pn;
-    a.w_last = a.cn - a.full * a.pn;
-    a.xn_shift = a.xn == 1 ? 0 : a.xn == 2 ? 1 : a.xn == 4 ? 2 : 3;
-    a.mg_cn = magic(a.cn);
-    a.mg_pp = magic(a.per_panel);
-    a.mg_pn = magic(a.pn);
-    a.mg_wl = magic(a.w_last);
-    const long wgs = (long)a.cm * a.cn;
-    if (wgs >= 65536) return 0;  // the tile walk's divisions are exact below 2^16 workgroups per XCD
-    return (unsigned)(wgs * 8);
+    return xcd_walk(a, m_wg, n_wg);
 }
 
 template <typename T, int kEpi, int TM, int TN, int KB, int DEPTH>
@@ -2261,6 +2486,48 @@ void launch_narrow(const GemmArgs& a, int p, hipStream_t st) {
         case 2: gemm_narrow_kernel<kEpi, kNorm, 4, 1, 4><<<grid, 256, 0, st>>>(a); break;
         default: gemm_narrow_kernel<kEpi, kNorm, 4, 2, 4><<<grid, 256, 0, st>>>(a); break;
     }
+}
+
+template <int MB, int NB, int NS>
+void launch_ring(GemmArgs a, hipStream_t st) {
+    const unsigned grid = xcd_split(a, (a.M + 32 * MB - 1) / (32 * MB), (a.N + 32 * NB - 1) / (32 * NB), 0.25, 32 * NB, 1.0);
+    ternary_gemm_ring_kernel<MB, NB, NS><<<grid, 256, 0, st>>>(a);
+}
+void launch_x16(GemmArgs a, hipStream_t st) {
+    const int m_wg = (a.M + 127) / 128, n_wg = (a.N + 255) / 256;
+    unsigned grid;
+    if (m_wg % 8 == 0) {
+        // whole M tiles per XCD: workgroups sharing an L2 share their activation rows, the larger
+        // operand, and stream the (4x smaller) packed weights tile column by tile column
+        a.xm = 8;
+        a.xn = a.pn = 1;
+        grid = xcd_walk(a, m_wg, n_wg);
+    } else {
+        grid = xcd_split(a, m_wg, n_wg, 0.25, 256, 1.0);
+    }
+    ternary_gemm_x16_kernel<<<grid, 256, 0, st>>>(a);
+}
+
+// Tile of a ternary GEMM (VLA_TERNARY_TILE codes) by predicted time: a launch costs `fixed`, and
+// `step` per 128 k while every workgroup has a CU of its own; up to two workgroups per CU
+// overlap to `two` steps, beyond that a step takes `more` times the workgroups per CU.  The
+// constants (us) are a fit to 75 measured shapes (40 to 4096 rows; N 640, 2560, 3840, 13824; K
+// 2560, 6912): the tile it picks is within 4 % of the fastest of the six on each of them.
+int ternary_tile(long M, long N, long K) {
+    const struct { int tile, rows, cols; double fixed, step, two, more; } t[] = {
+        {21, 32, 64, 3.23, 0.170, 1.48, 0.88},   {19, 64, 64, 3.35, 0.224, 1.32, 1.04},   {18, 64, 128, 4.55, 0.311, 1.56, 1.00},
+        {17, 128, 128, 6.09, 0.490, 1.65, 1.04}, {20, 64, 256, 5.30, 0.546, 1.53, 0.97}, {16, 128, 256, 6.79, 0.762, 1.36, 1.13}};
+    int best = 16;
+    double least = 1e30;
+    for (const auto& x : t) {
+        const double r = (double)(((M + x.rows - 1) / x.rows) * ((N + x.cols - 1) / x.cols)) / 256.0;
+        const double us = x.fixed + K / 128 * x.step * (r <= 1 ? 1.0 : r <= 2 ? x.two : (x.more * r > x.two ? x.more * r : x.two));
+        if (us < least) {
+            least = us;
+            best = x.tile;
+        }
+    }
+    return best;
 }
 
 template <typename T, int kEpi>
@@ -2370,7 +2637,7 @@ int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
             default: launch_cfg<T, kEpi, 1, 1, 128, 6>(a, st); break;
         }
     } else {
-        // VLA_TERNARY_TILE = 64 | 128 | 256 pins a tile of the 32x32x32 kernels, 16 the 16x16x64 kernel (tests and tuning); unset = by shape.
+        // VLA_TERNARY_TILE = 64 | 128 | 256 pins a tile of the 32x32x32 kernels, 16..21 one of the 16x16x64 kernels (tests and tuning); unset = by shape.
         const int force = tuning().ternary_tile;
         // Enough 128 x 256 tiles for half the chip: the large-M kernel, two workgroups per
         // CU (measured faster than one 256 x 256 workgroup: fewer wavefronts per barrier).
@@ -2386,13 +2653,19 @@ int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
             const unsigned grid = (unsigned)((a.N + 31) / 32);
             if (gemv_groups <= 10) ternary_gemv_kernel<10><<<grid, GEMV_WAVES * 64, 0, st>>>(a);
             else ternary_gemv_kernel<28><<<grid, GEMV_WAVES * 64, 0, st>>>(a);
+        } else if (x16_ok && (force == 0 || (force >= 16 && force < 64))) {
+            // the 16x16x64 kernels
+            switch (force ? force : ternary_tile(a.M, a.N, a.K)) {
+                case 17: launch_ring<4, 4, 4>(a, st); break;
+                case 18: launch_ring<2, 4, 5>(a, st); break;
+                case 19: launch_ring<2, 2, 6>(a, st); break;
+                case 20: launch_ring<2, 8, 4>(a, st); break;
+                case 21: launch_ring<1, 2, 8>(a, st); break;
+                default: launch_x16(a, st); break;  // 128 x 256 tiles, two workgroups per CU
+            }
         } else if (force == 256) {
             const unsigned grid = (unsigned)(((((a.M + 255) / 256) + 7) & ~7) * n256);
             ternary_gemm_big_kernel<4><<<grid, 512, 0, st>>>(a);
-        } else if (x16_ok && (force == 16 || (force == 0 && wg128 >= 128))) {
-            // the 16x16x64 kernel: 128 x 256 tiles, two workgroups per CU
-            const unsigned grid = (unsigned)(((((a.M + 127) / 128) + 7) & ~7) * n256);
-            ternary_gemm_x16_kernel<<<grid, 256, 0, st>>>(a);
         } else if (force == 128 || (force == 0 && wg128 >= 128)) {
             const unsigned grid = (unsigned)(((((a.M + 127) / 128) + 7) & ~7) * n256);
             ternary_gemm_big_kernel<2><<<grid, 256, 0, st>>>(a);
