@@ -252,6 +252,13 @@ VLA_KAPI int vla_qkv_split_rope_append(const void* qkv, const float* cos_tab, co
                                        void* k_cache, void* vt_cache, int dtype, int M, int S, int n_q_heads,
                                        int n_kv_heads, int head_dim, int t_max, int tok_offset, vla_stream_t stream);
 
+/* The same from three matrices, q [M][n_q_heads * D], k and v [M][n_kv_heads * D]: vla_rope_neox on
+ * q and k, then vla_kv_append, in one launch with the same bits.  q_out may be q.  bf16, head_dim a
+ * multiple of 16 and 16-byte aligned q, k, v, q_out, k_cache and tables; VLA_K_ERR_SHAPE otherwise. */
+VLA_KAPI int vla_rope_append(const void* q, const void* k, const void* v, const float* cos_tab, const float* sin_tab, void* q_out,
+                             void* k_cache, void* vt_cache, int dtype, int M, int S, int n_q_heads, int n_kv_heads, int head_dim,
+                             int t_max, int tok_offset, vla_stream_t stream);
+
 /* ------------------------------------------------------------------ attention */
 
 /* out = softmax(scale * Q K^T + mask) V over keys [0, n_keys) of the resident

@@ -1675,3 +1675,44 @@ def test_ternary_gemm_ring_tiles_bit_exact(tune, tile, M, N, K, ws_num):
     assert np.array_equal(host(acc), want_acc)
     assert np.array_equal(host(out, np.uint16), orc.ternary_epilogue(want_acc, s, ws))
     assert np.array_equal(host(h), host(want_sum))
+
+
+@pytest.mark.parametrize("rope", [True, False])
+@pytest.mark.parametrize("B,S,Hq,Hkv,D,off", [(1, 8, 2, 1, 16, 0), (2, 65, 4, 2, 64, 8), (1, 128, 3, 1, 48, 3), (3, 71, 5, 5, 128, 16),
+                                              (1, 64, 1, 1, 80, 0), (1, 9, 2, 1, 24, 0)])
+def test_rope_append_of_many_rows_is_the_element_kernels(B, S, Hq, Hkv, D, off, rope):
+    """Rows and head widths that end inside a 64 x 64 tile of V, unaligned cache slots, a width the
+    16-byte kernel leaves to the element kernel (24): from one fused matrix the bits of the same rows
+    appended token by token, from three those of rotation and append as launches of their own, and
+    nothing else of the caches touched."""
+    r = np.random.default_rng(B * S + D)
+    t_max, M = 160, B * S
+    q, k, v = (orc.to_bf16(r.standard_normal((M, h * D)).astype(np.float32)) for h in (Hq, Hkv, Hkv))
+    fill = r.integers(0, 65536, (2, B, Hkv, t_max * D)).astype(np.uint16)
+    cos, sin = (dev(t.astype(np.float32)) for t in orc.rope_tables(np.arange(off, off + S, dtype=np.int32), D, 10000.0))
+    tabs = (cos, sin) if rope else (None, None)
+    qkv = np.concatenate([q, k, v], 1).reshape(B, S, -1)
+    kc, vc, qt = dev(fill[0]), dev(fill[1]), torch.zeros((S, B, Hq * D), dtype=torch.int16, device="cuda")
+    rows = dev(np.ascontiguousarray(qkv.transpose(1, 0, 2)))
+    for s in range(S):
+        tok = (cos[s].clone(), sin[s].clone()) if rope else (None, None)
+        pkg.call("vla_qkv_split_rope_append", rows[s], *tok, qt[s], kc, vc, pkg.VLA_DT_BF16, B, 1, Hq, Hkv, D, t_max, off + s)
+    kc1, vc1, q1 = dev(fill[0]), dev(fill[1]), torch.zeros((B, S, Hq * D), dtype=torch.int16, device="cuda")
+    pkg.call("vla_qkv_split_rope_append", dev(qkv), *tabs, q1, kc1, vc1, pkg.VLA_DT_BF16, M, S, Hq, Hkv, D, t_max, off)
+    sync()
+    assert torch.equal(q1, qt.transpose(0, 1)) and torch.equal(kc1, kc) and torch.equal(vc1, vc)
+    dq, dk, dv = dev(q), dev(k), dev(v)
+    kc, vc = dev(fill[0]), dev(fill[1])
+    if rope:
+        pkg.call("vla_rope_neox", dq, cos, sin, pkg.VLA_DT_BF16, M, S, Hq, D)
+        pkg.call("vla_rope_neox", dk, cos, sin, pkg.VLA_DT_BF16, M, S, Hkv, D)
+    pkg.call("vla_kv_append", kc, vc, dk, dv, pkg.VLA_DT_BF16, B, Hkv, D, t_max, off, S)
+    q2, kc2, vc2, k2 = dev(q), dev(fill[0]), dev(fill[1]), dev(k)
+    args = (q2, k2, dv, *tabs, q2, kc2, vc2, pkg.VLA_DT_BF16, M, S, Hq, Hkv, D, t_max, off)
+    if D % 16:
+        ptr = [a.data_ptr() if isinstance(a, torch.Tensor) else a for a in args]
+        assert pkg.lib().vla_rope_append(*ptr, 0) == pkg.VLA_K_ERR_SHAPE
+        return
+    pkg.call("vla_rope_append", *args)
+    sync()
+    assert torch.equal(q2, dq) and torch.equal(kc2, kc) and torch.equal(vc2, vc)

@@ -91,6 +91,117 @@ __global__ void qkv_split_rope_append_kernel(const T* __restrict__ qkv, const fl
     }
 }
 
+// The same for bf16 rows of many tokens, Q, K and V each with a row stride of their own (one fused
+// matrix or three).  Bound by memory; the kernel above moves two bytes per lane and writes V^T one
+// element per cache line (4096 rows of 20 + 2 x 5 heads of 128, 63 MB: 41.7 us in the prefix build, this one
+// 12.5).  Here a thread rotates eight pairs with 16-byte loads and stores, and the first `v_blocks` workgroups
+// turn 64 tokens x 64 columns of V through LDS: token rows go in as 16-byte pieces, piece c of token t
+// at c ^ (t / 8) % 8, so that the eight token groups a wavefront reads of a column lie in distinct banks, and
+// a column leaves as up to 128 consecutive bytes.  V keeps its bits.  q_out may be q.  The second sum of a
+// pair is rounded as in the launches this one stands for: kSplit, the product x0 s as in
+// qkv_split_rope_append_kernel, else x1 c as in rope_neox_kernel.
+struct RopeAppend {
+    const bf16_t *q, *k, *v;
+    const float *cos_t, *sin_t;
+    bf16_t *q_out, *k_cache, *vt_cache;
+    int ldq, ldk, ldv, S, Hq, Hkv, D, t_max, tok_offset, s_tiles, d_tiles, v_vec;
+    unsigned v_blocks, rope_total;
+};
+template <bool kSplit>
+__global__ void __launch_bounds__(256) rope_append_rows_kernel(RopeAppend a) {
+    __shared__ u32x4_t tile[64 * 8];
+    const unsigned tid = threadIdx.x;
+    if (blockIdx.x < a.v_blocks) {
+        unsigned u = blockIdx.x;
+        const int st = u % a.s_tiles;
+        u /= a.s_tiles;
+        const int dt = u % a.d_tiles;
+        u /= a.d_tiles;
+        const int h = u % a.Hkv, b = u / a.Hkv;
+        const int s0 = st * 64, d0 = dt * 64;
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            const int t = p * 32 + (tid >> 3), c = tid & 7;
+            u32x4_t raw = {0u, 0u, 0u, 0u};
+            if (s0 + t < a.S && d0 + c * 8 < a.D)
+                raw = *reinterpret_cast<const u32x4_t*>(a.v + ((long)b * a.S + s0 + t) * a.ldv + h * a.D + d0 + c * 8);
+            tile[t * 8 + (c ^ (t >> 3))] = raw;
+        }
+        __syncthreads();
+        const bf16_t* el = reinterpret_cast<const bf16_t*>(tile);
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            const int i = p * 256 + tid, seg = i & 7, dd = (i >> 3) & 7, c = i >> 6;
+            const int d = d0 + c * 8 + dd, s = s0 + seg * 8;
+            if (d >= a.D || s >= a.S) continue;
+            bf16_t x[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) x[j] = el[(seg * 8 + j) * 64 + (c ^ seg) * 8 + dd];
+            bf16_t* dst = a.vt_cache + (((long)b * a.Hkv + h) * a.D + d) * (long)a.t_max + a.tok_offset + s;
+            if (a.v_vec && s + 8 <= a.S) {
+                u32x4_t o;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = (uint32_t)x[2 * e] | (uint32_t)x[2 * e + 1] << 16;
+                *reinterpret_cast<u32x4_t*>(dst) = o;
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if (s + j < a.S) dst[j] = x[j];
+            }
+        }
+        return;
+    }
+    const unsigned i = (blockIdx.x - a.v_blocks) * 256 + tid;
+    if (i >= a.rope_total) return;
+    const unsigned half = a.D >> 1, n8 = half >> 3, heads = a.Hq + a.Hkv;
+    const unsigned p = i % n8 * 8, rh = i / n8, hh = rh % heads, m = rh / heads;
+    const unsigned b = m / a.S, s = m % a.S;
+    const bool is_q = hh < (unsigned)a.Hq;
+    const bf16_t* src = is_q ? a.q + (long)m * a.ldq + hh * a.D : a.k + (long)m * a.ldk + (hh - a.Hq) * a.D;
+    u32x4_t lo = *reinterpret_cast<const u32x4_t*>(src + p), hi = *reinterpret_cast<const u32x4_t*>(src + p + half);
+    if (a.cos_t) {
+        const f32x4_t* cp = reinterpret_cast<const f32x4_t*>(a.cos_t + (long)s * half + p);
+        const f32x4_t* sp = reinterpret_cast<const f32x4_t*>(a.sin_t + (long)s * half + p);
+        const f32x4_t c[2] = {cp[0], cp[1]}, sn[2] = {sp[0], sp[1]};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float r0[2], r1[2];
+#pragma unroll
+            for (int w = 0; w < 2; ++w) {
+                const float x0 = __uint_as_float(w ? lo[e] & 0xffff0000u : lo[e] << 16);
+                const float x1 = __uint_as_float(w ? hi[e] & 0xffff0000u : hi[e] << 16);
+                const float cc = c[e >> 1][(e & 1) * 2 + w], ss = sn[e >> 1][(e & 1) * 2 + w];
+                r0[w] = fmaf(x0, cc, -(x1 * ss));
+                r1[w] = kSplit ? fmaf(x1, cc, x0 * ss) : fmaf(x0, ss, x1 * cc);
+            }
+            lo[e] = pack_bf2(r0[0], r0[1]);
+            hi[e] = pack_bf2(r1[0], r1[1]);
+        }
+    }
+    bf16_t* dst = is_q ? a.q_out + ((long)m * a.Hq + hh) * a.D
+                       : a.k_cache + (((long)b * a.Hkv + (hh - a.Hq)) * a.t_max + a.tok_offset + s) * a.D;
+    *reinterpret_cast<u32x4_t*>(dst + p) = lo;
+    *reinterpret_cast<u32x4_t*>(dst + p + half) = hi;
+}
+
+// false: shapes or addresses that the kernel above does not take (16-byte pieces of a half head, 32-bit indexes)
+template <bool kSplit>
+bool launch_rope_append(RopeAppend a, int M, hipStream_t st) {
+    auto off16 = [](const void* p) { return ((uintptr_t)p & 15) != 0; };
+    if (a.D % 16 || a.ldq % 8 || a.ldk % 8 || a.ldv % 8 || off16(a.q) || off16(a.k) || off16(a.v) || off16(a.q_out) || off16(a.k_cache) ||
+        (a.cos_t && (off16(a.cos_t) || off16(a.sin_t))))
+        return false;
+    a.s_tiles = (a.S + 63) / 64;
+    a.d_tiles = (a.D + 63) / 64;
+    a.v_vec = a.t_max % 8 == 0 && a.tok_offset % 8 == 0 && !off16(a.vt_cache);
+    const long v_blocks = (long)(M / a.S) * a.Hkv * a.s_tiles * a.d_tiles, total = (long)M * (a.Hq + a.Hkv) * (a.D / 16);
+    if (v_blocks >= (1l << 22) || total >= (1l << 30)) return false;
+    a.v_blocks = (unsigned)v_blocks;
+    a.rope_total = (unsigned)total;
+    rope_append_rows_kernel<kSplit><<<(unsigned)(v_blocks + (total + 255) / 256), 256, 0, st>>>(a);
+    return true;
+}
+
 // ----------------------------------------------------------------- norms ---
 template <typename T>
 __global__ void rms_norm_kernel(const T* __restrict__ x, const T* __restrict__ w, T* __restrict__ y, int K, float eps) {
@@ -957,6 +1068,14 @@ int vla_qkv_split_rope_append(const void* qkv, const float* cos_tab, const float
     if (total == 0) return VLA_K_OK;
     const unsigned blocks = (unsigned)((total + 255) / 256);
     hipStream_t st = (hipStream_t)stream;
+    // From eight tokens on; fewer would leave most of a 64-token tile of V empty.
+    if (dtype == VLA_DT_BF16 && S >= 8) {
+        const int ld = (n_q_heads + 2 * n_kv_heads) * head_dim;
+        const bf16_t* q = (const bf16_t*)qkv;
+        if (launch_rope_append<true>({q, q + n_q_heads * head_dim, q + (n_q_heads + n_kv_heads) * head_dim, cos_tab, sin_tab, (bf16_t*)q_out,
+                                (bf16_t*)k_cache, (bf16_t*)vt_cache, ld, ld, ld, S, n_q_heads, n_kv_heads, head_dim, t_max, tok_offset}, M, st))
+            return VLA_CHECK_LAUNCH();
+    }
     if (dtype == VLA_DT_F32)
         qkv_split_rope_append_kernel<float><<<blocks, 256, 0, st>>>((const float*)qkv, cos_tab, sin_tab, (float*)q_out,
                                                                    (float*)k_cache, (float*)vt_cache, S, n_q_heads,
@@ -967,6 +1086,21 @@ int vla_qkv_split_rope_append(const void* qkv, const float* cos_tab, const float
                                                                     n_kv_heads, head_dim, t_max, tok_offset, total);
     else
         return VLA_K_ERR_ARG;
+    return VLA_CHECK_LAUNCH();
+}
+
+int vla_rope_append(const void* q, const void* k, const void* v, const float* cos_tab, const float* sin_tab, void* q_out, void* k_cache,
+                    void* vt_cache, int dtype, int M, int S, int n_q_heads, int n_kv_heads, int head_dim, int t_max, int tok_offset,
+                    vla_stream_t stream) {
+    if (!q || !k || !v || !q_out || !k_cache || !vt_cache || M < 0 || S <= 0 || n_q_heads <= 0 || n_kv_heads <= 0) return VLA_K_ERR_ARG;
+    if ((cos_tab == nullptr) != (sin_tab == nullptr)) return VLA_K_ERR_ARG;
+    if (head_dim <= 0 || M % S || tok_offset < 0 || tok_offset + S > t_max || dtype != VLA_DT_BF16) return VLA_K_ERR_SHAPE;
+    if (M == 0) return VLA_K_OK;
+    const int kvd = n_kv_heads * head_dim;
+    if (!launch_rope_append<false>({(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, cos_tab, sin_tab, (bf16_t*)q_out, (bf16_t*)k_cache,
+                             (bf16_t*)vt_cache, n_q_heads * head_dim, kvd, kvd, S, n_q_heads, n_kv_heads, head_dim, t_max, tok_offset},
+                            M, (hipStream_t)stream))
+        return VLA_K_ERR_SHAPE;
     return VLA_CHECK_LAUNCH();
 }
 

@@ -44,9 +44,15 @@ int run(bitvla_lm_hip_ctx* c, const uint16_t* d_in, uint16_t* d_out, int seq, hi
         VLA_K(vla_ternary_gemm(q8, (const uint32_t*)w.q_packed, c->q.as<uint16_t>(), nullptr, s, rs, w.q_ws, 1, seq, hq, H, st));
         VLA_K(vla_ternary_gemm(q8, (const uint32_t*)w.k_packed, c->k.as<uint16_t>(), nullptr, s, rs, w.k_ws, 1, seq, hkv, H, st));
         VLA_K(vla_ternary_gemm(q8, (const uint32_t*)w.v_packed, c->v.as<uint16_t>(), nullptr, s, rs, w.v_ws, 1, seq, hkv, H, st));
-        VLA_K(vla_rope_neox(c->q.get(), c->cos.as<float>(), c->sin.as<float>(), VLA_DT_BF16, seq, seq, c->n_q, c->hd, st));
-        VLA_K(vla_rope_neox(c->k.get(), c->cos.as<float>(), c->sin.as<float>(), VLA_DT_BF16, seq, seq, c->n_kv, c->hd, st));
-        VLA_K(vla_kv_append(c->kc.get(), c->vtc.get(), c->k.get(), c->v.get(), VLA_DT_BF16, 1, c->n_kv, c->hd, c->t_max, 0, seq, st));
+        // rotation of Q and K and the cache append in one launch (same bits as the three below it)
+        const int ra = vla_rope_append(c->q.get(), c->k.get(), c->v.get(), c->cos.as<float>(), c->sin.as<float>(), c->q.get(), c->kc.get(),
+                                       c->vtc.get(), VLA_DT_BF16, seq, seq, c->n_q, c->n_kv, c->hd, c->t_max, 0, st);
+        if (ra != VLA_K_ERR_SHAPE) VLA_K(ra);
+        else {
+            VLA_K(vla_rope_neox(c->q.get(), c->cos.as<float>(), c->sin.as<float>(), VLA_DT_BF16, seq, seq, c->n_q, c->hd, st));
+            VLA_K(vla_rope_neox(c->k.get(), c->cos.as<float>(), c->sin.as<float>(), VLA_DT_BF16, seq, seq, c->n_kv, c->hd, st));
+            VLA_K(vla_kv_append(c->kc.get(), c->vtc.get(), c->k.get(), c->v.get(), VLA_DT_BF16, 1, c->n_kv, c->hd, c->t_max, 0, seq, st));
+        }
         VLA_K(vla_attn_prefix_suffix_ws(c->q.get(), c->kc.get(), c->vtc.get(), c->att.get(), VLA_DT_BF16_P2, 1, seq, c->n_q, c->n_kv,
                                         c->hd, c->t_max, seq, scale, VLA_MASK_NONE, seq, 0, 0, nullptr, c->attn_ws.get(),
                                         c->attn_ws.bytes(), st));
