@@ -1716,3 +1716,26 @@ def test_rope_append_of_many_rows_is_the_element_kernels(B, S, Hq, Hkv, D, off, 
     pkg.call("vla_rope_append", *args)
     sync()
     assert torch.equal(q2, dq) and torch.equal(kc2, kc) and torch.equal(vc2, vc)
+
+
+@pytest.mark.parametrize("M", [16, 50, 512, 2048])
+@pytest.mark.parametrize("K", [328, 1032, 320])
+def test_norm_inside_takes_multiples_of_16_at_every_number_of_rows(M, K):
+    """With a norm inside, K must be a multiple of 16: whether a call is taken does not depend on the
+    number of rows, so that a caller who probes one batch size knows the others."""
+    r = np.random.default_rng(K)
+    H, D, I = 4, 64, 128
+    N = 3 * H * D
+    x = to_dev(r.standard_normal((M, K)).astype(np.float32), BF16)
+    W = to_dev((0.05 * r.standard_normal((N, K))).astype(np.float32), BF16)
+    cs = dev(r.standard_normal(N).astype(np.float32))
+    q, kc, vc, y = empty((M, H * D), BF16), empty((1, H, M, D), BF16), empty((1, H, D, M), BF16), empty((M, I), BF16)
+    p = lambda t: t.data_ptr()
+    tail = (BF16, M, K, M, H, H, 1, 1, D, None, None, p(q), p(kc), p(vc), M, 0, 1e-5, pkg.stream())
+    got = [pkg.lib().vla_rmsnorm_attn_qkv_rope(p(x), p(W), None, *tail),
+           pkg.lib().vla_layernorm_attn_qkv_rope(p(x), p(W), p(cs), None, *tail),
+           pkg.lib().vla_glu_linear(p(x), p(W), None, p(y), BF16, BF16, M, I, K, pkg.VLA_ACT_SILU, 1e-5, pkg.stream())]
+    sync()
+    assert got == [pkg.VLA_K_OK if K % 16 == 0 else pkg.VLA_K_ERR_SHAPE] * 3
+    pkg.call("vla_glu_linear", x, W, None, y, BF16, BF16, M, I, K, pkg.VLA_ACT_SILU, -1.0)  # without a norm: multiples of 8
+    sync()

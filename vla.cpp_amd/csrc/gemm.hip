@@ -2549,6 +2549,7 @@ int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
                        (uintptr_t)a.A % 16 == 0 && (uintptr_t)a.W % 16 == 0 && !(a.colsum && a.norm_eps < 0.f) && !a.stats_out && !a.stats_in;
         if (kEpi == EPI_QKV) rows_ok = rows_ok && a.D % 16 == 0 && a.N % 16 == 0;  // 8 + 8 columns of one head
         if (kEpi == EPI_PLAIN) rows_ok = rows_ok && a.norm_eps < 0.f;
+        if (a.norm_eps >= 0.f) rows_ok = rows_ok && a.K % 16 == 0;  // what the tiled kernel takes with a norm inside, at every number of rows
         const int plan = rows_ok ? narrow_plan(a) : -1;
         if (plan >= 0) {
             if (a.norm_eps < 0.f) launch_narrow<kEpi, NORM_NONE>(a, plan, st);
