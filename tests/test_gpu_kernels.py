@@ -1739,3 +1739,20 @@ def test_norm_inside_takes_multiples_of_16_at_every_number_of_rows(M, K):
     assert got == [pkg.VLA_K_OK if K % 16 == 0 else pkg.VLA_K_ERR_SHAPE] * 3
     pkg.call("vla_glu_linear", x, W, None, y, BF16, BF16, M, I, K, pkg.VLA_ACT_SILU, -1.0)  # without a norm: multiples of 8
     sync()
+
+
+@pytest.mark.parametrize("M", [16, 50, 300, 2048])
+def test_register_staged_override_holds_at_every_number_of_rows(tune, M):
+    """VLA_GEMM_DL=0 pins the register-staged kernel, which takes no norm: a gated projection with a norm
+    inside is refused at every number of rows, and without one has the same bits as unpinned."""
+    r = np.random.default_rng(M)
+    I, K = 128, 320
+    x, W, y = (to_dev(r.standard_normal(s).astype(np.float32), BF16) for s in ((M, K), (2 * I, K), (M, I)))
+    args = (BF16, BF16, M, I, K, pkg.VLA_ACT_SILU)
+    pkg.call("vla_glu_linear", x, W, None, y, *args, -1.0)
+    tune.set("VLA_GEMM_DL", 0)
+    pinned = torch.empty_like(y)
+    pkg.call("vla_glu_linear", x, W, None, pinned, *args, -1.0)
+    assert pkg.lib().vla_glu_linear(x.data_ptr(), W.data_ptr(), None, pinned.data_ptr(), *args, 1e-5, pkg.stream()) == pkg.VLA_K_ERR_SHAPE
+    sync()
+    assert torch.equal(y, pinned)

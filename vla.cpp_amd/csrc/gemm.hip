@@ -2545,7 +2545,7 @@ int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
     }
     if constexpr (std::is_same<T, bf16_t>::value && kEpi != EPI_TERNARY) {
         // few bf16 rows (the suffix of one or a few observations through a projection): narrow tiles over the whole chip
-        bool rows_ok = a.M <= tuning().gemm_rows_max && a.K % 8 == 0 && a.K >= 64 && tuning().gemm_tile < 0 &&
+        bool rows_ok = a.M <= tuning().gemm_rows_max && a.K % 8 == 0 && a.K >= 64 && tuning().gemm_tile < 0 && tuning().gemm_dl != 0 &&
                        (uintptr_t)a.A % 16 == 0 && (uintptr_t)a.W % 16 == 0 && !(a.colsum && a.norm_eps < 0.f) && !a.stats_out && !a.stats_in;
         if (kEpi == EPI_QKV) rows_ok = rows_ok && a.D % 16 == 0 && a.N % 16 == 0;  // 8 + 8 columns of one head
         if (kEpi == EPI_PLAIN) rows_ok = rows_ok && a.norm_eps < 0.f;
