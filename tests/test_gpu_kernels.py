@@ -1756,3 +1756,22 @@ def test_register_staged_override_holds_at_every_number_of_rows(tune, M):
     assert pkg.lib().vla_glu_linear(x.data_ptr(), W.data_ptr(), None, pinned.data_ptr(), *args, 1e-5, pkg.stream()) == pkg.VLA_K_ERR_SHAPE
     sync()
     assert torch.equal(y, pinned)
+
+
+@pytest.mark.parametrize("tile,M,N", [(21, 16_800_000, 64), (0, 22_400_000, 288)])
+def test_ternary_gemm_of_more_tiles_than_the_tile_walk_counts(tune, tile, M, N):
+    """Millions of rows: from 65536 workgroups per XCD on, the call goes to the kernel whose grid has no
+    such limit.  Every output against the exact product (|acc| <= 127 * 128, exact in fp32)."""
+    K = 128
+    if torch.cuda.mem_get_info()[0] < 2 * M * (N + K):
+        pytest.skip("not enough device memory")
+    g = torch.Generator("cuda").manual_seed(N)
+    A = torch.randint(-127, 128, (M, K), generator=g, device="cuda", dtype=torch.int8)
+    t = np.random.default_rng(N).integers(-1, 2, (N, K)).astype(np.int8)
+    rowsum, one = A.sum(1, dtype=torch.int32), torch.ones(M, device="cuda")
+    out = torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
+    tune.set("VLA_TERNARY_TILE", tile)
+    pkg.call("vla_ternary_gemm", A, dev(_pack_plain(t)), out, None, one, rowsum, one, 1, M, N, K)
+    Wt = dev(t).float().T.contiguous()
+    for i in range(0, M, 1 << 20):
+        assert torch.equal(out[i:i + (1 << 20)], (A[i:i + (1 << 20)].float() @ Wt).to(torch.bfloat16))

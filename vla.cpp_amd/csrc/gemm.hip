@@ -2488,12 +2488,14 @@ void launch_narrow(const GemmArgs& a, int p, hipStream_t st) {
     }
 }
 
+// false, launching nothing: more workgroups than the tile walk can count (millions of rows)
 template <int MB, int NB, int NS>
-void launch_ring(GemmArgs a, hipStream_t st) {
+bool launch_ring(GemmArgs a, hipStream_t st) {
     const unsigned grid = xcd_split(a, (a.M + 32 * MB - 1) / (32 * MB), (a.N + 32 * NB - 1) / (32 * NB), 0.25, 32 * NB, 1.0);
-    ternary_gemm_ring_kernel<MB, NB, NS><<<grid, 256, 0, st>>>(a);
+    if (grid) ternary_gemm_ring_kernel<MB, NB, NS><<<grid, 256, 0, st>>>(a);
+    return grid != 0;
 }
-void launch_x16(GemmArgs a, hipStream_t st) {
+bool launch_x16(GemmArgs a, hipStream_t st) {
     const int m_wg = (a.M + 127) / 128, n_wg = (a.N + 255) / 256;
     unsigned grid;
     if (m_wg % 8 == 0) {
@@ -2505,7 +2507,8 @@ void launch_x16(GemmArgs a, hipStream_t st) {
     } else {
         grid = xcd_split(a, m_wg, n_wg, 0.25, 256, 1.0);
     }
-    ternary_gemm_x16_kernel<<<grid, 256, 0, st>>>(a);
+    if (grid) ternary_gemm_x16_kernel<<<grid, 256, 0, st>>>(a);
+    return grid != 0;
 }
 
 // Tile of a ternary GEMM (VLA_TERNARY_TILE codes) by predicted time: a launch costs `fixed`, and
@@ -2640,8 +2643,6 @@ int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
     } else {
         // VLA_TERNARY_TILE = 64 | 128 | 256 pins a tile of the 32x32x32 kernels, 16..21 one of the 16x16x64 kernels (tests and tuning); unset = by shape.
         const int force = tuning().ternary_tile;
-        // Enough 128 x 256 tiles for half the chip: the large-M kernel, two workgroups per
-        // CU (measured faster than one 256 x 256 workgroup: fewer wavefronts per barrier).
         const int n256 = (a.N + 255) / 256;
         const long wg128 = (long)((a.M + 127) / 128) * n256;
         const int gemv_groups = (a.K / 32 + GEMV_WAVES - 1) / GEMV_WAVES;  // k groups per wavefront
@@ -2650,24 +2651,31 @@ int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
         const int ws_group = a.N / (a.ws_num > 0 ? a.ws_num : 1);
         const bool x16_ok = a.N % 8 == 0 && (a.Y == nullptr || ws_group % 32 == 0) && (long)a.M * a.K < (1l << 32) &&
                             (long)((a.N + 31) / 32) * a.K * 8 < (1l << 32) && ((uintptr_t)a.A % 16 == 0) && a.K % 16 == 0;
+        const bool x16_asked = force == 0 || (force >= 16 && force < 64);
+        bool done = false;
         if (force == 0 && a.M <= 32 && gemv_groups <= 28) {
             const unsigned grid = (unsigned)((a.N + 31) / 32);
             if (gemv_groups <= 10) ternary_gemv_kernel<10><<<grid, GEMV_WAVES * 64, 0, st>>>(a);
             else ternary_gemv_kernel<28><<<grid, GEMV_WAVES * 64, 0, st>>>(a);
-        } else if (x16_ok && (force == 0 || (force >= 16 && force < 64))) {
+            done = true;
+        } else if (x16_ok && x16_asked) {
             // the 16x16x64 kernels
             switch (force ? force : ternary_tile(a.M, a.N, a.K)) {
-                case 17: launch_ring<4, 4, 4>(a, st); break;
-                case 18: launch_ring<2, 4, 5>(a, st); break;
-                case 19: launch_ring<2, 2, 6>(a, st); break;
-                case 20: launch_ring<2, 8, 4>(a, st); break;
-                case 21: launch_ring<1, 2, 8>(a, st); break;
-                default: launch_x16(a, st); break;  // 128 x 256 tiles, two workgroups per CU
+                case 17: done = launch_ring<4, 4, 4>(a, st); break;
+                case 18: done = launch_ring<2, 4, 5>(a, st); break;
+                case 19: done = launch_ring<2, 2, 6>(a, st); break;
+                case 20: done = launch_ring<2, 8, 4>(a, st); break;
+                case 21: done = launch_ring<1, 2, 8>(a, st); break;
+                default: done = launch_x16(a, st); break;  // 128 x 256 tiles, two workgroups per CU
             }
+        }
+        // What those do not take: the 32x32x32 kernels, with 128 x 256 tiles where they fill half the chip (two
+        // workgroups per CU, measured faster than one of 256 x 256: fewer wavefronts per barrier).
+        if (done) {
         } else if (force == 256) {
             const unsigned grid = (unsigned)(((((a.M + 255) / 256) + 7) & ~7) * n256);
             ternary_gemm_big_kernel<4><<<grid, 512, 0, st>>>(a);
-        } else if (force == 128 || (force == 0 && wg128 >= 128)) {
+        } else if (force == 128 || (x16_asked && wg128 >= 128)) {
             const unsigned grid = (unsigned)(((((a.M + 127) / 128) + 7) & ~7) * n256);
             ternary_gemm_big_kernel<2><<<grid, 256, 0, st>>>(a);
         } else {
