@@ -1775,3 +1775,31 @@ def test_ternary_gemm_of_more_tiles_than_the_tile_walk_counts(tune, tile, M, N):
     Wt = dev(t).float().T.contiguous()
     for i in range(0, M, 1 << 20):
         assert torch.equal(out[i:i + (1 << 20)], (A[i:i + (1 << 20)].float() @ Wt).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("tile", [0, 17, 18, 19, 20, 21])
+@pytest.mark.parametrize("M", [40, 300])
+@pytest.mark.parametrize("shift", ["words", "out", "residual"])
+def test_ternary_gemm_of_unaligned_buffers(tune, shift, M, tile):
+    """Packed words 4 bytes, output or residual rows 2 bytes off a 16-byte address: the bits of the aligned
+    call, whichever LDS-ring tile is asked for, and nothing written beside the output."""
+    r = np.random.default_rng(M)
+    N, K, pad = 320, 256, 8
+    A, s = dev(r.integers(-127, 128, (M, K)).astype(np.int8)), dev((40.0 + r.integers(0, 100, M)).astype(np.float32))
+    rowsum, ws = A.sum(1, dtype=torch.int32), dev(np.float32([0.02]))
+    W, res = dev(_pack_plain(r.integers(-1, 2, (N, K)).astype(np.int8))), dev(orc.to_bf16(r.standard_normal(M * N).astype(np.float32)))
+
+    def off(t, n):  # the same values n elements into a larger buffer
+        buf = torch.full((t.numel() + pad,), 77, dtype=t.dtype, device="cuda")
+        buf[n:n + t.numel()] = t.flatten()
+        return buf, buf.data_ptr() + n * t.element_size()
+
+    def run(w, y, rr):
+        (_, wp), (_, rp), (yb, yp) = off(W, w), off(res, rr), off(torch.zeros_like(res), y)
+        pkg.check(pkg.lib().vla_ternary_gemm_add(A.data_ptr(), wp, yp, rp, s.data_ptr(), rowsum.data_ptr(), ws.data_ptr(), 1, M, N, K, pkg.stream()))
+        sync()
+        assert torch.all(yb[:y] == 77) and torch.all(yb[y + M * N:] == 77)
+        return yb[y:y + M * N]
+
+    tune.set("VLA_TERNARY_TILE", tile)
+    assert torch.equal(run(int(shift == "words"), int(shift == "out"), int(shift == "residual")), run(0, 0, 0))

@@ -2651,6 +2651,10 @@ int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
         const int ws_group = a.N / (a.ws_num > 0 ? a.ws_num : 1);
         const bool x16_ok = a.N % 8 == 0 && (a.Y == nullptr || ws_group % 32 == 0) && (long)a.M * a.K < (1l << 32) &&
                             (long)((a.N + 31) / 32) * a.K * 8 < (1l << 32) && ((uintptr_t)a.A % 16 == 0) && a.K % 16 == 0;
+        // The LDS-ring tiles copy the weights and write the rows in 16-byte pieces; unaligned buffers stay with the other
+        // kernels, 128 x 256 tiles from half the chip on and the 64 x 64 ones, whose weight and row accesses are 4 bytes
+        // and less, below.
+        const bool ring_ok = (((uintptr_t)a.W | (uintptr_t)a.Y | (uintptr_t)a.residual) & 15) == 0;
         const bool x16_asked = force == 0 || (force >= 16 && force < 64);
         bool done = false;
         if (force == 0 && a.M <= 32 && gemv_groups <= 28) {
@@ -2658,9 +2662,9 @@ int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
             if (gemv_groups <= 10) ternary_gemv_kernel<10><<<grid, GEMV_WAVES * 64, 0, st>>>(a);
             else ternary_gemv_kernel<28><<<grid, GEMV_WAVES * 64, 0, st>>>(a);
             done = true;
-        } else if (x16_ok && x16_asked) {
+        } else if (x16_ok && x16_asked && (ring_ok || force == 16 || wg128 >= 128)) {
             // the 16x16x64 kernels
-            switch (force ? force : ternary_tile(a.M, a.N, a.K)) {
+            switch (!ring_ok ? 16 : force ? force : ternary_tile(a.M, a.N, a.K)) {
                 case 17: done = launch_ring<4, 4, 4>(a, st); break;
                 case 18: done = launch_ring<2, 4, 5>(a, st); break;
                 case 19: done = launch_ring<2, 2, 6>(a, st); break;
