@@ -1795,7 +1795,7 @@ def test_ternary_gemm_of_unaligned_buffers(tune, shift, M, tile):
         return buf, buf.data_ptr() + n * t.element_size()
 
     def run(w, y, rr):
-        (_, wp), (_, rp), (yb, yp) = off(W, w), off(res, rr), off(torch.zeros_like(res), y)
+        (wb, wp), (rb, rp), (yb, yp) = off(W, w), off(res, rr), off(torch.zeros_like(res), y)
         pkg.check(pkg.lib().vla_ternary_gemm_add(A.data_ptr(), wp, yp, rp, s.data_ptr(), rowsum.data_ptr(), ws.data_ptr(), 1, M, N, K, pkg.stream()))
         sync()
         assert torch.all(yb[:y] == 77) and torch.all(yb[y + M * N:] == 77)
@@ -1803,3 +1803,40 @@ def test_ternary_gemm_of_unaligned_buffers(tune, shift, M, tile):
 
     tune.set("VLA_TERNARY_TILE", tile)
     assert torch.equal(run(int(shift == "words"), int(shift == "out"), int(shift == "residual")), run(0, 0, 0))
+
+
+@pytest.mark.parametrize("M", [16, 50, 102])
+@pytest.mark.parametrize("out", [BF16, F32])
+def test_narrow_tile_projection_of_unaligned_outputs(M, out):
+    """Outputs, residual, Q and caches, or the rotation tables, one element off a 16-byte address (inside a
+    larger buffer): the bits of the aligned calls and nothing written beside the outputs, plain, gated, QKV."""
+    r = np.random.default_rng(M)
+    H, D, K = 2, 64, 320
+    N, tdt = 3 * H * D, torch.bfloat16 if out == BF16 else torch.float32
+    x, W = (to_dev((0.3 * r.standard_normal(s)).astype(np.float32), BF16) for s in ((M, K), (N, K)))
+    res = dev(r.standard_normal(M * N).astype(np.float32)).to(tdt)
+    ang = r.uniform(0, 6.28, (M, D // 2)).astype(np.float32)
+
+    def off(t, n):  # (buffer, address of t's values n elements into it)
+        buf = torch.full((t.numel() + 8,), 77.0, dtype=t.dtype, device="cuda")
+        buf[n:n + t.numel()] = t.flatten()
+        return buf, buf.data_ptr() + n * t.element_size()
+
+    def run(n, n_tab):
+        st, L, outs = pkg.stream(), pkg.lib(), []
+        zero = lambda count, dt: off(torch.zeros(count, dtype=dt, device="cuda"), n)
+        (y, yp), (rb, rp), (g, gp) = zero(M * N, tdt), off(res, n), zero(M * N // 2, tdt)
+        pkg.check(L.vla_linear(x.data_ptr(), W.data_ptr(), None, rp, yp, BF16, out, M, N, K, st))
+        pkg.check(L.vla_glu_linear(x.data_ptr(), W.data_ptr(), None, gp, BF16, out, M, N // 2, K, pkg.VLA_ACT_SILU, -1.0, st))
+        (cb, cp), (sb, sp) = off(dev(np.cos(ang)), n_tab), off(dev(np.sin(ang)), n_tab)
+        (q, qp), (k, kp), (v, vp) = (zero(M * H * D, torch.bfloat16) for _ in range(3))
+        pkg.check(L.vla_attn_qkv_rope(x.data_ptr(), W.data_ptr(), None, BF16, M, K, M, H, H, 1, 1, D, cp, sp, qp, kp, vp, M, 0, st))
+        sync()
+        for buf in (y, g, q, k, v):
+            assert torch.all(buf[:n] == 77) and torch.all(buf[buf.numel() - 8 + n:] == 77)
+            outs.append(buf[n:buf.numel() - 8 + n])
+        return outs
+
+    want = run(0, 0)
+    for got in (run(1, 0), run(0, 1)):
+        assert all(torch.equal(g, w) for g, w in zip(got, want))

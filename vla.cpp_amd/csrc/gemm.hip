@@ -1187,6 +1187,10 @@ __global__ void __launch_bounds__(256) gemm_narrow_kernel(GemmArgs a) {
             f = rsqrtf(sq * inv_k + a.norm_eps);
         }
     }
+    // Four columns at a time where the output's and residual's addresses allow it (uniform), else one by one; the
+    // operands' and rotation tables' addresses are checked by the launcher.
+    const uintptr_t io = kEpi == EPI_QKV ? (uintptr_t)a.q_out | (uintptr_t)a.k_cache : (uintptr_t)a.Y | (uintptr_t)a.residual;
+    const bool vec_io = (io & (kEpi == EPI_QKV || a.out_bf16 ? 7 : 15)) == 0;
     const int m = m0 + rb * 16 + c;
 #pragma unroll
     for (int j = 0; j < MY_NB; ++j) {
@@ -1218,7 +1222,7 @@ __global__ void __launch_bounds__(256) gemm_narrow_kernel(GemmArgs a) {
             }
             if (!live) continue;
             const long o = (long)m * a.N + n0;
-            if (a.N % 4 == 0) {  // 4 consecutive columns are inside the row or outside as a whole
+            if (a.N % 4 == 0 && vec_io) {  // 4 consecutive columns are inside the row or outside as a whole
                 if (n0 >= a.N) continue;
                 if (a.out_bf16) {
                     if (a.residual) {
@@ -1263,8 +1267,17 @@ __global__ void __launch_bounds__(256) gemm_narrow_kernel(GemmArgs a) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) y[e] = apply_act(v[e], a.act) * other[e];
             const long o = (long)m * (a.N / 2) + n0;
-            if (a.out_bf16) *reinterpret_cast<u32x2_t*>((bf16_t*)a.Y + o) = u32x2_t{pack_bf2(y[0], y[1]), pack_bf2(y[2], y[3])};
-            else *reinterpret_cast<f32x4_t*>((float*)a.Y + o) = f32x4_t{y[0], y[1], y[2], y[3]};
+            if (!vec_io) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (a.out_bf16) ((bf16_t*)a.Y)[o + e] = f2bf(y[e]);
+                    else ((float*)a.Y)[o + e] = y[e];
+                }
+            } else if (a.out_bf16) {
+                *reinterpret_cast<u32x2_t*>((bf16_t*)a.Y + o) = u32x2_t{pack_bf2(y[0], y[1]), pack_bf2(y[2], y[3])};
+            } else {
+                *reinterpret_cast<f32x4_t*>((float*)a.Y + o) = f32x4_t{y[0], y[1], y[2], y[3]};
+            }
             continue;
         }
         // QKV: rotation, scatter
@@ -1282,12 +1295,20 @@ __global__ void __launch_bounds__(256) gemm_narrow_kernel(GemmArgs a) {
         if (!live) continue;
         const int col = q < 2 ? t.col_lo + 4 * q : t.col_hi + 4 * q - 8;  // segment-local, 4 consecutive columns of one head
         const u32x2_t pk = {pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+        auto store = [&](bf16_t* dst) __attribute__((always_inline)) {
+            if (vec_io) {
+                *reinterpret_cast<u32x2_t*>(dst) = pk;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) dst[e] = (bf16_t)(pk[e >> 1] >> (16 * (e & 1)));
+            }
+        };
         if (t.seg == 0) {
-            *reinterpret_cast<u32x2_t*>((bf16_t*)a.q_out + (long)m * (a.Hq * a.D) + col) = pk;
+            store((bf16_t*)a.q_out + (long)m * (a.Hq * a.D) + col);
         } else {
             const int head = col / a.D, d = col % a.D;
             if (t.seg == 1) {
-                *reinterpret_cast<u32x2_t*>((bf16_t*)a.k_cache + (((long)b * a.Hkv + head) * a.t_max + a.tok_offset + s) * a.D + d) = pk;
+                store((bf16_t*)a.k_cache + (((long)b * a.Hkv + head) * a.t_max + a.tok_offset + s) * a.D + d);
             } else {
                 bf16_t* vt = (bf16_t*)a.vt_cache + (((long)b * a.Hkv + head) * a.D + d) * (long)a.t_max + a.tok_offset + s;
 #pragma unroll
@@ -2550,7 +2571,8 @@ int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
         // few bf16 rows (the suffix of one or a few observations through a projection): narrow tiles over the whole chip
         bool rows_ok = a.M <= tuning().gemm_rows_max && a.K % 8 == 0 && a.K >= 64 && tuning().gemm_tile < 0 && tuning().gemm_dl != 0 &&
                        (uintptr_t)a.A % 16 == 0 && (uintptr_t)a.W % 16 == 0 && !(a.colsum && a.norm_eps < 0.f) && !a.stats_out && !a.stats_in;
-        if (kEpi == EPI_QKV) rows_ok = rows_ok && a.D % 16 == 0 && a.N % 16 == 0;  // 8 + 8 columns of one head
+        if (kEpi == EPI_QKV)  // 8 + 8 columns of one head, rotation tables read 16 bytes at a time
+            rows_ok = rows_ok && a.D % 16 == 0 && a.N % 16 == 0 && (((uintptr_t)a.cos_t | (uintptr_t)a.sin_t) & 15) == 0;
         if (kEpi == EPI_PLAIN) rows_ok = rows_ok && a.norm_eps < 0.f;
         if (a.norm_eps >= 0.f) rows_ok = rows_ok && a.K % 16 == 0;  // what the tiled kernel takes with a norm inside, at every number of rows
         const int plan = rows_ok ? narrow_plan(a) : -1;
