@@ -1,0 +1,41 @@
+"""The kernels' routing rules on sizes (csrc/tile_rules.h), over their whole range, on the host."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+from util import ROOT
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    d = tmp_path_factory.mktemp("rules")
+    src, so = str(d / "rules.cpp"), str(d / "rules.so")
+    with open(src, "w") as f:
+        f.write('''#include "tile_rules.h"
+extern "C" int plan(int M, int N) { return vla_rules::narrow_plan(M, N); }
+extern "C" int rows(int p) { return 16 * vla_rules::NARROW_PLANS[p][0]; }
+extern "C" int cols(int p) { return 16 * vla_rules::NARROW_PLANS[p][1]; }
+''')
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", "-I", os.path.join(ROOT, "vla.cpp_amd", "csrc"), src, "-o", so],
+                   check=True)
+    return ctypes.CDLL(so)
+
+
+# 16-column steps up to the widest model, then wider
+WIDTHS = list(range(16, 8449, 16)) + [12288, 16384, 32768, 151936]
+
+
+def test_no_xcd_gets_more_narrow_tiles_of_64_x_32_than_it_has_cus(rules):
+    """A CU holds one workgroup of that size (96 KiB of LDS each) and an XCD has 32 CUs; the column groups are
+    dealt out over eight XCDs, each with all of its row groups."""
+    taken = 0
+    for M in range(65, 513):
+        for N in WIDTHS:
+            p = rules.plan(M, N)
+            if p >= 0 and (rules.rows(p), rules.cols(p)) == (64, 32):
+                taken += 1
+                groups = -(-N // 32)
+                assert -(-groups // 8) * -(-M // 64) <= 32, (M, N)
+    assert taken > 10000

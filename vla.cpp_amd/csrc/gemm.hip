@@ -28,6 +28,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "tile_rules.h"
 #include "vla_kernels.h"
 
 namespace {
@@ -2462,46 +2463,21 @@ void launch_dl(GemmArgs a, hipStream_t st) {
     gemm_dl_kernel<kEpi, TM, TN, KB, NS, NORM_NONE><<<grid, 256, 0, st>>>(a);
 }
 
-// Row blocks and column tiles per workgroup of the narrow-tile kernel: the split with the least
-// operand traffic per CU among those whose workgroups are all on the chip at once.  A column
-// tile (weights, from memory) weighs 2.2 times a row block (activations, from the L2): the
-// ratio under which the rule picks the fastest split on the models' shapes at batch 1.  Without
-// such a split the tiled kernel is the faster one -- 98 rows through 4608 x 1536: 288 narrow
-// workgroups 14.0 us, tiled 11.0; 147 rows through 1536 x 6144: 144 workgroups 17.0, tiled 23.0 --
-// and -1 is returned.
-constexpr int NARROW_PLANS[4][2] = {{1, 1}, {2, 1}, {4, 1}, {4, 2}};
-inline long narrow_wgs(const GemmArgs& a, int p) {
-    const int rb = NARROW_PLANS[p][0], nb = NARROW_PLANS[p][1], n_t16 = (a.N + 15) / 16;
-    return (long)((n_t16 + nb - 1) / nb) * ((a.M + 16 * rb - 1) / (16 * rb));
-}
+// rows x columns per workgroup, or -1 for the tiled kernel
 int narrow_plan(const GemmArgs& a) {
     const int force = tuning().gemm_rows_plan;
-    if (force > 0 && force <= 4) return force - 1;
-    int p = -1, best = 1 << 30;
-    for (int i = 0; i < 4; ++i) {
-        const int rb = NARROW_PLANS[i][0], nb = NARROW_PLANS[i][1];
-        if (rb > 1 && (rb / 2) * 16 >= a.M) continue;  // a smaller block holds every row
-        const int cost = 5 * rb + 11 * nb;
-        if (narrow_wgs(a, i) <= 256 && cost < best) {
-            best = cost;
-            p = i;
-        }
-    }
-    // more columns than one round holds: still this kernel where a single row block takes every row
-    return p < 0 && a.M <= 64 ? (a.M <= 16 ? 0 : a.M <= 32 ? 1 : 3) : p;
+    return force > 0 && force <= 4 ? force - 1 : vla_rules::narrow_plan(a.M, a.N);
 }
 
 template <int kEpi, int kNorm>
 void launch_narrow(const GemmArgs& a, int p, hipStream_t st) {
-    const int rb = NARROW_PLANS[p][0], nb = NARROW_PLANS[p][1];
-    const int n_rg = (a.M + 16 * rb - 1) / (16 * rb), n_cg = ((a.N + 15) / 16 + nb - 1) / nb;
-    const unsigned grid = (unsigned)((n_cg + 7) / 8 * 8 * n_rg);
+    const unsigned grid = (unsigned)vla_rules::narrow_grid(a.M, a.N, p);
     // Ring depths: more stages only delay the first one, fewer leave a CU short of requests; with
     // more workgroups than CUs two of them share a CU's LDS and its requests.
     switch (p) {
         case 0: gemm_narrow_kernel<kEpi, kNorm, 1, 1, 6><<<grid, 256, 0, st>>>(a); break;
         case 1:
-            if (narrow_wgs(a, 1) > 256) gemm_narrow_kernel<kEpi, kNorm, 2, 1, 4><<<grid, 256, 0, st>>>(a);
+            if (vla_rules::narrow_wgs(a.M, a.N, 1) > 256) gemm_narrow_kernel<kEpi, kNorm, 2, 1, 4><<<grid, 256, 0, st>>>(a);
             else gemm_narrow_kernel<kEpi, kNorm, 2, 1, 6><<<grid, 256, 0, st>>>(a);
             break;
         case 2: gemm_narrow_kernel<kEpi, kNorm, 4, 1, 4><<<grid, 256, 0, st>>>(a); break;
