@@ -39,3 +39,11 @@ def test_no_xcd_gets_more_narrow_tiles_of_64_x_32_than_it_has_cus(rules):
                 groups = -(-N // 32)
                 assert -(-groups // 8) * -(-M // 64) <= 32, (M, N)
     assert taken > 10000
+
+
+def test_narrow_tiles_of_more_columns_than_one_round_only_up_to_32_rows(rules):
+    """Beyond, a workgroup of the 64-row tiles fills a CU and the columns would take several rounds."""
+    for N in WIDTHS:
+        if N > 8192:
+            assert all(rules.plan(M, N) >= 0 for M in range(1, 33)), N
+            assert all(rules.plan(M, N) < 0 for M in range(33, 513)), N

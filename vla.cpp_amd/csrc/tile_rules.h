@@ -35,8 +35,10 @@ inline int narrow_plan(int M, int N) {
             p = i;
         }
     }
-    // more columns than one round holds: still this kernel where a single row block takes every row
-    return p < 0 && M <= 64 ? (M <= 16 ? 0 : M <= 32 ? 1 : 3) : p;
+    // More columns than one round holds: still this kernel up to 32 rows, where several of its workgroups share a CU (16
+    // rows through 12288 x 1024 7.8 us, tiled 10.4).  From 33 rows on one fills a CU: 50 rows through 16384 x 1024, gated,
+    // 12.7 us, tiled 11.6.
+    return p < 0 && M <= 32 ? (M <= 16 ? 0 : 1) : p;
 }
 
 }  // namespace vla_rules
