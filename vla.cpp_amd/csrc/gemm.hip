@@ -2464,9 +2464,9 @@ void launch_dl(GemmArgs a, hipStream_t st) {
 }
 
 // rows x columns per workgroup, or -1 for the tiled kernel
-int narrow_plan(const GemmArgs& a) {
+int narrow_plan(const GemmArgs& a, bool qkv) {
     const int force = tuning().gemm_rows_plan;
-    return force > 0 && force <= 4 ? force - 1 : vla_rules::narrow_plan(a.M, a.N);
+    return force > 0 && force <= 4 ? force - 1 : vla_rules::narrow_plan(a.M, a.N, a.K, qkv);
 }
 
 template <int kEpi, int kNorm>
@@ -2551,7 +2551,7 @@ int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
             rows_ok = rows_ok && a.D % 16 == 0 && a.N % 16 == 0 && (((uintptr_t)a.cos_t | (uintptr_t)a.sin_t) & 15) == 0;
         if (kEpi == EPI_PLAIN) rows_ok = rows_ok && a.norm_eps < 0.f;
         if (a.norm_eps >= 0.f) rows_ok = rows_ok && a.K % 16 == 0;  // what the tiled kernel takes with a norm inside, at every number of rows
-        const int plan = rows_ok ? narrow_plan(a) : -1;
+        const int plan = rows_ok ? narrow_plan(a, kEpi == EPI_QKV) : -1;
         if (plan >= 0) {
             if (a.norm_eps < 0.f) launch_narrow<kEpi, NORM_NONE>(a, plan, st);
             else if constexpr (kEpi == EPI_QKV) {

@@ -21,11 +21,14 @@ inline long narrow_grid(int M, int N, int p) { return (long)((narrow_col_groups(
 // such a split the tiled kernel is the faster one -- 98 rows through 4608 x 1536: 288 narrow
 // workgroups 14.0 us, tiled 11.0; 147 rows through 1536 x 6144: 144 workgroups 17.0, tiled 23.0 --
 // and -1 is returned.
-inline int narrow_plan(int M, int N) {
+inline int narrow_plan(int M, int N, int K, bool qkv) {
     int p = -1, best = 1 << 30;
     for (int i = 0; i < 4; ++i) {
         const int rb = NARROW_PLANS[i][0], nb = NARROW_PLANS[i][1];
         if (rb > 1 && (rb / 2) * 16 >= M) continue;  // a smaller block holds every row
+        // The QKV epilogue of 64 x 32 tiles (rotation, scatter) outweighs what so short a K saves: 64 rows of 6144 x 64 with the
+        // norm inside 5.0 us, tiled 4.4; from K = 256 on the two are level or this one is ahead.
+        if (qkv && i == 3 && K < 256) continue;
         const int cost = 5 * rb + 11 * nb;
         // The 96 KiB ring of 64 x 32 tiles leaves a CU to one workgroup: the 33rd on an XCD waits for a whole round.  300 rows
         // through 1600 x 720 with the norm inside: 250 workgroups, 35 on the busiest XCD, 10.2 us; tiled 6.9.
