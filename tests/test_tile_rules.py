@@ -15,6 +15,7 @@ def rules(tmp_path_factory):
     with open(src, "w") as f:
         f.write('''#include "tile_rules.h"
 extern "C" int plan(int M, int N, int K, int qkv) { return vla_rules::narrow_plan(M, N, K, qkv); }
+extern "C" int ternary(int M, int N, int K) { return vla_rules::ternary_tile(M, N, K); }
 extern "C" int rows(int p) { return 16 * vla_rules::NARROW_PLANS[p][0]; }
 extern "C" int cols(int p) { return 16 * vla_rules::NARROW_PLANS[p][1]; }
 ''')
@@ -57,3 +58,32 @@ def test_short_fused_qkv_projections_stay_off_64_x_32_tiles(rules):
             long_k, short_k = rules.plan(M, N, 256, 1), rules.plan(M, N, 128, 1)
             assert long_k == rules.plan(M, N, 128, 0)
             assert short_k == (-1 if long_k == 3 else long_k), (M, N)
+
+
+# M, N, K -> measured us on the tiles 16 (128 x 256), 17 (128 x 128), 18 (64 x 128), 19 (64 x 64), 20 (64 x 256), 21 (32 x 64)
+TERNARY_US = [
+    ((2048, 3840, 2560), (21.8, 22.1, 25.7, 32.1, 22.6, 37.0)),
+    ((2048, 2560, 6912), (43.9, 44.0, 45.2, 46.8, 49.4, 58.2)),
+    ((3000, 2560, 2560), (21.7, 22.3, 25.9, 32.1, 22.8, 37.3)),
+    ((4096, 3840, 2560), (33.0, 41.0, 48.0, 58.7, 43.3, 69.6)),
+    ((4664, 13824, 2560), (132.7, 159.4, 184.2, 234.8, 155.7, 275.2)),
+    ((512, 2560, 2560), (20.8, 15.6, 10.8, 9.2, 16.2, 10.3)),
+    ((583, 13824, 2560), (31.4, 32.9, 31.5, 36.4, 33.7, 41.2)),
+    ((583, 2560, 6912), (42.7, 31.8, 22.2, 18.0, 34.3, 28.1)),
+    ((1024, 3840, 2560), (21.0, 16.0, 14.3, 17.7, 16.7, 21.6)),
+    ((64, 640, 2560), (20.4, 15.3, 10.5, 7.8, 16.1, 6.9)),
+    ((300, 4096, 4096), (28.3, 21.0, 14.6, 11.9, 22.6, 13.7)),
+    ((4096, 512, 512), (10.1, 8.0, 5.8, 5.2, 7.7, 6.3)),
+    ((1500, 8192, 1024), (17.8, 19.4, 20.5, 26.7, 19.3, 31.4)),
+]
+
+
+@pytest.mark.parametrize("shape,us", TERNARY_US)
+def test_ternary_tile_is_near_the_fastest_and_not_slower_than_the_large_tiles(rules, shape, us):
+    """Within the prediction's error (4 %) of the fastest tile, and 128 x 256 tiles, where they fill half the
+    chip, are left only for a faster one (2 %: two runs of one tile)."""
+    M, N, K = shape
+    took = us[rules.ternary(M, N, K) - 16]
+    assert took <= 1.04 * min(us)
+    if -(-M // 128) * -(-N // 256) >= 128:
+        assert took <= 1.02 * us[0]

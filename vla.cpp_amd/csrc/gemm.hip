@@ -2508,28 +2508,6 @@ bool launch_x16(GemmArgs a, hipStream_t st) {
     return grid != 0;
 }
 
-// Tile of a ternary GEMM (VLA_TERNARY_TILE codes) by predicted time: a launch costs `fixed`, and
-// `step` per 128 k while every workgroup has a CU of its own; up to two workgroups per CU
-// overlap to `two` steps, beyond that a step takes `more` times the workgroups per CU.  The
-// constants (us) are a fit to 75 measured shapes (40 to 4096 rows; N 640, 2560, 3840, 13824; K
-// 2560, 6912): the tile it picks is within 4 % of the fastest of the six on each of them.
-int ternary_tile(long M, long N, long K) {
-    const struct { int tile, rows, cols; double fixed, step, two, more; } t[] = {
-        {21, 32, 64, 3.23, 0.170, 1.48, 0.88},   {19, 64, 64, 3.35, 0.224, 1.32, 1.04},   {18, 64, 128, 4.55, 0.311, 1.56, 1.00},
-        {17, 128, 128, 6.09, 0.490, 1.65, 1.04}, {20, 64, 256, 5.30, 0.546, 1.53, 0.97}, {16, 128, 256, 6.79, 0.762, 1.36, 1.13}};
-    int best = 16;
-    double least = 1e30;
-    for (const auto& x : t) {
-        const double r = (double)(((M + x.rows - 1) / x.rows) * ((N + x.cols - 1) / x.cols)) / 256.0;
-        const double us = x.fixed + K / 128 * x.step * (r <= 1 ? 1.0 : r <= 2 ? x.two : (x.more * r > x.two ? x.more * r : x.two));
-        if (us < least) {
-            least = us;
-            best = x.tile;
-        }
-    }
-    return best;
-}
-
 template <typename T, int kEpi>
 int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
     if (a.M == 0 || n_tiles == 0) return VLA_K_OK;
@@ -2662,7 +2640,7 @@ int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
             done = true;
         } else if (x16_ok && x16_asked && (ring_ok || force == 16 || wg128 >= 128)) {
             // the 16x16x64 kernels
-            switch (!ring_ok ? 16 : force ? force : ternary_tile(a.M, a.N, a.K)) {
+            switch (!ring_ok ? 16 : force ? force : vla_rules::ternary_tile(a.M, a.N, a.K)) {
                 case 17: done = launch_ring<4, 4, 4>(a, st); break;
                 case 18: done = launch_ring<2, 4, 5>(a, st); break;
                 case 19: done = launch_ring<2, 2, 6>(a, st); break;

@@ -44,4 +44,30 @@ inline int narrow_plan(int M, int N, int K, bool qkv) {
     return p < 0 && M <= 32 ? (M <= 16 ? 0 : 1) : p;
 }
 
+// Tile of a ternary GEMM (VLA_TERNARY_TILE codes) by predicted time: a launch costs `fixed`, and
+// `step` per 128 k while every workgroup has a CU of its own; up to two workgroups per CU
+// overlap to `two` steps, beyond that a step takes `more` times the workgroups per CU.  The
+// constants (us) are a fit to 75 measured shapes (40 to 4096 rows; N 640, 2560, 3840, 13824; K
+// 2560, 6912).  On 234 shapes (33 to 4664 rows; N 256 to 32000; K 512 to 16384) the picked tile is within
+// 4 % of the fastest of the six on 227 and within 11 % on all.  The prediction's error is a few per cent, so
+// that 128 x 256 tiles, where they fill half the chip, give way only to a tile predicted 4 % faster: 2048 x
+// 2560 x 6912 45.4 -> 44.0 us, 2048 x 3840 x 2560 22.6 -> 21.9 (64 x 128 and 64 x 256 tiles without the margin).
+inline int ternary_tile(long M, long N, long K) {
+    const struct { int tile, rows, cols; double fixed, step, two, more; } t[] = {
+        {21, 32, 64, 3.23, 0.170, 1.48, 0.88},   {19, 64, 64, 3.35, 0.224, 1.32, 1.04},   {18, 64, 128, 4.55, 0.311, 1.56, 1.00},
+        {17, 128, 128, 6.09, 0.490, 1.65, 1.04}, {20, 64, 256, 5.30, 0.546, 1.53, 0.97}, {16, 128, 256, 6.79, 0.762, 1.36, 1.13}};
+    int best = 16;
+    double least = 1e30;
+    for (const auto& x : t) {
+        const double r = (double)(((M + x.rows - 1) / x.rows) * ((N + x.cols - 1) / x.cols)) / 256.0;
+        const double us = x.fixed + K / 128 * x.step * (r <= 1 ? 1.0 : r <= 2 ? x.two : (x.more * r > x.two ? x.more * r : x.two));
+        const double margin = x.tile == 16 && r >= 0.5 ? 0.96 : 1.0;
+        if (us * margin < least) {
+            least = us * margin;
+            best = x.tile;
+        }
+    }
+    return best;
+}
+
 }  // namespace vla_rules
