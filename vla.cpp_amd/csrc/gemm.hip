@@ -1071,7 +1071,7 @@ template <int kEpi, int kNorm, int RB, int NB, int NS>  // RB: 16-row blocks, NB
 __global__ void __launch_bounds__(256) gemm_narrow_kernel(GemmArgs a) {
     constexpr int KB = 256, BK = 128, STAGE = (RB + NB) * 16 * KB, NLOAD = RB + NB;
     constexpr int IN_FLIGHT = (NS - 2) * NLOAD;
-    constexpr int MY_NB = RB == 4 ? NB : 1;  // 16-column tiles per wavefront
+    static_assert(NB == 1 || RB == 4, "a wavefront per row block; fewer than four repeat each other's products");
     static_assert(IN_FLIGHT <= 63, "ring depth exceeds the vector-memory counter");
     __shared__ __attribute__((aligned(1024))) unsigned char lds[NS * STAGE];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1108,27 +1108,26 @@ __global__ void __launch_bounds__(256) gemm_narrow_kernel(GemmArgs a) {
     for (int t = 0; t < NS - 1; ++t)
         if (t < nkt) issue(t, t);  // uniform
 
-    // wavefront -> row block, first column tile
-    const bool active = RB * NB >= 4 || wave < RB * NB;
-    const int rb = RB == 4 ? wave : RB == 2 ? (NB == 2 ? wave >> 1 : wave & 1) : 0;
-    const int nb0 = RB == 4 ? 0 : NB == 2 ? wave & 1 : 0;
-    f32x4_t acc[MY_NB];
+    // wavefront -> row block; each multiplies it with all NB column tiles
+    const bool active = wave < RB;
+    const int rb = wave % RB;
+    f32x4_t acc[NB];
 #pragma unroll
-    for (int j = 0; j < MY_NB; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < NB; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     // Row sums for the norm, in the tiled kernels' order: lane (c, q) sums its piece of every 32
     // k with one accumulator per word; the pairs q, q ^ 1 are those kernels' two lane halves, the
     // pairs q, q ^ 2 their two wavefronts.
     float ssq[4] = {0.f, 0.f, 0.f, 0.f}, ssum[4] = {0.f, 0.f, 0.f, 0.f};
-    const int fx0 = (rb * 16 + c) * KB, fw0 = ((RB + nb0) * 16 + c) * KB;
+    const int fx0 = (rb * 16 + c) * KB, fw0 = (RB * 16 + c) * KB;
     auto multiply = [&](int stage, int k_left) __attribute__((always_inline)) {  // k_left: k of this tile inside K (the partial last tile), or BK
         const unsigned char* base = lds + stage * STAGE;
-        u32x4_t fx[4], fw[4][MY_NB];
+        u32x4_t fx[4], fw[4][NB];
 #pragma unroll
         for (int ch = 0; ch < 4; ++ch) {
             const int off = ((4 * ch + q) ^ c) * 16;
             fx[ch] = *reinterpret_cast<const u32x4_t*>(base + fx0 + off);
 #pragma unroll
-            for (int j = 0; j < MY_NB; ++j) fw[ch][j] = *reinterpret_cast<const u32x4_t*>(base + fw0 + j * 16 * KB + off);
+            for (int j = 0; j < NB; ++j) fw[ch][j] = *reinterpret_cast<const u32x4_t*>(base + fw0 + j * 16 * KB + off);
         }
         if (k_left < BK) {  // K is a multiple of 8: a piece is inside or outside as a whole
             const u32x4_t z = {0u, 0u, 0u, 0u};
@@ -1137,14 +1136,14 @@ __global__ void __launch_bounds__(256) gemm_narrow_kernel(GemmArgs a) {
                 if (ch * 32 + 8 * q >= k_left) {
                     fx[ch] = z;
 #pragma unroll
-                    for (int j = 0; j < MY_NB; ++j) fw[ch][j] = z;
+                    for (int j = 0; j < NB; ++j) fw[ch][j] = z;
                 }
         }
         __builtin_amdgcn_sched_barrier(0);  // all reads requested before the first product: left alone they are spread for fewer registers
 #pragma unroll
         for (int ch = 0; ch < 4; ++ch) {
 #pragma unroll
-            for (int j = 0; j < MY_NB; ++j)
+            for (int j = 0; j < NB; ++j)
                 acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, fw[ch][j]), __builtin_bit_cast(bf16x8_t, fx[ch]),
                                                                  acc[j], 0, 0, 0);
             if (kNorm) {
@@ -1194,9 +1193,9 @@ __global__ void __launch_bounds__(256) gemm_narrow_kernel(GemmArgs a) {
     const bool vec_io = (io & (kEpi == EPI_QKV || a.out_bf16 ? 7 : 15)) == 0;
     const int m = m0 + rb * 16 + c;
 #pragma unroll
-    for (int j = 0; j < MY_NB; ++j) {
-        const RowCols& t = rc[nb0 + j];
-        const bool live = m < a.M && tg * NB + nb0 + j < n_t16;
+    for (int j = 0; j < NB; ++j) {
+        const RowCols& t = rc[j];
+        const bool live = m < a.M && tg * NB + j < n_t16;
         const int n0 = q < 2 ? t.base_lo + 4 * q : t.base_hi + 4 * q - 8;  // W row (= bias, column-sum index) of v[0]
         float v[4];
 #pragma unroll
