@@ -1067,7 +1067,8 @@ __device__ __forceinline__ void narrow_tail(int nkt, Body body) {
     if constexpr (LEFT > 1) narrow_tail<LEFT - 1, NLOAD>(nkt, body);
 }
 
-template <int kEpi, int kNorm, int RB, int NB, int NS>  // RB: 16-row blocks, NB: 16-column tiles per workgroup
+// RB: 16-row blocks, NB: 16-column tiles per workgroup; VEC: outputs and residual four columns at a time, else one by one
+template <int kEpi, int kNorm, int RB, int NB, int NS, bool VEC = true>
 __global__ void __launch_bounds__(256) gemm_narrow_kernel(GemmArgs a) {
     constexpr int KB = 256, BK = 128, STAGE = (RB + NB) * 16 * KB, NLOAD = RB + NB;
     constexpr int IN_FLIGHT = (NS - 2) * NLOAD;
@@ -1187,10 +1188,6 @@ __global__ void __launch_bounds__(256) gemm_narrow_kernel(GemmArgs a) {
             f = rsqrtf(sq * inv_k + a.norm_eps);
         }
     }
-    // Four columns at a time where the output's and residual's addresses allow it (uniform), else one by one; the
-    // operands' and rotation tables' addresses are checked by the launcher.
-    const uintptr_t io = kEpi == EPI_QKV ? (uintptr_t)a.q_out | (uintptr_t)a.k_cache : (uintptr_t)a.Y | (uintptr_t)a.residual;
-    const bool vec_io = (io & (kEpi == EPI_QKV || a.out_bf16 ? 7 : 15)) == 0;
     const int m = m0 + rb * 16 + c;
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
@@ -1222,7 +1219,7 @@ __global__ void __launch_bounds__(256) gemm_narrow_kernel(GemmArgs a) {
             }
             if (!live) continue;
             const long o = (long)m * a.N + n0;
-            if (a.N % 4 == 0 && vec_io) {  // 4 consecutive columns are inside the row or outside as a whole
+            if (VEC && a.N % 4 == 0) {  // 4 consecutive columns are inside the row or outside as a whole
                 if (n0 >= a.N) continue;
                 if (a.out_bf16) {
                     if (a.residual) {
@@ -1267,7 +1264,7 @@ __global__ void __launch_bounds__(256) gemm_narrow_kernel(GemmArgs a) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) y[e] = apply_act(v[e], a.act) * other[e];
             const long o = (long)m * (a.N / 2) + n0;
-            if (!vec_io) {
+            if (!VEC) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     if (a.out_bf16) ((bf16_t*)a.Y)[o + e] = f2bf(y[e]);
@@ -1296,7 +1293,7 @@ __global__ void __launch_bounds__(256) gemm_narrow_kernel(GemmArgs a) {
         const int col = q < 2 ? t.col_lo + 4 * q : t.col_hi + 4 * q - 8;  // segment-local, 4 consecutive columns of one head
         const u32x2_t pk = {pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
         auto store = [&](bf16_t* dst) __attribute__((always_inline)) {
-            if (vec_io) {
+            if (VEC) {
                 *reinterpret_cast<u32x2_t*>(dst) = pk;
             } else {
 #pragma unroll
@@ -2470,6 +2467,13 @@ int narrow_plan(const GemmArgs& a, bool qkv) {
 
 template <int kEpi, int kNorm>
 void launch_narrow(const GemmArgs& a, int p, hipStream_t st) {
+    // Outputs or a residual that four columns at a time would not hit aligned: a form of its own (a branch in the others'
+    // epilogues costs 0.05 us of a launch of 5).  The caller checks the operands and the rotation tables.
+    const uintptr_t io = kEpi == EPI_QKV ? (uintptr_t)a.q_out | (uintptr_t)a.k_cache : (uintptr_t)a.Y | (uintptr_t)a.residual;
+    if (io & (kEpi == EPI_QKV || a.out_bf16 ? 7 : 15)) {
+        gemm_narrow_kernel<kEpi, kNorm, 1, 1, 6, false><<<(unsigned)vla_rules::narrow_grid(a.M, a.N, 0), 256, 0, st>>>(a);
+        return;
+    }
     const unsigned grid = (unsigned)vla_rules::narrow_grid(a.M, a.N, p);
     // Ring depths: more stages only delay the first one, fewer leave a CU short of requests; with
     // more workgroups than CUs two of them share a CU's LDS and its requests.
