@@ -427,7 +427,8 @@ VLA_KAPI int vla_ternary_repack_ladder_host(const uint8_t* ladder, int N, int K,
  * acc = sum_k A[m][k] * t[n][k] exact in int32
  * (ladder_int8xint2_kernel_m_wide, bitnet_kernels.h:285-409).  acc_out
  * (int32 [M][N]) receives the raw accumulators when not NULL; out may then be
- * NULL. */
+ * NULL.  The tiles for a few hundred rows ask for 16-byte aligned W_packed, out and
+ * residual; other addresses are served by slower ones. */
 VLA_KAPI int vla_ternary_gemm(const int8_t* A, const uint32_t* W_packed, uint16_t* out, int32_t* acc_out,
                               const float* s, const int32_t* rowsum, const float* ws, int ws_num, int M, int N,
                               int K, vla_stream_t stream);
