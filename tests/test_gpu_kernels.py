@@ -1821,14 +1821,15 @@ def test_narrow_tile_projection_of_unaligned_outputs(M, out):
     def run(n, n_tab):
         st, L, outs = pkg.stream(), pkg.lib(), []
         zero = lambda count, dt: off(torch.zeros(count, dtype=dt, device="cuda"), n)
-        (y, yp), (rb, rp), (g, gp) = zero(M * N, tdt), off(res, n), zero(M * N // 2, tdt)
+        (y, yp), (rb, rp), (g, gp), (z, zp) = zero(M * N, tdt), off(res, n), zero(M * N // 2, tdt), zero(M * (N - 1), tdt)
         pkg.check(L.vla_linear(x.data_ptr(), W.data_ptr(), None, rp, yp, BF16, out, M, N, K, st))
+        pkg.check(L.vla_linear(x.data_ptr(), W.data_ptr(), None, None, zp, BF16, out, M, N - 1, K, st))  # odd rows
         pkg.check(L.vla_glu_linear(x.data_ptr(), W.data_ptr(), None, gp, BF16, out, M, N // 2, K, pkg.VLA_ACT_SILU, -1.0, st))
         (cb, cp), (sb, sp) = off(dev(np.cos(ang)), n_tab), off(dev(np.sin(ang)), n_tab)
         (q, qp), (k, kp), (v, vp) = (zero(M * H * D, torch.bfloat16) for _ in range(3))
         pkg.check(L.vla_attn_qkv_rope(x.data_ptr(), W.data_ptr(), None, BF16, M, K, M, H, H, 1, 1, D, cp, sp, qp, kp, vp, M, 0, st))
         sync()
-        for buf in (y, g, q, k, v):
+        for buf in (y, z, g, q, k, v):
             assert torch.all(buf[:n] == 77) and torch.all(buf[buf.numel() - 8 + n:] == 77)
             outs.append(buf[n:buf.numel() - 8 + n])
         return outs

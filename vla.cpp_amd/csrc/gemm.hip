@@ -2473,7 +2473,7 @@ void launch_narrow(const GemmArgs& a, int p, hipStream_t st) {
     // Outputs or a residual that four columns at a time would not hit aligned: a form of its own (a branch in the others'
     // epilogues costs 0.05 us of a launch of 5).  The caller checks the operands and the rotation tables.
     const uintptr_t io = kEpi == EPI_QKV ? (uintptr_t)a.q_out | (uintptr_t)a.k_cache : (uintptr_t)a.Y | (uintptr_t)a.residual;
-    if (io & (kEpi == EPI_QKV || a.out_bf16 ? 7 : 15)) {
+    if ((kEpi != EPI_PLAIN || a.N % 4 == 0) && (io & (kEpi == EPI_QKV || a.out_bf16 ? 7 : 15))) {  // other N go one by one anyway
         gemm_narrow_kernel<kEpi, kNorm, 1, 1, 6, false><<<(unsigned)vla_rules::narrow_grid(a.M, a.N, 0), 256, 0, st>>>(a);
         return;
     }
