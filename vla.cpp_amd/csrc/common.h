@@ -304,6 +304,27 @@ __device__ __forceinline__ float apply_act(float x, int act) {
     return x;
 }
 
+// The same for values that are rounded to bf16 next, N at a time.  The exact division and tanhf above are some 25 and 45
+// instructions per value, and a 128 x 128 tile has 64 per thread: 1323 x 6144 x 1536 took 64.6 us with GELU and 52.8 without.  Here
+// 5 and 7 instructions (51.7 us; 408 rows 29.4 -> 20.3): the reciprocal is the hardware's (1 ulp), and GELU's tanh form is
+// written as the sigmoid it is, 0.5 x (1 + tanh u) = x / (1 + exp(-2 u)).  Against float64 over all bf16 x in (-8, 30): SiLU
+// 4.2e-7 of the value (as above), GELU 3.9e-6 (above: 1, where 1 + tanh u cancels), beside the 2^-8 of the rounding that follows.
+// The multiply-add is spelled out: every kernel gives the same bits.
+template <int N>
+__device__ __forceinline__ void apply_act_bf16(float (&v)[N], int act) {
+    if (act == VLA_ACT_SILU) {
+#pragma unroll
+        for (int e = 0; e < N; ++e) v[e] *= __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(v[e] * -1.44269504088896341f));
+    } else if (act == VLA_ACT_GELU) {
+        constexpr float k1 = -2.0f * 0.79788456080286535588f * 1.44269504088896341f, k3 = k1 * 0.044715f;
+#pragma unroll
+        for (int e = 0; e < N; ++e) v[e] *= __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(v[e] * fmaf(k3, v[e] * v[e], k1)));
+    } else if (act == VLA_ACT_RELU) {
+#pragma unroll
+        for (int e = 0; e < N; ++e) v[e] = v[e] > 0.f ? v[e] : 0.f;
+    }
+}
+
 // s_waitcnt on the vector-memory counter alone (vmcnt[3:0] in bits 3:0, vmcnt[5:4] in bits
 // 15:14; the export and LDS/scalar counter fields at their maxima, i.e. not waited on).
 template <int N>
