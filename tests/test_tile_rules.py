@@ -15,6 +15,7 @@ def rules(tmp_path_factory):
     with open(src, "w") as f:
         f.write('''#include "tile_rules.h"
 extern "C" int plan(int M, int N, int K, int qkv) { return vla_rules::narrow_plan(M, N, K, qkv); }
+extern "C" int plan_f32(int M, int N) { return vla_rules::narrow_plan_f32(M, N); }
 extern "C" int ternary(int M, int N, int K) { return vla_rules::ternary_tile(M, N, K); }
 extern "C" int rows(int p) { return 16 * vla_rules::NARROW_PLANS[p][0]; }
 extern "C" int cols(int p) { return 16 * vla_rules::NARROW_PLANS[p][1]; }
@@ -87,3 +88,14 @@ def test_ternary_tile_is_near_the_fastest_and_not_slower_than_the_large_tiles(ru
     assert took <= 1.04 * min(us)
     if -(-M // 128) * -(-N // 256) >= 128:
         assert took <= 1.02 * us[0]
+
+
+def test_fp32_narrow_tiles_of_more_than_one_round(rules):
+    """16 x 16 tiles up to one round of two per CU, up to four rounds where the 64-row tiles would repeat the
+    weights or waste rows, and always a narrow tile for up to 64 rows."""
+    for M in list(range(1, 130)) + [200, 300, 400, 512]:
+        for N in WIDTHS:
+            wgs, p = -(-M // 16) * (N // 16), rules.plan_f32(M, N)
+            if M <= 64:
+                assert p in (0, 2), (M, N)
+            assert (p == 0) == (wgs <= 512 or (wgs <= 2048 and not 32 < M <= 64)), (M, N)

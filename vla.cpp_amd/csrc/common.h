@@ -26,8 +26,8 @@ struct Tuning {
     bool attn_no_arrive = false; // VLA_ATTN_NO_ARRIVE: no in-launch merge by the last slice to arrive
     bool attn_no_direct = false; // VLA_ATTN_NO_DIRECT: never the register-direct kernel
     bool attn_no_stream = false; // VLA_ATTN_NO_STREAM: never the streaming (LDS-ring) form of the register-direct kernel
-    int gemm_rows_max = 512;     // VLA_GEMM_ROWS_MAX: bf16 projections of at most this many rows may take the narrow-tile kernel, 0 = never
-    int gemm_rows_plan = 0;      // VLA_GEMM_ROWS_PLAN: 1..4 pins that kernel's rows x columns per workgroup (16x16, 32x16, 64x16, 64x32), 0 = by shape
+    int gemm_rows_max = 512;     // VLA_GEMM_ROWS_MAX: projections of at most this many rows may take the narrow-tile kernels, 0 = never
+    int gemm_rows_plan = 0;      // VLA_GEMM_ROWS_PLAN: 1..4 pins those kernels' rows x columns per workgroup (16x16, 32x16, 64x16, 64x32; fp32: 1 and 3), 0 = by shape
     bool attn_no_small = false;  // VLA_ATTN_NO_SMALL: fp32 launches with few row tiles do not split their keys beyond the usual rule
     int attn_direct_rows = 32;   // VLA_ATTN_DIRECT_ROWS: row limit of the register-direct kernel
     int gemm_tile = -1;          // VLA_GEMM_TILE: 0..5

@@ -29,6 +29,7 @@
 
 #include "common.h"
 #include "gemm_common.h"
+#include "gemm_f32.h"
 #include "tile_rules.h"
 #include "vla_kernels.h"
 
@@ -607,64 +608,6 @@ __global__ void __launch_bounds__(256) gemm_dl_kernel(GemmArgs a) {
 // Against the tiled kernel (us, weights not in the caches): 16 rows x 1536 x 1536 7.9 -> 4.2, 50 x 720 x 2048
 // 9.3 -> 4.7, 50 x 4096 x 720 gated 7.0 -> 4.9, 50 x 1536 x 6144 28.4 -> 11.3.  At 2 to 5 TB/s out of the L2s such a
 // launch is mostly its fixed cost: start, first loads, epilogue.
-struct RowCols {
-    int base_lo, base_hi;  // rows of W of tile columns [0, 8) and [8, 16)
-    int seg;               // 0 Q, 1 K, 2 V (QKV mode)
-    int col_lo, col_hi;    // segment-local column of tile column 0 and of tile column 8
-    bool rope;
-};
-template <int kEpi>
-__device__ __forceinline__ RowCols row_cols(const GemmArgs& a, int t) {
-    RowCols rc;
-    rc.seg = 0;
-    rc.rope = false;
-    if (kEpi == EPI_GLU) {
-        rc.base_lo = rc.col_lo = t * 8;
-        rc.base_hi = rc.col_hi = a.N / 2 + t * 8;
-        return rc;
-    }
-    if (kEpi != EPI_QKV) {
-        rc.base_lo = rc.col_lo = t * 16;
-        rc.base_hi = rc.col_hi = t * 16 + 8;
-        return rc;
-    }
-    const int tq = a.Hq * a.D / 16, tk = a.nk * a.D / 16;
-    int lt = t, seg_base = 0;
-    if (t >= tq + tk) {
-        rc.seg = 2;
-        lt = t - tq - tk;
-        seg_base = (a.Hq + a.nk) * a.D;
-    } else if (t >= tq) {
-        rc.seg = 1;
-        lt = t - tq;
-        seg_base = a.Hq * a.D;
-    }
-    rc.rope = (a.cos_t != nullptr) && rc.seg != 2;
-    if (rc.rope) {
-        const int tph = a.D / 16;  // tiles per head
-        const int head = lt / tph, chunk = lt % tph;
-        rc.col_lo = head * a.D + chunk * 8;
-        rc.col_hi = rc.col_lo + a.D / 2;
-    } else {
-        rc.col_lo = lt * 16;
-        rc.col_hi = rc.col_lo + 8;
-    }
-    rc.base_lo = seg_base + rc.col_lo;
-    rc.base_hi = seg_base + rc.col_hi;
-    return rc;
-}
-
-// The last min(nkt, LEFT) tiles of the ring: with LEFT tiles in flight, the oldest has landed
-// when at most (LEFT - 1) NLOAD loads are still due.
-template <int LEFT, int NLOAD, typename Body>
-__device__ __forceinline__ void narrow_tail(int nkt, Body body) {
-    if (LEFT <= nkt) {  // uniform
-        wait_vmcnt<(LEFT - 1) * NLOAD>();
-        body(LEFT == 1);
-    }
-    if constexpr (LEFT > 1) narrow_tail<LEFT - 1, NLOAD>(nkt, body);
-}
-
 // RB: 16-row blocks, NB: 16-column tiles per workgroup; VEC: outputs and residual four columns at a time, else one by one
 template <int kEpi, int kNorm, int RB, int NB, int NS, bool VEC = true>
 __global__ void __launch_bounds__(256) gemm_narrow_kernel(GemmArgs a) {
@@ -1655,141 +1598,6 @@ __global__ void __launch_bounds__(256) ternary_gemm_ring_kernel(GemmArgs a) {
     }
 }
 
-// fp32 projection of a few rows (M <= 64: the suffix of one observation in the reference's
-// own fp32 case).  The fp32 MFMA gives a CU 256 flop per clock, no more than its plain FMA
-// rate, and the MFMA kernel's 64 x 64 tiles leave a 50 x 720 x 960 problem on 12 CUs that walk
-// K one after the other (22 us).  Here a wavefront owns 4 rows and 8 output columns and its
-// lanes share K: lane l sums k = 256 j + 4 l + (0..3), so a load instruction reads 1 KiB of
-// consecutive bytes of a row of x or W, K = 960 is four rounds of loads (two in flight at a
-// time), and a 50 x 720 problem is 1170 wavefronts.  The 64 partial sums of an output meet
-// through six xor-shuffles, in that order whatever the launch.  The 8 columns are two runs
-// of 4: next to each other for a plain projection, half a head apart where the QKV epilogue
-// rotates, so that lane ks < 16 ends up with both members of a rotation pair (row ks / 4 of
-// the four, columns ks % 4 of either run).
-constexpr int SKINNY_MAX_M = 64;
-template <int kEpi>
-__global__ void __launch_bounds__(256) linear_f32_skinny_kernel(GemmArgs a) {
-    const int tid = threadIdx.x, ks = tid & 63, rg = (tid >> 6) + 4 * blockIdx.y;
-    const int K = a.K;
-    // W rows of the two runs, and for QKV the segment and the segment-local columns
-    int base0 = blockIdx.x * 8, base1 = base0 + 4, seg = 0, col0 = base0, col1 = base1;
-    bool rope = false;
-    if (kEpi == EPI_QKV) {
-        const int gq = a.Hq * a.D / 8, gk = a.nk * a.D / 8;
-        int lt = blockIdx.x, seg_base = 0;
-        if (lt >= gq + gk) {
-            seg = 2;
-            lt -= gq + gk;
-            seg_base = (a.Hq + a.nk) * a.D;
-        } else if (lt >= gq) {
-            seg = 1;
-            lt -= gq;
-            seg_base = a.Hq * a.D;
-        }
-        rope = a.cos_t != nullptr && seg != 2;
-        if (rope) {
-            const int gph = a.D / 8;  // groups per head
-            col0 = (lt / gph) * a.D + (lt % gph) * 4;
-            col1 = col0 + a.D / 2;
-        } else {
-            col0 = lt * 8;
-            col1 = col0 + 4;
-        }
-        base0 = seg_base + col0;
-        base1 = seg_base + col1;
-    }
-    const float* xr[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) xr[i] = (const float*)a.A + (long)min(4 * rg + i, a.M - 1) * K;
-    const float* wr[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) wr[c] = (const float*)a.W + (long)min((c < 4 ? base0 : base1 - 4) + c, a.N - 1) * K;
-    float acc[4][8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int c = 0; c < 8; ++c) acc[i][c] = 0.f;
-    if (4 * rg < a.M) {  // whole wavefronts
-#pragma unroll 2
-        for (int k = 4 * ks; k < K; k += 256) {
-            f32x4_t xv[4], wv[8];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) xv[i] = *reinterpret_cast<const f32x4_t*>(xr[i] + k);
-#pragma unroll
-            for (int c = 0; c < 8; ++c) wv[c] = *reinterpret_cast<const f32x4_t*>(wr[c] + k);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int c = 0; c < 8; ++c)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[i][c] = fmaf(xv[i][e], wv[c][e], acc[i][c]);
-        }
-    }
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int c = 0; c < 8; ++c) acc[i][c] += __shfl_xor(acc[i][c], off, 64);
-    if (ks >= 16) return;
-    float lo = 0.f, hi = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int cp = 0; cp < 4; ++cp)
-            if (ks == i * 4 + cp) {
-                lo = acc[i][cp];
-                hi = acc[i][cp + 4];
-            }
-    const int m = 4 * rg + (ks >> 2), cp = ks & 3;
-    if (m >= a.M) return;
-    if (kEpi == EPI_PLAIN) {
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const int n = (e ? base1 : base0) + cp;
-            if (n >= a.N) continue;
-            float y = e ? hi : lo;
-            if (a.bias) y += a.bias[n];
-            if (a.act != VLA_ACT_NONE) y = apply_act(y, a.act);
-            if (a.col_gate) y *= a.col_gate[n];
-            const long o = (long)m * a.N + n;
-            if (a.out_bf16) {
-                if (a.residual) y += bf2f(((const bf16_t*)a.residual)[o]);
-                ((bf16_t*)a.Y)[o] = f2bf(y);
-            } else {
-                if (a.residual) y += ((const float*)a.residual)[o];
-                ((float*)a.Y)[o] = y;
-            }
-        }
-        return;
-    }
-    // QKV: bias, rotation, scatter (the MFMA kernel's epilogue, two columns per lane)
-    const int b = m / a.S, sq = m % a.S;
-    if (a.bias) {
-        lo += a.bias[base0 + cp];
-        hi += a.bias[base1 + cp];
-    }
-    if (rope) {
-        const int half = a.D >> 1, p0 = (col0 % a.D) + cp;
-        const float c = a.cos_t[(long)sq * half + p0], sn = a.sin_t[(long)sq * half + p0];
-        const float x0 = lo, x1 = hi;
-        lo = x0 * c - x1 * sn;
-        hi = x1 * c + x0 * sn;
-    }
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-        const float v = e ? hi : lo;
-        const int col = (e ? col1 : col0) + cp;
-        if (seg == 0) {
-            ((float*)a.q_out)[(long)m * (a.Hq * a.D) + col] = v;
-        } else {
-            const int head = col / a.D, d = col % a.D;
-            if (seg == 1) ((float*)a.k_cache)[(((long)b * a.Hkv + head) * a.t_max + a.tok_offset + sq) * a.D + d] = v;
-            else ((float*)a.vt_cache)[(((long)b * a.Hkv + head) * a.D + d) * a.t_max + a.tok_offset + sq] = v;
-        }
-    }
-}
-
 // Ternary GEMV for a handful of rows (single-token decode, M <= 32).  A workgroup owns 32
 // output columns; its 8 wavefronts each take one eighth of K and multiply it with
 // v_mfma_i32_32x32x32_i8 as C[n][m] = sum_k W[n][k] * A[m][k] (weight fragment as the A
@@ -2065,11 +1873,13 @@ int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
     if (a.M == 0 || n_tiles == 0) return VLA_K_OK;
     a.n_tiles = n_tiles;
     hipStream_t st = (hipStream_t)stream;
-    if constexpr (std::is_same<T, float>::value && (kEpi == EPI_PLAIN || kEpi == EPI_QKV)) {
-        // a few fp32 rows: the FMA kernel (VLA_GEMM_TILE pins the MFMA kernel's tiles instead)
-        if (a.M <= SKINNY_MAX_M && a.K % 4 == 0 && a.norm_eps < 0.f && tuning().gemm_tile < 0 && (uintptr_t)a.A % 16 == 0 &&
-            (uintptr_t)a.W % 16 == 0 && (kEpi == EPI_PLAIN || a.D % 8 == 0)) {
-            linear_f32_skinny_kernel<kEpi><<<dim3((unsigned)((a.N + 7) / 8), (unsigned)((a.M + 15) / 16)), 256, 0, st>>>(a);
+    if constexpr (std::is_same<T, float>::value) {
+        // a few fp32 rows: narrow tiles (VLA_GEMM_TILE pins the tiled kernel instead)
+        bool rows_ok = a.M <= tuning().gemm_rows_max && a.norm_eps < 0.f && tuning().gemm_tile < 0 && ((uintptr_t)a.A | (uintptr_t)a.W) % 16 == 0;
+        const int force = tuning().gemm_rows_plan;
+        const int plan = !rows_ok ? -1 : force == 1 || force == 3 ? force - 1 : vla_rules::narrow_plan_f32(a.M, a.N);
+        if (plan >= 0) {
+            launch_narrow_f32<kEpi>(a, plan, st);
             return hipGetLastError() == hipSuccess ? VLA_K_OK : VLA_K_ERR_LAUNCH;
         }
     }

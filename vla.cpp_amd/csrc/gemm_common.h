@@ -151,6 +151,65 @@ __device__ __forceinline__ TileCols tile_cols(const GemmArgs& a, int nt) {
     return t;
 }
 
+// Rows of W of a narrow tile's 16 columns: 8 + 8 (see gemm_narrow_kernel).
+struct RowCols {
+    int base_lo, base_hi;  // rows of W of tile columns [0, 8) and [8, 16)
+    int seg;               // 0 Q, 1 K, 2 V (QKV mode)
+    int col_lo, col_hi;    // segment-local column of tile column 0 and of tile column 8
+    bool rope;
+};
+template <int kEpi>
+__device__ __forceinline__ RowCols row_cols(const GemmArgs& a, int t) {
+    RowCols rc;
+    rc.seg = 0;
+    rc.rope = false;
+    if (kEpi == EPI_GLU) {
+        rc.base_lo = rc.col_lo = t * 8;
+        rc.base_hi = rc.col_hi = a.N / 2 + t * 8;
+        return rc;
+    }
+    if (kEpi != EPI_QKV) {
+        rc.base_lo = rc.col_lo = t * 16;
+        rc.base_hi = rc.col_hi = t * 16 + 8;
+        return rc;
+    }
+    const int tq = a.Hq * a.D / 16, tk = a.nk * a.D / 16;
+    int lt = t, seg_base = 0;
+    if (t >= tq + tk) {
+        rc.seg = 2;
+        lt = t - tq - tk;
+        seg_base = (a.Hq + a.nk) * a.D;
+    } else if (t >= tq) {
+        rc.seg = 1;
+        lt = t - tq;
+        seg_base = a.Hq * a.D;
+    }
+    rc.rope = (a.cos_t != nullptr) && rc.seg != 2;
+    if (rc.rope) {
+        const int tph = a.D / 16;  // tiles per head
+        const int head = lt / tph, chunk = lt % tph;
+        rc.col_lo = head * a.D + chunk * 8;
+        rc.col_hi = rc.col_lo + a.D / 2;
+    } else {
+        rc.col_lo = lt * 16;
+        rc.col_hi = rc.col_lo + 8;
+    }
+    rc.base_lo = seg_base + rc.col_lo;
+    rc.base_hi = seg_base + rc.col_hi;
+    return rc;
+}
+
+// The last min(nkt, LEFT) tiles of the ring: with LEFT tiles in flight, the oldest has landed
+// when at most (LEFT - 1) NLOAD loads are still due.
+template <int LEFT, int NLOAD, typename Body>
+__device__ __forceinline__ void narrow_tail(int nkt, Body body) {
+    if (LEFT <= nkt) {  // uniform
+        wait_vmcnt<(LEFT - 1) * NLOAD>();
+        body(LEFT == 1);
+    }
+    if constexpr (LEFT > 1) narrow_tail<LEFT - 1, NLOAD>(nkt, body);
+}
+
 // acc + lo^2 + hi^2 of the two bf16 values packed in u (taken by value: a bit_cast applied
 // directly to a vector element expression reads element 0).
 __device__ __forceinline__ float add_squares_bf16x2(uint32_t u, float acc) {

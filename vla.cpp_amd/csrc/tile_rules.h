@@ -44,6 +44,18 @@ inline int narrow_plan(int M, int N, int K, bool qkv) {
     return p < 0 && M <= 32 ? (M <= 16 ? 0 : 1) : p;
 }
 
+// Rows per workgroup of the fp32 narrow-tile kernel, as an index of NARROW_PLANS (16 x 16 or 64 x 16), or -1 for the tiled
+// kernel.  Two workgroups of 16 x 16 share a CU; beyond one round of them (512), 64-row tiles read the weights a quarter as
+// often while they cover 33 to 64 rows (50 x 4096 x 720 gated 11.4 -> 9.3 us, 51 x 8192 x 1024 22.1 -> 18.9), and 16 x 16 tiles stay ahead
+// of the tiled kernel up to four rounds: 200 x 1600 x 720 14.0 us, tiled 19.0; 482 x 640 x 960 14.9, 22.6; 100 x 4096 x 720 gated (1792
+// workgroups) 18.9, 19.8; 150 x 4096 x 720 gated (2560) 23.4, 20.0.
+inline int narrow_plan_f32(int M, int N) {
+    const long wgs = narrow_wgs(M, N, 0);
+    if (wgs <= 512) return 0;
+    if (M <= 64) return M > 32 || wgs > 2048 ? 2 : 0;
+    return wgs <= 2048 ? 0 : -1;
+}
+
 // Tile of a ternary GEMM (VLA_TERNARY_TILE codes) by predicted time: a launch costs `fixed`, and
 // `step` per 128 k while every workgroup has a CU of its own; up to two workgroups per CU
 // overlap to `two` steps, beyond that a step takes `more` times the workgroups per CU.  The
