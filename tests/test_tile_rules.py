@@ -16,6 +16,7 @@ def rules(tmp_path_factory):
         f.write('''#include "tile_rules.h"
 extern "C" int plan(int M, int N, int K, int qkv) { return vla_rules::narrow_plan(M, N, K, qkv); }
 extern "C" int plan_f32(int M, int N) { return vla_rules::narrow_plan_f32(M, N); }
+extern "C" int wide(int M, int N, int K, int kind) { return vla_rules::wide_tile(M, N, K, kind); }
 extern "C" int ternary(int M, int N, int K) { return vla_rules::ternary_tile(M, N, K); }
 extern "C" int rows(int p) { return 16 * vla_rules::NARROW_PLANS[p][0]; }
 extern "C" int cols(int p) { return 16 * vla_rules::NARROW_PLANS[p][1]; }
@@ -99,3 +100,42 @@ def test_fp32_narrow_tiles_of_more_than_one_round(rules):
             if M <= 64:
                 assert p in (0, 2), (M, N)
             assert (p == 0) == (wgs <= 512 or (wgs <= 2048 and not 32 < M <= 64)), (M, N)
+
+
+# M, N, K, kind (0 plain or gated, 1 QKV, 2 with a LayerNorm) -> measured us of the direct-to-LDS kernel and on the wide tiles
+# 256 x 256, 192 x 192, 256 x 128, 192 x 128, 128 x 128, 128 x 128 in pairs
+WIDE_US = [
+    ((1323, 6144, 1536, 0), 53.3, (45.2, 30.2, 47.2, 45.5, 47.1, 46.1)),
+    ((816, 8192, 1024, 0), 22.3, (28.5, 20.7, 19.8, 28.6, 23.8, 20.0)),
+    ((1600, 4096, 720, 0), 17.1, (22.9, 16.7, 16.6, 24.2, 20.5, 16.5)),
+    ((408, 6144, 1536, 0), 21.1, (45.6, 25.1, 25.7, 21.3, 18.0, 26.0)),
+    ((1323, 4608, 1536, 2), 34.8, (44.8, 30.9, 30.5, 45.0, 36.2, 30.8)),
+    ((13824, 3072, 2048, 1), 202.2, (160.0, 163.7, 173.4, 177.5, 199.3, 175.9)),
+    ((4096, 4096, 4096, 0), 149.3, (106.6, 166.1, 117.2, 144.6, 146.7, 138.5)),
+    ((816, 1024, 4096, 0), 19.5, (85.8, 47.2, 44.6, 38.8, 32.4, 55.8)),
+    ((816, 2560, 1024, 1), 11.3, (28.3, 19.2, 17.7, 15.9, 13.3, 15.3)),
+    ((1088, 1536, 1536, 0), 12.1, (36.8, 22.4, 21.2, 18.2, 15.3, 19.1)),
+    ((5300, 4864, 4576, 1), 332.9, (239.2, 237.4, 297.1, 287.4, 352.1, 337.8)),
+    ((4886, 448, 288, 0), 8.7, (17.9, 12.0, 11.9, 10.0, 8.8, 8.3)),
+    ((600, 1344, 336, 1), 5.2, (19.2, 13.8, 12.8, 11.4, 9.8, 9.4)),
+    ((8362, 4160, 496, 0), 75.2, (73.7, 69.8, 73.3, 78.6, 87.2, 64.6)),
+    ((3570, 8512, 1440, 0), 133.2, (141.7, 112.2, 118.2, 135.9, 142.3, 121.7)),
+]
+
+
+@pytest.mark.parametrize("shape,dl,wide", WIDE_US)
+def test_wide_tiles_are_taken_where_they_are_faster(rules, shape, dl, wide):
+    """The picked kernel is not slower than the direct-to-LDS one, and within the prediction's error (11 %) of the fastest."""
+    t = rules.wide(*shape)
+    took = dl if t < 0 else wide[t]
+    assert took <= dl
+    assert took <= 1.11 * min(wide + (dl,))
+
+
+def test_a_wide_tile_is_named_for_every_size(rules):
+    """From one row to millions the rule answers with a tile or none (no size divides by zero or overflows)."""
+    for M in (1, 63, 64, 513, 1000, 65536, 1 << 24):
+        for N in (8, 64, 200, 4096, 151936):
+            for K in (16, 720, 8192, 1 << 20):
+                for kind in (0, 1, 2):
+                    assert -1 <= rules.wide(M, N, K, kind) < 6

@@ -51,7 +51,7 @@ def _check_no_spill(src, remarks):
 # itself the compiler parks them in the accumulation registers and copies them back and forth
 # around the products (1300 copies in the K loop of dit_self.hip; every product of gemm.hip's
 # narrow-tile kernel).
-EXTRA_FLAGS = {"attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"], "dit_self.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"], "gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"], "gemm_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+EXTRA_FLAGS = {"attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"], "dit_self.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"], "gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"], "gemm_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"], "gemm_wide.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 
 def _compile(src):

@@ -30,6 +30,7 @@
 #include "common.h"
 #include "gemm_common.h"
 #include "gemm_f32.h"
+#include "gemm_wide.h"
 #include "tile_rules.h"
 #include "vla_kernels.h"
 
@@ -1905,24 +1906,13 @@ int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
     }
     if constexpr (kEpi != EPI_TERNARY) {
         // VLA_GEMM_TILE = 0..5 pins the tile configuration and VLA_GEMM_STAGES the ring depth
-        // of the direct-to-LDS kernel (tests and tuning); unset = by shape.
+        // of the direct-to-LDS kernel, 16..21 a tile of the wide-tile kernel (tests and tuning); unset = by shape.
         int cfg = tuning().gemm_tile;
+        const bool pinned = cfg >= 0;
+        const int pinned_wide = cfg >= 16 && cfg < 16 + vla_rules::WIDE_TILES ? cfg - 16 : -1;
         const long m128 = (a.M + 127) / 128, m64 = (a.M + 63) / 64;
         const long wgs0 = m128 * ((n_tiles + 1) / 2), wgs2 = m128 * n_tiles, wgs4 = m64 * n_tiles;
-        if (cfg < 0) {
-            // Enough 128x128 tiles to occupy the chip: use them (half the LDS and L2 traffic
-            // per multiply); else 128x64 tiles if those fill it; else 64x64 tiles, with
-            // 256-byte K rows (half the barriers per K) while one workgroup per CU covers them.
-            cfg = wgs0 >= 128 ? 0 : (wgs2 >= 150 ? 2 : (wgs4 <= 256 ? 1 : 4));
-            // 128x128 tiles that leave more than a third of the CUs idle lose to 128x64 tiles
-            // that cover the chip in little more than one round (pi0's fused QKV: 140 -> 280)
-            if (cfg == 0 && wgs0 < 160 && wgs2 <= 288) cfg = 2;
-            // Between one and one and a half rounds of 128x128 tiles, some CUs would run two
-            // workgroups while the rest run one; 128x192 tiles cover the same grid in a single
-            // round of 1.5x workgroups (GR00T's fused QKV: 324 -> 216 workgroups).
-            const long wgs5 = m128 * ((n_tiles + 2) / 3);
-            if (cfg == 0 && wgs0 > 256 && wgs0 <= 384 && wgs5 <= 256) cfg = 5;
-        }
+        if (!pinned) cfg = vla_rules::dl_tile(a.M, n_tiles);
         // bf16 operands with 16-byte aligned rows and K a multiple of the MFMA depth take the
         // direct-to-LDS kernel (VLA_GEMM_DL=0 pins the register-staged one).  Its ring depth
         // trades loads in flight against LDS per workgroup: a workgroup is short-lived, so
@@ -1934,6 +1924,14 @@ int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
         }
         if (a.norm_eps >= 0.f && !(dl && (kEpi == EPI_QKV || kEpi == EPI_GLU))) return VLA_K_ERR_SHAPE;  // only that kernel takes the row statistics
         if (a.colsum && kEpi != EPI_QKV) return VLA_K_ERR_SHAPE;
+        if constexpr (std::is_same<T, bf16_t>::value) {
+            // The wide tiles where they are predicted faster (32-bit lane offsets inside a tile; row sums handed from launch
+            // to launch stay with the kernel below).
+            if (dl && a.K <= (1 << 20) && !a.stats_in && !a.stats_out) {
+                const int wide = pinned ? pinned_wide : vla_rules::wide_tile(a.M, a.N, a.K, kEpi != EPI_QKV ? 0 : a.colsum ? 2 : 1);
+                if (wide >= 0 && launch_wide<kEpi>(a, wide, st)) return hipGetLastError() == hipSuccess ? VLA_K_OK : VLA_K_ERR_LAUNCH;
+            }
+        }
         if (dl) {
             int ns = tuning().gemm_stages;
             const long wgs = cfg == 0 ? wgs0 : (cfg == 2 || cfg == 3 ? wgs2 : wgs4);

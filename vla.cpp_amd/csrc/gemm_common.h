@@ -3,6 +3,7 @@
 #pragma once
 
 #include "common.h"
+#include "tile_rules.h"
 #include "vla_kernels.h"
 
 namespace vk {
@@ -64,6 +65,7 @@ struct GemmArgs {
     // for x < 2^16); xn_shift = log2 xn.
     int cn, cm, per_panel, full, w_last, xn_shift;
     unsigned mg_cn, mg_pp, mg_pn, mg_wl;
+    DivC div_s;  // QKV, wide tiles: rows per observation
 };
 
 // Workgroup -> tile.  Workgroup i runs on XCD i % 8; the XCDs form an xm x xn grid over the
@@ -507,32 +509,12 @@ inline unsigned xcd_walk(GemmArgs& a, int m_wg, int n_wg) {
     return (unsigned)(wgs * 8);
 }
 
-// XCD grid xm x xn = 8 for a tile grid of m_wg x n_wg workgroup tiles of tile_cols columns:
-// every L2 reads its N tiles' rows of W once and its M tiles' rows of A once per panel of N
-// tiles (xcd_tile).  One panel while an XCD's rows of W fit in half of its 4 MiB L2 beside
-// the streaming A and C; else panels of about 2 MiB of W.  The split with the least total,
-// counting the padding of the tile grid.  Returns the grid size.
+// The same with the XCD grid by shape (xcd_grid in tile_rules.h).
 inline unsigned xcd_split(GemmArgs& a, int m_wg, int n_wg, double w_bytes_per_elem, int tile_cols, double a_bytes_per_elem) {
-    const double bytes_a = (double)a.M * a.K * a_bytes_per_elem, bytes_w = (double)a.N * a.K * w_bytes_per_elem;
-    const double tile_w = (double)tile_cols * a.K * w_bytes_per_elem, l2_panel = 2.0 * 1024 * 1024;
-    const int forced = tuning().gemm_panel;  // 0 = by size, > 0 = that many tiles per panel
-    double best = -1;
-    for (int xm = 1; xm <= 8; xm *= 2) {
-        const int xn = 8 / xm;
-        const int cn = (n_wg + xn - 1) / xn, cm = (m_wg + xm - 1) / xm;
-        int pn = cn;
-        if (forced > 0) pn = forced < cn ? forced : cn;
-        else if (cn * tile_w > l2_panel && cm >= 4) pn = tile_w >= l2_panel ? 1 : (int)(l2_panel / tile_w);
-        const int panels = (cn + pn - 1) / pn;
-        const long wgs = (long)cm * cn * 8;
-        const double cost = (bytes_a * xn * panels + bytes_w * xm) * (double)wgs / ((double)m_wg * n_wg);
-        if (best < 0 || cost < best) {
-            best = cost;
-            a.xm = xm;
-            a.xn = xn;
-            a.pn = pn;
-        }
-    }
+    const vla_rules::XcdGrid g = vla_rules::xcd_grid(a.M, a.N, a.K, m_wg, n_wg, w_bytes_per_elem, tile_cols, a_bytes_per_elem, tuning().gemm_panel);
+    a.xm = g.xm;
+    a.xn = g.xn;
+    a.pn = g.pn;
     return xcd_walk(a, m_wg, n_wg);
 }
 

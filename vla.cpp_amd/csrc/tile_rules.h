@@ -56,6 +56,102 @@ inline int narrow_plan_f32(int M, int N) {
     return wgs <= 2048 ? 0 : -1;
 }
 
+// XCD grid xm x xn = 8 for a tile grid of m_wg x n_wg workgroup tiles of tile_cols columns:
+// every L2 reads its N tiles' rows of W once and its M tiles' rows of A once per panel of pn N
+// tiles.  One panel while an XCD's rows of W fit in half of its 4 MiB L2 beside
+// the streaming A and C; else panels of about 2 MiB of W.  The split with the least total,
+// counting the padding of the tile grid.  forced_pn: 0 = by size, > 0 = that many tiles per panel.
+struct XcdGrid {
+    int xm, xn, pn;
+    long wgs;  // workgroups of an XCD
+};
+inline XcdGrid xcd_grid(int M, int N, int K, int m_wg, int n_wg, double w_bytes_per_elem, int tile_cols, double a_bytes_per_elem, int forced_pn) {
+    const double bytes_a = (double)M * K * a_bytes_per_elem, bytes_w = (double)N * K * w_bytes_per_elem;
+    const double tile_w = (double)tile_cols * K * w_bytes_per_elem, l2_panel = 2.0 * 1024 * 1024;
+    double best = -1;
+    XcdGrid g = {1, 8, 1, 0};
+    for (int xm = 1; xm <= 8; xm *= 2) {
+        const int xn = 8 / xm;
+        const int cn = (n_wg + xn - 1) / xn, cm = (m_wg + xm - 1) / xm;
+        int pn = cn;
+        if (forced_pn > 0) pn = forced_pn < cn ? forced_pn : cn;
+        else if (cn * tile_w > l2_panel && cm >= 4) pn = tile_w >= l2_panel ? 1 : (int)(l2_panel / tile_w);
+        const int panels = (cn + pn - 1) / pn;
+        const long wgs = (long)cm * cn;
+        const double cost = (bytes_a * xn * panels + bytes_w * xm) * (double)(wgs * 8) / ((double)m_wg * n_wg);
+        if (best < 0 || cost < best) {
+            best = cost;
+            g = {xm, xn, pn, wgs};
+        }
+    }
+    return g;
+}
+
+// Tile of the direct-to-LDS bf16 kernel (VLA_GEMM_TILE codes): enough 128 x 128 tiles to occupy the chip: use them (half the
+// LDS and L2 traffic per multiply); else 128 x 64 tiles if those fill it; else 64 x 64 tiles, with 256-byte K rows (half the
+// barriers per K) while one workgroup per CU covers them.
+inline int dl_tile(int M, int n_tiles) {
+    const long m128 = (M + 127) / 128, m64 = (M + 63) / 64;
+    const long wgs0 = m128 * ((n_tiles + 1) / 2), wgs2 = m128 * n_tiles, wgs4 = m64 * n_tiles, wgs5 = m128 * ((n_tiles + 2) / 3);
+    int cfg = wgs0 >= 128 ? 0 : (wgs2 >= 150 ? 2 : (wgs4 <= 256 ? 1 : 4));
+    // 128x128 tiles that leave more than a third of the CUs idle lose to 128x64 tiles
+    // that cover the chip in little more than one round (pi0's fused QKV: 140 -> 280)
+    if (cfg == 0 && wgs0 < 160 && wgs2 <= 288) cfg = 2;
+    // Between one and one and a half rounds of 128x128 tiles, some CUs would run two
+    // workgroups while the rest run one; 128x192 tiles cover the same grid in a single
+    // round of 1.5x workgroups (GR00T's fused QKV: 324 -> 216 workgroups).
+    if (cfg == 0 && wgs0 > 256 && wgs0 <= 384 && wgs5 <= 256) cfg = 5;
+    return cfg;
+}
+
+// Predicted time (us) of a bf16 projection on a tile: `fixed`, and per round of workgroups on the busiest XCD (32 CUs) its
+// prologue and epilogue `round` (QKV: + `qkv`, with a LayerNorm inside + `layer`) and `step` per 64 k, which grows by `load` with the
+// share of the CUs that are busy.  Tiles of which two share a CU: round2 and step2 for the rounds of two.  Fitted to 3362
+// measured shapes (200 to 16000 rows, N 256 to 10240, K 128 to 8192, plain, gated, QKV); the prediction is off by 11 % (rms).
+struct TileTime {
+    int rows, cols;
+    bool pairs;
+    double fixed, round, step, load, round2, step2, qkv, layer;
+    double us(int M, int N, int K, int kind) const {
+        const XcdGrid g = xcd_grid(M, N, K, (M + rows - 1) / rows, (N + cols - 1) / cols, 2.0, cols, 2.0, 0);
+        const double w = g.wgs / 32.0, kt = (K + 63) / 64, extra = kind == 0 ? 0.0 : kind == 1 ? qkv : layer;
+        const long n = (g.wgs + 31) / 32, n2 = pairs ? n / 2 : 0, n1 = n - 2 * n2;
+        return fixed + n2 * (round2 + 1.5 * extra + kt * step2) + n1 * (round + extra + kt * (step + load * (w < 1 ? w : 1)));
+    }
+};
+
+// Tile of the wide-tile kernel: rows x columns, and whether two workgroups share a CU.
+enum { WIDE_256X256 = 0, WIDE_192X192, WIDE_256X128, WIDE_192X128, WIDE_128X128, WIDE_128X128_PAIRS, WIDE_TILES };
+
+// The wide tile with the least predicted time, or -1 where the direct-to-LDS kernel's tile is not predicted 6 % slower.  kind:
+// 0 plain or gated, 1 QKV, 2 QKV with a LayerNorm inside.  On the fitted shapes the wide tile is taken on 60 %, where it needs
+// 0.83 of the time (geometric mean; 0.90 over all, 0.89 if the faster one were always known); 1 % of them are 3 to 6 %
+// slower, none more.  1323 x 6144 x 1536 53 -> 28 us (192 x 192: 224 workgroups, one round, where 528 of 128 x 128 left 16 for a second
+// one), 816 x 8192 x 1024 gated 23 -> 20, 13824 x 3072 x 2048 203 -> 161 (256 x 256), 4096 x 4096 x 4096 150 -> 107.
+inline int wide_tile(int M, int N, int K, int kind) {
+    static const TileTime wide[WIDE_TILES] = {
+        {256, 256, false, 0.18, 11.50, 1.234, 0.314, 0, 0, 1.57, 3.50}, {192, 192, false, 1.05, 7.02, 0.703, 0.225, 0, 0, 2.04, 3.15},
+        {256, 128, false, 1.05, 6.86, 0.676, 0.188, 0, 0, 1.31, 2.89},  {192, 128, false, 1.38, 5.32, 0.565, 0.152, 0, 0, 1.51, 2.93},
+        {128, 128, false, 1.85, 3.90, 0.455, 0.115, 0, 0, 1.10, 2.04},  {128, 128, true, 1.41, 2.86, 0.664, 0.198, 4.82, 0.982, 1.08, 1.63}};
+    static const TileTime dl[6] = {
+        {128, 128, true, 2.34, 4.32, 0.249, 0.410, 5.77, 1.132, -0.38, 0.29}, {64, 64, false, 2.23, 2.14, 0.194, 0.029, 0, 0, -0.16, 0.87},
+        {128, 64, true, 3.53, 1.36, 0.335, 0.063, 2.32, 0.662, 0.13, 0.81},   {128, 64, true, 3.53, 1.36, 0.335, 0.063, 2.32, 0.662, 0.13, 0.81},
+        {64, 64, true, 4.86, 1.00, 0.300, 0.300, 0.00, 0.378, -0.42, 0.31},   {128, 192, false, 6.38, 2.96, 0.637, 0.119, 0, 0, 0.21, 0.71}};
+    const int cfg = dl_tile(M, (N + 63) / 64);
+    double least = 0.94 * dl[cfg].us(M, N, K, kind);
+    int best = -1;
+    for (int t = 0; t < WIDE_TILES; ++t) {
+        // one 128 x 128 tile per CU, where 128 x 64 tiles cover the chip: up to 18 % slower than those
+        if (t == WIDE_128X128 && cfg != 0) continue;
+        const double us = wide[t].us(M, N, K, kind);
+        if (us < least) {
+            least = us;
+            best = t;
+        }
+    }
+    return best;
+}
+
 // Tile of a ternary GEMM (VLA_TERNARY_TILE codes) by predicted time: a launch costs `fixed`, and
 // `step` per 128 k while every workgroup has a CU of its own; up to two workgroups per CU
 // overlap to `two` steps, beyond that a step takes `more` times the workgroups per CU.  The
