@@ -1031,12 +1031,14 @@ extern "C" {
 int vla_rope_tables_host(const int32_t* pos, int n, int head_dim, double base, float* cos_tab, float* sin_tab) {
     if (!pos || !cos_tab || !sin_tab || n < 0 || head_dim <= 0 || (head_dim & 1)) return VLA_K_ERR_ARG;
     const int half = head_dim / 2;
-    for (int s = 0; s < n; ++s)
-        for (int i = 0; i < half; ++i) {
-            const double ang = (double)pos[s] * pow(base, -2.0 * (double)i / (double)head_dim);
+    for (int i = 0; i < half; ++i) {
+        const double freq = pow(base, -2.0 * (double)i / (double)head_dim);
+        for (int s = 0; s < n; ++s) {
+            const double ang = (double)pos[s] * freq;
             cos_tab[(size_t)s * half + i] = (float)cos(ang);
             sin_tab[(size_t)s * half + i] = (float)sin(ang);
         }
+    }
     return VLA_K_OK;
 }
 

@@ -27,6 +27,7 @@
 #include "checkpoint.h"
 #include "layers.h"
 #include "model.h"
+#include "staging.h"
 
 namespace vla {
 namespace {
@@ -126,6 +127,7 @@ class BitvlaLm : public ModelArch {
     std::shared_ptr<RowSource> lang_rows_;
     DevBuf out_norm_, W_out_, b_out_;
     RopeTable rope_;
+    PinnedBuf stage_;  // host staging of the embeddings (page-locked)
     AttnWorkspace attn_ws_;
     DevBuf h_, hn_, q8_, s_, rowsum_, qkv_, q_, att_, o_, emb_bcast_, hfin_, x_, gu_, act_;
     hipStream_t last_stream_ = nullptr;
@@ -236,10 +238,15 @@ void BitvlaLm::prefill(const Inputs* in, int batch) {
                 for (int c = 0; c < H_; ++c) eb[((size_t)t * B + b) * H_ + c] = f32_to_bf16(act_emb_[(size_t)t * H_ + c]);
         emb_bcast_.upload(eb.data(), eb.size() * 2);
     }
-    std::vector<uint16_t> emb((size_t)B * P * H_);
-    for (int b = 0; b < B; ++b) {
-        uint16_t* dst = emb.data() + (size_t)b * P * H_;
-        for (size_t i = 0; i < (size_t)n_img_ * H_; ++i) dst[i] = f32_to_bf16(in[b].precomputed_img_emb[i]);
+    // embeddings to bf16 in page-locked staging memory, sent to the device in groups of observations
+    Ctx C;  // prefill runs on the default stream and is synchronous
+    stage_.reserve((size_t)B * P * H_ * 2);
+    uint16_t* const emb = stage_.as<uint16_t>();
+    const size_t n_feat = (size_t)n_img_ * H_, obs = (size_t)P * H_;
+    const int n_groups = std::min(B, 4), pieces = stage_pieces(n_feat * sizeof(float)), per_obs = pieces + 1;
+    std::vector<int> first(n_groups + 1);
+    for (int g = 0; g <= n_groups; ++g) first[g] = (int)((long)B * g / n_groups) * per_obs;
+    auto stage_text = [&](int b) {
         std::vector<float> fetched;
         if (lang_rows_) {
             fetched.resize((size_t)n_lang_ * H_);
@@ -248,11 +255,21 @@ void BitvlaLm::prefill(const Inputs* in, int batch) {
         }
         for (int i = 0; i < n_lang_; ++i) {
             const float* e = lang_rows_ ? fetched.data() + (size_t)i * H_ : E_lang_.data() + (size_t)in[b].lang_tokens[i] * H_;
-            for (int c = 0; c < H_; ++c) dst[(size_t)(n_img_ + i) * H_ + c] = f32_to_bf16(e[c]);
+            convert_scaled(emb + b * obs + n_feat + (size_t)i * H_, e, (size_t)H_, 1.0f, VLA_DT_BF16);
         }
-    }
-    h_.upload(emb.data(), emb.size() * 2);
-    Ctx C;
+    };
+    run_staged(
+        first, 1,  // 2.6 MB an observation: see stage_threads
+        [&](int t) {
+            const int b = t / per_obs, piece = t % per_obs - 1;
+            if (piece < 0) return stage_text(b);
+            const size_t e0 = n_feat * piece / pieces, e1 = n_feat * (piece + 1) / pieces;
+            convert_scaled(emb + b * obs + e0, in[b].precomputed_img_emb + e0, e1 - e0, 1.0f, VLA_DT_BF16);
+        },
+        [&](int g) {
+            const size_t e0 = first[g] / per_obs * obs, e1 = first[g + 1] / per_obs * obs;
+            VLA_HIP(hipMemcpyAsync(h_.as<uint16_t>() + e0, emb + e0, (e1 - e0) * 2, hipMemcpyHostToDevice, C.stream));
+        });
     prof_start("prefill", C.stream);
     run_layers(C, B * P, P, 0, P);
     VLA_HIP(hipDeviceSynchronize());

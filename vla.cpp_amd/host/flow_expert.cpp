@@ -30,6 +30,7 @@
 #include "checkpoint.h"
 #include "layers.h"
 #include "model.h"
+#include "staging.h"
 
 namespace vla {
 namespace {
@@ -118,6 +119,7 @@ class FlowExpert : public ModelArch {
 
   private:
     void allocate(int B, int P, int P_txt = 0);
+    void rope_positions(int64_t n);
     uint32_t alloc_gen_ = 0;
     int tuning_gen_ = -1;
 
@@ -157,9 +159,9 @@ class FlowExpert : public ModelArch {
 
     // per-call state
     int B_ = 0, P_ = 0, pad_start_ = 0, pad_end_ = 0;
-    RopeTable rope_prefill_, rope_self_, rope_cross_;
+    RopeTable rope_all_, rope_prefill_, rope_self_;  // every position the model can meet (formed once); this call's rows of it
     DevBuf prefix_, prefix_n_, tmpk_, tmpv_, lead_, x0_, xt_, h_, hn_, q_, att_, mid_;
-    PinnedBuf stage_;  // host staging of the prefix embeddings (page-locked)
+    PinnedBuf stage_, stage_f32_;  // host staging (page-locked): prefix embeddings; lead rows and noise
     KVLayer tmp_kv_;
     AttnWorkspace attn_ws_;
     std::mt19937 rng_{std::random_device{}()};
@@ -236,6 +238,9 @@ FlowExpert::FlowExpert(const Checkpoint& ck) {
     if (!config_is_sane(cfg)) throw std::runtime_error("vla: real_* dims exceed max_* dims");
 
     if (S_ <= n_lead_) throw std::runtime_error("vla: n_suffix leaves no action rows");
+    // Every position that max_views and n_lang allow; formed per call, the table was 2.3 of the 3 ms in front of the first
+    // launch of a three-view pi0 observation.
+    if (rope_) rope_positions(std::min<int64_t>((int64_t)max_views_ * n_img_ + n_lang_max_ + 1 + S_, 1 << 16));
     const int64_t qd = (int64_t)Hq_ * D_, kvd = (int64_t)Hkv_ * D_;
     if (vocab_ > 0) {
         lang_rows_ = ck.row_source("prefix.E_lang");
@@ -602,6 +607,15 @@ void FlowExpert::allocate(int B, int P, int P_txt) {
     }
 }
 
+// rope_all_ with positions 0 .. n - 1 at least
+void FlowExpert::rope_positions(int64_t n) {
+    if (n <= rope_all_.rows) return;
+    std::vector<int32_t> pos((size_t)n);
+    for (size_t i = 0; i < pos.size(); ++i) pos[i] = (int32_t)i;
+    rope_all_.build(RopeSpec{D_, cfg.rope_freq_base}, pos);
+    ++alloc_gen_;  // captured graphs hold its address
+}
+
 void FlowExpert::prefill(const Inputs* in, int batch) {
     if (!in || batch <= 0) throw std::invalid_argument("vla: prefill needs at least one observation");
     const int views = in[0].n_img_views, n_lang = (arch_ == Arch::GR00T && !alt_vl_) ? 0 : in[0].n_lang;
@@ -628,25 +642,28 @@ void FlowExpert::prefill(const Inputs* in, int batch) {
     Ctx C;  // prefill runs on the default stream and is synchronous
 
     // ---- prefix embeddings: scaled and converted to the model's dtype straight from the
-    // callers' buffers into page-locked staging memory by a few threads, an observation per
+    // callers' buffers into page-locked staging memory by a few threads, a piece of an observation per
     // task, and sent to the device in groups while the next group is being converted (the
     // copies are asynchronous; everything below runs on the same stream, after them)
-    const size_t es = dtype_size(dt_);
+    const size_t es = dtype_size(dt_), nx = (size_t)(S_ - n_lead_) * A_, n_lead_row = (size_t)std::max(n_lead_, 0) * W_;
     stage_.reserve((size_t)B * P * Wv_ * es);
+    stage_f32_.reserve(((size_t)B * n_lead_row + (size_t)B * nx) * sizeof(float));
     char* const pe = stage_.as<char>();
+    float* const lead_host = stage_f32_.as<float>();  // the state (and future) rows in front of the actions
+    float* const noise_host = lead_host + (size_t)B * n_lead_row;
     const float lang_scale = std::sqrt((float)Wv_);
     const float img_scale = arch_ == Arch::SMOLVLA ? lang_scale : 1.0f;  // smolvla.cpp:1363 vs pi0.cpp:554-555
-    std::vector<float> lead_host((size_t)B * std::max(n_lead_, 0) * W_);  // the state (and future) rows in front of the actions
-    auto stage_obs = [&](int b) {
-        char* dst = pe + (size_t)b * P * Wv_ * es;
-        // alternating layers project the image rows and the text rows separately: all image
-        // rows of the batch first, then all text rows, each block [B][rows][Wv]
-        char* txt_dst = dst + (size_t)n_img_tot * Wv_ * es;
-        if (alt_vl_) {
-            dst = pe + (size_t)b * n_img_tot * Wv_ * es;
-            txt_dst = pe + ((size_t)B * n_img_tot + (size_t)b * n_lang) * Wv_ * es;
-        }
-        convert_scaled(dst, in[b].precomputed_img_emb, (size_t)n_img_tot * Wv_, img_scale, dt_);
+    // alternating layers project the image rows and the text rows separately: all image
+    // rows of the batch first, then all text rows, each block [B][rows][Wv]
+    const size_t img_rows = (size_t)n_img_tot, obs_rows = alt_vl_ ? img_rows : (size_t)P;
+    const int pieces = stage_pieces(img_rows * Wv_ * sizeof(float));
+    auto stage_img = [&](int b, int piece) {
+        const size_t n = img_rows * Wv_, e0 = n * piece / pieces, e1 = n * (piece + 1) / pieces;
+        convert_scaled(pe + ((size_t)b * obs_rows * Wv_ + e0) * es, in[b].precomputed_img_emb + e0, e1 - e0, img_scale, dt_);
+    };
+    auto stage_rest = [&](int b) {
+        char* dst = pe + (size_t)b * obs_rows * Wv_ * es;
+        char* txt_dst = alt_vl_ ? pe + ((size_t)B * img_rows + (size_t)b * n_lang) * Wv_ * es : dst + img_rows * Wv_ * es;
         if (arch_ != Arch::GR00T || alt_vl_) {
             const int rows = arch_ == Arch::SMOLVLA ? n_lang_max_ : n_lang;
             const float ls = alt_vl_ ? 1.0f : lang_scale;  // N1.6: the rows stand for backbone features, unscaled
@@ -665,72 +682,75 @@ void FlowExpert::prefill(const Inputs* in, int batch) {
         }
         std::vector<float> st(max_state_, 0.f);
         if (in[b].state) std::copy(in[b].state, in[b].state + max_state_, st.begin());
+        float* const ld = lead_host + (size_t)b * n_lead_row;
         if (arch_ == Arch::SMOLVLA) {
             std::vector<float> row(Wv_);
             host_linear(Wstate_.data(), bstate_.data(), st.data(), row.data(), Wv_, max_state_);
             convert_scaled(dst + (size_t)(P - 1) * Wv_ * es, row.data(), (size_t)Wv_, 1.0f, dt_);
         } else if (head_io_) {
             // encode_state (relu between the two projections), then the learned future tokens
-            std::vector<float> h1(Hs_), ld((size_t)n_lead_ * W_);
+            std::vector<float> h1(Hs_);
             host_linear(se_l1W_.data(), se_l1b_.data(), st.data(), h1.data(), Hs_, max_state_);
             for (float& v : h1) v = v > 0.f ? v : 0.f;
-            host_linear(se_l2W_.data(), se_l2b_.data(), h1.data(), ld.data(), W_, Hs_);
-            std::copy(future_.begin(), future_.end(), ld.begin() + W_);
-            std::copy(ld.begin(), ld.end(), lead_host.begin() + (size_t)b * n_lead_ * W_);
+            host_linear(se_l2W_.data(), se_l2b_.data(), h1.data(), ld, W_, Hs_);
+            std::copy(future_.begin(), future_.end(), ld + W_);
         } else if (n_lead_ > 0) {
-            host_linear(W_sp_.data(), b_sp_.data(), st.data(), lead_host.data() + (size_t)b * W_, W_, max_state_);
+            host_linear(W_sp_.data(), b_sp_.data(), st.data(), ld, W_, max_state_);
         }
     };
-    {
-        const int nthr = std::max(1, std::min(default_cpu_threads(), B));
-        const int n_groups = alt_vl_ ? 1 : std::min(B, 4);  // the alternating layout interleaves observations: one copy at the end
-        for (int gi = 0; gi < n_groups; ++gi) {
-            const int b0 = (int)((long)B * gi / n_groups), b1 = (int)((long)B * (gi + 1) / n_groups);
-            if (nthr == 1 || b1 - b0 == 1) {
-                for (int b = b0; b < b1; ++b) stage_obs(b);
-            } else {
-                std::vector<std::thread> pool;
-                std::vector<std::string> errors(nthr);
-                for (int t = 0; t < nthr; ++t)
-                    pool.emplace_back([&, t]() {
-                        try {
-                            for (int b = b0 + t; b < b1; b += nthr) stage_obs(b);
-                        } catch (const std::exception& e) {
-                            errors[t] = e.what();
-                        }
-                    });
-                for (auto& th : pool) th.join();
-                for (const std::string& e : errors)
-                    if (!e.empty()) throw std::runtime_error(e);
-            }
-            const size_t off = alt_vl_ ? 0 : (size_t)b0 * P * Wv_ * es;
-            const size_t len = alt_vl_ ? (size_t)B * P * Wv_ * es : (size_t)(b1 - b0) * P * Wv_ * es;
-            VLA_HIP(hipMemcpyAsync((char*)prefix_.get() + off, pe + off, len, hipMemcpyHostToDevice, C.stream));
+    // initial noise (the generator's draws in order of the observations)
+    for (int b = 0; b < B; ++b) {
+        if (in[b].noise) {
+            std::copy(in[b].noise, in[b].noise + nx, noise_host + (size_t)b * nx);
+        } else {
+            std::normal_distribution<float> nd(0.f, 1.f);
+            for (size_t i = 0; i < nx; ++i) noise_host[(size_t)b * nx + i] = nd(rng_);
         }
-        if (!lead_host.empty()) VLA_HIP(hipMemcpy(lead_.get(), lead_host.data(), lead_host.size() * sizeof(float), hipMemcpyHostToDevice));
+    }
+    {
+        const int n_groups = std::min(B, 4), per_obs = pieces + 1;
+        std::vector<int> first(n_groups + 1);
+        for (int g = 0; g <= n_groups; ++g) first[g] = (int)((long)B * g / n_groups) * per_obs;
+        auto copy_rows = [&](size_t r0, size_t rows) {
+            VLA_HIP(hipMemcpyAsync((char*)prefix_.get() + r0 * Wv_ * es, pe + r0 * Wv_ * es, rows * Wv_ * es, hipMemcpyHostToDevice, C.stream));
+        };
+        run_staged(
+            first, stage_threads(B),
+            [&](int t) {
+                // the small remainder first: it may wait for a file
+                if (t % per_obs == 0) stage_rest(t / per_obs);
+                else stage_img(t / per_obs, t % per_obs - 1);
+            },
+            [&](int g) {
+                const size_t b0 = first[g] / per_obs, b1 = first[g + 1] / per_obs;
+                copy_rows(b0 * obs_rows, (b1 - b0) * obs_rows);
+                if (g + 1 < n_groups) return;
+                if (alt_vl_ && n_lang > 0) copy_rows((size_t)B * img_rows, (size_t)B * n_lang);
+                if (n_lead_row > 0)
+                    VLA_HIP(hipMemcpyAsync(lead_.get(), lead_host, (size_t)B * n_lead_row * sizeof(float), hipMemcpyHostToDevice, C.stream));
+                VLA_HIP(hipMemcpyAsync(x0_.get(), noise_host, (size_t)B * nx * sizeof(float), hipMemcpyHostToDevice, C.stream));
+            });
     }
 
-    // ---- positions and masks (smolvla.cpp:1633-1672, pi0.cpp:612-616)
+    // ---- positions and masks (smolvla.cpp:1633-1672, pi0.cpp:612-616).  The rows of the tables come from the one that the
+    // handle formed when it was loaded: position i is its row i.
     pad_start_ = pad_end_ = 0;
+    const RopeTable* rope_prefix = &rope_all_;  // prefix row i is at position i
     if (rope_) {
-        const RopeSpec rs{D_, cfg.rope_freq_base};
-        std::vector<int32_t> pp(P), ps(S_), pc(S_);
-        for (int i = 0; i < P; ++i) pp[i] = i;
+        rope_positions((int64_t)P + S_);
         int suffix_base = P;
-        if (arch_ == Arch::SMOLVLA) {
+        if (arch_ == Arch::SMOLVLA) {  // the state row, behind the padded text, is at the position behind the text
             const int state_pos = n_img_tot + n_lang;
-            pp[P - 1] = state_pos;
+            rope_prefill_.reserve(rope_all_, P);
+            rope_prefill_.copy_rows(0, rope_all_, 0, P - 1, C.stream);
+            rope_prefill_.copy_rows(P - 1, rope_all_, state_pos, 1, C.stream);
+            rope_prefix = &rope_prefill_;
             suffix_base = state_pos + 1;
             pad_start_ = n_img_tot + n_lang;
             pad_end_ = n_img_tot + n_lang_max_;
         }
-        for (int i = 0; i < S_; ++i) {
-            ps[i] = suffix_base + i;
-            pc[i] = i;
-        }
-        rope_prefill_.build(rs, pp);
-        rope_self_.build(rs, ps);
-        rope_cross_.build(rs, pc);
+        rope_self_.reserve(rope_all_, S_);
+        rope_self_.copy_rows(0, rope_all_, suffix_base, S_, C.stream);
     }
 
     // ---- vlln: the affine LayerNorm between the backbone and the DiT head
@@ -764,7 +784,7 @@ void FlowExpert::prefill(const Inputs* in, int batch) {
         prof_mark("prefix_norm");
         if (arch_ == Arch::SMOLVLA && !w.is_self) {
             // expert_cross_kv: K = Wk_x . cachedK_flat, V = Wv_x . cachedV_flat, no second rotation
-            qkv_rope_append(C, xn, Wkv, bkv, P, 0, true, true, &rope_prefill_, nullptr, tmp_kv_, 0);
+            qkv_rope_append(C, xn, Wkv, bkv, P, 0, true, true, rope_prefix, nullptr, tmp_kv_, 0);
             VLA_K(vla_kv_gather(tmp_kv_.k.get(), tmp_kv_.vt.get(), tmpk_.get(), tmpv_.get(), dt_, B, Hkv_, D_,
                                 tmp_kv_.t_max, 0, P, C.stream));
             Tensor tk = tensor_2d(tmpk_.get(), dt_, kvd, (int64_t)B * P), tv = tensor_2d(tmpv_.get(), dt_, kvd, (int64_t)B * P);
@@ -773,23 +793,11 @@ void FlowExpert::prefill(const Inputs* in, int batch) {
             qkv_rope_append(C, tv, Wvx, nullptr, P, 0, false, true, nullptr, nullptr, w.kv, 0);
             prof_mark("prefix_kv_proj_and_cross_reprojection");
         } else {
-            qkv_rope_append(C, xn, Wkv, bkv, P, 0, true, true, &rope_prefill_, nullptr, w.kv, 0);
+            qkv_rope_append(C, xn, Wkv, bkv, P, 0, true, true, rope_prefix, nullptr, w.kv, 0);
             prof_mark("prefix_kv_proj");
         }
     }
 
-    // ---- initial noise
-    const size_t nx = (size_t)(S_ - n_lead_) * A_;
-    std::vector<float> x0((size_t)B * nx);
-    for (int b = 0; b < B; ++b) {
-        if (in[b].noise) {
-            std::copy(in[b].noise, in[b].noise + nx, x0.begin() + (size_t)b * nx);
-        } else {
-            std::normal_distribution<float> nd(0.f, 1.f);
-            for (size_t i = 0; i < nx; ++i) x0[(size_t)b * nx + i] = nd(rng_);
-        }
-    }
-    x0_.upload(x0.data(), x0.size() * sizeof(float));
     VLA_HIP(hipDeviceSynchronize());
 }
 
@@ -846,7 +854,7 @@ void FlowExpert::run_steps(int n_steps, void* stream) {
                 const bool leave_stats = stats_path && l + 1 < L_ && (bool)layers_[l + 1].Wqkv_ada;
                 const float* bq = w.bqkv ? w.bqkv.as<float>() : nullptr;
                 const int64_t n_rows_w = w.is_self ? (int64_t)(Hq_ + 2 * Hkv_) * D_ : (int64_t)Hq_ * D_;
-                const RopeTable* tab = rope_ ? (w.is_self ? &rope_self_ : &rope_cross_) : nullptr;
+                const RopeTable* tab = rope_ ? (w.is_self ? &rope_self_ : &rope_all_) : nullptr;  // cross layers: positions 0 .. S - 1
                 const int tok = w.is_self ? w.kv.n_prefix : 0;
                 // pi0.5: this step's (scale, shift, gate) of the layer's two norm sites
                 const float* mod_in = adarms_ ? ada_.as<float>() + ((size_t)s * (2 * L_ + 1) + 2 * l) * 3 * W_ : nullptr;

@@ -46,14 +46,29 @@ struct RopeSpec {
 
 struct RopeTable {
     DevBuf cos, sin;
-    int rows = 0;
+    int rows = 0, half = 0;
     void build(const RopeSpec& r, const std::vector<int32_t>& pos) {
         rows = (int)pos.size();
-        const size_t n = pos.size() * (size_t)(r.n_dims / 2);
+        half = r.n_dims / 2;
+        const size_t n = pos.size() * (size_t)half;
         std::vector<float> c(n), s(n);
         VLA_K(vla_rope_tables_host(pos.data(), rows, r.n_dims, (double)r.freq_base, c.data(), s.data()));
         cos.upload(c.data(), n * sizeof(float));
         sin.upload(s.data(), n * sizeof(float));
+    }
+    // Room for n rows that copy_rows() fills from table `of` on the device.
+    void reserve(const RopeTable& of, int n) {
+        rows = n;
+        half = of.half;
+        cos.reserve((size_t)n * half * sizeof(float));
+        sin.reserve((size_t)n * half * sizeof(float));
+    }
+    void copy_rows(int at, const RopeTable& of, int first, int n, hipStream_t st) {
+        if (first < 0 || n < 0 || first + n > of.rows || at + n > rows) throw std::logic_error("vla: rotation table rows out of range");
+        const size_t d = (size_t)at * half, s = (size_t)first * half, bytes = (size_t)n * half * sizeof(float);
+        if (bytes == 0) return;
+        VLA_HIP(hipMemcpyAsync(cos.as<float>() + d, of.cos.as<float>() + s, bytes, hipMemcpyDeviceToDevice, st));
+        VLA_HIP(hipMemcpyAsync(sin.as<float>() + d, of.sin.as<float>() + s, bytes, hipMemcpyDeviceToDevice, st));
     }
 };
 
