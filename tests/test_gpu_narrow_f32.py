@@ -93,3 +93,31 @@ def test_qkv(tune, B, S, Hq, Hkv, D, K, rope, kv):
             assert off(kc[:, :, P:P + S], y[:, :, Hq:Hq + Hkv].transpose(1, 2)) < TOL, plan
             assert off(vc[:, :, :, P:P + S], y[:, :, Hq + Hkv:].permute(0, 2, 3, 1)) < TOL, plan
             assert not kc[:, :, :P].any() and not kc[:, :, P + S:].any() and not vc[..., :P].any() and not vc[..., P + S:].any(), plan
+
+
+@pytest.mark.parametrize("arch,batch", [("smolvla", 1), ("smolvla", 3), ("smolvla", 11), ("pi0", 1)])
+def test_norms_inside_the_projection_launches(tmp_path, monkeypatch, arch, batch):
+    """An fp32 model with its RMSNorms inside the projections (few rows) against the same model with norms as launches of
+    their own: a norm inside rounds x w once and scales the sum, one apart rounds x rstd and times w; 1e-5 of the largest
+    output as for the models themselves.  Batch 3 mixes both (the gated projection has too many tiles), from batch 11 on
+    every projection of the suffix is the tiled one."""
+    import os
+
+    import numpy as np
+    from test_gpu_chunk import ckpt, ffi, make_obs
+
+    cfg = ckpt.smolvla_config(2, "f32", suffix_mask=1) if arch == "smolvla" else dict(ckpt.pi0_config(1), dtype="f32")
+    cfg = dict(cfg, ffn_dim=1024)
+    path = os.path.join(str(tmp_path), "m.vlaw")
+    ckpt.write_synthetic(path, cfg, ckpt.synth_weights(cfg, seed=77))
+    r = np.random.default_rng(5)
+    obs = [make_obs(cfg, r, n_views=2) for _ in range(batch)]
+    out = []
+    for apart in (False, True):
+        if apart:
+            monkeypatch.setenv("VLA_NO_NORM_FUSION", "1")
+        m = ffi.Model(path)
+        out.append(np.asarray(m.predict_batch(obs), np.float64))
+        m.close()
+    assert np.abs(out[0] - out[1]).max() / np.abs(out[1]).max() < 1e-5
+    assert not np.array_equal(out[0], out[1])  # the two are different launches (the final norm's too)

@@ -29,6 +29,7 @@
 
 #include "common.h"
 #include "gemm_common.h"
+#include "fused_f32.h"
 #include "gemm_f32.h"
 #include "gemm_wide.h"
 #include "tile_rules.h"
@@ -1876,7 +1877,7 @@ int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
     hipStream_t st = (hipStream_t)stream;
     if constexpr (std::is_same<T, float>::value) {
         // a few fp32 rows: narrow tiles (VLA_GEMM_TILE pins the tiled kernel instead)
-        bool rows_ok = a.M <= tuning().gemm_rows_max && a.norm_eps < 0.f && tuning().gemm_tile < 0 && ((uintptr_t)a.A | (uintptr_t)a.W) % 16 == 0;
+        bool rows_ok = a.M <= tuning().gemm_rows_max && (a.norm_eps < 0.f || (a.norm_w && a.K <= F32_NORM_MAX_K && (uintptr_t)a.norm_w % 16 == 0)) && tuning().gemm_tile < 0 && ((uintptr_t)a.A | (uintptr_t)a.W) % 16 == 0;
         const int force = tuning().gemm_rows_plan;
         const int plan = !rows_ok ? -1 : force == 1 || force == 3 ? force - 1 : vla_rules::narrow_plan_f32(a.M, a.N);
         if (plan >= 0) {
@@ -2081,7 +2082,8 @@ int vla_linear(const void* x, const void* W, const float* bias, const void* resi
 static int qkv_rope_impl(const void* x, const void* W, const float* bias, int dtype, int M, int K, int S, int n_q_heads,
                          int n_kv_heads, int has_k, int has_v, int head_dim, const float* cos_tab, const float* sin_tab,
                          void* q_out, void* k_cache, void* vt_cache, int t_max, int tok_offset, float rms_eps,
-                         vla_stream_t stream, const float* colsum = nullptr, const float* stats_in = nullptr, int n_stat = 0) {
+                         vla_stream_t stream, const float* colsum = nullptr, const float* stats_in = nullptr, int n_stat = 0,
+                         const float* norm_w = nullptr) {
     if (!x || !W || M < 0 || K <= 0 || S <= 0 || n_q_heads < 0 || n_kv_heads < 0 || head_dim <= 0) return VLA_K_ERR_ARG;
     const int nk = has_k ? n_kv_heads : 0, nv = has_v ? n_kv_heads : 0;
     if (n_q_heads > 0 && !q_out) return VLA_K_ERR_ARG;
@@ -2098,6 +2100,7 @@ static int qkv_rope_impl(const void* x, const void* W, const float* bias, int dt
     a.colsum = colsum;
     a.stats_in = stats_in;
     a.n_stat = n_stat;
+    a.norm_w = norm_w;
     a.A = x; a.W = W; a.bias = bias; a.M = M; a.K = K;
     a.N = (n_q_heads + nk + nv) * D;
     a.S = S; a.Hq = n_q_heads; a.nk = nk; a.nv = nv; a.D = D; a.Hkv = n_kv_heads;
@@ -2457,3 +2460,28 @@ int vla_ternary_repack_ladder_host(const uint8_t* ladder, int N, int K, uint32_t
 }
 
 }  // extern "C"
+
+namespace vk {
+
+int f32_rmsnorm_attn_qkv_rope(const float* x, const float* norm_w, float eps, const float* W, const float* bias, int M, int K, int S,
+                              int n_q_heads, int n_kv_heads, int has_k, int has_v, int head_dim, const float* cos_tab,
+                              const float* sin_tab, void* q_out, void* k_cache, void* vt_cache, int t_max, int tok_offset,
+                              vla_stream_t stream) {
+    if (!norm_w || eps < 0.f) return VLA_K_ERR_ARG;
+    return qkv_rope_impl(x, W, bias, VLA_DT_F32, M, K, S, n_q_heads, n_kv_heads, has_k, has_v, head_dim, cos_tab, sin_tab, q_out, k_cache,
+                         vt_cache, t_max, tok_offset, eps, stream, nullptr, nullptr, 0, norm_w);
+}
+
+int f32_rmsnorm_glu_linear(const float* x, const float* norm_w, float eps, const float* W_gate_up, void* y, int M, int I, int K, int act,
+                           vla_stream_t stream) {
+    if (!x || !norm_w || !W_gate_up || !y || eps < 0.f || M < 0 || I <= 0 || K <= 0) return VLA_K_ERR_ARG;
+    if (I % 32 || K % 4) return VLA_K_ERR_SHAPE;
+    GemmArgs a = {};
+    a.norm_eps = eps;
+    a.norm_w = norm_w;
+    a.A = x; a.W = W_gate_up; a.M = M; a.N = 2 * I; a.K = K;
+    a.Y = y; a.act = act;
+    return launch<float, EPI_GLU>(a, I / 32, stream);
+}
+
+}  // namespace vk

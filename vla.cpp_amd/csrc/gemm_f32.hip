@@ -14,13 +14,15 @@ using namespace vk;
 // keeps 16 accumulators in turn, which also shortens the sums: K / 64 products (four row blocks: K / 16) follow one
 // another before the partial sums are added in pairs, as in the FMA kernel this replaces, whose error against float64 it has
 // (50 x 720 x 960: 9.8e-8 of the norm both; tiled kernel 5.6e-7).  Half as many accumulators cost 1.2e-7 and gained 0.2 us.
+// NORM: the rows' RMSNorm inside.  The operand is x w (the weight, resident in LDS, is applied to the fragments), the sum of
+// squares is taken from the fragments, and row c of the result is scaled by 1 / sqrt(mean + eps).
 // A lane (c, q) reads 16 bytes, k = 4 q .. 4 q + 3 of a 16-k group, of row c; product t of the group takes element t of both
 // operands (k = t, 4 + t, 8 + t, 12 + t).  W is the left operand, so that a lane ends with columns 4 q .. 4 q + 3 of row c.
 // What bounds it: start and first loads (3 us), then per 256 k and wavefront 512 clocks of products beside 32 KiB of fill.
 // Against the FMA kernel (8 columns per workgroup, weights through L1; us): 50 x 720 x 960 10.8 -> 4.9, 50 x 1600 x 720 12.4 -> 6.1,
 // 50 x 720 x 2048 13.1 -> 6.5; against the tiled kernel: 50 x 4096 x 720 gated 19.8 -> 9.3, 241 x 640 x 960 22.5 -> 10.5, 100 x 720 x 2048
 // 43.5 -> 10.3.
-template <int kEpi, int RB, int KB, int NS, bool VEC>
+template <int kEpi, int RB, int KB, int NS, bool VEC, bool NORM>
 __global__ void __launch_bounds__(256) gemm_narrow_f32_kernel(GemmArgs a) {
     constexpr int BK = KB / 4, STAGE = (RB + 1) * 16 * KB, LPS = KB / 256, NLOAD = (RB + 1) * LPS;  // LPS: loads per thread and slab of 16 rows
     constexpr int KS = 4 / RB;        // wavefronts sharing a row block's K
@@ -29,7 +31,9 @@ __global__ void __launch_bounds__(256) gemm_narrow_f32_kernel(GemmArgs a) {
     static_assert((RB == 1 || RB == 4) && NG % 4 == 0, "one row block per workgroup or per wavefront; every accumulator has its turn in a stage");
     constexpr int IN_FLIGHT = (NS - 2) * NLOAD;
     static_assert(IN_FLIGHT <= 63 && NS * STAGE <= 160 * 1024, "ring depth");
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[NS * STAGE];
+    // NORM: the norm's weight and, after the walk, the wavefronts' partial sums of squares
+    constexpr int NORM_BYTES = NORM ? F32_NORM_MAX_K * 4 : 0;
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[NS * STAGE + NORM_BYTES];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, q = lane >> 4;
     const int n_t16 = (a.N + 15) / 16;
@@ -63,6 +67,10 @@ __global__ void __launch_bounds__(256) gemm_narrow_f32_kernel(GemmArgs a) {
             for (int i = 0; i <= RB; ++i) load_to_lds16(src[i * LPS + j] + k, lds0 + stage * STAGE + (i * LPS + j) * 4096);
         }
     };
+    if (NORM) {  // older than every operand load, so that the first stage's wait covers it
+        for (int k = wave * 256; k < a.K; k += 1024)  // uniform
+            load_to_lds16((const float*)a.norm_w + min(k + lane * 4, a.K - 4), (uint32_t)(uintptr_t)lds + NS * STAGE + k * 4);
+    }
 #pragma unroll
     for (int t = 0; t < NS - 1; ++t)
         if (t < nkt) issue(t, t);  // uniform
@@ -71,8 +79,9 @@ __global__ void __launch_bounds__(256) gemm_narrow_f32_kernel(GemmArgs a) {
     f32x4_t acc[NACC];
 #pragma unroll
     for (int j = 0; j < NACC; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    f32x4_t ssq = {0.f, 0.f, 0.f, 0.f};  // squares of this lane's pieces of its row
     const int fx0 = (rb * 16 + c) * KB, fw0 = (RB * 16 + c) * KB;
-    auto multiply = [&](int stage, int k_left) __attribute__((always_inline)) {  // k_left: k of this tile inside K (the last tile), or BK
+    auto multiply = [&](int stage, int kt, int k_left) __attribute__((always_inline)) {  // k_left: k of this tile inside K (the last tile), or BK
         const unsigned char* base = lds + stage * STAGE;
         f32x4_t fx[NG], fw[NG];
 #pragma unroll
@@ -81,6 +90,11 @@ __global__ void __launch_bounds__(256) gemm_narrow_f32_kernel(GemmArgs a) {
             fx[g] = *reinterpret_cast<const f32x4_t*>(base + fx0 + off);
             fw[g] = *reinterpret_cast<const f32x4_t*>(base + fw0 + off);
         }
+        f32x4_t nw[NORM ? NG : 1];
+        if (NORM) {  // past K: some weight, beside an operand that is zeroed
+#pragma unroll
+            for (int g = 0; g < NG; ++g) nw[g] = *reinterpret_cast<const f32x4_t*>(lds + NS * STAGE + min(kt * BK + (g * KS + ks) * 16 + 4 * q, F32_NORM_MAX_K - 4) * 4);
+        }
         if (k_left < BK) {  // K is a multiple of 4: a piece is inside or outside as a whole
             const f32x4_t z = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -88,6 +102,14 @@ __global__ void __launch_bounds__(256) gemm_narrow_f32_kernel(GemmArgs a) {
                 if ((g * KS + ks) * 16 + 4 * q >= k_left) fx[g] = fw[g] = z;
         }
         __builtin_amdgcn_sched_barrier(0);  // all reads requested before the first product
+        if (NORM) {
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) ssq[e] = fmaf(fx[g][e], fx[g][e], ssq[e]);
+                fx[g] *= nw[g];
+            }
+        }
 #pragma unroll
         for (int g = 0; g < NG; ++g)
 #pragma unroll
@@ -99,13 +121,14 @@ __global__ void __launch_bounds__(256) gemm_narrow_f32_kernel(GemmArgs a) {
         wait_vmcnt<IN_FLIGHT>();
         __syncthreads();  // this stage has landed for every wavefront; stage ls has been read by everyone
         issue(kt + NS - 1, ls);
-        multiply(cs, BK);
+        multiply(cs, kt, BK);
         cs = (cs + 1 == NS) ? 0 : cs + 1;
         ls = (ls + 1 == NS) ? 0 : ls + 1;
     }
     narrow_tail<NS - 1, NLOAD>(nkt, [&](bool last) __attribute__((always_inline)) {
         __syncthreads();
-        multiply(cs, last ? a.K - (nkt - 1) * BK : BK);
+        multiply(cs, kt, last ? a.K - (nkt - 1) * BK : BK);
+        ++kt;
         cs = (cs + 1 == NS) ? 0 : cs + 1;
     });
 #pragma unroll
@@ -113,13 +136,23 @@ __global__ void __launch_bounds__(256) gemm_narrow_f32_kernel(GemmArgs a) {
 #pragma unroll
         for (int j = 0; j < w; ++j) acc[j] += acc[j + w];
     f32x4_t sum = acc[0];
+    float sq = NORM ? rows_sum((ssq[0] + ssq[1]) + (ssq[2] + ssq[3])) : 0.f;  // of row c, over this wavefront's share of K
     if (KS > 1) {
         __syncthreads();  // the ring has been read by everyone
         f32x4_t* part = reinterpret_cast<f32x4_t*>(lds);  // [ks][rb][lane]
-        if (ks > 0) part[(ks * RB + rb) * 64 + lane] = sum;
+        float* part_sq = reinterpret_cast<float*>(lds + KS * RB * 1024);  // [ks][rb][c]
+        if (ks > 0) {
+            part[(ks * RB + rb) * 64 + lane] = sum;
+            if (NORM && q == 0) part_sq[(ks * RB + rb) * 16 + c] = sq;
+        }
         __syncthreads();
         if (ks > 0) return;
         sum = (sum + part[(RB + rb) * 64 + lane]) + (part[(2 * RB + rb) * 64 + lane] + part[(3 * RB + rb) * 64 + lane]);
+        if (NORM) sq = (sq + part_sq[(RB + rb) * 16 + c]) + (part_sq[(2 * RB + rb) * 16 + c] + part_sq[(3 * RB + rb) * 16 + c]);
+    }
+    if (NORM) {
+        const float rstd = 1.0f / sqrtf(sq / (float)a.K + a.norm_eps);
+        sum *= f32x4_t{rstd, rstd, rstd, rstd};
     }
 
     const int m = m0 + rb * 16 + c;
@@ -206,14 +239,14 @@ __global__ void __launch_bounds__(256) gemm_narrow_f32_kernel(GemmArgs a) {
     }
 }
 
-template <int kEpi, bool VEC>
+template <int kEpi, bool VEC, bool NORM>
 void launch_plan(const GemmArgs& a, int plan, hipStream_t st) {
     const unsigned grid = (unsigned)vla_rules::narrow_grid(a.M, a.N, plan);
     // Three stages (96 KiB: all of K = 720 requested at once) while every workgroup has a CU of its own, else two (64 KiB), so
     // that two share a CU: 50 x 720 x 960 (180 workgroups) 4.9 us and 5.2, 50 x 1600 x 720 (400) 7.4 us and 6.1.
-    if (plan) gemm_narrow_f32_kernel<kEpi, 4, 512, 3, VEC><<<grid, 256, 0, st>>>(a);
-    else if (grid <= 256) gemm_narrow_f32_kernel<kEpi, 1, 1024, 3, VEC><<<grid, 256, 0, st>>>(a);
-    else gemm_narrow_f32_kernel<kEpi, 1, 1024, 2, VEC><<<grid, 256, 0, st>>>(a);
+    if (plan) gemm_narrow_f32_kernel<kEpi, 4, 512, 3, VEC, NORM><<<grid, 256, 0, st>>>(a);
+    else if (grid <= 256) gemm_narrow_f32_kernel<kEpi, 1, 1024, 3, VEC, NORM><<<grid, 256, 0, st>>>(a);
+    else gemm_narrow_f32_kernel<kEpi, 1, 1024, 2, VEC, NORM><<<grid, 256, 0, st>>>(a);
 }
 
 }  // namespace
@@ -224,8 +257,16 @@ template <int kEpi>
 void launch_narrow_f32(const GemmArgs& a, int plan, hipStream_t st) {
     // four columns at a time where they are inside a row as a whole and aligned, else one by one
     const uintptr_t io = kEpi == EPI_QKV ? (uintptr_t)a.q_out | (uintptr_t)a.k_cache : (uintptr_t)a.Y | (uintptr_t)a.residual;
-    if ((kEpi != EPI_PLAIN || a.N % 4 == 0) && io % 16 == 0) launch_plan<kEpi, true>(a, plan, st);
-    else launch_plan<kEpi, false>(a, plan, st);
+    const bool vec = (kEpi != EPI_PLAIN || a.N % 4 == 0) && io % 16 == 0;
+    if constexpr (kEpi != EPI_PLAIN) {
+        if (a.norm_eps >= 0.f) {
+            if (vec) launch_plan<kEpi, true, true>(a, plan, st);
+            else launch_plan<kEpi, false, true>(a, plan, st);
+            return;
+        }
+    }
+    if (vec) launch_plan<kEpi, true, false>(a, plan, st);
+    else launch_plan<kEpi, false, false>(a, plan, st);
 }
 template void launch_narrow_f32<EPI_PLAIN>(const GemmArgs&, int, hipStream_t);
 template void launch_narrow_f32<EPI_QKV>(const GemmArgs&, int, hipStream_t);

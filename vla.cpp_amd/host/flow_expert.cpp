@@ -149,6 +149,7 @@ class FlowExpert : public ModelArch {
     int text_every_ = 2, P_txt_ = 0;
     DevBuf vlln_sc_, vlln_sh_;  // vlln as (weight - 1, bias) fp32 [Wv]: the modulated-norm launch computes xn (1 + sc) + sh
     float vlln_eps_ = 1e-5f;
+    bool fuse_f32_norm_ = false;   // fp32 RMS archs: norms inside the projection launches where the rows are few
     bool fuse_final_norm_ = true;  // the final norm runs inside the Euler launch
     bool fuse_self_block_ = true;  // GR00T self blocks: norm, projections and attention in one launch (VLA_NO_FUSED_SELF_BLOCK=1: off)
     bool hand_row_stats_ = true;   // GR00T from batch 32: a block's Wo launch leaves the row sums the next block's LayerNorm needs (VLA_NO_ROW_STATS=1: off)
@@ -299,6 +300,7 @@ FlowExpert::FlowExpert(const Checkpoint& ck) {
 
     const bool no_norm_fusion = std::getenv("VLA_NO_NORM_FUSION") != nullptr;  // read once, at load
     fuse_final_norm_ = !no_norm_fusion;
+    fuse_f32_norm_ = !no_norm_fusion && dt_ == VLA_DT_F32 && arch_ != Arch::GR00T && !adarms_;
     fuse_self_block_ = !no_norm_fusion && std::getenv("VLA_NO_FUSED_SELF_BLOCK") == nullptr;
     hand_row_stats_ = !no_norm_fusion && std::getenv("VLA_NO_ROW_STATS") == nullptr;
     layers_.resize(L_);
@@ -780,11 +782,14 @@ void FlowExpert::prefill(const Inputs* in, int batch) {
             prof_mark("prefix_kv_proj");
             continue;
         }
-        rms_norm(C, xp, w.vlm_ln.get(), eps_, xn);
-        prof_mark("prefix_norm");
+        KVLayer& kv_first = arch_ == Arch::SMOLVLA && !w.is_self ? tmp_kv_ : w.kv;  // cross layers project these K and V again
+        if (!(fuse_f32_norm_ && f32_rmsnorm_qkv_rope_append(C, xp, w.vlm_ln, eps_, Wkv, bkv, P, 0, true, true, rope_prefix, nullptr, kv_first, 0))) {
+            rms_norm(C, xp, w.vlm_ln.get(), eps_, xn);
+            prof_mark("prefix_norm");
+            qkv_rope_append(C, xn, Wkv, bkv, P, 0, true, true, rope_prefix, nullptr, kv_first, 0);
+        }
         if (arch_ == Arch::SMOLVLA && !w.is_self) {
             // expert_cross_kv: K = Wk_x . cachedK_flat, V = Wv_x . cachedV_flat, no second rotation
-            qkv_rope_append(C, xn, Wkv, bkv, P, 0, true, true, rope_prefix, nullptr, tmp_kv_, 0);
             VLA_K(vla_kv_gather(tmp_kv_.k.get(), tmp_kv_.vt.get(), tmpk_.get(), tmpv_.get(), dt_, B, Hkv_, D_,
                                 tmp_kv_.t_max, 0, P, C.stream));
             Tensor tk = tensor_2d(tmpk_.get(), dt_, kvd, (int64_t)B * P), tv = tensor_2d(tmpv_.get(), dt_, kvd, (int64_t)B * P);
@@ -793,7 +798,6 @@ void FlowExpert::prefill(const Inputs* in, int batch) {
             qkv_rope_append(C, tv, Wvx, nullptr, P, 0, false, true, nullptr, nullptr, w.kv, 0);
             prof_mark("prefix_kv_proj_and_cross_reprojection");
         } else {
-            qkv_rope_append(C, xn, Wkv, bkv, P, 0, true, true, rope_prefix, nullptr, w.kv, 0);
             prof_mark("prefix_kv_proj");
         }
     }
@@ -871,6 +875,10 @@ void FlowExpert::run_steps(int n_steps, void* stream) {
                 if (!done && w.Wqkv_ln) {
                     Tensor Wf = tensor_2d(w.Wqkv_ln.get(), dt_, W_, n_rows_w);
                     done = rmsnorm_qkv_rope_append(C, h, Wf, bq, eps_, S_, Hq_, w.is_self, w.is_self, tab, Q.data, w.kv, tok);
+                }
+                if (!done && fuse_f32_norm_) {
+                    Tensor Wqkv = tensor_2d(w.Wqkv.get(), dt_, W_, n_rows_w);
+                    done = f32_rmsnorm_qkv_rope_append(C, h, w.ln, eps_, Wqkv, bq, S_, Hq_, w.is_self, w.is_self, tab, Q.data, w.kv, tok);
                 }
                 // a GR00T self block without prefix rows, mask or rotation: norm, projections and attention in one launch
                 // (from batch 32 on: a workgroup of that launch takes eight observations and one head, and below
@@ -964,9 +972,10 @@ void FlowExpert::run_steps(int n_steps, void* stream) {
                             Tensor Wf = tensor_2d(w.Wgu_ln.get(), dt_, W_, 2 * (int64_t)I_);
                             fused = ffn_glu(C, Wf, act, Wd, h, eps_, h.data, mid, h);
                         }
+                        Tensor Wgu = tensor_2d(w.Wgu.get(), dt_, W_, 2 * (int64_t)I_);
+                        if (!fused && fuse_f32_norm_) fused = f32_rmsnorm_ffn_glu(C, h, w.ln2, eps_, Wgu, act, Wd, h.data, mid, h);
                         if (!fused) {
                             rms_norm(C, h, w.ln2.get(), eps_, hn);
-                            Tensor Wgu = tensor_2d(w.Wgu.get(), dt_, W_, 2 * (int64_t)I_);
                             ffn_glu(C, Wgu, act, Wd, hn, -1.f, h.data, mid, h);
                         }
                         prof_mark("ffn_gate_up_down");

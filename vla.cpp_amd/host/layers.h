@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "device.h"
+#include "fused_f32.h"
 #include "vla_kernels.h"
 
 namespace vla {
@@ -201,6 +202,30 @@ inline bool rmsnorm_qkv_rope_append(Ctx& C, const Tensor& x, const Tensor& W_fol
                                              q_out, kv.k.get(), kv.vt.get(), kv.t_max, tok_offset, eps, C.stream);
     if (rc == VLA_K_ERR_SHAPE) return false;
     VLA_K(rc);
+    return true;
+}
+
+// The two launches of an fp32 stream in which its RMSNorm is taken inside, weights as they are; false where the rows are too
+// many for them (nothing was launched then).
+inline bool f32_rmsnorm_qkv_rope_append(Ctx& C, const Tensor& x, const DevBuf& norm_w, float eps, const Tensor& W, const float* bias, int S,
+                                        int n_q_heads, bool has_k, bool has_v, const RopeTable* tab, void* q_out, KVLayer& kv,
+                                        int tok_offset) {
+    const int rc = vk::f32_rmsnorm_attn_qkv_rope((const float*)x.data, norm_w.as<float>(), eps, (const float*)W.data, bias, (int)x.rows(),
+                                                 (int)x.ne[0], S, n_q_heads, kv.n_kv_heads, has_k ? 1 : 0, has_v ? 1 : 0, kv.head_dim,
+                                                 tab ? tab->cos.as<float>() : nullptr, tab ? tab->sin.as<float>() : nullptr, q_out,
+                                                 kv.k.get(), kv.vt.get(), kv.t_max, tok_offset, C.stream);
+    if (rc == VLA_K_ERR_SHAPE) return false;
+    VLA_K(rc);
+    return true;
+}
+inline bool f32_rmsnorm_ffn_glu(Ctx& C, const Tensor& x, const DevBuf& norm_w, float eps, const Tensor& Wgu, int act, const Tensor& Wd,
+                                const void* residual, Tensor& mid, Tensor& y) {
+    const int rc = vk::f32_rmsnorm_glu_linear((const float*)x.data, norm_w.as<float>(), eps, (const float*)Wgu.data, mid.data, (int)x.rows(),
+                                              (int)(Wgu.ne[1] / 2), (int)Wgu.ne[0], act, C.stream);
+    if (rc == VLA_K_ERR_SHAPE) return false;
+    VLA_K(rc);
+    VLA_K(vla_linear(mid.data, Wd.data, nullptr, residual, y.data, mid.dtype, y.dtype, (int)mid.rows(), (int)Wd.ne[1],
+                     (int)Wd.ne[0], C.stream));
     return true;
 }
 
