@@ -16,6 +16,7 @@ def rules(tmp_path_factory):
         f.write('''#include "tile_rules.h"
 extern "C" int plan(int M, int N, int K, int qkv) { return vla_rules::narrow_plan(M, N, K, qkv); }
 extern "C" int plan_f32(int M, int N) { return vla_rules::narrow_plan_f32(M, N); }
+extern "C" int rows_kernel(int bf16, int grid, int blocks, int sliced) { return vla_rules::attn_rows(bf16, grid, blocks, sliced); }
 extern "C" int wide(int M, int N, int K, int kind) { return vla_rules::wide_tile(M, N, K, kind); }
 extern "C" int ternary(int M, int N, int K) { return vla_rules::ternary_tile(M, N, K); }
 extern "C" int rows(int p) { return 16 * vla_rules::NARROW_PLANS[p][0]; }
@@ -139,3 +140,11 @@ def test_a_wide_tile_is_named_for_every_size(rules):
             for K in (16, 720, 8192, 1 << 20):
                 for kind in (0, 1, 2):
                     assert -1 <= rules.wide(M, N, K, kind) < 6
+
+
+def test_attention_rows_only_while_the_workgroups_are_few(rules):
+    for blocks in (1, 8, 9, 20, 21, 1000):
+        for sliced in (0, 1):
+            assert rules.rows_kernel(1, 448, blocks, sliced) and not rules.rows_kernel(1, 513, blocks, sliced)
+            assert rules.rows_kernel(1, 512, blocks, sliced) == (blocks <= 8)
+            assert rules.rows_kernel(0, 512, blocks, sliced) == (blocks <= 20 or not sliced) and not rules.rows_kernel(0, 513, blocks, sliced)

@@ -42,6 +42,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "tile_rules.h"
 #include "vla_kernels.h"
 
 namespace {
@@ -1756,6 +1757,247 @@ __global__ void __launch_bounds__(256, 1) attn_stream_kernel(AttnArgs a, int n_u
     wait_vm_mem<0>();  // the ring's trailing loads still target this wavefront's LDS
 }
 
+// ---- 48- and 64-wide heads, some tens to a few hundred query rows per kv head, few workgroups (one or a few observations) ----
+// The tiled kernel gives such a launch few workgroups (15 at batch 1) that walk the keys one tile after the other, a barrier
+// and a trip to memory each; fp32 has to slice the keys over workgroups and pay a merge launch for it.  Here a workgroup
+// owns 16 rows of a (batch, kv head) and its wavefronts own the 32-key blocks, one each while there are no more blocks than
+// wavefronts: every byte of K and V^T is requested at the start of the launch, one trip to memory deep.  A wavefront's block
+// goes straight into LDS of its own (K rows are contiguous, V^T rows one 32-key run each), so no barrier is needed until the
+// wavefronts' (max, sum, output) meet in LDS.
+// Products as in the decode kernel: S^T = K Q^T as two 16-key products, row i of product j standing for key 8 (i / 4) + 4 j +
+// i % 4 of the block, so that lane (c, q) holds the scores of keys 8 q .. 8 q + 7 against row c: already the right operand of
+// O^T += V^T P^T.  bf16: 16x16x32; fp32: 16x16x4, product t of a 16-d group taking element t of the lanes' 16-byte pieces.
+// LDS pieces (16 bytes) are XOR-swizzled so that the fragment reads, served sixteen lanes at a time (lanes 0-3, 12-15, 20-27 and
+// so on), are free of bank conflicts: K by the lane that reads the row, V^T rows of 64 bytes by row / 4 times 2 in GF(4),
+// of 128 bytes by row / 2 + 2.
+// K rows of 48-wide heads are kept as if 64 wide; what lies past the head repeats its last piece and meets zeros of Q.
+template <typename T, int D> struct RowsT {
+    static constexpr int EB = sizeof(T), KROW = 64 * EB, VROW = 32 * EB, BLK = 32 * KROW + D * VROW;
+    static constexpr int WAVES = sizeof(T) == 2 ? 16 : 10;  // that a CU's LDS and registers hold
+};
+// W: wavefronts that the workgroup's LDS has room for; as many are launched as the blocks are shared out over evenly.
+template <typename T, int D, int W>
+__global__ void __launch_bounds__(W * 64) attn_rows_kernel(AttnArgs a) {
+    typedef RowsT<T, D> RT;
+    constexpr int EB = RT::EB, NDB = D / 16, KPR = RT::KROW / 16, VPR = RT::VROW / 16, VE = 16 / EB, PIECES = D * EB / 16;
+    constexpr int OSTRIDE = D + 4;  // floats between the rows of a wavefront's partial output
+    constexpr int NK = 32 * RT::KROW / 1024, NV = D * RT::VROW / 1024;  // load instructions of a block
+    constexpr int NQ = (PIECES + 3) / 4;  // 16-byte pieces of a row per lane
+    static_assert(OSTRIDE * 16 * 4 + 128 <= RT::BLK, "partial rows fit a wavefront's LDS");
+    constexpr bool F32 = EB == 4;
+    __shared__ __attribute__((aligned(1024))) unsigned char rows_lds[W * RT::BLK];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = (int)(blockDim.x >> 6);
+    const int c = lane & 15, q = lane >> 4;
+    // the row tiles of a pair sit eight workgroups apart, on one XCD: they share its L2's copy of K and V^T
+    const int R = a.grp * a.S, local = (int)blockIdx.x >> 3, p8 = (int)div_c(local, a.dGS);
+    const int tile = local - p8 * a.n_groups, pair = p8 * 8 + ((int)blockIdx.x & 7);  // n_groups: row tiles of a pair
+    if (pair >= a.batch * a.Hkv) return;
+    const int b = (int)div_c(pair, a.dHkv), hk = pair - b * a.Hkv;
+    const int nb = (a.n_keys + 31) / 32;
+
+    unsigned char* const kl = rows_lds + wave * RT::BLK;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)kl;
+    const unsigned char* kbase = (const unsigned char*)a.k_cache + ((long)b * a.Hkv + hk) * a.t_max * D * EB;
+    const unsigned char* vbase = (const unsigned char*)a.vt_cache + ((long)b * a.Hkv + hk) * D * (long)a.t_max * EB;
+    // row of the block -> lane c whose fragment it is
+    auto k_lane = [](int row) __attribute__((always_inline)) { return (row & 3) | (((row >> 3) & 3) << 2); };
+    auto v_swz = [](int row) __attribute__((always_inline)) {
+        const int x = (row >> 2) & 3;
+        return F32 ? ((row >> 1) + 2) & 7 : ((x << 1) ^ ((x >> 1) * 3)) & 3;
+    };
+    // K rows past n_keys repeat the last key (their scores are masked); V^T runs past the cache row are moved back into it and
+    // those past n_keys zeroed as fragments (stale cache contents may be NaN).
+    auto issue = [&](int kb) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NK; ++i) {
+            const int row = i * (32 / NK) + lane / KPR, piece = (lane % KPR) ^ (F32 ? k_lane(row) : k_lane(row) >> 1);
+            load_to_lds16(kbase + ((long)min(kb * 32 + row, a.n_keys - 1) * D * EB + min(piece, PIECES - 1) * 16), lds0 + i * 1024);
+        }
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int row = i * (D / NV) + lane / VPR, piece = (lane % VPR) ^ v_swz(row);
+            load_to_lds16(vbase + ((long)row * a.t_max + min(kb * 32 + piece * VE, a.t_max - VE)) * EB, lds0 + 32 * RT::KROW + i * 1024);
+        }
+    };
+    issue(wave);  // nw <= nb: every wavefront has a block
+
+    const int row = tile * 16 + c;
+    const bool row_valid = row < R;
+    const int rr = row_valid ? row : 0, hg = (int)div_c(rr, a.dS), s = rr - hg * a.S, h = hk * a.grp + hg;
+    u32x4_t qf[NQ];
+    {
+        const unsigned char* qrow = (const unsigned char*)a.q + (((long)b * a.S + s) * a.Hq + h) * D * EB + q * 16;
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) {
+            const u32x4_t z = {0u, 0u, 0u, 0u};
+            qf[i] = 4 * i + 3 < PIECES || 4 * i + q < PIECES ? *reinterpret_cast<const u32x4_t*>(qrow + i * 64) : z;
+        }
+    }
+    int hi = a.n_keys;
+    if (a.mask_kind == VLA_MASK_CAUSAL_SUFFIX) hi = min(a.n_keys, a.n_prefix + s + 1);
+    else if (a.mask_kind == VLA_MASK_PI0_STATE && s == 0) hi = min(a.n_keys, a.n_prefix + 1);
+    const int pad_lo = a.pad_start, pad_hi = min(a.pad_end, a.n_prefix);
+    constexpr float LOG2E = 1.4426950408889634f;
+    const float c2 = a.scale * LOG2E;
+    f32x4_t o[NDB];
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) o[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    float m_run = -INFINITY, l_run = 0.f;
+
+    for (int kb = wave; kb < nb; kb += nw) {
+        wait_vmcnt<0>();
+        asm volatile("" ::: "memory");
+        u32x4_t kf[2][NQ], vf[NDB][F32 ? 2 : 1];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int i = 0; i < NQ; ++i)
+                kf[j][i] = *reinterpret_cast<const u32x4_t*>(kl + (8 * (c >> 2) + (c & 3) + 4 * j) * RT::KROW + (((4 * i + q) ^ (F32 ? c : c >> 1)) * 16));
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+            for (int i = 0; i < (F32 ? 2 : 1); ++i) {
+                const int d = db * 16 + c, piece = F32 ? 2 * q + i : q;
+                vf[db][i] = *reinterpret_cast<const u32x4_t*>(kl + 32 * RT::KROW + d * RT::VROW + ((piece ^ v_swz(d)) * 16));
+            }
+        if (4 * NQ > PIECES) {  // beside the zeros of Q, or an infinity in K's last piece would be a NaN
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                if (4 * (NQ - 1) + q >= PIECES) kf[j][NQ - 1] = u32x4_t{0u, 0u, 0u, 0u};
+        }
+        f32x4_t sc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int i = 0; i < NQ; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                if constexpr (F32) {
+                    const f32x4_t kv = __builtin_bit_cast(f32x4_t, kf[j][i]), qv = __builtin_bit_cast(f32x4_t, qf[i]);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) sc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[t], qv[t], sc[j], 0, 0, 0);
+                } else {
+                    sc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[j][i]), __builtin_bit_cast(bf16x8_t, qf[i]), sc[j], 0, 0, 0);
+                }
+            }
+        const int k0 = kb * 32, key0 = k0 + 8 * q, nvalid = a.n_keys - key0;  // real keys among this lane's 8, may be <= 0
+        if (k0 + 32 > a.n_keys) {  // uniform
+#pragma unroll
+            for (int db = 0; db < NDB; ++db)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if constexpr (F32) {
+                        vf[db][0][e] = e < nvalid ? vf[db][0][e] : 0u;
+                        vf[db][1][e] = 4 + e < nvalid ? vf[db][1][e] : 0u;
+                    } else {
+                        vf[db][0][e] &= (2 * e < nvalid ? 0xffffu : 0u) | (2 * e + 1 < nvalid ? 0xffff0000u : 0u);
+                    }
+                }
+        }
+        float p[8];  // keys key0 + i
+#pragma unroll
+        for (int i = 0; i < 8; ++i) p[i] = sc[i >> 2][i & 3] * c2;
+        if (a.mask) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) p[i] = i < nvalid ? p[i] + a.mask[(long)s * a.n_keys + key0 + i] * LOG2E : -INFINITY;
+        } else if (k0 + 32 > a.n_keys || (k0 < pad_hi && k0 + 32 > pad_lo) || (a.mask_kind != VLA_MASK_NONE && k0 + 32 > a.n_prefix)) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int key = key0 + i;
+                const bool visible = (key < hi) & !((key >= pad_lo) & (key < pad_hi));
+                p[i] = visible ? p[i] : -INFINITY;
+            }
+        }
+        float m_new = m_run;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) m_new = fmaxf(m_new, p[i]);
+        m_new = rows_max(m_new);
+        const float m_use = m_new == -INFINITY ? 0.f : m_new, alpha = __builtin_amdgcn_exp2f(m_run - m_use);  // first block: 0
+        m_run = m_new;
+        float psum = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            p[i] = __builtin_amdgcn_exp2f(p[i] - m_use);
+            psum += p[i];
+        }
+        l_run = l_run * alpha + rows_sum(psum);
+        u32x4_t pf;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) pf[e] = pack_bf2(p[2 * e], p[2 * e + 1]);
+#pragma unroll
+        for (int db = 0; db < NDB; ++db) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[db][e] *= alpha;
+            if constexpr (F32) {
+#pragma unroll
+                for (int t = 0; t < 8; ++t)
+                    o[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(f32x4_t, vf[db][t >> 2])[t & 3], p[t], o[db], 0, 0, 0);
+            } else {
+                o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, vf[db][0]), __builtin_bit_cast(bf16x8_t, pf), o[db], 0, 0, 0);
+            }
+        }
+        if (kb + nw < nb) {  // uniform; only with more blocks than wavefronts
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this block's fragments are in registers
+            issue(kb + nw);
+        }
+    }
+
+    // The wavefronts' partial rows meet in the LDS that each has read by now: output [16][D + 4], then (max, sum) [16].
+    float* const po = reinterpret_cast<float*>(kl);
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) *reinterpret_cast<f32x4_t*>(po + c * OSTRIDE + db * 16 + 4 * q) = o[db];
+    if (q == 0) *reinterpret_cast<f32x2_t*>(po + 16 * OSTRIDE + 2 * c) = f32x2_t{m_run, l_run};
+    __syncthreads();
+    for (int item = tid; item < 16 * (D / 4); item += (int)blockDim.x) {  // four columns of a row each
+        const int r = item / (D / 4), d0 = (item % (D / 4)) * 4, orow = tile * 16 + r;
+        if (orow >= R) continue;
+        f32x2_t ml[W];
+        f32x4_t ow[W];
+#pragma unroll
+        for (int w = 0; w < W; ++w) {  // all requested before the first is used; past nw the last one again
+            const float* pw = reinterpret_cast<const float*>(rows_lds + min(w, nw - 1) * RT::BLK);
+            ml[w] = *reinterpret_cast<const f32x2_t*>(pw + 16 * OSTRIDE + 2 * r);
+            ow[w] = *reinterpret_cast<const f32x4_t*>(pw + r * OSTRIDE + d0);
+        }
+        float m = ml[0][0];
+#pragma unroll
+        for (int w = 1; w < W; ++w) m = fmaxf(m, ml[w][0]);
+        const float m_use = m == -INFINITY ? 0.f : m;
+        float l = 0.f;
+        f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            const float f = w < nw ? __builtin_amdgcn_exp2f(ml[w][0] - m_use) : 0.f;
+            l += ml[w][1] * f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] += ow[w][e] * f;
+        }
+        const float inv = l > 0.f ? 1.0f / l : 0.f;
+        const int og = (int)div_c(orow, a.dS), os = orow - og * a.S;
+        const long oo = (((long)b * a.S + os) * a.Hq + hk * a.grp + og) * D + d0;
+        if constexpr (F32) *reinterpret_cast<f32x4_t*>((float*)a.out + oo) = f32x4_t{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
+        else *reinterpret_cast<u32x2_t*>((bf16_t*)a.out + oo) = u32x2_t{pack_bf2(acc[0] * inv, acc[1] * inv), pack_bf2(acc[2] * inv, acc[3] * inv)};
+    }
+}
+
+// The launch of attn_rows_kernel: false, launching nothing, where the call is not one of its.
+template <typename T, int D>
+bool launch_rows(AttnArgs& a, hipStream_t st) {
+    const Tuning& tn = tuning();
+    if (tn.attn_rows == 0 || a.p2 || (((uintptr_t)a.q | (uintptr_t)a.k_cache | (uintptr_t)a.vt_cache | (uintptr_t)a.out) & 15)) return false;
+    constexpr int W = RowsT<T, D>::WAVES;
+    const int R = (a.Hq / a.Hkv) * a.S, n_tiles = (R + 15) / 16, nb = (a.n_keys + 31) / 32;
+    const long grid = ((long)a.batch * a.Hkv + 7) / 8 * 8 * n_tiles;
+    if (grid >= (1l << 31)) return false;
+    if (tn.attn_rows < 0 && !vla_rules::attn_rows(sizeof(T) == 2, grid, nb, a.n_split > 1)) return false;
+    const int steps = (nb + W - 1) / W, nw = (nb + steps - 1) / steps;
+    a.n_groups = n_tiles;
+    a.n_split = 1;
+    set_divisors(a, grid);
+    // half the LDS while that is room enough: two workgroups then share a CU
+    if (nw <= W / 2) attn_rows_kernel<T, D, W / 2><<<(unsigned)grid, nw * 64, 0, st>>>(a);
+    else attn_rows_kernel<T, D, W><<<(unsigned)grid, nw * 64, 0, st>>>(a);
+    return true;
+}
+
 // Merge of key-split partials as a launch of its own: one wavefront per (pair, row).
 template <typename T, bool HALF>
 __global__ void __launch_bounds__(256) attn_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
@@ -2050,6 +2292,10 @@ int launch_d(AttnArgs& a, vla_stream_t stream, Scratch& sc) {
     }
     if (sc.kind == Scratch::DRY) return VLA_K_OK;
     a.arrive = nullptr;
+    // (after the scratch is bound: a call is refused for want of it whichever kernel serves it)
+    if constexpr (D == 64 || D == 48) {
+        if (launch_rows<T, D>(a, st)) return hipGetLastError() == hipSuccess ? VLA_K_OK : VLA_K_ERR_LAUNCH;
+    }
     switch (nw) {
         case 1: return launch_nw<T, D, 1>(a, st);
         case 2: return launch_nw<T, D, 2>(a, st);

@@ -178,4 +178,16 @@ inline int ternary_tile(long M, long N, long K) {
     return best;
 }
 
+// Whether an attention launch of 48- or 64-wide heads takes 16 rows per workgroup with the 32-key blocks shared out over
+// its wavefronts (`grid` workgroups, `blocks` key blocks) instead of the tiled kernel, which reads K and V^T once per 64 to
+// 128 rows but walks the keys.  About two rounds of workgroups: 50 rows x 15 heads on 5, 227 keys: 1, 4, 8, 16 observations (50,
+// 200, 400, 800 workgroups) 8.9, 9.1, 9.2, 9.8 us tiled and 4.9, 5.1, 6.2, 9.9 here; with more than eight blocks a CU holds one
+// workgroup: 512 keys 10.5, 10.8, 11.1, 11.6 and 5.8, 6.3, 10.7, 18.2.  fp32: 13.0, 25.2, 25.9, 26.6 and 7.3, 7.8, 13.4, 23.9; where the tiled
+// kernel slices the keys over workgroups, more than two blocks per wavefront (ten of them) are left to it: 16 rows x 16 heads on
+// 4, 1000 keys 14.8 us, here 16.0 (one slice only: 50 x 15 on 5, two observations 87.9, here 17.1).
+inline bool attn_rows(bool bf16, long grid, int blocks, bool sliced) {
+    if (bf16) return grid <= (blocks <= 8 ? 512 : 448);
+    return grid <= 512 && (blocks <= 20 || !sliced);
+}
+
 }  // namespace vla_rules
