@@ -82,6 +82,26 @@ void host_linear(const float* W, const float* b, const float* x, float* y, int N
         y[n] = (float)(a + (b ? (double)b[n] : 0.0));
     }
 }
+// W [N][K] -> W^T [K][N]
+std::vector<float> transposed(const std::vector<float>& W, int N, int K) {
+    std::vector<float> t(W.size());
+    for (int n = 0; n < N; ++n)
+        for (int k = 0; k < K; ++k) t[(size_t)k * N + n] = W[(size_t)n * K + k];
+    return t;
+}
+// The same product from W^T: every output's sum in the same order, hence the same bits, but the outputs side by side in vector
+// registers instead of one chain of dependent additions (the DiT head's state encoder, 1.6 M products per observation, was
+// 1.2 ms of a GR00T prediction).
+void host_linear_t(const float* Wt, const float* b, const float* x, float* y, int N, int K) {
+    std::vector<double> acc((size_t)N, 0.0);
+    double* const a = acc.data();
+    for (int k = 0; k < K; ++k) {
+        const double xk = (double)x[k];
+        const float* wr = Wt + (size_t)k * N;
+        for (int n = 0; n < N; ++n) a[n] += (double)wr[n] * xk;
+    }
+    for (int n = 0; n < N; ++n) y[n] = (float)(a[n] + (b ? (double)b[n] : 0.0));
+}
 float host_silu(float x) { return x / (1.0f + std::exp(-x)); }
 
 struct LayerW {
@@ -134,7 +154,7 @@ class FlowExpert : public ModelArch {
 
     std::vector<LayerW> layers_;
     // small fp32 tensors kept on the host for per-observation work
-    std::vector<float> E_lang_, Wstate_, bstate_, W_sp_, b_sp_;
+    std::vector<float> E_lang_, Wstate_, bstate_, W_sp_, b_sp_;  // W*: transposed (host_linear_t)
     DevBuf W_in_, W_out_, b_out_, final_norm_;
     DevBuf W_at2_, b_at2_, m1_;  // action-time MLP: second projection, fp32 scratch [B*S][W]
     bool time_mlp_ = false;
@@ -260,19 +280,19 @@ FlowExpert::FlowExpert(const Checkpoint& ck) {
         vlln_eps_ = (float)ck.f64("vlln_eps", 1e-5);
     }
     if (arch_ == Arch::SMOLVLA) {
-        Wstate_ = host_f32(ck, "prefix.Wstate", {Wv_, max_state_});
+        Wstate_ = transposed(host_f32(ck, "prefix.Wstate", {Wv_, max_state_}), Wv_, max_state_);
         bstate_ = host_f32(ck, "prefix.bstate", {Wv_});
     } else if (head_io_) {
         O_ = (int)ck.i64("dit_out_dim");
         Hd_ = (int)ck.i64("dec_hidden");
         Hs_ = (int)ck.i64("state_hidden");
-        se_l1W_ = host_f32(ck, "aex.se_l1W", {Hs_, max_state_});
+        se_l1W_ = transposed(host_f32(ck, "aex.se_l1W", {Hs_, max_state_}), Hs_, max_state_);
         se_l1b_ = host_f32(ck, "aex.se_l1b", {Hs_});
-        se_l2W_ = host_f32(ck, "aex.se_l2W", {W_, Hs_});
+        se_l2W_ = transposed(host_f32(ck, "aex.se_l2W", {W_, Hs_}), W_, Hs_);
         se_l2b_ = host_f32(ck, "aex.se_l2b", {W_});
         if (n_future_ > 0) future_ = host_f32(ck, "aex.future_tokens", {n_future_, W_});  // N1.6 / N1.7 have none
     } else if (n_lead_ > 0) {
-        W_sp_ = host_f32(ck, "act.W_sp", {W_, max_state_});
+        W_sp_ = transposed(host_f32(ck, "act.W_sp", {W_, max_state_}), W_, max_state_);
         b_sp_ = host_f32(ck, "act.b_sp", {W_});
     }
     if (head_io_) {
@@ -687,17 +707,17 @@ void FlowExpert::prefill(const Inputs* in, int batch) {
         float* const ld = lead_host + (size_t)b * n_lead_row;
         if (arch_ == Arch::SMOLVLA) {
             std::vector<float> row(Wv_);
-            host_linear(Wstate_.data(), bstate_.data(), st.data(), row.data(), Wv_, max_state_);
+            host_linear_t(Wstate_.data(), bstate_.data(), st.data(), row.data(), Wv_, max_state_);
             convert_scaled(dst + (size_t)(P - 1) * Wv_ * es, row.data(), (size_t)Wv_, 1.0f, dt_);
         } else if (head_io_) {
             // encode_state (relu between the two projections), then the learned future tokens
             std::vector<float> h1(Hs_);
-            host_linear(se_l1W_.data(), se_l1b_.data(), st.data(), h1.data(), Hs_, max_state_);
+            host_linear_t(se_l1W_.data(), se_l1b_.data(), st.data(), h1.data(), Hs_, max_state_);
             for (float& v : h1) v = v > 0.f ? v : 0.f;
-            host_linear(se_l2W_.data(), se_l2b_.data(), h1.data(), ld, W_, Hs_);
+            host_linear_t(se_l2W_.data(), se_l2b_.data(), h1.data(), ld, W_, Hs_);
             std::copy(future_.begin(), future_.end(), ld + W_);
         } else if (n_lead_ > 0) {
-            host_linear(W_sp_.data(), b_sp_.data(), st.data(), ld, W_, max_state_);
+            host_linear_t(W_sp_.data(), b_sp_.data(), st.data(), ld, W_, max_state_);
         }
     };
     // initial noise (the generator's draws in order of the observations)
@@ -717,7 +737,7 @@ void FlowExpert::prefill(const Inputs* in, int batch) {
             VLA_HIP(hipMemcpyAsync((char*)prefix_.get() + r0 * Wv_ * es, pe + r0 * Wv_ * es, rows * Wv_ * es, hipMemcpyHostToDevice, C.stream));
         };
         run_staged(
-            first, stage_threads(B),
+            first, stage_threads(B, alt_vl_),
             [&](int t) {
                 // the small remainder first: it may wait for a file
                 if (t % per_obs == 0) stage_rest(t / per_obs);

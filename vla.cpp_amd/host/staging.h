@@ -63,11 +63,12 @@ void run_staged(const std::vector<int>& first, int threads, Work work, Ready rea
     if (failed) throw std::runtime_error(error);
 }
 
-// Pieces of 1 MiB and more that an observation's `bytes` are cut into for run_staged, and the threads for a batch.  Fewer than
-// eight observations are left to the calling thread: the caller's next writes to lines that other cores have read take
-// longer than the shares gain (three views of pi0, 6.3 MB: six threads made the call 0.2 ms shorter and the refill of the
-// same buffer by the caller 4.5 ms longer).
+// Pieces of 1 MiB and more that an observation's `bytes` are cut into for run_staged, and the threads for a batch.  A single
+// observation is left to the calling thread: the caller's next writes to lines that other cores have read take longer than the
+// shares gain (three views of pi0, 6.3 MB: six threads made the call 0.2 ms shorter and the refill of the same buffer by the
+// caller 4.5 ms longer).  From there on a thread per two observations; with text rows and a state encoder for each (`texts`) one
+// per observation.
 inline int stage_pieces(size_t bytes) { return (int)std::max<size_t>(1, bytes >> 20); }
-inline int stage_threads(int batch) { return batch < 8 ? 1 : std::min(default_cpu_threads(), batch); }
+inline int stage_threads(int batch, bool texts) { return batch < 2 ? 1 : std::min(default_cpu_threads(), texts || batch >= 8 ? batch : (batch + 1) / 2); }
 
 }  // namespace vla
