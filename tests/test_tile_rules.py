@@ -17,6 +17,7 @@ def rules(tmp_path_factory):
 extern "C" int plan(int M, int N, int K, int qkv) { return vla_rules::narrow_plan(M, N, K, qkv); }
 extern "C" int plan_f32(int M, int N) { return vla_rules::narrow_plan_f32(M, N); }
 extern "C" int rows_kernel(int bf16, int grid, int blocks, int sliced) { return vla_rules::attn_rows(bf16, grid, blocks, sliced); }
+extern "C" int f32_tile(int M, int n_tiles) { return vla_rules::f32_tile(M, n_tiles); }
 extern "C" int wide(int M, int N, int K, int kind) { return vla_rules::wide_tile(M, N, K, kind); }
 extern "C" int ternary(int M, int N, int K) { return vla_rules::ternary_tile(M, N, K); }
 extern "C" int rows(int p) { return 16 * vla_rules::NARROW_PLANS[p][0]; }
@@ -148,3 +149,15 @@ def test_attention_rows_only_while_the_workgroups_are_few(rules):
             assert rules.rows_kernel(1, 448, blocks, sliced) and not rules.rows_kernel(1, 513, blocks, sliced)
             assert rules.rows_kernel(1, 512, blocks, sliced) == (blocks <= 8)
             assert rules.rows_kernel(0, 512, blocks, sliced) == (blocks <= 20 or not sliced) and not rules.rows_kernel(0, 513, blocks, sliced)
+
+
+# M, N, K -> measured us on the tiles 0 (128 x 128), 1 (64 x 64, 256-byte K rows), 2 (128 x 64), 4 (64 x 64)
+F32_US = [((1323, 1536, 1536), (113.1, 65.2, 110.0, 62.8)), ((408, 1536, 1536), (111.2, 36.6, 63.1, 37.7)), ((1600, 720, 720), (57.7, 33.7, 33.8, 32.2)),
+          ((816, 1024, 1024), (75.7, 26.0, 43.6, 26.2)), ((3549, 704, 960), (75.1, 59.7, 71.4, 57.2)), ((3144, 896, 1536), (113.7, 117.9, 108.8, 111.0)),
+          ((964, 640, 960), (72.0, 23.7, 40.6, 25.0)), ((700, 1536, 1536), (111.1, 61.1, 62.9, 61.1))]
+
+
+@pytest.mark.parametrize("shape,us", F32_US)
+def test_fp32_tile_is_near_the_fastest(rules, shape, us):
+    took = dict(zip((0, 1, 2, 4), us))[rules.f32_tile(shape[0], -(-shape[1] // 64))]
+    assert took <= 1.04 * min(us)

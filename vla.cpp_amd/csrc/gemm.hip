@@ -1913,7 +1913,7 @@ int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
         const int pinned_wide = cfg >= 16 && cfg < 16 + vla_rules::WIDE_TILES ? cfg - 16 : -1;
         const long m128 = (a.M + 127) / 128, m64 = (a.M + 63) / 64;
         const long wgs0 = m128 * ((n_tiles + 1) / 2), wgs2 = m128 * n_tiles, wgs4 = m64 * n_tiles;
-        if (!pinned) cfg = vla_rules::dl_tile(a.M, n_tiles);
+        if (!pinned) cfg = sizeof(T) == 4 ? vla_rules::f32_tile(a.M, n_tiles) : vla_rules::dl_tile(a.M, n_tiles);
         // bf16 operands with 16-byte aligned rows and K a multiple of the MFMA depth take the
         // direct-to-LDS kernel (VLA_GEMM_DL=0 pins the register-staged one).  Its ring depth
         // trades loads in flight against LDS per workgroup: a workgroup is short-lived, so

@@ -104,6 +104,23 @@ inline int dl_tile(int M, int n_tiles) {
     return cfg;
 }
 
+// Tile of an fp32 projection (VLA_GEMM_TILE codes): the fp32 MFMA is its whole time, a 128 x 64 tile takes 1.6 times as long
+// as a 64 x 64 one and a 128 x 128 one three times, and further rounds of workgroups cost somewhat less than the first because
+// two share a CU.  A grid just past a round is what the bf16 rule got wrong here: 1323 x 1536 x 1536 on 264 of 128 x 64 110 us, on
+// 504 of 64 x 64 63; 3549 x 704 x 960 75 and 57.  On 140 measured shapes (65 to 6500 rows, N 256 to 4096) 0.95 of the time of that
+// rule's tiles (geometric mean), none more than 3 % slower; 3144 x 896 x 1536 stays level (112 us on each).
+inline int f32_tile(int M, int n_tiles) {
+    const long m128 = (M + 127) / 128, m64 = (M + 63) / 64;
+    const long wgs0 = m128 * ((n_tiles + 1) / 2), wgs2 = m128 * n_tiles, wgs4 = m64 * n_tiles;
+    auto rounds = [](long wgs, double more) {
+        const long n = (wgs + 255) / 256;
+        return n == 1 ? 1.0 : more * n;
+    };
+    const double t4 = rounds(wgs4, 0.72), t2 = 1.6 * rounds(wgs2, 0.9), t0 = 3.05 * rounds(wgs0, 0.9);
+    if (t4 <= t2 && t4 <= t0) return wgs4 <= 256 ? 1 : 4;
+    return t2 <= t0 ? 2 : 0;
+}
+
 // Predicted time (us) of a bf16 projection on a tile: `fixed`, and per round of workgroups on the busiest XCD (32 CUs) its
 // prologue and epilogue `round` (QKV: + `qkv`, with a LayerNorm inside + `layer`) and `step` per 64 k, which grows by `load` with the
 // share of the CUs that are busy.  Tiles of which two share a CU: round2 and step2 for the rounds of two.  Fitted to 3362
