@@ -36,7 +36,7 @@ int main() {
     bool thrown = false;  // an announcement that throws
     try { vla::run_staged({0, 4, 8}, 4, [](int) {}, [](int) { throw std::runtime_error("copy"); }); } catch (const std::runtime_error&) { thrown = true; }
     CHECK(thrown);
-    CHECK(vla::stage_pieces(0) == 1 && vla::stage_pieces(5 << 20) == 5 && vla::stage_threads(100, false) == 8 && vla::stage_threads(7, false) == 4 && vla::stage_threads(7, true) == 7 && vla::stage_threads(1, true) == 1);
+    CHECK(vla::stage_pieces(0) == 1 && vla::stage_pieces(5 << 20) == 5 && vla::stage_threads(100, false) == 8 && vla::stage_threads(7, false) == 2 && vla::stage_threads(4, false) == 1 && vla::stage_threads(7, true) == 7 && vla::stage_threads(1, true) == 1);
     std::printf("ok\n");
 }
 '''

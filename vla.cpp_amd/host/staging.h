@@ -63,12 +63,15 @@ void run_staged(const std::vector<int>& first, int threads, Work work, Ready rea
     if (failed) throw std::runtime_error(error);
 }
 
-// Pieces of 1 MiB and more that an observation's `bytes` are cut into for run_staged, and the threads for a batch.  A single
-// observation is left to the calling thread: the caller's next writes to lines that other cores have read take longer than the
+// Pieces of 1 MiB and more that an observation's `bytes` are cut into for run_staged, and the threads for a batch.  Up to four
+// observations are left to the calling thread: the caller's next writes to lines that other cores have read take longer than the
 // shares gain (three views of pi0, 6.3 MB: six threads made the call 0.2 ms shorter and the refill of the same buffer by the
-// caller 4.5 ms longer).  From there on a thread per two observations; with text rows and a state encoder for each (`texts`) one
-// per observation.
+// caller 4.5 ms longer; four observations of two views: two threads 0.6 and 6 ms).  Five to seven go to two threads (six
+// observations of GR00T: three made the refill 5 ms longer), from there on a thread an observation; with text rows and a
+// state encoder for each (`texts`) always.
 inline int stage_pieces(size_t bytes) { return (int)std::max<size_t>(1, bytes >> 20); }
-inline int stage_threads(int batch, bool texts) { return batch < 2 ? 1 : std::min(default_cpu_threads(), texts || batch >= 8 ? batch : (batch + 1) / 2); }
+inline int stage_threads(int batch, bool texts) {
+    return texts || batch >= 8 ? std::max(1, std::min(default_cpu_threads(), batch)) : batch < 5 ? 1 : std::min(default_cpu_threads(), 2);
+}
 
 }  // namespace vla
