@@ -1,5 +1,5 @@
-"""Attention of 48- and 64-wide heads on 16 query rows per workgroup, the key blocks shared out over its wavefronts (pinned with
-VLA_ATTN_ROWS=1), against float64."""
+"""Attention of 48- and 64-wide heads with the key blocks shared out over a workgroup's wavefronts (pinned with VLA_ATTN_ROWS=1; bf16:
+32 rows a workgroup, up to ten 64-key tiles, fp32: 16 rows), against float64."""
 import pytest
 import torch
 
@@ -22,7 +22,7 @@ def reference(q, k, v, scale, bias):
 
 
 # row tiles with a ragged last one; key blocks: one of a single key, a partial last one, as many as wavefronts, more than those
-# (bf16 16, fp32 10), a cache row that ends inside the last block (t_max = 40, 104)
+# (fp32 10 of 32 keys; bf16 keys past its ten tiles take the tiled kernel), a cache row that ends inside the last block (t_max = 40, 104)
 @pytest.mark.parametrize("D", [48, 64])
 @pytest.mark.parametrize("dtype", [BF16, F32])
 @pytest.mark.parametrize("B,S,Hq,Hkv,n_keys,t_max", [(1, 50, 15, 5, 227, 256), (2, 50, 15, 5, 291, 320), (3, 7, 4, 2, 33, 40), (1, 17, 9, 3, 1, 8), (1, 40, 3, 3, 100, 104),

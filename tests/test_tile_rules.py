@@ -16,7 +16,8 @@ def rules(tmp_path_factory):
         f.write('''#include "tile_rules.h"
 extern "C" int plan(int M, int N, int K, int qkv) { return vla_rules::narrow_plan(M, N, K, qkv); }
 extern "C" int plan_f32(int M, int N) { return vla_rules::narrow_plan_f32(M, N); }
-extern "C" int rows_kernel(int bf16, int grid, int blocks, int sliced) { return vla_rules::attn_rows(bf16, grid, blocks, sliced); }
+extern "C" int rows_kernel(int grid, int blocks, int sliced) { return vla_rules::attn_rows(grid, blocks, sliced); }
+extern "C" int tiles_kernel(int grid, int tiles) { return vla_rules::attn_tiles(grid, tiles); }
 extern "C" int f32_tile(int M, int n_tiles) { return vla_rules::f32_tile(M, n_tiles); }
 extern "C" int wide(int M, int N, int K, int kind) { return vla_rules::wide_tile(M, N, K, kind); }
 extern "C" int ternary(int M, int N, int K) { return vla_rules::ternary_tile(M, N, K); }
@@ -146,9 +147,10 @@ def test_a_wide_tile_is_named_for_every_size(rules):
 def test_attention_rows_only_while_the_workgroups_are_few(rules):
     for blocks in (1, 8, 9, 20, 21, 1000):
         for sliced in (0, 1):
-            assert rules.rows_kernel(1, 448, blocks, sliced) and not rules.rows_kernel(1, 513, blocks, sliced)
-            assert rules.rows_kernel(1, 512, blocks, sliced) == (blocks <= 8)
-            assert rules.rows_kernel(0, 512, blocks, sliced) == (blocks <= 20 or not sliced) and not rules.rows_kernel(0, 513, blocks, sliced)
+            assert rules.rows_kernel(512, blocks, sliced) == (blocks <= 20 or not sliced) and not rules.rows_kernel(513, blocks, sliced)
+    for tiles in range(1, 11):
+        assert rules.tiles_kernel(256, tiles) and not rules.tiles_kernel(513, tiles)
+        assert rules.tiles_kernel(512, tiles) == (tiles <= 4)
 
 
 # M, N, K -> measured us on the tiles 0 (128 x 128), 1 (64 x 64, 256-byte K rows), 2 (128 x 64), 4 (64 x 64)

@@ -1757,34 +1757,275 @@ __global__ void __launch_bounds__(256, 1) attn_stream_kernel(AttnArgs a, int n_u
     wait_vm_mem<0>();  // the ring's trailing loads still target this wavefront's LDS
 }
 
-// ---- 48- and 64-wide heads, some tens to a few hundred query rows per kv head, few workgroups (one or a few observations) ----
+// ---- 48- and 64-wide heads, more than 32 query rows per kv head, few workgroups (one or a few observations): bf16 ----
 // The tiled kernel gives such a launch few workgroups (15 at batch 1) that walk the keys one tile after the other, a barrier
-// and a trip to memory each; fp32 has to slice the keys over workgroups and pay a merge launch for it.  Here a workgroup
-// owns 16 rows of a (batch, kv head) and its wavefronts own the 32-key blocks, one each while there are no more blocks than
-// wavefronts: every byte of K and V^T is requested at the start of the launch, one trip to memory deep.  A wavefront's block
-// goes straight into LDS of its own (K rows are contiguous, V^T rows one 32-key run each), so no barrier is needed until the
-// wavefronts' (max, sum, output) meet in LDS.
+// and a trip to memory each.  Here a workgroup owns one 32-row tile of a (batch, kv head) and wavefront t the 64-key tile t:
+// every byte of K and V^T is requested at the start of the launch, one trip to memory deep, straight into LDS.
+//
+// Which of the two kernels a launch takes depends on its batch, and an observation's bits must not: every value here is formed by
+// the tiled kernel's instructions in the tiled kernel's order (compared bit for bit in the tests).  What that kernel does one
+// tile after the other and is not independent of the tiles before is short, and is done again from every tile's row maxima and sums:
+//   1. wavefront t: scores of tile t, row maxima to LDS;
+//   2. wavefront t: the running reference maximum that the tiled kernel has at tile t (its lazy update is a vote of the 32 rows,
+//      hence row tiles of 32), probabilities against it; P as fragments and row sums to LDS, over K's tile;
+//   3. wavefront (slice, 32-column block of the output): the chain of products and rescalings over the slice's tiles; with two
+//      key slices (tiles t, t + 2, ... as in the tiled kernel) the second's output meets the first's in LDS.
+// What bounds it: launch and one trip to memory (some 3.5 us), then three short phases; the serial part is four products a tile.
+// 50 rows x 15 heads on 5, 227 keys, one observation 7.9 -> 5.5 us, nine 8.2 -> 5.8.  Row tiles of 16 with a running maximum per 32-key
+// block are faster at one observation (4.4 us) but add in another order.  Two wavefronts per tile, one per 32 keys, are
+// slower from three tiles on (227 keys 6.1 us: one barrier more and the row sums' hand-over).
+// LDS of a tile: K rows of 128 bytes (a 48-wide row's last piece repeated, never read), V^T rows of 128 bytes, 16-byte pieces
+// XOR-swizzled by (row >> 1) & 7 as in the tiled kernel's ring.  Once its wavefront has read K's 8 KiB, P takes the lower half, the
+// rows' maxima and sums the last 256 bytes, the slices' exchange what lies between.
+// W: tiles that the workgroup's LDS has room for.
+template <int D, int W, int NSL>
+__global__ void __launch_bounds__(W * 64) attn_tiles_kernel(AttnArgs a) {
+    typedef AT<bf16_t> A;
+    constexpr int NQ = D / 16, PIECES = D / 8, KBYTES = 64 * 128, TILE = KBYTES + D * 128;
+    constexpr int P_BYTES = 4096, XCH_SLOTS = (KBYTES - 256 - P_BYTES) / 256, NDB = 2;  // (48-wide: the second block is half empty)
+    constexpr int WS = (W + NSL - 1) / NSL, AHEAD = 2;  // tiles of a slice; of these, tiles whose V^T a chain reads during phase 2
+    static_assert(W >= 2 * NSL && W * TILE <= 160 * 1024 && 3 * XCH_SLOTS >= 16 * NDB + 2 && WS >= AHEAD, "wavefronts of the chains, LDS, room for the exchange");
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[W * TILE];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 5, r = lane & 31;
+    // the row tiles of a pair sit eight workgroups apart, on one XCD: they share its L2's copy of K and V^T
+    const int R = a.grp * a.S, local = (int)blockIdx.x >> 3, p8 = (int)div_c(local, a.dGS);
+    const int tile = local - p8 * a.n_groups, pair = p8 * 8 + ((int)blockIdx.x & 7);  // n_groups: row tiles of a pair
+    if (pair >= a.batch * a.Hkv) return;
+    const int b = (int)div_c(pair, a.dHkv), hk = pair - b * a.Hkv;
+    const int n_t = (a.n_keys + 63) / 64;  // at most W; with fewer tiles than chains the other wavefronts own none
+
+    const int row = tile * 32 + r;
+    const bool row_valid = row < R;
+    const int hg = row_valid ? (int)div_c(row, a.dS) : 0, s = row_valid ? row - hg * a.S : 0, h = hk * a.grp + hg;
+    constexpr float LOG2E = 1.4426950408889634f;
+    const float c2 = a.scale * LOG2E;
+    auto row_max = [&](int t) __attribute__((always_inline)) { return reinterpret_cast<float*>(lds + t * TILE + KBYTES - 256) + r; };
+    auto row_sum = [&](int t) __attribute__((always_inline)) { return reinterpret_cast<float*>(lds + t * TILE + KBYTES - 128) + r; };
+
+    unsigned char* const own = lds + wave * TILE;
+    const int k0 = wave * 64;
+    float p[2][16];
+    if (wave < n_t) {  // uniform
+        const uint32_t lds0 = (uint32_t)(uintptr_t)own;
+        const unsigned char* kbase = (const unsigned char*)a.k_cache + ((long)b * a.Hkv + hk) * a.t_max * D * 2;
+        const unsigned char* vbase = (const unsigned char*)a.vt_cache + ((long)b * a.Hkv + hk) * D * (long)a.t_max * 2;
+        // K rows past n_keys repeat the last key (their scores are masked); V^T runs past the cache row are moved back into it and
+        // those past n_keys zeroed as fragments (stale cache contents may be NaN).
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int rowi = i * 8 + (lane >> 3), piece = (lane & 7) ^ ((rowi >> 1) & 7);
+            load_to_lds16(kbase + ((long)min(k0 + rowi, a.n_keys - 1) * D * 2 + min(piece, PIECES - 1) * 16), lds0 + i * 1024);
+        }
+        u32x4_t qf[NQ];
+        const unsigned char* qrow = (const unsigned char*)a.q + (((long)b * a.S + s) * a.Hq + h) * D * 2;
+#pragma unroll
+        for (int c = 0; c < NQ; ++c) {
+            const u32x4_t z = {0u, 0u, 0u, 0u};
+            qf[c] = row_valid ? *reinterpret_cast<const u32x4_t*>(qrow + (c * 16 + g * 8) * 2) : z;
+        }
+#pragma unroll
+        for (int i = 0; i < D / 8; ++i) {
+            const int rowi = i * 8 + (lane >> 3), piece = (lane & 7) ^ ((rowi >> 1) & 7);
+            load_to_lds16(vbase + ((long)rowi * a.t_max + min(k0 + piece * 8, a.t_max - 8)) * 2, lds0 + KBYTES + i * 1024);
+        }
+        wait_vmcnt<0>();
+        asm volatile("" ::: "memory");
+        const int kr = key_of_score_row(r), kx = g ^ ((kr >> 1) & 7);
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+            f32x16_t sc;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) sc[i] = 0.f;
+#pragma unroll
+            for (int c = 0; c < NQ; ++c) A::mma(sc, *reinterpret_cast<const u32x4_t*>(own + (kb * 32 + kr) * 128 + (((2 * c) ^ kx) * 16)), qf[c]);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) p[kb][i] = sc[i] * c2;
+        }
+        const int pad_lo = a.pad_start, pad_hi = min(a.pad_end, a.n_prefix);
+        if (a.mask) {  // mask given as data: additive, one fp32 per (query, key)
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const int key = k0 + kb * 32 + key_of_element(e, g);
+                    p[kb][e] = key < a.n_keys ? p[kb][e] + a.mask[(long)s * a.n_keys + key] * LOG2E : -INFINITY;
+                }
+        } else if (k0 + 64 > a.n_keys || (k0 < pad_hi && k0 + 64 > pad_lo) || (a.mask_kind != VLA_MASK_NONE && k0 + 64 > a.n_prefix)) {
+            int hi = a.n_keys;
+            if (a.mask_kind == VLA_MASK_CAUSAL_SUFFIX) hi = min(a.n_keys, a.n_prefix + s + 1);
+            else if (a.mask_kind == VLA_MASK_PI0_STATE && s == 0) hi = min(a.n_keys, a.n_prefix + 1);
+            const int kl = k0 + 8 * g, left = hi - kl;  // this lane's keys from kl on that its row may see
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) p[kb][e] = kb * 32 + key_of_element(e, 0) < left ? p[kb][e] : -INFINITY;
+            if (k0 < pad_hi && k0 + 64 > pad_lo) {  // uniform
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        const int key = kl + kb * 32 + key_of_element(e, 0);
+                        p[kb][e] = (key >= pad_lo) & (key < pad_hi) ? -INFINITY : p[kb][e];
+                    }
+            }
+        }
+        float m_tile = -INFINITY;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) m_tile = fmaxf(m_tile, p[kb][i]);
+        m_tile = halves_max(m_tile);
+        if (g == 0) *row_max(wave) = m_tile;
+    }
+    __syncthreads();
+
+    const int sl = wave / NDB, db = wave % NDB;  // this wavefront's chain, if sl < NSL
+    const int vrow = min(db * 32 + r, D - 1), vx = g ^ ((vrow >> 1) & 7);
+    auto read_v = [&](int t, u32x4_t (&vf)[4]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int f = 0; f < 4; ++f) vf[f] = *reinterpret_cast<const u32x4_t*>(lds + t * TILE + KBYTES + vrow * 128 + (((2 * f) ^ vx) * 16));
+    };
+    u32x4_t ahead[AHEAD][4];
+    float mt[W];  // past n_t: not used
+#pragma unroll
+    for (int t = 0; t < W; ++t) mt[t] = *row_max(t);
+    if (sl < NSL) {  // uniform
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j)
+            if (sl + j * NSL < n_t) read_v(sl + j * NSL, ahead[j]);  // uniform
+    }
+    if (wave < n_t) {
+        float m_run = -INFINITY;
+#pragma unroll
+        for (int t = 0; t < W; ++t)
+            if (t <= wave && (wave - t) % NSL == 0) {  // uniform
+                if (__builtin_amdgcn_ballot_w64(mt[t] > m_run + RESCALE_LOG2) != 0) m_run = fmaxf(m_run, mt[t]);
+            }
+        const float m_use = (m_run == -INFINITY) ? 0.f : m_run;
+        float psum = 0.f;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const float e = A::fexp2(p[kb][i] - m_use);
+                p[kb][i] = e;
+                psum += e;
+            }
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {  // f = 2 kb + hh: the lane's eight probabilities of a 16-key product
+            const float* pp = &p[f >> 1][(f & 1) * 8];
+            *reinterpret_cast<u32x4_t*>(own + f * 1024 + lane * 16) = u32x4_t{pack_bf2(pp[0], pp[1]), pack_bf2(pp[2], pp[3]), pack_bf2(pp[4], pp[5]), pack_bf2(pp[6], pp[7])};
+        }
+        psum = halves_sum(psum);
+        if (g == 0) *row_sum(wave) = psum;
+    }
+    __syncthreads();
+
+    f32x16_t o;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[i] = 0.f;
+    float m_run = -INFINITY, l_run = 0.f;
+    if (sl < NSL) {  // uniform
+#pragma unroll
+        for (int j = 0; j < WS; ++j) {
+            const int t = sl + j * NSL;
+            if (t >= n_t) break;  // uniform
+            u32x4_t pf[4], vf[4];
+#pragma unroll
+            for (int f = 0; f < 4; ++f) pf[f] = *reinterpret_cast<const u32x4_t*>(lds + t * TILE + f * 1024 + lane * 16);
+            const float psum = *row_sum(t);
+            if (j < AHEAD) {
+#pragma unroll
+                for (int f = 0; f < 4; ++f) vf[f] = ahead[j < AHEAD ? j : 0][f];
+            } else {
+                read_v(t, vf);
+            }
+#pragma unroll
+            for (int f = 0; f < 4; ++f)
+                if (t * 64 + 16 * f + 16 > a.n_keys) {  // uniform
+                    const int nvalid = a.n_keys - (t * 64 + 16 * f + 8 * g);  // real keys among this lane's 8, may be <= 0
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) vf[f][e] &= (2 * e < nvalid ? 0xffffu : 0u) | (2 * e + 1 < nvalid ? 0xffff0000u : 0u);
+                }
+            const float m_tile = NSL == 2 && sl == 1 ? mt[j * NSL + 1 < W ? j * NSL + 1 : 0] : mt[j * NSL];
+            if (__builtin_amdgcn_ballot_w64(m_tile > m_run + RESCALE_LOG2) != 0) {
+                const float m_new = fmaxf(m_run, m_tile);
+                const float alpha = A::fexp2(m_run - ((m_new == -INFINITY) ? 0.f : m_new));  // 2^-inf = 0 at the first visible tile
+                l_run *= alpha;
+                m_run = m_new;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) o[i] *= alpha;
+            }
+            l_run += psum;
+#pragma unroll
+            for (int f = 0; f < 4; ++f) A::mma(o, vf[f], pf[f]);
+        }
+    }
+    if constexpr (NSL == 2) {
+        // element i of block db, and after them the second slice's (maximum, sum): slot x % XCH_SLOTS of tile x / XCH_SLOTS
+        auto slot = [&](int x) __attribute__((always_inline)) {
+            return reinterpret_cast<float*>(lds + (x / XCH_SLOTS) * TILE + P_BYTES + (x % XCH_SLOTS) * 256) + lane;
+        };
+        if (sl == 1) {
+            if (db == 0) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) *slot(i) = o[i];
+                *slot(32) = m_run;
+                *slot(33) = l_run;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) *slot(16 + i) = o[i];
+            }
+        }
+        __syncthreads();
+        if (sl != 0) return;
+        const float m2 = *slot(32), l2 = *slot(33);
+        const float m_new = fmaxf(m_run, m2);
+        const float mm = (m_new == -INFINITY) ? 0.f : m_new;
+        const float w1 = A::fexp2(m_run - mm), w2 = A::fexp2(m2 - mm);  // 2^-inf = 0 for an empty side
+        l_run = l_run * w1 + l2 * w2;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[i] = o[i] * w1 + (db == 0 ? *slot(i) : *slot(16 + i)) * w2;
+    } else {
+        if (sl != 0) return;
+    }
+    if (!row_valid) return;
+    const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
+    bf16_t* const orow = (bf16_t*)a.out + (((long)b * a.S + s) * a.Hq + h) * D;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int d = db * 32 + 8 * j + 4 * g;
+        if (d >= D) continue;
+        *reinterpret_cast<u32x2_t*>(orow + d) = u32x2_t{pack_bf2(o[4 * j] * inv, o[4 * j + 1] * inv), pack_bf2(o[4 * j + 2] * inv, o[4 * j + 3] * inv)};
+    }
+}
+
+// ---- the same launches in fp32 ----
+// The tiled kernel has to slice the keys over workgroups there and pays a merge launch for it (how many slices depends on the
+// batch: fp32 results do, in the last bits, with either kernel).  Here a workgroup owns 16 rows of a (batch, kv head) and its
+// wavefronts own the 32-key blocks, one each while there are no more blocks than wavefronts, requested at the start of the launch.
+// A wavefront's block goes straight into LDS of its own (K rows are contiguous, V^T rows one 32-key run each), so no barrier is
+// needed until the wavefronts' (max, sum, output) meet in LDS.
 // Products as in the decode kernel: S^T = K Q^T as two 16-key products, row i of product j standing for key 8 (i / 4) + 4 j +
 // i % 4 of the block, so that lane (c, q) holds the scores of keys 8 q .. 8 q + 7 against row c: already the right operand of
-// O^T += V^T P^T.  bf16: 16x16x32; fp32: 16x16x4, product t of a 16-d group taking element t of the lanes' 16-byte pieces.
+// O^T += V^T P^T.  16x16x4 MFMA, product t of a 16-d group taking element t of the lanes' 16-byte pieces.
 // LDS pieces (16 bytes) are XOR-swizzled so that the fragment reads, served sixteen lanes at a time (lanes 0-3, 12-15, 20-27 and
-// so on), are free of bank conflicts: K by the lane that reads the row, V^T rows of 64 bytes by row / 4 times 2 in GF(4),
-// of 128 bytes by row / 2 + 2.
+// so on), are free of bank conflicts: K by the lane that reads the row, V^T by row / 2 + 2.
 // K rows of 48-wide heads are kept as if 64 wide; what lies past the head repeats its last piece and meets zeros of Q.
-template <typename T, int D> struct RowsT {
-    static constexpr int EB = sizeof(T), KROW = 64 * EB, VROW = 32 * EB, BLK = 32 * KROW + D * VROW;
-    static constexpr int WAVES = sizeof(T) == 2 ? 16 : 10;  // that a CU's LDS and registers hold
+template <int D> struct RowsT {
+    static constexpr int KROW = 256, VROW = 128, BLK = 32 * KROW + D * VROW;
+    static constexpr int WAVES = 10;  // that a CU's LDS and registers hold
 };
 // W: wavefronts that the workgroup's LDS has room for; as many are launched as the blocks are shared out over evenly.
-template <typename T, int D, int W>
+template <int D, int W>
 __global__ void __launch_bounds__(W * 64) attn_rows_kernel(AttnArgs a) {
-    typedef RowsT<T, D> RT;
-    constexpr int EB = RT::EB, NDB = D / 16, KPR = RT::KROW / 16, VPR = RT::VROW / 16, VE = 16 / EB, PIECES = D * EB / 16;
+    typedef RowsT<D> RT;
+    constexpr int EB = 4, NDB = D / 16, KPR = RT::KROW / 16, VPR = RT::VROW / 16, VE = 16 / EB, PIECES = D * EB / 16;
     constexpr int OSTRIDE = D + 4;  // floats between the rows of a wavefront's partial output
     constexpr int NK = 32 * RT::KROW / 1024, NV = D * RT::VROW / 1024;  // load instructions of a block
     constexpr int NQ = (PIECES + 3) / 4;  // 16-byte pieces of a row per lane
     static_assert(OSTRIDE * 16 * 4 + 128 <= RT::BLK, "partial rows fit a wavefront's LDS");
-    constexpr bool F32 = EB == 4;
     __shared__ __attribute__((aligned(1024))) unsigned char rows_lds[W * RT::BLK];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = (int)(blockDim.x >> 6);
     const int c = lane & 15, q = lane >> 4;
@@ -1801,16 +2042,13 @@ __global__ void __launch_bounds__(W * 64) attn_rows_kernel(AttnArgs a) {
     const unsigned char* vbase = (const unsigned char*)a.vt_cache + ((long)b * a.Hkv + hk) * D * (long)a.t_max * EB;
     // row of the block -> lane c whose fragment it is
     auto k_lane = [](int row) __attribute__((always_inline)) { return (row & 3) | (((row >> 3) & 3) << 2); };
-    auto v_swz = [](int row) __attribute__((always_inline)) {
-        const int x = (row >> 2) & 3;
-        return F32 ? ((row >> 1) + 2) & 7 : ((x << 1) ^ ((x >> 1) * 3)) & 3;
-    };
+    auto v_swz = [](int row) __attribute__((always_inline)) { return ((row >> 1) + 2) & 7; };
     // K rows past n_keys repeat the last key (their scores are masked); V^T runs past the cache row are moved back into it and
     // those past n_keys zeroed as fragments (stale cache contents may be NaN).
     auto issue = [&](int kb) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < NK; ++i) {
-            const int row = i * (32 / NK) + lane / KPR, piece = (lane % KPR) ^ (F32 ? k_lane(row) : k_lane(row) >> 1);
+            const int row = i * (32 / NK) + lane / KPR, piece = (lane % KPR) ^ k_lane(row);
             load_to_lds16(kbase + ((long)min(kb * 32 + row, a.n_keys - 1) * D * EB + min(piece, PIECES - 1) * 16), lds0 + i * 1024);
         }
 #pragma unroll
@@ -1847,18 +2085,18 @@ __global__ void __launch_bounds__(W * 64) attn_rows_kernel(AttnArgs a) {
     for (int kb = wave; kb < nb; kb += nw) {
         wait_vmcnt<0>();
         asm volatile("" ::: "memory");
-        u32x4_t kf[2][NQ], vf[NDB][F32 ? 2 : 1];
+        u32x4_t kf[2][NQ], vf[NDB][2];
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int i = 0; i < NQ; ++i)
-                kf[j][i] = *reinterpret_cast<const u32x4_t*>(kl + (8 * (c >> 2) + (c & 3) + 4 * j) * RT::KROW + (((4 * i + q) ^ (F32 ? c : c >> 1)) * 16));
+                kf[j][i] = *reinterpret_cast<const u32x4_t*>(kl + (8 * (c >> 2) + (c & 3) + 4 * j) * RT::KROW + (((4 * i + q) ^ c) * 16));
 #pragma unroll
         for (int db = 0; db < NDB; ++db)
 #pragma unroll
-            for (int i = 0; i < (F32 ? 2 : 1); ++i) {
-                const int d = db * 16 + c, piece = F32 ? 2 * q + i : q;
-                vf[db][i] = *reinterpret_cast<const u32x4_t*>(kl + 32 * RT::KROW + d * RT::VROW + ((piece ^ v_swz(d)) * 16));
+            for (int i = 0; i < 2; ++i) {
+                const int d = db * 16 + c;
+                vf[db][i] = *reinterpret_cast<const u32x4_t*>(kl + 32 * RT::KROW + d * RT::VROW + (((2 * q + i) ^ v_swz(d)) * 16));
             }
         if (4 * NQ > PIECES) {  // beside the zeros of Q, or an infinity in K's last piece would be a NaN
 #pragma unroll
@@ -1870,13 +2108,9 @@ __global__ void __launch_bounds__(W * 64) attn_rows_kernel(AttnArgs a) {
         for (int i = 0; i < NQ; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                if constexpr (F32) {
-                    const f32x4_t kv = __builtin_bit_cast(f32x4_t, kf[j][i]), qv = __builtin_bit_cast(f32x4_t, qf[i]);
+                const f32x4_t kv = __builtin_bit_cast(f32x4_t, kf[j][i]), qv = __builtin_bit_cast(f32x4_t, qf[i]);
 #pragma unroll
-                    for (int t = 0; t < 4; ++t) sc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[t], qv[t], sc[j], 0, 0, 0);
-                } else {
-                    sc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[j][i]), __builtin_bit_cast(bf16x8_t, qf[i]), sc[j], 0, 0, 0);
-                }
+                for (int t = 0; t < 4; ++t) sc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[t], qv[t], sc[j], 0, 0, 0);
             }
         const int k0 = kb * 32, key0 = k0 + 8 * q, nvalid = a.n_keys - key0;  // real keys among this lane's 8, may be <= 0
         if (k0 + 32 > a.n_keys) {  // uniform
@@ -1884,12 +2118,8 @@ __global__ void __launch_bounds__(W * 64) attn_rows_kernel(AttnArgs a) {
             for (int db = 0; db < NDB; ++db)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    if constexpr (F32) {
-                        vf[db][0][e] = e < nvalid ? vf[db][0][e] : 0u;
-                        vf[db][1][e] = 4 + e < nvalid ? vf[db][1][e] : 0u;
-                    } else {
-                        vf[db][0][e] &= (2 * e < nvalid ? 0xffffu : 0u) | (2 * e + 1 < nvalid ? 0xffff0000u : 0u);
-                    }
+                    vf[db][0][e] = e < nvalid ? vf[db][0][e] : 0u;
+                    vf[db][1][e] = 4 + e < nvalid ? vf[db][1][e] : 0u;
                 }
         }
         float p[8];  // keys key0 + i
@@ -1919,20 +2149,13 @@ __global__ void __launch_bounds__(W * 64) attn_rows_kernel(AttnArgs a) {
             psum += p[i];
         }
         l_run = l_run * alpha + rows_sum(psum);
-        u32x4_t pf;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) pf[e] = pack_bf2(p[2 * e], p[2 * e + 1]);
 #pragma unroll
         for (int db = 0; db < NDB; ++db) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[db][e] *= alpha;
-            if constexpr (F32) {
 #pragma unroll
-                for (int t = 0; t < 8; ++t)
-                    o[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(f32x4_t, vf[db][t >> 2])[t & 3], p[t], o[db], 0, 0, 0);
-            } else {
-                o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, vf[db][0]), __builtin_bit_cast(bf16x8_t, pf), o[db], 0, 0, 0);
-            }
+            for (int t = 0; t < 8; ++t)
+                o[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(f32x4_t, vf[db][t >> 2])[t & 3], p[t], o[db], 0, 0, 0);
         }
         if (kb + nw < nb) {  // uniform; only with more blocks than wavefronts
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this block's fragments are in registers
@@ -1973,28 +2196,44 @@ __global__ void __launch_bounds__(W * 64) attn_rows_kernel(AttnArgs a) {
         const float inv = l > 0.f ? 1.0f / l : 0.f;
         const int og = (int)div_c(orow, a.dS), os = orow - og * a.S;
         const long oo = (((long)b * a.S + os) * a.Hq + hk * a.grp + og) * D + d0;
-        if constexpr (F32) *reinterpret_cast<f32x4_t*>((float*)a.out + oo) = f32x4_t{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
-        else *reinterpret_cast<u32x2_t*>((bf16_t*)a.out + oo) = u32x2_t{pack_bf2(acc[0] * inv, acc[1] * inv), pack_bf2(acc[2] * inv, acc[3] * inv)};
+        *reinterpret_cast<f32x4_t*>((float*)a.out + oo) = f32x4_t{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
     }
 }
 
-// The launch of attn_rows_kernel: false, launching nothing, where the call is not one of its.
+// The launch of attn_tiles_kernel (bf16) or attn_rows_kernel (fp32): false, launching nothing, where the call is not one of theirs.
 template <typename T, int D>
 bool launch_rows(AttnArgs& a, hipStream_t st) {
     const Tuning& tn = tuning();
     if (tn.attn_rows == 0 || a.p2 || (((uintptr_t)a.q | (uintptr_t)a.k_cache | (uintptr_t)a.vt_cache | (uintptr_t)a.out) & 15)) return false;
-    constexpr int W = RowsT<T, D>::WAVES;
-    const int R = (a.Hq / a.Hkv) * a.S, n_tiles = (R + 15) / 16, nb = (a.n_keys + 31) / 32;
+    constexpr bool BF16 = sizeof(T) == 2;
+    const int R = (a.Hq / a.Hkv) * a.S, n_tiles = BF16 ? (R + 31) / 32 : (R + 15) / 16, blocks = BF16 ? (a.n_keys + 63) / 64 : (a.n_keys + 31) / 32;
     const long grid = ((long)a.batch * a.Hkv + 7) / 8 * 8 * n_tiles;
     if (grid >= (1l << 31)) return false;
-    if (tn.attn_rows < 0 && !vla_rules::attn_rows(sizeof(T) == 2, grid, nb, a.n_split > 1)) return false;
-    const int steps = (nb + W - 1) / W, nw = (nb + steps - 1) / steps;
+    if (BF16 && (blocks > vla_rules::ATTN_TILES_MAX || a.n_split > 1)) return false;  // (split keys: another order, and pinned)
+    if (tn.attn_rows < 0 && !(BF16 ? vla_rules::attn_tiles(grid, blocks) : vla_rules::attn_rows(grid, blocks, a.n_split > 1))) return false;
     a.n_groups = n_tiles;
     a.n_split = 1;
     set_divisors(a, grid);
-    // half the LDS while that is room enough: two workgroups then share a CU
-    if (nw <= W / 2) attn_rows_kernel<T, D, W / 2><<<(unsigned)grid, nw * 64, 0, st>>>(a);
-    else attn_rows_kernel<T, D, W><<<(unsigned)grid, nw * 64, 0, st>>>(a);
+    if constexpr (BF16) {
+        constexpr int MAX = vla_rules::ATTN_TILES_MAX;
+        // n_slices: the key slices that the tiled kernel takes (64-wide heads); a wavefront per tile, and as many as own the chains
+        const int nw = std::max(blocks, 2 * a.n_slices);
+        if constexpr (D == 64) {
+            if (a.n_slices == 2) {
+                if (blocks <= MAX / 2) attn_tiles_kernel<D, MAX / 2, 2><<<(unsigned)grid, nw * 64, 0, st>>>(a);
+                else attn_tiles_kernel<D, MAX, 2><<<(unsigned)grid, nw * 64, 0, st>>>(a);
+                return true;
+            }
+        }
+        if (blocks <= MAX / 2) attn_tiles_kernel<D, MAX / 2, 1><<<(unsigned)grid, nw * 64, 0, st>>>(a);
+        else attn_tiles_kernel<D, MAX, 1><<<(unsigned)grid, nw * 64, 0, st>>>(a);
+    } else {
+        constexpr int W = RowsT<D>::WAVES;
+        const int steps = (blocks + W - 1) / W, nw = (blocks + steps - 1) / steps;
+        // half the LDS while that is room enough: two workgroups then share a CU
+        if (nw <= W / 2) attn_rows_kernel<D, W / 2><<<(unsigned)grid, nw * 64, 0, st>>>(a);
+        else attn_rows_kernel<D, W><<<(unsigned)grid, nw * 64, 0, st>>>(a);
+    }
     return true;
 }
 

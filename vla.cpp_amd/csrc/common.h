@@ -29,7 +29,7 @@ struct Tuning {
     int gemm_rows_max = 512;     // VLA_GEMM_ROWS_MAX: projections of at most this many rows may take the narrow-tile kernels, 0 = never
     int gemm_rows_plan = 0;      // VLA_GEMM_ROWS_PLAN: 1..4 pins those kernels' rows x columns per workgroup (16x16, 32x16, 64x16, 64x32; fp32: 1 and 3), 0 = by shape
     bool attn_no_small = false;  // VLA_ATTN_NO_SMALL: fp32 launches with few row tiles do not split their keys beyond the usual rule
-    int attn_rows = -1;          // VLA_ATTN_ROWS: 0 never, 1 always the kernel of 16 rows per workgroup for 64-wide heads; unset = by shape
+    int attn_rows = -1;          // VLA_ATTN_ROWS: 0 never, 1 always (as far as they serve the shape) the kernels of a wavefront per key block for 48- and 64-wide heads; unset = by shape
     int attn_direct_rows = 32;   // VLA_ATTN_DIRECT_ROWS: row limit of the register-direct kernel
     int gemm_tile = -1;          // VLA_GEMM_TILE: 0..5, wide tiles 16..21
     int gemm_panel = 0;          // VLA_GEMM_PANEL: N tiles per panel of an XCD's walk over its tiles; 0 = by size

@@ -196,16 +196,22 @@ inline int ternary_tile(long M, long N, long K) {
     return best;
 }
 
-// Whether an attention launch of 48- or 64-wide heads takes 16 rows per workgroup with the 32-key blocks shared out over
-// its wavefronts (`grid` workgroups, `blocks` key blocks) instead of the tiled kernel, which reads K and V^T once per 64 to
-// 128 rows but walks the keys.  About two rounds of workgroups: 50 rows x 15 heads on 5, 227 keys: 1, 4, 8, 16 observations (50,
-// 200, 400, 800 workgroups) 8.9, 9.1, 9.2, 9.8 us tiled and 4.9, 5.1, 6.2, 9.9 here; with more than eight blocks a CU holds one
-// workgroup: 512 keys 10.5, 10.8, 11.1, 11.6 and 5.8, 6.3, 10.7, 18.2.  fp32: 13.0, 25.2, 25.9, 26.6 and 7.3, 7.8, 13.4, 23.9; where the tiled
-// kernel slices the keys over workgroups, more than two blocks per wavefront (ten of them) are left to it: 16 rows x 16 heads on
-// 4, 1000 keys 14.8 us, here 16.0 (one slice only: 50 x 15 on 5, two observations 87.9, here 17.1).
-inline bool attn_rows(bool bf16, long grid, int blocks, bool sliced) {
-    if (bf16) return grid <= (blocks <= 8 ? 512 : 448);
-    return grid <= 512 && (blocks <= 20 || !sliced);
+// Whether a bf16 attention launch of 48- or 64-wide heads (`grid` workgroups of 32 rows, `blocks` 64-key tiles) takes a wavefront
+// per tile (attn_tiles_kernel, the bits of the tiled kernel) instead of the tiled kernel, which reads K and V^T once per 64
+// to 128 rows but walks the keys.  Two rounds of workgroups while a CU holds two of them, else one: 50 rows x 15 heads on 5, 227
+// keys: 1, 4, 8, 16, 20 observations (40, 120, 200, 400, 520 workgroups) 7.9, 8.2, 8.2, 8.4, 9.6 us tiled and 5.5, 5.7, 5.8, 6.9, 9.8
+// here; 291 keys (five tiles) 1, 4, 9, 10 observations (40, 120, 240, 280) 9.2, 9.4, 9.6, 9.5 and 6.0, 6.2, 6.4, 10.0; 512 keys 1 and 9
+// observations 9.5, 9.9 and 6.6, 7.1; 48-wide, 49 rows, 32 heads: 227 keys 1, 4, 8 observations (64, 256, 512) 6.9, 7.1, 7.2 and 5.1, 5.4, 6.3.
+constexpr int ATTN_TILES_MAX = 10;  // tiles that a workgroup's LDS holds
+inline bool attn_tiles(long grid, int blocks) {
+    return grid <= (blocks <= 4 ? 512 : 256);
 }
+
+// Whether an fp32 attention launch of 48- or 64-wide heads takes 16 rows per workgroup with the 32-key blocks shared out over
+// its wavefronts (`grid` workgroups, `blocks` key blocks) instead of the tiled kernel.  About two rounds of workgroups: 50 rows x
+// 15 heads on 5, 227 keys: 1, 4, 8, 16 observations (50, 200, 400, 800 workgroups) 13.0, 25.2, 25.9, 26.6 us tiled and 7.3, 7.8, 13.4, 23.9
+// here; where the tiled kernel slices the keys over workgroups, more than two blocks per wavefront (ten of them) are left to
+// it: 16 rows x 16 heads on 4, 1000 keys 14.8 us, here 16.0 (one slice only: 50 x 15 on 5, two observations 87.9, here 17.1).
+inline bool attn_rows(long grid, int blocks, bool sliced) { return grid <= 512 && (blocks <= 20 || !sliced); }
 
 }  // namespace vla_rules
