@@ -305,21 +305,30 @@ __device__ __forceinline__ float apply_act(float x, int act) {
     return x;
 }
 
+// x / (1 + e) in seven instructions, correctly rounded: the hardware reciprocal (1 ulp), the quotient, and one step on its exact
+// remainder.  On 2^24 values from -87 to 30 and over all exponents the bits of the division (which is some 15 instructions), but for
+// |x| < 2^-124, where it is the nearest denormal or the one beside it.  A quarter of both sides, so that the reciprocal is a
+// normal number up to e = 2^128; v_div_fixup puts right what infinities make of the remainder.
+__device__ __forceinline__ float div_1p(float x, float e) {
+    const float d = fmaf(e, 0.25f, 0.25f), n = 0.25f * x, r = __builtin_amdgcn_rcpf(d), q = n * r;
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, n), r, q), d, n);
+}
 // The same for values that are rounded to bf16 next, N at a time.  The exact division and tanhf above are some 25 and 45
-// instructions per value, and a 128 x 128 tile has 64 per thread: 1323 x 6144 x 1536 took 64.6 us with GELU and 52.8 without.  Here
-// 5 and 7 instructions (51.7 us; 408 rows 29.4 -> 20.3): the reciprocal is the hardware's (1 ulp), and GELU's tanh form is
-// written as the sigmoid it is, 0.5 x (1 + tanh u) = x / (1 + exp(-2 u)).  Against float64 over all bf16 x in (-8, 30): SiLU
-// 4.2e-7 of the value (as above), GELU 3.9e-6 (above: 1, where 1 + tanh u cancels), beside the 2^-8 of the rounding that follows.
+// instructions per value, and a 128 x 128 tile has 64 per thread: 12 of the 65 us that 1323 x 6144 x 1536 with GELU took on such
+// tiles (on the wide tiles now 29.3 us, 25.9 without an activation).  Here 9 and 11: GELU's tanh form is written as the sigmoid
+// it is, 0.5 x (1 + tanh u) = x / (1 + exp(-2 u)).  SiLU has the bits of the exact form.  GELU against float64, 4 M values of N(0, 1):
+// 4.2e-8 of the norm (tanhf 3.8e-8; N(0, 0.3^2) 4.0e-8, tanhf 4.2e-8), largest error 1.6e-6 of the value (tanhf 0.35, where 1 + tanh u
+// cancels); rounded to bf16 both are 1.665157630e-3 of the norm, and 29 values are not the nearest (tanhf 111).
 // The multiply-add is spelled out: every kernel gives the same bits.
 template <int N>
 __device__ __forceinline__ void apply_act_bf16(float (&v)[N], int act) {
     if (act == VLA_ACT_SILU) {
 #pragma unroll
-        for (int e = 0; e < N; ++e) v[e] *= __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(v[e] * -1.44269504088896341f));
+        for (int e = 0; e < N; ++e) v[e] = div_1p(v[e], __builtin_amdgcn_exp2f(v[e] * -1.44269504088896341f));
     } else if (act == VLA_ACT_GELU) {
         constexpr float k1 = -2.0f * 0.79788456080286535588f * 1.44269504088896341f, k3 = k1 * 0.044715f;
 #pragma unroll
-        for (int e = 0; e < N; ++e) v[e] *= __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(v[e] * fmaf(k3, v[e] * v[e], k1)));
+        for (int e = 0; e < N; ++e) v[e] = div_1p(v[e], __builtin_amdgcn_exp2f(v[e] * fmaf(k3, v[e] * v[e], k1)));
     } else if (act == VLA_ACT_RELU) {
 #pragma unroll
         for (int e = 0; e < N; ++e) v[e] = v[e] > 0.f ? v[e] : 0.f;
