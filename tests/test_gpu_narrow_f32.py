@@ -95,6 +95,27 @@ def test_qkv(tune, B, S, Hq, Hkv, D, K, rope, kv):
             assert not kc[:, :, :P].any() and not kc[:, :, P + S:].any() and not vc[..., :P].any() and not vc[..., P + S:].any(), plan
 
 
+@pytest.mark.parametrize("M,N,K,heads", [(50, 720, 960, None), (33, 2816, 1024, None), (51, 2560, 2048, None), (48, 8192, 720, None), (64, 8192, 2048, None), (17, 8192, 1024, None),
+                                         (51, 2560, 1024, (8, 1, 256)), (51, 2560, 2048, (8, 1, 256)), (50, 2880, 720, (15, 15, 64)), (64, 3072, 1024, (16, 16, 64))])
+def test_default_tiles_add_in_short_sums(M, N, K, heads):
+    """Plain and QKV products of up to 64 rows and 8192 columns: 64 partial sums of n = K / 64 products each, added in pairs.  An
+    addition is off by a 0.24 (2^-24)^2 share of its result's square (uniform rounding errors, values spread over a binade),
+    a partial sum's square grows with its length: n / 2 + 6 times that in all.  Four times as long sums are off by 1.5 to 1.7 times as much."""
+    g = torch.Generator().manual_seed(N + K)
+    x, W = torch.randn(M, K, generator=g).cuda(), (torch.randn(N, K, generator=g) / K ** 0.5).cuda()
+    if heads:
+        Hq, Hkv, D = heads
+        q, kc, vc = torch.zeros(M, Hq * D, device="cuda"), torch.zeros(1, Hkv, 64, D, device="cuda"), torch.zeros(1, Hkv, D, 64, device="cuda")
+        pkg.call("vla_attn_qkv_rope", x, W, None, F32, M, K, M, Hq, Hkv, 1, 1, D, None, None, q, kc, vc, 64, 0)
+        y = torch.cat([q, kc[0, :, :M].transpose(0, 1).reshape(M, -1), vc[0, :, :, :M].permute(2, 0, 1).reshape(M, -1)], 1)
+    else:
+        y = torch.zeros(M, N, device="cuda")
+        pkg.call("vla_linear", x, W, None, None, y, F32, F32, M, N, K)
+    want = x.double() @ W.double().T
+    err = ((y.double() - want).norm() / want.norm()).item()
+    assert err < 2.0 ** -24 * (0.24 * (K / 128 + 6)) ** 0.5, err
+
+
 @pytest.mark.parametrize("arch,batch", [("smolvla", 1), ("smolvla", 3), ("smolvla", 11), ("pi0", 1)])
 def test_norms_inside_the_projection_launches(tmp_path, monkeypatch, arch, batch):
     """An fp32 model with its RMSNorms inside the projections (few rows) against the same model with norms as launches of

@@ -15,7 +15,7 @@ def rules(tmp_path_factory):
     with open(src, "w") as f:
         f.write('''#include "tile_rules.h"
 extern "C" int plan(int M, int N, int K, int qkv) { return vla_rules::narrow_plan(M, N, K, qkv); }
-extern "C" int plan_f32(int M, int N) { return vla_rules::narrow_plan_f32(M, N); }
+extern "C" int plan_f32(int M, int N, int gated) { return vla_rules::narrow_plan_f32(M, N, gated); }
 extern "C" int rows_kernel(int grid, int blocks, int sliced) { return vla_rules::attn_rows(grid, blocks, sliced); }
 extern "C" int tiles_kernel(int grid, int tiles) { return vla_rules::attn_tiles(grid, tiles); }
 extern "C" int f32_tile(int M, int n_tiles) { return vla_rules::f32_tile(M, n_tiles); }
@@ -96,13 +96,14 @@ def test_ternary_tile_is_near_the_fastest_and_not_slower_than_the_large_tiles(ru
 
 def test_fp32_narrow_tiles_of_more_than_one_round(rules):
     """16 x 16 tiles up to one round of two per CU, up to four rounds where the 64-row tiles would repeat the
-    weights or waste rows, and always a narrow tile for up to 64 rows."""
+    weights or waste rows or make the sums of plain and QKV products longer, and always a narrow tile for up to 64 rows."""
     for M in list(range(1, 130)) + [200, 300, 400, 512]:
         for N in WIDTHS:
-            wgs, p = -(-M // 16) * (N // 16), rules.plan_f32(M, N)
-            if M <= 64:
-                assert p in (0, 2), (M, N)
-            assert (p == 0) == (wgs <= 512 or (wgs <= 2048 and not 32 < M <= 64)), (M, N)
+            for gated in (0, 1):
+                wgs, p = -(-M // 16) * (N // 16), rules.plan_f32(M, N, gated)
+                if M <= 64:
+                    assert p in (0, 2), (M, N)
+                assert (p == 0) == (wgs <= 512 or (wgs <= 2048 and not (gated and 32 < M <= 64))), (M, N)
 
 
 # M, N, K, kind (0 plain or gated, 1 QKV, 2 with a LayerNorm) -> measured us of the direct-to-LDS kernel and on the wide tiles

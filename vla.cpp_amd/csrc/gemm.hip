@@ -1879,7 +1879,7 @@ int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
         // a few fp32 rows: narrow tiles (VLA_GEMM_TILE pins the tiled kernel instead)
         bool rows_ok = a.M <= tuning().gemm_rows_max && (a.norm_eps < 0.f || (a.norm_w && a.K <= F32_NORM_MAX_K && (uintptr_t)a.norm_w % 16 == 0)) && tuning().gemm_tile < 0 && ((uintptr_t)a.A | (uintptr_t)a.W) % 16 == 0;
         const int force = tuning().gemm_rows_plan;
-        const int plan = !rows_ok ? -1 : force == 1 || force == 3 ? force - 1 : vla_rules::narrow_plan_f32(a.M, a.N);
+        const int plan = !rows_ok ? -1 : force == 1 || force == 3 ? force - 1 : vla_rules::narrow_plan_f32(a.M, a.N, kEpi == EPI_GLU);
         if (plan >= 0) {
             launch_narrow_f32<kEpi>(a, plan, st);
             return hipGetLastError() == hipSuccess ? VLA_K_OK : VLA_K_ERR_LAUNCH;

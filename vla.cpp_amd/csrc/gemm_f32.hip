@@ -11,16 +11,18 @@ using namespace vk;
 // fragment reads free of bank conflicts), NS - 1 stages in flight, one barrier per stage.
 // v_mfma_f32_16x16x4_f32 multiplies full fp32 at twice the rate of plain FMAs, but one block over all of K is K / 4
 // products of 32 clocks in a row: with one row block the four wavefronts share K (16-k groups in turn).  A wavefront
-// keeps 16 accumulators in turn, which also shortens the sums: K / 64 products (four row blocks: K / 16) follow one
-// another before the partial sums are added in pairs, as in the FMA kernel this replaces, whose error against float64 it has
-// (50 x 720 x 960: 9.8e-8 of the norm both; tiled kernel 5.6e-7).  Half as many accumulators cost 1.2e-7 and gained 0.2 us.
+// keeps 16 accumulators in turn, which also shortens the sums: K / 64 values of k follow one another (K / 256 MFMA products of four) before
+// the partial sums are added in pairs, as in an FMA kernel with a value of k per lane, whose error against float64 it has (50 x
+// 720 x 960: 9.9e-8 of the norm; tiled kernel 5.6e-7).  Half as many accumulators cost 1.2e-7 and gained 0.2 us.  With four row blocks a
+// wavefront has all of K to itself, K / 16 values: 1.5e-7 for K = 1024 (tiled kernel 8e-7).  Adding its accumulators up every 128 k would make
+// that 0.95e-7, but the additions are not hidden behind the products: 51 x 2560 x 1024 9.0 -> 10.4 us, where 16 x 16 tiles take 9.1.
 // NORM: the rows' RMSNorm inside.  The operand is x w (the weight, resident in LDS, is applied to the fragments), the sum of
 // squares is taken from the fragments, and row c of the result is scaled by 1 / sqrt(mean + eps).
 // A lane (c, q) reads 16 bytes, k = 4 q .. 4 q + 3 of a 16-k group, of row c; product t of the group takes element t of both
 // operands (k = t, 4 + t, 8 + t, 12 + t).  W is the left operand, so that a lane ends with columns 4 q .. 4 q + 3 of row c.
 // What bounds it: start and first loads (3 us), then per 256 k and wavefront 512 clocks of products beside 32 KiB of fill.
-// Against the FMA kernel (8 columns per workgroup, weights through L1; us): 50 x 720 x 960 10.8 -> 4.9, 50 x 1600 x 720 12.4 -> 6.1,
-// 50 x 720 x 2048 13.1 -> 6.5; against the tiled kernel: 50 x 4096 x 720 gated 19.8 -> 9.3, 241 x 640 x 960 22.5 -> 10.5, 100 x 720 x 2048
+// Against an FMA kernel of 8 columns per workgroup (us): 50 x 720 x 960 10.8 -> 4.9, 50 x 1600 x 720 12.4 -> 6.1, 50 x 720 x 2048 13.1 -> 6.5,
+// 51 x 2560 x 1024 QKV 18.0 -> 10.3; against the tiled kernel: 50 x 4096 x 720 gated 19.8 -> 9.3, 241 x 640 x 960 22.5 -> 10.5, 100 x 720 x 2048
 // 43.5 -> 10.3.
 template <int kEpi, int RB, int KB, int NS, bool VEC, bool NORM>
 __global__ void __launch_bounds__(256) gemm_narrow_f32_kernel(GemmArgs a) {

@@ -45,14 +45,16 @@ inline int narrow_plan(int M, int N, int K, bool qkv) {
 }
 
 // Rows per workgroup of the fp32 narrow-tile kernel, as an index of NARROW_PLANS (16 x 16 or 64 x 16), or -1 for the tiled
-// kernel.  Two workgroups of 16 x 16 share a CU; beyond one round of them (512), 64-row tiles read the weights a quarter as
-// often while they cover 33 to 64 rows (50 x 4096 x 720 gated 11.4 -> 9.3 us, 51 x 8192 x 1024 22.1 -> 18.9), and 16 x 16 tiles stay ahead
-// of the tiled kernel up to four rounds: 200 x 1600 x 720 14.0 us, tiled 19.0; 482 x 640 x 960 14.9, 22.6; 100 x 4096 x 720 gated (1792
-// workgroups) 18.9, 19.8; 150 x 4096 x 720 gated (2560) 23.4, 20.0.
-inline int narrow_plan_f32(int M, int N) {
+// kernel.  Two workgroups of 16 x 16 share a CU; beyond one round of them (512), 64-row tiles read the weights of gated products
+// a quarter as often while they cover 33 to 64 rows (50 x 4096 x 720 10.8 -> 8.6 us, 51 x 8192 x 1024 21.2 -> 18.2).  Their sums are four
+// times as long (errors of 1.5e-7 and 2.1e-7 of the norm for K of 1024 and 2048, 16 x 16 tiles 1.0e-7 and 1.2e-7): plain and QKV
+// products stay with 16 x 16 tiles, which are as fast there (51 x 2560 x 1024 9.1 us, 64-row tiles 9.0; 51 x 2560 x 2048 13.9, 15.4).  16 x 16
+// tiles are ahead of the tiled kernel up to four rounds: 200 x 1600 x 720 14.0 us, tiled 19.0; 482 x 640 x 960 14.9, 22.6; 100 x 4096 x 720
+// gated (1792 workgroups) 18.9, 19.8; 150 x 4096 x 720 gated (2560) 23.4, 20.0.
+inline int narrow_plan_f32(int M, int N, bool gated) {
     const long wgs = narrow_wgs(M, N, 0);
     if (wgs <= 512) return 0;
-    if (M <= 64) return M > 32 || wgs > 2048 ? 2 : 0;
+    if (M <= 64) return (gated && M > 32) || wgs > 2048 ? 2 : 0;
     return wgs <= 2048 ? 0 : -1;
 }
 
