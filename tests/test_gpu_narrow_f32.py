@@ -96,9 +96,10 @@ def test_qkv(tune, B, S, Hq, Hkv, D, K, rope, kv):
 
 
 @pytest.mark.parametrize("M,N,K,heads", [(50, 720, 960, None), (33, 2816, 1024, None), (51, 2560, 2048, None), (48, 8192, 720, None), (64, 8192, 2048, None), (17, 8192, 1024, None),
+                                         (16, 36864, 720, None), (32, 40960, 256, None), (51, 20480, 1024, None),
                                          (51, 2560, 1024, (8, 1, 256)), (51, 2560, 2048, (8, 1, 256)), (50, 2880, 720, (15, 15, 64)), (64, 3072, 1024, (16, 16, 64))])
 def test_default_tiles_add_in_short_sums(M, N, K, heads):
-    """Plain and QKV products of up to 64 rows and 8192 columns: 64 partial sums of n = K / 64 products each, added in pairs.  An
+    """Plain and QKV products of up to 64 rows: 64 partial sums of n = K / 64 products each, added in pairs.  An
     addition is off by a 0.24 (2^-24)^2 share of its result's square (uniform rounding errors, values spread over a binade),
     a partial sum's square grows with its length: n / 2 + 6 times that in all.  Four times as long sums are off by 1.5 to 1.7 times as much."""
     g = torch.Generator().manual_seed(N + K)

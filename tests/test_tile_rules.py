@@ -95,15 +95,14 @@ def test_ternary_tile_is_near_the_fastest_and_not_slower_than_the_large_tiles(ru
 
 
 def test_fp32_narrow_tiles_of_more_than_one_round(rules):
-    """16 x 16 tiles up to one round of two per CU, up to four rounds where the 64-row tiles would repeat the
-    weights or waste rows or make the sums of plain and QKV products longer, and always a narrow tile for up to 64 rows."""
+    """16 x 16 tiles up to four rounds of two per CU and always a narrow tile for up to 64 rows; 64-row tiles only for gated products of
+    33 to 64 rows beyond one round (elsewhere they repeat the weights, waste rows or make sums longer)."""
     for M in list(range(1, 130)) + [200, 300, 400, 512]:
         for N in WIDTHS:
             for gated in (0, 1):
                 wgs, p = -(-M // 16) * (N // 16), rules.plan_f32(M, N, gated)
-                if M <= 64:
-                    assert p in (0, 2), (M, N)
-                assert (p == 0) == (wgs <= 512 or (wgs <= 2048 and not (gated and 32 < M <= 64))), (M, N)
+                want = -1 if M > 64 and wgs > 2048 else 2 if gated and 32 < M <= 64 and wgs > 512 else 0
+                assert p == want, (M, N, gated)
 
 
 # M, N, K, kind (0 plain or gated, 1 QKV, 2 with a LayerNorm) -> measured us of the direct-to-LDS kernel and on the wide tiles

@@ -50,11 +50,14 @@ inline int narrow_plan(int M, int N, int K, bool qkv) {
 // times as long (errors of 1.5e-7 and 2.1e-7 of the norm for K of 1024 and 2048, 16 x 16 tiles 1.0e-7 and 1.2e-7): plain and QKV
 // products stay with 16 x 16 tiles, which are as fast there (51 x 2560 x 1024 9.1 us, 64-row tiles 9.0; 51 x 2560 x 2048 13.9, 15.4).  16 x 16
 // tiles are ahead of the tiled kernel up to four rounds: 200 x 1600 x 720 14.0 us, tiled 19.0; 482 x 640 x 960 14.9, 22.6; 100 x 4096 x 720
-// gated (1792 workgroups) 18.9, 19.8; 150 x 4096 x 720 gated (2560) 23.4, 20.0.
+// gated (1792 workgroups) 18.9, 19.8; 150 x 4096 x 720 gated (2560) 23.4, 20.0.  Up to 64 rows any number of rounds, for the tiled
+// kernel's sums are the longest (5.7e-7 for K = 1024): up to 32 rows 16 x 16 tiles there too, since 64-row tiles would multiply
+// repeated rows (16 x 36864 x 720 28.7 us, 64-row tiles 60.8, tiled 44.8; 8 x 151936 x 1024 130, 285, 192; 17 x 20480 x 720 21.5, 33.0, 30.1;
+// 32 x 24576 x 2048 60.6, 86.7, 77.3; 32 x 65536 x 960 92.9, 132.6, 76.0).
 inline int narrow_plan_f32(int M, int N, bool gated) {
     const long wgs = narrow_wgs(M, N, 0);
-    if (wgs <= 512) return 0;
-    if (M <= 64) return (gated && M > 32) || wgs > 2048 ? 2 : 0;
+    if (wgs <= 512 || M <= 32 || (M <= 64 && !gated)) return 0;
+    if (M <= 64) return 2;
     return wgs <= 2048 ? 0 : -1;
 }
 
