@@ -3,8 +3,7 @@
 
 #include <algorithm>
 #include <atomic>
-#include <stdexcept>
-#include <string>
+#include <exception>
 #include <system_error>
 #include <thread>
 #include <vector>
@@ -16,8 +15,9 @@ namespace vla {
 // Runs `work(task)` for every task of every group (group g: tasks first[g] .. first[g + 1] - 1) on up to `threads` threads,
 // the calling one among them, in order; `ready(g)` is called on the calling thread, in order of g, as soon as it sees
 // that the tasks of groups 0 .. g are done (an upload then overlaps the next groups' work).  The threads live for this
-// call only: one start per call, where a start per group cost 27 observations 24 of them.  The first error is thrown
-// when all threads are back; ready() is not called for groups from there on.
+// call only: one start per call, where a start per group cost 27 observations 24 of them.  The first exception, of a task or
+// of ready(), is thrown again when all threads are back: no further task starts, and ready() is not called for groups from there
+// on (a task that throws never counts as done, so its group is not announced whoever looks at it when).
 template <typename Work, typename Ready>
 void run_staged(const std::vector<int>& first, int threads, Work work, Ready ready) {
     const int n_groups = (int)first.size() - 1, n_tasks = first.back();
@@ -25,16 +25,20 @@ void run_staged(const std::vector<int>& first, int threads, Work work, Ready rea
     std::atomic<bool> failed{false};
     std::vector<std::atomic<int>> left(n_groups);
     for (int g = 0; g < n_groups; ++g) left[g] = first[g + 1] - first[g];
-    std::string error;
+    std::exception_ptr error;
     std::atomic_flag has_error = ATOMIC_FLAG_INIT;
+    auto fail = [&]() {
+        if (!has_error.test_and_set()) error = std::current_exception();
+        failed = true;
+    };
     auto one = [&]() {  // false: no task left
         const int t = next.fetch_add(1);
         if (t >= n_tasks || failed) return false;
         try {
             work(t);
-        } catch (const std::exception& e) {
-            if (!has_error.test_and_set()) error = e.what();
-            failed = true;
+        } catch (...) {
+            fail();
+            return true;
         }
         const int g = (int)(std::upper_bound(first.begin(), first.end(), t) - first.begin()) - 1;
         left[g].fetch_sub(1, std::memory_order_release);
@@ -47,20 +51,24 @@ void run_staged(const std::vector<int>& first, int threads, Work work, Ready rea
     };
     int done = 0;
     auto announce = [&]() {
-        while (done < n_groups && !failed && left[done].load(std::memory_order_acquire) == 0) ready(done++);
+        while (done < n_groups && left[done].load(std::memory_order_acquire) == 0) ready(done++);
     };
     {
         Join join{pool};
         try {
             for (int t = 1; t < std::min(threads, n_tasks); ++t) pool.emplace_back([&]() { while (one()) {} });
         } catch (const std::system_error&) {}  // no more threads to be had: the ones there are do the work
-        while (one()) announce();
-        while (done < n_groups && !failed) {  // the others' last tasks
-            announce();
-            std::this_thread::yield();
+        try {
+            while (one()) announce();
+            while (done < n_groups && !failed) {  // the others' last tasks
+                announce();
+                std::this_thread::yield();
+            }
+        } catch (...) {
+            fail();
         }
     }
-    if (failed) throw std::runtime_error(error);
+    if (failed) std::rethrow_exception(error);
 }
 
 // Pieces of 1 MiB and more that an observation's `bytes` are cut into for run_staged, and the threads for a batch.  Up to four
