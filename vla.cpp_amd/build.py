@@ -26,8 +26,11 @@ def sources():
 
 # Kernels that keep registers "in flight" between an inline-assembly load and its wait must
 # not spill: a spilled in-flight register is stored before its data arrives and reused while
-# the load is still due.  Their scratch size is read from the compiler's resource remarks.
-NO_SPILL_KERNELS = {"gemm.hip": ["ternary_gemm_x16_kernel"], "dit_self.hip": ["dit_self_block_kernel"]}
+# the load is still due.  Kernels that count their vector-memory waits by hand must not either: spills add operations
+# to the count, and the waits no longer leave in flight what they were meant to.  Their scratch size is read from the
+# compiler's resource remarks.
+NO_SPILL_KERNELS = {"gemm.hip": ["ternary_gemm_x16_kernel"], "dit_self.hip": ["dit_self_block_kernel"], "gemm_wide.hip": ["gemm_wide_kernel"],
+                    "gemm_f32.hip": ["gemm_narrow_f32_kernel"], "attention.hip": ["attn_tiles_kernel", "attn_rows_kernel"]}
 
 
 def _check_no_spill(src, remarks):
@@ -41,7 +44,7 @@ def _check_no_spill(src, remarks):
                         seen = True
                         size = int(m.split("ScratchSize [bytes/lane]:")[1].split()[0])
                         if size != 0:
-                            raise RuntimeError("%s spills %d bytes per lane: its in-flight registers are not safe" % (kernel, size))
+                            raise RuntimeError("%s spills %d bytes per lane: its in-flight registers or counted waits are not safe" % (kernel, size))
                         break
         if not seen:
             raise RuntimeError("no resource remarks for %s in %s" % (kernel, src))

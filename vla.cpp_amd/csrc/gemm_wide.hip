@@ -225,18 +225,12 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_wide_kernel(GemmArgs a) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) cs[e] = a.colsum[(e < 8 ? tc.base0 : tc.base1) + jg + (e & 7)];
     }
-    // A bf16 residual of all the lane's rows is requested before the first row is stored (it may be the output buffer).
+    // A bf16 residual of up to four of the lane's rows is requested before the first of them is stored (it may be the output
+    // buffer: a lane stores no other lane's elements).  All eight of the 256 x 256 tile at once are 64 registers beside 128
+    // accumulators and spilled.
+    constexpr int RG = RM < 4 ? RM : 4;
     const bool have_res = kEpi == EPI_PLAIN && a.residual != nullptr && a.out_bf16 && a.N % 8 == 0;
-    u32x4_t res[RM][2] = {};
-    if (have_res) {
-#pragma unroll
-        for (int i = 0; i < RM; ++i)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int m = min(m0 + (wm * RM + i) * 16 + c, a.M - 1), n = min(nt * 64 + h * 32 + jg, a.N - 8);
-                res[i][h] = *reinterpret_cast<const u32x4_t*>((const bf16_t*)a.residual + (long)m * a.N + n);
-            }
-    }
+    u32x4_t res[RG][2] = {};
     // QKV: what belongs to the lane's columns is formed once for all of its rows.  dst[h]: element (b = 0, s = 0) of half h's
     // first column; rows are s_stride apart within an observation, observations b_stride.
     bf16_t* dst[2] = {nullptr, nullptr};
@@ -256,6 +250,15 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_wide_kernel(GemmArgs a) {
     }
 #pragma unroll
     for (int i = 0; i < RM; ++i) {
+        if (have_res && i % RG == 0) {
+#pragma unroll
+            for (int j = 0; j < RG; ++j)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int m = min(m0 + (wm * RM + i + j) * 16 + c, a.M - 1), n = min(nt * 64 + h * 32 + jg, a.N - 8);
+                    res[j][h] = *reinterpret_cast<const u32x4_t*>((const bf16_t*)a.residual + (long)m * a.N + n);
+                }
+        }
         const int mr = (wm * RM + i) * 16 + c;
         float lo[8], hi[8];
 #pragma unroll
@@ -274,7 +277,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_wide_kernel(GemmArgs a) {
         }
         if (m0 + mr >= a.M) continue;
         if (kEpi != EPI_QKV) {
-            epilogue_16<bf16_t, kEpi, true>(a, m0 + mr, nt, tc, jg, lo, hi, have_res, res[i][0], res[i][1], bias);
+            epilogue_16<bf16_t, kEpi, true>(a, m0 + mr, nt, tc, jg, lo, hi, have_res, res[i % RG][0], res[i % RG][1], bias);
             continue;
         }
         const int b = (int)div_c((unsigned)(m0 + mr), a.div_s), s = m0 + mr - b * a.S;
