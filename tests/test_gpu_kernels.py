@@ -195,9 +195,9 @@ def test_linear_bias_residual(dtype, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(50, 720, 960), (3, 37, 2048), (64, 1601, 52), (33, 8, 4), (50, 64, 2052)])
-def test_fp32_rows_of_one_observation_take_the_fma_kernel(M, N, K, monkeypatch):
-    """At most 64 fp32 rows go through the FMA kernel (8 columns per workgroup, 16 partial sums
-    per output).  It and the MFMA kernel (pinned with VLA_GEMM_TILE) against the oracle at the
+def test_fp32_rows_of_one_observation_on_narrow_and_on_large_tiles(M, N, K, monkeypatch):
+    """At most 64 fp32 rows go through the narrow-tile kernel (16 columns per workgroup, K shared out
+    over wavefronts).  It and the tiled kernel (pinned with VLA_GEMM_TILE) against the oracle at the
     fp32 bar and against each other, with ragged N, K not a multiple of 64, bias, activation,
     column gate and residual."""
     r = np.random.default_rng(1700 + N)
@@ -901,6 +901,16 @@ def test_attention_cache_rows_of_any_multiple_of_8(dtype, case):
         assert rel_err(got, want) < FP32_TOL, rel_err(got, want)
     else:
         assert bf16_close(got, want) and rel_err(got, want) < 1e-2
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("case", [c for c in CASES if c[5] in (48, 64)], ids=[c[0] for c in CASES if c[5] in (48, 64)])
+def test_tiled_attention_where_few_workgroups_take_another_kernel(tune, dtype, case):
+    """48- and 64-wide heads: launches of the size of CASES take the kernels with a wavefront per key block.  The tiled kernel that
+    larger launches take (in fp32 with its key slices and the merge launch) on the same cases."""
+    tune.set("VLA_ATTN_ROWS", 0)
+    test_attention_against_oracle(tune, dtype, "auto", case)
+    test_attention_cache_rows_of_any_multiple_of_8(dtype, case)
 
 
 @pytest.mark.parametrize("split", [1, 2, 5, 8, 64])
