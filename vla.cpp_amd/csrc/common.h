@@ -315,7 +315,7 @@ __device__ __forceinline__ float div_1p(float x, float e) {
 }
 // The same for values that are rounded to bf16 next, N at a time.  The exact division and tanhf above are some 25 and 45
 // instructions per value, and a 128 x 128 tile has 64 per thread: 12 of the 65 us that 1323 x 6144 x 1536 with GELU took on such
-// tiles (on the wide tiles now 29.3 us, 25.9 without an activation).  Here 9 and 11: GELU's tanh form is written as the sigmoid
+// tiles (on the wide tiles now 30.9 us, 28.3 without an activation).  Here 9 and 11: GELU's tanh form is written as the sigmoid
 // it is, 0.5 x (1 + tanh u) = x / (1 + exp(-2 u)).  SiLU has the bits of the exact form.  GELU against float64, 4 M values of N(0, 1):
 // 4.2e-8 of the norm (tanhf 3.8e-8; N(0, 0.3^2) 4.0e-8, tanhf 4.2e-8), largest error 1.6e-6 of the value (tanhf 0.35, where 1 + tanh u
 // cancels); rounded to bf16 both are 1.665157630e-3 of the norm, and 29 values are not the nearest (tanhf 111).

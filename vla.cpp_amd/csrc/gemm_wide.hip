@@ -40,8 +40,8 @@ __device__ __forceinline__ void wait_tiles(int tiles) {
 // issues its products first instead of alternating, and the others' reads fall behind them (4096 x 4096 x 4096 113 -> 100 us
 // as a kernel without epilogue variants).
 // Against the direct-to-LDS kernel (128 x 128 tiles of four wavefronts, 32x32x16; us, weights not in the caches): 1323 x 6144 x 1536
-// 53.3 -> 30.2 (0.83 PFLOP/s; loads alone 26, MFMA and LDS alone 23), 816 x 8192 x 1024 gated 22.3 -> 19.8, 1323 x 4608 x 1536 with the
-// LayerNorm inside 34.8 -> 30.5, 13824 x 3072 x 2048 202 -> 160, 4096 x 4096 x 4096 149 -> 107 (1.29 PFLOP/s).
+// 46.3 -> 28.3 (0.88 PFLOP/s; loads alone 22 to 26, MFMA and LDS alone 23), 816 x 8192 x 1024 gated 21.4 -> 19.6, 1323 x 4608 x 1536 with the
+// LayerNorm inside 34.8 -> 30.5, 13824 x 3072 x 2048 186 -> 144, 4096 x 4096 x 4096 147 -> 102 (1.35 PFLOP/s).
 template <int kEpi, int kNorm, int RM, int WM, int WN, int NS>
 __global__ void __launch_bounds__(64 * WM * WN) gemm_wide_kernel(GemmArgs a) {
     constexpr int RN = 4, BM = 16 * RM * WM, BW = 64 * WN, NW = WM * WN, KB = 128, BK = 64;

@@ -147,10 +147,10 @@ enum { WIDE_256X256 = 0, WIDE_192X192, WIDE_256X128, WIDE_192X128, WIDE_128X128,
 
 // The wide tile with the least predicted time, or -1 where the direct-to-LDS kernel's tile is not predicted 6 % slower.  kind:
 // 0 plain or gated, 1 QKV, 2 QKV with a LayerNorm inside.  On the fitted shapes the wide tile is taken on 60 %, where it needs
-// 0.83 of the time (geometric mean; 0.90 over all, 0.89 if the faster one were always known); 1 % of them are 3 to 7 %
-// slower, one 15 % (576 x 2752 x 5552 gated, 71.6 -> 82.0 us).  1323 x 6144 x 1536 53 -> 28 us (192 x 192: 224 workgroups, one
-// round, where 528 of 128 x 128 left 16 for a second one), 816 x 8192 x 1024 gated 23 -> 20, 13824 x 3072 x 2048 203 -> 161
-// (256 x 256), 4096 x 4096 x 4096 150 -> 107.
+// 0.84 of the time (geometric mean; 0.90 over all, 0.89 if the faster one were always known); 1 % of them are 3 to 7 %
+// slower, one 15 % (576 x 2752 x 5552 gated, 71.6 -> 82.0 us).  1323 x 6144 x 1536 46.3 -> 28.3 us (192 x 192: 224 workgroups, one
+// round, where 528 of 128 x 128 left 16 for a second one), 816 x 8192 x 1024 gated 21.4 -> 19.6, 13824 x 3072 x 2048 186 -> 144
+// (256 x 256), 4096 x 4096 x 4096 147 -> 102 (weights not in the caches).
 inline int wide_tile(int M, int N, int K, int kind) {
     static const TileTime wide[WIDE_TILES] = {
         {256, 256, false, 0.18, 11.50, 1.234, 0.314, 0, 0, 1.57, 3.50}, {192, 192, false, 1.05, 7.02, 0.703, 0.225, 0, 0, 2.04, 3.15},

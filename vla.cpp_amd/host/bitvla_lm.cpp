@@ -259,7 +259,9 @@ void BitvlaLm::prefill(const Inputs* in, int batch) {
         }
     };
     run_staged(
-        first, 1,  // 2.6 MB an observation: see stage_threads
+        // One thread at every batch.  2.6 MB of features and 256 rows of text an observation: with eight threads eight observations
+        // take 23.7 ms a call where they take 25.8, twelve 31.0 and 34.1; the caller's refill of its buffers takes 0.6 and 1.1 ms with either.
+        first, 1,
         [&](int t) {
             const int b = t / per_obs, piece = t % per_obs - 1;
             if (piece < 0) return stage_text(b);
