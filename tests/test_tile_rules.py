@@ -21,6 +21,10 @@ extern "C" int tiles_kernel(int grid, int tiles) { return vla_rules::attn_tiles(
 extern "C" int f32_tile(int M, int n_tiles) { return vla_rules::f32_tile(M, n_tiles); }
 extern "C" int wide(int M, int N, int K, int kind) { return vla_rules::wide_tile(M, N, K, kind); }
 extern "C" int ternary(int M, int N, int K) { return vla_rules::ternary_tile(M, N, K); }
+extern "C" int heads256(int pairs, int rows, int units, int part_rows, int forced) {
+    const vla_rules::WideHeads h = vla_rules::wide_heads(pairs, rows, units, part_rows, forced);
+    return h.rb * 100 + h.slices;
+}
 extern "C" int rows(int p) { return 16 * vla_rules::NARROW_PLANS[p][0]; }
 extern "C" int cols(int p) { return 16 * vla_rules::NARROW_PLANS[p][1]; }
 ''')
@@ -163,3 +167,25 @@ F32_US = [((1323, 1536, 1536), (113.1, 65.2, 110.0, 62.8)), ((408, 1536, 1536), 
 def test_fp32_tile_is_near_the_fastest(rules, shape, us):
     took = dict(zip((0, 1, 2, 4), us))[rules.f32_tile(shape[0], -(-shape[1] // 64))]
     assert took <= 1.04 * min(us)
+
+
+def test_256_wide_heads_keep_to_their_scratch_and_to_one_round(rules):
+    """A split fits the partial rows that the tiled kernel would have used, leaves no slice empty and no XCD more than 32
+    workgroups; what does not fit one round is the tiled kernel's, unless forced."""
+    taken = 0
+    for pairs in list(range(1, 34)) + [64, 100, 1000]:
+        for rows in (1, 8, 16, 17, 32, 33, 136, 400, 408, 800, 1600, 5000):
+            for units in list(range(1, 40)) + [128, 1000]:
+                for part_rows in (0, 512, 2560, 3584, 100000):
+                    rb, s = divmod(rules.heads256(pairs, rows, units, part_rows, 0), 100)
+                    assert divmod(rules.heads256(pairs, rows, units, part_rows, 1), 100)[0] in (1, 2)
+                    if not rb:
+                        continue
+                    taken += 1
+                    tiles, per = -(-rows // (16 * rb)), -(-units // s)
+                    assert rb in (1, 2) and (s - 1) * per < units <= s * per
+                    assert s == 1 or pairs * s * tiles * 16 * rb <= part_rows
+                    assert -(-pairs * s // 8) * tiles <= 32
+    assert taken > 10000
+    assert rules.heads256(1, 400, 15, 2560, 0) == 104 and rules.heads256(8, 400, 15, 10240, 0) == 101 and rules.heads256(16, 400, 15, 32768, 0) == 201
+    assert rules.heads256(20, 400, 15, 100000, 0) < 100

@@ -30,7 +30,7 @@ def sources():
 # to the count, and the waits no longer leave in flight what they were meant to.  Their scratch size is read from the
 # compiler's resource remarks.
 NO_SPILL_KERNELS = {"gemm.hip": ["ternary_gemm_x16_kernel"], "dit_self.hip": ["dit_self_block_kernel"], "gemm_wide.hip": ["gemm_wide_kernel"],
-                    "gemm_f32.hip": ["gemm_narrow_f32_kernel"], "attention.hip": ["attn_tiles_kernel", "attn_rows_kernel"]}
+                    "gemm_f32.hip": ["gemm_narrow_f32_kernel"], "attention.hip": ["attn_tiles_kernel", "attn_rows_kernel", "attn_wide_kernel"]}
 
 
 def _check_no_spill(src, remarks):

@@ -2237,6 +2237,351 @@ bool launch_rows(AttnArgs& a, hipStream_t st) {
     return true;
 }
 
+// ---- 256-wide bf16 heads (pi0 and pi0.5: eight query heads on one kv head) ----
+// The tiled kernel gives such a launch few workgroups of 128 rows, cuts the keys into slices until the chip is covered and pays for it
+// with partials and a merge launch (18.9 + 6.1 us at 16 observations of 955 keys, 13.1 + 4.7 at one).  Here a workgroup owns 16 RB rows of a
+// (batch, kv head) and each of its W wavefronts 64-key units of its own, W units further on each time: no barrier between the first
+// and the last.  What the wavefronts have summed up meets in LDS, so the keys of 16 observations need no slices at all.
+//
+// A unit is eight parts of 8 KiB: the sixteen keys of each of four score products, then 64 rows of V^T at a time.  They go
+// straight into a ring of NS parts in the wavefront's own LDS, in order, each requested when the part four before it has been read, and a part's
+// fragments are read one part ahead of their products.  16x16x32 products as in the decode kernel: S^T = K Q^T, two of 16 keys per 32, row x of
+// product j standing for key 8 (x / 4) + 4 j + x % 4, so that lane (c, q) holds the scores of keys 8 q .. + 7 of both halves
+// against query row c: already the right operand of O^T += V^T P^T.  LDS pieces (16 bytes) are XOR-swizzled, K and Q by the row, V^T by
+// row / 2: the fragment reads, sixteen lanes at a time, are free of bank conflicts.
+//
+// What bounds it: 8 KiB a part is 512 clocks of a CU's 64 bytes a clock from the L2 for four wavefronts, and a wavefront whose request has to wait its
+// turn cannot go on with its products either: of some 7000 clocks that a unit takes (32 rows, 2.1 GHz), 4096 are that, 2048 products and 1900
+// the softmax.  Hence requests, fragment reads and products take turns; one wavefront a SIMD, since 32 rows x 256 of output and the query
+// fragments are 192 registers.  50 positions x 8 heads, 955 keys, keys from memory: 16 observations 27.8 -> 21.9 us, 8 21.9 -> 16.2 (16 rows a
+// workgroup), one 16.6 -> 10.8 (four slices, merged by a launch).  Tried: K through registers (the compiler's waits drain V^T's
+// requests with them), two wavefronts a workgroup and twice the slices (level at one observation), fragments in two sets
+// (registers moved about: 21.3 us with the keys in the caches, now 20.2).
+// RB: 16-row blocks; W: wavefronts; GIVEN: the mask is data (added to the scaled scores; zeros and -inf give the generated masks' bits).
+template <int RB, int W, bool GIVEN>
+__global__ void __launch_bounds__(W * 64, 1) attn_wide_kernel(AttnArgs a) {
+    constexpr int D = 256, NDB = D / 16, STAGE = 8192, NS = 4, NL = STAGE / 1024, RING = NS * STAGE, ROWS = 16 * RB;
+    constexpr int QL = RB * NL / W;  // a wavefront's share of the query rows' load instructions
+    static_assert(RB * NL % W == 0 && ROWS <= 64, "the wavefronts share the query rows out evenly");
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[W * RING + RB * STAGE];  // rings, Q
+    __shared__ f32x2_t row_ml[W][ROWS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane & 15, q = lane >> 4;
+    const int local = (int)blockIdx.x >> 3, p8 = (int)div_c(local, a.dGS);
+    const int tile = local - p8 * a.n_groups, ps = p8 * 8 + ((int)blockIdx.x & 7);  // (pair, slice)
+    if (ps >= a.batch * a.Hkv * a.n_split) return;
+    const int pair = (int)div_c(ps, a.dns), split = ps - pair * a.n_split;
+    const int b = (int)div_c(pair, a.dHkv), hk = pair - b * a.Hkv;
+    const int R = a.grp * a.S;
+    // This wavefront's units: u0, u0 + W, ...  Where it starts depends on the row tile, so that the tiles of a pair, which walk side by
+    // side, do not all wait for the same unit to come from memory; a unit that reaches past n_keys stays the last.
+    const int units = (a.n_keys + 63) / 64, u0 = split * a.tiles_per_split + wave, u_end = min(units, (split + 1) * a.tiles_per_split);
+    const int count = u0 < u_end ? (u_end - u0 + W - 1) / W : 0;
+    const int turning = count - (count > 0 && (a.n_keys & 63) && u0 + (count - 1) * W == units - 1);  // units whose order turns
+    int at = turning > 0 ? tile % turning : 0, u = u0 + at * W;
+
+    // lane x's query position and row of q / out, for row x of the tile
+    const int row_x = min(tile * ROWS + (lane & (ROWS - 1)), R - 1), hg_x = (int)div_c(row_x, a.dS), s_x = row_x - hg_x * a.S;
+    const int out_x = (b * a.S + s_x) * a.Hq + hk * a.grp + hg_x;
+    unsigned char* const ring = lds + wave * RING;
+    const uint32_t ring0 = (uint32_t)(uintptr_t)ring;  // low 32 bits of a shared-aperture address = LDS offset
+    const int r2 = lane >> 5, p32 = lane & 31, r8 = lane >> 3;
+#pragma unroll
+    for (int i = 0; i < QL; ++i) {
+        const int l = i * W + wave, x = 2 * l + r2;
+        load_to_lds16((const unsigned char*)a.q + (long)__shfl(out_x, x) * (D * 2) + (p32 ^ (x & 15)) * 16, (uint32_t)(uintptr_t)lds + W * RING + l * 1024);
+    }
+    // Part j of unit uu into slot j % NS: j < 4 the sixteen keys of score product j (row x: key 32 (j / 2) + 8 (x / 4) + 4 (j % 2) + x % 4
+    // of the unit), else 64 rows of V^T.  Lane offsets are formed once; those of the unit that reaches past n_keys again: keys
+    // there repeat the last one (their scores are masked), V^T runs are kept inside the cache row.
+    const unsigned char* kbase = (const unsigned char*)a.k_cache + ((long)b * a.Hkv + hk) * a.t_max * (D * 2);
+    const unsigned char* vbase = (const unsigned char*)a.vt_cache + ((long)b * a.Hkv + hk) * D * (long)a.t_max * 2;
+    uint32_t koff[NL], voff[NL];
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+        koff[i] = (uint32_t)((8 * (i >> 1) + 2 * (i & 1) + r2) * (D * 2) + (p32 ^ (2 * i + r2)) * 16);
+        voff[i] = (uint32_t)((i * 8 + r8) * a.t_max * 2 + ((lane & 7) ^ (((i & 1) * 4 + (r8 >> 1)) & 7)) * 16);
+    }
+    const unsigned char* src = nullptr;
+    auto begin_part = [&](int uu, int j) __attribute__((always_inline)) {
+        if (j < 4) {
+            const int first = min(uu * 64 + 32 * (j >> 1) + 4 * (j & 1), a.n_keys - 1);
+            if (uu * 64 + 64 > a.n_keys) {  // uniform; the last unit: no whole one follows
+#pragma unroll
+                for (int i = 0; i < NL; ++i)
+                    koff[i] = (min(koff[i] >> 9, (uint32_t)(a.n_keys - 1 - first)) << 9) | (koff[i] & 511);  // (fewer rows are left with every part)
+            }
+            src = kbase + (long)first * (D * 2);
+        } else {
+            if (j == 4 && uu * 64 + 64 > a.n_keys) {  // uniform
+#pragma unroll
+                for (int i = 0; i < NL; ++i) voff[i] -= (uint32_t)max(((lane & 7) ^ (((i & 1) * 4 + (r8 >> 1)) & 7)) * 16 - (a.t_max - 8 - uu * 64) * 2, 0);
+            }
+            src = vbase + ((long)(j - 4) * 64 * a.t_max + uu * 64) * 2;
+        }
+    };
+    auto load = [&](int j, int i) __attribute__((always_inline)) { load_to_lds16_plus(src, j < 4 ? koff[i] : voff[i], ring0, (j % NS) * STAGE + i * 1024); };
+    auto load_if = [&](bool c, int j, int i) __attribute__((always_inline)) { load_to_lds16_plus_if(c, src, koff[i], ring0, (j % NS) * STAGE + i * 1024); };
+    typedef u32x4_t Frag[8];
+    const int fsw = (c >> 1) & 7;
+    auto row_frag = [&](const unsigned char* part, int ch) __attribute__((always_inline)) {  // Q, K: piece 4 ch + q of row c
+        return *reinterpret_cast<const u32x4_t*>(part + c * 512 + (((4 * ch + q) ^ c) * 16));
+    };
+    auto v_frag = [&](const unsigned char* part, int x) __attribute__((always_inline)) {  // 2 d + hh: keys 32 hh + 8 q .. + 7 of row 16 d + c
+        return *reinterpret_cast<const u32x4_t*>(part + ((x >> 1) * 16 + c) * 128 + (((4 * (x & 1) + q) ^ fsw) * 16));
+    };
+    // V^T elements past n_keys (stale cache contents, possibly NaN) to zero, lane = row of the part
+    auto zero_tail = [&](unsigned char* part, int valid) __attribute__((always_inline)) {
+        unsigned char* rowp = part + lane * 128;
+        const int sw = (lane >> 1) & 7;
+        int p = valid >> 3;
+        if (valid & 7) {  // uniform; the piece that has real keys too
+            u32x4_t* at = reinterpret_cast<u32x4_t*>(rowp + ((p ^ sw) * 16));
+            u32x4_t v = *at;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] &= (2 * e < (valid & 7) ? 0xffffu : 0u) | (2 * e + 1 < (valid & 7) ? 0xffff0000u : 0u);
+            *at = v;
+            ++p;
+        }
+        for (; p < 8; ++p) *reinterpret_cast<u32x4_t*>(rowp + ((p ^ sw) * 16)) = u32x4_t{0u, 0u, 0u, 0u};
+    };
+
+    int hi[RB], srow[RB];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+        const int s = __shfl(s_x, rb * 16 + c);
+        srow[rb] = s;
+        hi[rb] = a.n_keys;
+        if (a.mask_kind == VLA_MASK_CAUSAL_SUFFIX) hi[rb] = min(a.n_keys, a.n_prefix + s + 1);
+        else if (a.mask_kind == VLA_MASK_PI0_STATE && s == 0) hi[rb] = min(a.n_keys, a.n_prefix + 1);
+    }
+    const int pad_lo = a.pad_start, pad_hi = min(a.pad_end, a.n_prefix);
+    if (count) {  // uniform
+#pragma unroll
+        for (int j = 0; j < NS; ++j) {
+            begin_part(u, j);
+#pragma unroll
+            for (int i = 0; i < NL; ++i) load(j, i);
+        }
+        wait_vmcnt<NS * NL>();
+    } else {
+        wait_vmcnt<0>();
+    }
+    __syncthreads();
+    Frag qf[RB], f;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int ch = 0; ch < 8; ++ch) qf[rb][ch] = row_frag(lds + W * RING + rb * STAGE, ch);
+    constexpr float LOG2E = 1.4426950408889634f;
+    const float c2 = a.scale * LOG2E;
+    f32x4_t o[RB][NDB];
+    float m_run[RB], l_run[RB];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+        m_run[rb] = -INFINITY;
+        l_run[rb] = 0.f;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db) o[rb][db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    if (count) {
+        wait_vmcnt<(NS - 1) * NL>();
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int ch = 0; ch < 8; ++ch) f[ch] = row_frag(ring, ch);
+    }
+    for (int n = 0; n < count; ++n) {
+        const bool more = n + 1 < count;  // uniform
+        at = n + 1 >= turning ? turning : (at + 1 == turning ? 0 : at + 1);
+        const int u_next = u0 + at * W;
+        const int k0 = u * 64;
+        const bool partial = k0 + 64 > a.n_keys;
+        f32x4_t sc[RB][2][4];
+        u32x4_t pf[RB][2];
+        // Part j: its fragments are on their way (read a part earlier).  Once they are here its slot takes the part four
+        // further on; requests, the next part's fragment reads and this part's products take turns.
+        auto step = [&](auto jt) __attribute__((always_inline)) {
+            constexpr int j = decltype(jt)::value, nx = (j + 1) % 8;
+            unsigned char* const next = ring + nx % NS * STAGE;
+            if (j < 4) begin_part(u, j + 4);
+            else if (more) begin_part(u_next, j - 4);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (j < 4 || more) wait_vmcnt<2 * NL>();
+            else wait_vmcnt<(j < 6 ? 6 - j : 0) * NL>();
+            asm volatile("" ::: "memory");
+            if (nx >= 4 && partial) zero_tail(next, a.n_keys - k0);  // uniform
+            {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    if (j < 4) load(j + 4, i);
+                    else load_if(more, j - 4, i);
+#pragma unroll
+                    for (int rb = 0; rb < RB; ++rb) {
+                        if constexpr (j < 4) {
+                            constexpr int NA = RB == 1 ? 2 : 1;  // chains of products that depend on each other, so that one need not wait for another
+                            const f32x4_t z = {0.f, 0.f, 0.f, 0.f};
+                            sc[rb][i % NA][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, f[i]), __builtin_bit_cast(bf16x8_t, qf[rb][i]), i < NA ? z : sc[rb][i % NA][j], 0, 0, 0);
+                        } else {
+                            const int d = i / 2, hh = i % 2;
+                            o[rb][(j - 4) * 4 + d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, f[2 * d + hh]), __builtin_bit_cast(bf16x8_t, pf[rb][hh]), o[rb][(j - 4) * 4 + d], 0, 0, 0);
+                        }
+                    }
+                    if (nx >= 4) f[i] = v_frag(next, i);
+                    else f[i] = row_frag(next, i);  // (behind the last unit: not used)
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        };
+        step(std::integral_constant<int, 0>{});
+        step(std::integral_constant<int, 1>{});
+        step(std::integral_constant<int, 2>{});
+        step(std::integral_constant<int, 3>{});
+        const bool masked = partial || (k0 < pad_hi && k0 + 64 > pad_lo) || (a.mask_kind != VLA_MASK_NONE && k0 + 64 > a.n_prefix);
+        float p[RB][16], m_tile[RB];  // key k0 + 32 (i / 8) + 8 q + i % 8; scores, then probabilities
+        float add[RB][16];
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) p[rb][i] = RB == 1 ? sc[rb][0][i >> 2][i & 3] + sc[rb][1][i >> 2][i & 3] : sc[rb][0][i >> 2][i & 3];
+            const int key0 = k0 + 8 * q;
+            if (GIVEN) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int key = key0 + (i >> 3) * 32 + (i & 7);
+                    const float mv = a.mask[(long)srow[rb] * a.n_keys + min(key, a.n_keys - 1)] * LOG2E;
+                    add[rb][i] = key < a.n_keys ? mv : -INFINITY;
+                }
+            } else if (masked) {  // uniform
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int key = key0 + (i >> 3) * 32 + (i & 7);
+                    const bool visible = (key < hi[rb]) & !((key >= pad_lo) & (key < pad_hi));
+                    p[rb][i] = visible ? p[rb][i] : -INFINITY;
+                }
+            }
+            m_tile[rb] = -INFINITY;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) m_tile[rb] = fmaxf(m_tile[rb], GIVEN ? fmaf(p[rb][i], c2, add[rb][i]) : p[rb][i]);
+            m_tile[rb] = rows_max(m_tile[rb]) * (GIVEN ? 1.f : c2);  // (the scale is positive)
+        }
+        // the lazily updated reference of the tiled kernel, moved for all of the wavefront's rows at once
+        bool moves = m_tile[0] > m_run[0] + RESCALE_LOG2;
+#pragma unroll
+        for (int rb = 1; rb < RB; ++rb) moves |= m_tile[rb] > m_run[rb] + RESCALE_LOG2;
+        if (__builtin_amdgcn_ballot_w64(moves) != 0) {
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+                const float m_new = fmaxf(m_run[rb], m_tile[rb]);
+                const float alpha = __builtin_amdgcn_exp2f(m_run[rb] - (m_new == -INFINITY ? 0.f : m_new));
+                l_run[rb] *= alpha;
+                m_run[rb] = m_new;
+                if (n) {  // uniform; before that the sums are zero
+#pragma unroll
+                    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) o[rb][db][e] *= alpha;
+                }
+            }
+        }
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            const float m_use = m_run[rb] == -INFINITY ? 0.f : m_run[rb];
+            float psum[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                // (a mask value is added before the reference is taken off: beside a very low one the score has to vanish)
+                const float x = GIVEN && add[rb][i] != 0.f ? fmaf(p[rb][i], c2, add[rb][i]) - m_use : fmaf(p[rb][i], c2, -m_use);
+                p[rb][i] = __builtin_amdgcn_exp2f(x);
+                psum[i & 3] += p[rb][i];
+            }
+            l_run[rb] += rows_sum((psum[0] + psum[1]) + (psum[2] + psum[3]));
+#pragma unroll
+            for (int hh = 0; hh < 2; ++hh)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) pf[rb][hh][e] = pack_bf2(p[rb][8 * hh + 2 * e], p[rb][8 * hh + 2 * e + 1]);
+        }
+        step(std::integral_constant<int, 4>{});
+        step(std::integral_constant<int, 5>{});
+        step(std::integral_constant<int, 6>{});
+        step(std::integral_constant<int, 7>{});
+        u = u_next;
+    }
+
+    // The wavefronts' partial rows meet in LDS, each in the ring of its owner (32 rows of 1 KiB fill one): 16-byte piece pc of row
+    // r at position pc ^ (r % 16).
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+#pragma unroll
+        for (int db = 0; db < NDB; ++db) *reinterpret_cast<f32x4_t*>(ring + (rb * 16 + c) * 1024 + (((db * 4 + q) ^ c) * 16)) = o[rb][db];
+        if (q == 0) row_ml[wave][rb * 16 + c] = f32x2_t{m_run[rb], l_run[rb]};
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ROWS / W; ++i) {
+        const int r = i * W + wave, row = tile * ROWS + r;
+        f32x2_t ml[W];
+        f32x4_t ow[W];
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            ml[w] = row_ml[w][r];
+            ow[w] = *reinterpret_cast<const f32x4_t*>(lds + w * RING + r * 1024 + ((lane ^ (r & 15)) * 16));
+        }
+        float m = ml[0][0];
+#pragma unroll
+        for (int w = 1; w < W; ++w) m = fmaxf(m, ml[w][0]);
+        const float m_use = m == -INFINITY ? 0.f : m;
+        float l = 0.f;
+        f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            const float f = __builtin_amdgcn_exp2f(ml[w][0] - m_use);  // 2^-inf = 0 for a wavefront without a visible key
+            l += ml[w][1] * f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] += ow[w][e] * f;
+        }
+        if (row >= R) return;  // uniform
+        if (a.n_split > 1) {
+            const long prow = ((long)pair * a.n_split + split) * a.r_pad + row;
+            *reinterpret_cast<f32x4_t*>(a.part_o + prow * D + lane * 4) = acc;
+            if (lane == 0) *reinterpret_cast<f32x2_t*>(a.part_ml + prow * 2) = f32x2_t{m, l};
+        } else {
+            const float inv = l > 0.f ? 1.0f / l : 0.f;
+            *reinterpret_cast<u32x2_t*>((bf16_t*)a.out + (long)__builtin_amdgcn_readlane(out_x, r) * D + lane * 4) =
+                u32x2_t{pack_bf2(acc[0] * inv, acc[1] * inv), pack_bf2(acc[2] * inv, acc[3] * inv)};
+        }
+    }
+}
+
+// The launch of attn_wide_kernel (and, with the keys sliced over workgroups, what a merge launch needs): false, launching nothing, where
+// the call is not one of its.  part_rows: rows of partials that the bound scratch has room for.
+bool launch_wide_heads(AttnArgs& a, hipStream_t st, long part_rows) {
+    const Tuning& tn = tuning();
+    if (tn.attn_rows == 0 || a.p2 || !(a.scale > 0.f) || (((uintptr_t)a.q | (uintptr_t)a.k_cache | (uintptr_t)a.vt_cache | (uintptr_t)a.out) & 15)) return false;
+    const long pairs = (long)a.batch * a.Hkv;
+    const int R = (a.Hq / a.Hkv) * a.S, units = (a.n_keys + 63) / 64;
+    const vla_rules::WideHeads p = vla_rules::wide_heads(pairs, R, units, part_rows, tn.attn_rows > 0);
+    if (!p.rb) return false;
+    const int tiles = (R + 16 * p.rb - 1) / (16 * p.rb);
+    const long grid = (pairs * p.slices + 7) / 8 * 8 * tiles;
+    // rows of q and out are 32-bit indices, a part's V^T offsets 32-bit bytes
+    if (grid >= (1l << 31) || (long)a.batch * a.S * a.Hq >= (1l << 31) || (long)a.t_max * 128 >= (1l << 31)) return false;
+    a.tiles_per_split = (units + p.slices - 1) / p.slices;
+    a.n_split = p.slices;
+    a.r_pad = tiles * 16 * p.rb;
+    a.part_half = 0;
+    a.n_groups = tiles;
+    set_divisors(a, grid);
+    a.dGS = make_divc(tiles, grid);
+    if (a.mask) {
+        if (p.rb == 2) attn_wide_kernel<2, 4, true><<<(unsigned)grid, 256, 0, st>>>(a);
+        else attn_wide_kernel<1, 4, true><<<(unsigned)grid, 256, 0, st>>>(a);
+    } else {
+        if (p.rb == 2) attn_wide_kernel<2, 4, false><<<(unsigned)grid, 256, 0, st>>>(a);
+        else attn_wide_kernel<1, 4, false><<<(unsigned)grid, 256, 0, st>>>(a);
+    }
+    return true;
+}
+
 // Merge of key-split partials as a launch of its own: one wavefront per (pair, row).
 template <typename T, bool HALF>
 __global__ void __launch_bounds__(256) attn_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
@@ -2534,6 +2879,10 @@ int launch_d(AttnArgs& a, vla_stream_t stream, Scratch& sc) {
     // (after the scratch is bound: a call is refused for want of it whichever kernel serves it)
     if constexpr (D == 64 || D == 48) {
         if (launch_rows<T, D>(a, st)) return hipGetLastError() == hipSuccess ? VLA_K_OK : VLA_K_ERR_LAUNCH;
+    }
+    if constexpr (sizeof(T) == 2 && D == 256) {
+        const long rows = a.n_split > 1 ? (long)a.batch * a.Hkv * a.n_split * a.r_pad : 0;
+        if (launch_wide_heads(a, st, rows)) return hipGetLastError() == hipSuccess ? launch_merge<T, D>(a, st) : VLA_K_ERR_LAUNCH;
     }
     switch (nw) {
         case 1: return launch_nw<T, D, 1>(a, st);

@@ -5,11 +5,6 @@ namespace {
 
 using namespace vk;
 
-// One 16-byte load per lane from uniform base + 32-bit lane offset straight into LDS (see load_to_lds16).
-__device__ __forceinline__ void load_to_lds16_at(const void* base, uint32_t off, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(off), "s"(base) : "memory");
-}
-
 // wait until at most `tiles` tiles of NL loads are due (uniform run-time count, at most MAX)
 template <int NL, int MAX>
 __device__ __forceinline__ void wait_tiles(int tiles) {

@@ -219,4 +219,37 @@ inline bool attn_tiles(long grid, int blocks) {
 // it: 16 rows x 16 heads on 4, 1000 keys 14.8 us, here 16.0 (one slice only: 50 x 15 on 5, two observations 87.9, here 17.1).
 inline bool attn_rows(long grid, int blocks, bool sliced) { return grid <= 512 && (blocks <= 20 || !sliced); }
 
+// Row blocks (of 16) per workgroup and key slices of a bf16 attention launch of 256-wide heads on attn_wide_kernel, or rb = 0 for the tiled
+// kernel.  pairs: (observation, kv head); units: 64-key units, four of which a workgroup walks at a time; part_rows: rows of partials
+// that the call's scratch holds (what the tiled kernel asks for, so that no call needs more than it did).  A workgroup fills a CU, so only splits whose
+// workgroups all run at once (32 on the busiest XCD) are taken: behind them the tiled kernel is the faster one, which reads K and
+// V^T once per 128 rows (50 positions x 8 heads on 955 keys, 20 observations, 260 workgroups: tiled 40.5 us, here 41.7; 32: 34.6, 46.8).  Of
+// these the least predicted time (us): start and end 5.5, a round of units 2.5 (16 rows) or 3.3 (32), the merge launch 1.8 and 0.75 per
+// 1000 partial rows.  Against the tiled kernel and its merge, 50 positions, 955 keys from memory: 1, 2, 4, 8, 12, 16 observations 16.6, 18.3, 19.1,
+// 22.0, 31.2, 27.8 us, here 10.8, 13.1, 15.6, 16.2, 21.2, 21.9; 60 to 330 keys at 1 to 16 observations 0.59 to 0.95 of its time.  16 rows or
+// fewer on 5 to 8 units: two rounds for what one wavefront row of the tiled kernel's slices does as fast (8 rows, 281 keys 9.1 us,
+// here 9.8): left to it.
+struct WideHeads {
+    int rb, slices;
+};
+inline WideHeads wide_heads(long pairs, int rows, int units, long part_rows, bool forced) {
+    WideHeads best = {0, 1};
+    if (rows <= 16 && units > 4 && units <= 8 && !forced) return best;
+    double least = 1e30;
+    for (int rb = 1; rb <= 2; ++rb) {
+        const long tiles = (rows + 16 * rb - 1) / (16 * rb);
+        for (int s = 1; s <= 16 && s <= units; ++s) {
+            const int per = (units + s - 1) / s;
+            const long partials = s > 1 ? pairs * s * tiles * 16 * rb : 0, rounds = ((pairs * s + 7) / 8 * tiles + 31) / 32;
+            if ((units + per - 1) / per != s || partials > part_rows || (rounds > 1 && !forced)) continue;  // (no empty slice)
+            const double us = rounds * (2.9 + (per + 3) / 4 * (rb == 1 ? 2.5 : 3.3)) + 2.6 + (s > 1 ? 1.8 + 0.75e-3 * partials : 0.0);
+            if (us < least) {
+                least = us;
+                best = {rb, s};
+            }
+        }
+    }
+    return best;
+}
+
 }  // namespace vla_rules
