@@ -189,6 +189,9 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
 // index in it, vectors lane, lane + 64 WAVES, ...; `red` = 16 floats of LDS for the three
 // reductions; every thread of the workgroup calls).  The squares are then added in another
 // order than by one wavefront, so the two forms agree to rounding, not bit for bit.
+// (Loads, weights and rounding under a branch per vector and word: a launch of the decode projections, 2560-wide rows, 0.65 us longer.)
+// Two loads per vector and no other branch than the stores': addresses past the row are clamped and the values replaced by zeros
+// (which change neither sums nor maxima), a missing or unaligned weight is read or made up once, in front of the arithmetic.
 template <int NV, bool GLU = false, int WAVES = 1>
 __device__ __forceinline__ void rms_act_quant_row(const bf16_t* __restrict__ xr, const bf16_t* __restrict__ w, int K,
                                                   float eps, int lane, int8_t* qrow, float& scale_out, int& sum_out,
@@ -197,41 +200,46 @@ __device__ __forceinline__ void rms_act_quant_row(const bf16_t* __restrict__ xr,
     const int nvec = K / 8;
     // Every value kept between the passes is a bf16 (the input, then the rounded normalised
     // row), so the row stays packed: 4 registers per 16-byte vector.
-    u32x4_t xp[NV];
-    u32x4_t wraw[NV];  // the weight's vectors, requested with the row's so that one round trip covers both
-    const bool w_vec = w && !((uintptr_t)w & 15);
+    u32x4_t xp[NV], up[GLU ? NV : 1];
+    u32x4_t wv[NV];  // the weight's vectors, requested with the row's so that one round trip covers both
     auto lo = [](uint32_t u) { return __uint_as_float(u << 16); };
     auto hi = [](uint32_t u) { return __uint_as_float(u & 0xffff0000u); };
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const long k0 = (long)min(lane + LS * i, nvec - 1) * 8;
+        xp[i] = *reinterpret_cast<const u32x4_t*>(xr + k0);
+        if (GLU) up[i] = *reinterpret_cast<const u32x4_t*>(xr + K + k0);
+    }
+    if (w && !((uintptr_t)w & 15)) {  // uniform
+#pragma unroll
+        for (int i = 0; i < NV; ++i) wv[i] = *reinterpret_cast<const u32x4_t*>(w + (long)min(lane + LS * i, nvec - 1) * 8);
+    } else {
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const bf16_t* we = w ? w + (long)min(lane + LS * i, nvec - 1) * 8 + 2 * e : nullptr;
+                wv[i][e] = we ? (uint32_t)we[0] | ((uint32_t)we[1] << 16) : 0x3f803f80u;  // none: ones
+            }
+    }
     float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-        const int vec = lane + LS * i;
-        u32x4_t raw = {0u, 0u, 0u, 0u}, upr = {0u, 0u, 0u, 0u};
-        wraw[i] = raw;
-        if (vec < nvec) {
-            raw = *reinterpret_cast<const u32x4_t*>(xr + (long)vec * 8);
-            if (GLU) upr = *reinterpret_cast<const u32x4_t*>(xr + K + (long)vec * 8);
-            if (w_vec) wraw[i] = *reinterpret_cast<const u32x4_t*>(w + (long)vec * 8);
-        }
-        if (GLU) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                float g0 = lo(raw[e]), g1 = hi(raw[e]);
-                if (g0 < 0.f) g0 = 0.f;
-                if (g1 < 0.f) g1 = 0.f;
-                raw[e] = pack_bf2(g0 * g0 * lo(upr[e]), g1 * g1 * hi(upr[e]));
-            }
-        }
-        xp[i] = raw;
-    }
-#pragma unroll
-    for (int i = 0; i < NV; ++i)
+        const bool in = lane + LS * i < nvec;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
+            if (GLU) {
+                float g0 = lo(xp[i][e]), g1 = hi(xp[i][e]);
+                if (g0 < 0.f) g0 = 0.f;
+                if (g1 < 0.f) g1 = 0.f;
+                xp[i][e] = pack_bf2(g0 * g0 * lo(up[i][e]), g1 * g1 * hi(up[i][e]));
+            }
+            xp[i][e] = in ? xp[i][e] : 0u;
             const float a = lo(xp[i][e]), b = hi(xp[i][e]);
             ss += a * a;
             ss += b * b;
         }
+    }
     const float inv = 1.0f / sqrtf((WAVES > 1 ? block_sum(ss, red) : wave_sum(ss)) / (float)K + eps);
     // the packed words are opaque from here on, or the compiler keeps the first pass's unpacked
     // floats alive across the reduction (8 registers per vector instead of 4)
@@ -242,20 +250,11 @@ __device__ __forceinline__ void rms_act_quant_row(const bf16_t* __restrict__ xr,
     float amax = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-        const int vec = lane + LS * i;
-        if (vec >= nvec) continue;
-        const int k0 = vec * 8;
+        const bool in = lane + LS * i < nvec;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            float o0 = lo(xp[i][e]) * inv, o1 = hi(xp[i][e]) * inv;
-            if (w_vec) {
-                o0 *= lo(wraw[i][e]);
-                o1 *= hi(wraw[i][e]);
-            } else if (w) {
-                o0 *= bf2f(w[k0 + 2 * e]);
-                o1 *= bf2f(w[k0 + 2 * e + 1]);
-            }
-            const uint32_t pr = pack_bf2(o0, o1);  // the activation as the bf16 it would be stored as
+            const float o0 = lo(xp[i][e]) * inv * lo(wv[i][e]), o1 = hi(xp[i][e]) * inv * hi(wv[i][e]);
+            const uint32_t pr = in ? pack_bf2(o0, o1) : 0u;  // the activation as the bf16 it would be stored as (0 x inv may be NaN past the row)
             xp[i][e] = pr;
             amax = fmaxf(amax, fmaxf(fabsf(lo(pr)), fabsf(hi(pr))));
         }
@@ -270,19 +269,22 @@ __device__ __forceinline__ void rms_act_quant_row(const bf16_t* __restrict__ xr,
     int sum = 0;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-        const int vec = lane + LS * i;
-        if (vec >= nvec) continue;
-        uint32_t pk[2] = {0u, 0u};
+        // Clamped, then rounded to the nearest even integer by adding 1.5 x 2^23, whose ulp is 1: the low byte of the sum's bits is
+        // the integer's (rounding first gives the same, the bounds being integers; NaN becomes -128 as before).
+        uint32_t t[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const uint32_t u = xp[i][e >> 1];
-            float qf = rintf(((e & 1) ? hi(u) : lo(u)) * scale);
-            qf = fminf(fmaxf(qf, -128.0f), 127.0f);
-            pk[e >> 2] |= (uint32_t)((int)qf & 0xff) << (8 * (e & 3));
+            const float qf = fminf(fmaxf(((e & 1) ? hi(u) : lo(u)) * scale, -128.0f), 127.0f);
+            t[e] = __float_as_uint(qf + 12582912.0f);
         }
+        uint32_t pk[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)  // bytes 0 of four words
+            pk[h] = __builtin_amdgcn_perm(t[4 * h + 1], t[4 * h], 0x0c0c0400u) | (__builtin_amdgcn_perm(t[4 * h + 3], t[4 * h + 2], 0x0c0c0400u) << 16);
         sum = __builtin_amdgcn_sdot4((int)pk[0], 0x01010101, sum, false);  // + the four signed bytes
         sum = __builtin_amdgcn_sdot4((int)pk[1], 0x01010101, sum, false);
-        *reinterpret_cast<u32x2_t*>(qrow + (long)vec * 8) = u32x2_t{pk[0], pk[1]};
+        if (lane + LS * i < nvec) *reinterpret_cast<u32x2_t*>(qrow + (long)(lane + LS * i) * 8) = u32x2_t{pk[0], pk[1]};
     }
     scale_out = scale;
     sum = wave_sum_i(sum);

@@ -406,6 +406,7 @@ bool launch_row_norm(const void* x, const void* w, const float* sc, const float*
     row_norm_kernel<T, NV, MODE, GLU><<<blocks, 256, 0, st>>>((const T*)x, (const T*)w, sc, sh, (T*)y, q, scales, rowsum, M, K, eps)
     if (nvec <= 64 * 2) VLA_ROW_NORM(2);
     else if (nvec <= 64 * 4) VLA_ROW_NORM(4);
+    else if (MODE == NORM_RMS_AQ && sizeof(T) == 2 && nvec <= 64 * 5) VLA_ROW_NORM(5);  // the 2560-wide model
     else if (nvec <= 64 * 8) VLA_ROW_NORM(8);
     else if constexpr (MODE == NORM_RMS_AQ && sizeof(T) == 2) {  // the 6912-wide BitNet FFN rows
         if (nvec > 64 * 16) return false;
