@@ -20,6 +20,7 @@ extern "C" int rows_kernel(int grid, int blocks, int sliced) { return vla_rules:
 extern "C" int tiles_kernel(int grid, int tiles) { return vla_rules::attn_tiles(grid, tiles); }
 extern "C" int f32_tile(int M, int n_tiles) { return vla_rules::f32_tile(M, n_tiles); }
 extern "C" int wide(int M, int N, int K, int kind) { return vla_rules::wide_tile(M, N, K, kind); }
+extern "C" int plain(int M, int N, int K) { return vla_rules::plain_tile(M, N, K); }
 extern "C" int ternary(int M, int N, int K) { return vla_rules::ternary_tile(M, N, K); }
 extern "C" int heads256(int pairs, int rows, int units, int part_rows, int forced) {
     const vla_rules::WideHeads h = vla_rules::wide_heads(pairs, rows, units, part_rows, forced);
@@ -189,3 +190,33 @@ def test_256_wide_heads_keep_to_their_scratch_and_to_one_round(rules):
     assert taken > 10000
     assert rules.heads256(1, 400, 15, 2560, 0) == 104 and rules.heads256(8, 400, 15, 10240, 0) == 101 and rules.heads256(16, 400, 15, 32768, 0) == 201
     assert rules.heads256(20, 400, 15, 100000, 0) < 100
+
+
+# M, N, K -> measured us of what wide_tile takes and on the plain tiles 96 x 96, 128 x 96, 96 x 64
+PLAIN_US = [
+    ((1323, 1536, 6144), 55.2, (46.1, 42.6, 51.1)),
+    ((1323, 1536, 1536), 15.1, (12.9, 15.5, 14.6)),
+    ((1600, 720, 960), 9.2, (9.6, 11.5, 8.0)),
+    ((1600, 720, 2048), 13.8, (14.3, 16.7, 12.0)),
+    ((2000, 1536, 6144), 59.6, (60.3, 48.4, 73.2)),
+    ((408, 1536, 6144), 24.4, (42.5, 39.5, 29.4)),
+    ((816, 1024, 4096), 15.6, (23.5, 26.7, 18.5)),
+    ((1323, 6144, 1536), 29.7, (42.8, 50.5, 43.8)),
+]
+
+
+@pytest.mark.parametrize("shape,wide,plain", PLAIN_US)
+def test_plain_tiles_are_taken_where_they_are_faster(rules, shape, wide, plain):
+    t = rules.plain(*shape)
+    took = wide if t < 6 else plain[t - 6]
+    assert took <= 1.05 * min(plain + (wide,))
+
+
+def test_a_plain_tile_is_named_for_every_size(rules):
+    for M in (1, 33, 512, 513, 1323, 4000, 18944, 1 << 20):
+        for N in (8, 64, 720, 1536, 8192, 151936):
+            for K in (16, 960, 6144, 1 << 20):
+                t = rules.plain(M, N, K)
+                assert -1 <= t < 9
+                if t < 6:
+                    assert t == rules.wide(M, N, K, 0)

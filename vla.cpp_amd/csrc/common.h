@@ -31,7 +31,7 @@ struct Tuning {
     bool attn_no_small = false;  // VLA_ATTN_NO_SMALL: fp32 launches with few row tiles do not split their keys beyond the usual rule
     int attn_rows = -1;          // VLA_ATTN_ROWS: 0 never, 1 always (as far as they serve the shape) the kernels of a wavefront per key block for 48- and 64-wide heads; unset = by shape
     int attn_direct_rows = 32;   // VLA_ATTN_DIRECT_ROWS: row limit of the register-direct kernel
-    int gemm_tile = -1;          // VLA_GEMM_TILE: 0..5, wide tiles 16..21
+    int gemm_tile = -1;          // VLA_GEMM_TILE: 0..5, wide tiles 16..24
     int gemm_panel = 0;          // VLA_GEMM_PANEL: N tiles per panel of an XCD's walk over its tiles; 0 = by size
     int gemm_dl = -1;            // VLA_GEMM_DL: 0 pins the register-staged GEMM
     int gemm_stages = 0;         // VLA_GEMM_STAGES: ring depth of the direct-to-LDS GEMM

@@ -1907,10 +1907,10 @@ int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
     }
     if constexpr (kEpi != EPI_TERNARY) {
         // VLA_GEMM_TILE = 0..5 pins the tile configuration and VLA_GEMM_STAGES the ring depth
-        // of the direct-to-LDS kernel, 16..21 a tile of the wide-tile kernel (tests and tuning); unset = by shape.
+        // of the direct-to-LDS kernel, 16..24 a tile of the wide-tile kernel (tests and tuning; 22..24 plain products only, 16 in their place elsewhere); unset = by shape.
         int cfg = tuning().gemm_tile;
         const bool pinned = cfg >= 0;
-        const int pinned_wide = cfg >= 16 && cfg < 16 + vla_rules::WIDE_TILES ? cfg - 16 : -1;
+        const int pinned_wide = cfg >= 16 && cfg < 16 + vla_rules::PLAIN_TILES ? (kEpi == EPI_PLAIN || cfg < 16 + vla_rules::WIDE_TILES ? cfg - 16 : 0) : -1;
         const long m128 = (a.M + 127) / 128, m64 = (a.M + 63) / 64;
         const long wgs0 = m128 * ((n_tiles + 1) / 2), wgs2 = m128 * n_tiles, wgs4 = m64 * n_tiles;
         if (!pinned) cfg = sizeof(T) == 4 ? vla_rules::f32_tile(a.M, n_tiles) : vla_rules::dl_tile(a.M, n_tiles);
@@ -1929,7 +1929,7 @@ int launch(GemmArgs a, int n_tiles, vla_stream_t stream) {
             // The wide tiles where they are predicted faster (32-bit lane offsets inside a tile; row sums handed from launch
             // to launch stay with the kernel below).
             if (dl && a.K <= (1 << 20) && !a.stats_in && !a.stats_out) {
-                const int wide = pinned ? pinned_wide : vla_rules::wide_tile(a.M, a.N, a.K, kEpi != EPI_QKV ? 0 : a.colsum ? 2 : 1);
+                const int wide = pinned ? pinned_wide : kEpi == EPI_PLAIN ? vla_rules::plain_tile(a.M, a.N, a.K) : vla_rules::wide_tile(a.M, a.N, a.K, kEpi != EPI_QKV ? 0 : a.colsum ? 2 : 1);
                 if (wide >= 0 && launch_wide<kEpi>(a, wide, st)) return hipGetLastError() == hipSuccess ? VLA_K_OK : VLA_K_ERR_LAUNCH;
             }
         }

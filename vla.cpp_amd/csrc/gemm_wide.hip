@@ -16,7 +16,104 @@ __device__ __forceinline__ void wait_tiles(int tiles) {
     }
 }
 
-// Workgroup tile (16 RM WM) x (64 WN); wavefront (wm, wn) of WM x WN owns RM x 4 blocks of 16 x 16 over all of K:
+// NV (4 or 8) consecutive columns from n0 on of row m, plain epilogue: bias (fetched by the caller), activation, gate, residual (have_res: the
+// first NV / 2 words of res), store.
+template <int NV>
+__device__ __forceinline__ void plain_cols(const GemmArgs& a, int m, int n0, float (&v)[NV], const float (&bias)[NV], bool have_res, u32x4_t res) {
+    if (n0 >= a.N) return;
+    const long o = (long)m * a.N + n0;
+    if (a.bias) {
+#pragma unroll
+        for (int e = 0; e < NV; ++e) v[e] += bias[e];
+    }
+    if (a.act != VLA_ACT_NONE) epilogue_act(v, a.act, a.out_bf16);
+    if (a.col_gate) {
+#pragma unroll
+        for (int e = 0; e < NV; ++e) v[e] *= a.col_gate[min(n0 + e, a.N - 1)];
+    }
+    if (a.N % 8 == 0 && a.out_bf16) {
+        if (a.residual) {
+            if (!have_res) {
+                const bf16_t* r = (const bf16_t*)a.residual + o;
+                if constexpr (NV == 8) {
+                    res = *reinterpret_cast<const u32x4_t*>(r);
+                } else {
+                    const u32x2_t h = *reinterpret_cast<const u32x2_t*>(r);
+                    res[0] = h[0];
+                    res[1] = h[1];
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < NV / 2; ++e) {
+                v[2 * e] += __uint_as_float(res[e] << 16);
+                v[2 * e + 1] += __uint_as_float(res[e] & 0xffff0000u);
+            }
+        }
+        bf16_t* y = (bf16_t*)a.Y + o;
+        if constexpr (NV == 8) *reinterpret_cast<u32x4_t*>(y) = u32x4_t{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]), pack_bf2(v[4], v[5]), pack_bf2(v[6], v[7])};
+        else *reinterpret_cast<u32x2_t*>(y) = u32x2_t{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+    } else if (a.N % 8 == 0) {
+#pragma unroll
+        for (int h = 0; h < NV / 4; ++h) {
+            f32x4_t x = {v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]};
+            if (a.residual) x += *reinterpret_cast<const f32x4_t*>((const float*)a.residual + o + 4 * h);
+            *reinterpret_cast<f32x4_t*>((float*)a.Y + o + 4 * h) = x;
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < NV; ++e) {
+            if (n0 + e >= a.N) continue;
+            if (a.out_bf16) {
+                const float r = a.residual ? bf2f(((const bf16_t*)a.residual)[o + e]) : 0.f;
+                ((bf16_t*)a.Y)[o + e] = f2bf(a.residual ? v[e] + r : v[e]);
+            } else {
+                const float r = a.residual ? ((const float*)a.residual)[o + e] : 0.f;
+                ((float*)a.Y)[o + e] = a.residual ? v[e] + r : v[e];
+            }
+        }
+    }
+}
+
+// The epilogue of a wavefront of RM x RN blocks, RN < 4: rows m + 16 i, columns n0 + 8 q .. + 7 and, RN = 3, n0 + 32 + 4 q .. + 3.  Bias and a bf16
+// residual (which may be the output buffer: a lane stores no other lane's elements) are requested ahead of the first store.
+template <int RM, int RN>
+__device__ __forceinline__ void plain_rows(const GemmArgs& a, const f32x4_t (&acc)[RM][RN], int m, int n0, int q) {
+    const int n8 = n0 + 8 * q, n4 = n0 + 32 + 4 * q;
+    float b8[8] = {}, b4[4] = {};
+    if (a.bias) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) b8[e] = a.bias[min(n8 + e, a.N - 1)];
+        if (RN == 3) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) b4[e] = a.bias[min(n4 + e, a.N - 1)];
+        }
+    }
+    const bool have_res = a.residual != nullptr && a.out_bf16 && a.N % 8 == 0;
+    u32x4_t res[RM] = {};
+    u32x2_t res4[RM] = {};
+    if (have_res) {
+#pragma unroll
+        for (int i = 0; i < RM; ++i) {
+            const bf16_t* r = (const bf16_t*)a.residual + (long)min(m + 16 * i, a.M - 1) * a.N;
+            res[i] = *reinterpret_cast<const u32x4_t*>(r + min(n8, a.N - 8));
+            if (RN == 3) res4[i] = *reinterpret_cast<const u32x2_t*>(r + min(n4, a.N - 4));
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < RM; ++i) {
+        if (m + 16 * i >= a.M) continue;
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = acc[i][e >> 2][e & 3];
+        plain_cols(a, m + 16 * i, n8, v, b8, have_res, res[i]);
+        if constexpr (RN == 3) {
+            float u[4] = {acc[i][2][0], acc[i][2][1], acc[i][2][2], acc[i][2][3]};
+            plain_cols(a, m + 16 * i, n4, u, b4, have_res, u32x4_t{res4[i][0], res4[i][1], 0u, 0u});
+        }
+    }
+}
+
+// Workgroup tile (16 RM WM) x (16 RN WN); wavefront (wm, wn) of WM x WN owns RM x RN blocks (RN = 4 if not said otherwise) of 16 x 16 over all of K:
 // v_mfma_f32_16x16x32_bf16, ascending k, whose sums have the bits of the 32x32x16 kernels.  W is the left operand, so
 // that a lane (c, q) = (lane % 16, lane / 16) ends with four columns of row c per block; the loader places the rows of W
 // so that a wavefront's four blocks are columns 8 q .. 8 q + 7 of both 32-column halves of a 64-column sub-tile (the
@@ -37,19 +134,26 @@ __device__ __forceinline__ void wait_tiles(int tiles) {
 // Against the direct-to-LDS kernel (128 x 128 tiles of four wavefronts, 32x32x16; us, weights not in the caches): 1323 x 6144 x 1536
 // 46.3 -> 28.3 (0.88 PFLOP/s; loads alone 22 to 26, MFMA and LDS alone 23), 816 x 8192 x 1024 gated 21.4 -> 19.6, 1323 x 4608 x 1536 with the
 // LayerNorm inside 34.8 -> 30.5, 13824 x 3072 x 2048 186 -> 144, 4096 x 4096 x 4096 147 -> 102 (1.35 PFLOP/s).
-template <int kEpi, int kNorm, int RM, int WM, int WN, int NS>
+//
+// RN = 2, 3 (plain epilogue): 32- and 48-column wavefronts of tiles that cover a narrow product in one round.  Such a launch is bound by what its
+// CUs draw from the L2s (12 to 14 TB/s in all when the weights come from memory, 21 to 25 when every line hits, loads alone; requesting the
+// lines ahead of the ring changes nothing), so that of the tiles that fit a round the one with the fewest operand rows per output is the
+// fastest: 1323 x 1536 x 6144 264 tiles of 128 x 64 55.2 us, 176 of 128 x 96 42.6; 1323 x 1536 x 1536 15.1 -> 12.9 (96 x 96, two a CU); 1600 x 720 x 2048
+// 13.8 -> 12.0 (96 x 64, two a CU).
+template <int kEpi, int kNorm, int RM, int RN, int WM, int WN, int NS>
 __global__ void __launch_bounds__(64 * WM * WN) gemm_wide_kernel(GemmArgs a) {
-    constexpr int RN = 4, BM = 16 * RM * WM, BW = 64 * WN, NW = WM * WN, KB = 128, BK = 64;
+    constexpr int CW = 16 * RN, BM = 16 * RM * WM, BW = CW * WN, NW = WM * WN, KB = 128, BK = 64;
     constexpr int STAGE = (BM + BW) * KB, VA = BM / 8 / NW, VW = BW / 8 / NW, NL = VA + VW;
     constexpr int SB = (RM + WN - 1) / WN;  // row blocks whose norm a wavefront sums up
     static_assert(BM % (8 * NW) == 0 && BW % (8 * NW) == 0, "a load instruction of a wavefront fills eight rows of one operand");
+    static_assert(RN == 4 || (RN >= 2 && RN < 4 && kEpi == EPI_PLAIN && kNorm == NORM_NONE), "narrower wavefront tiles know the plain epilogue only");
     static_assert(NS >= 2 && NS * STAGE <= 160 * 1024, "ring exceeds the LDS");
     static_assert((NS - 1) * NL <= 63, "ring depth exceeds the vector-memory counter");
     __shared__ __attribute__((aligned(1024))) unsigned char lds[NS * STAGE];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WN, wn = wave % WN, c = lane & 15, q = lane >> 4;
-    const int n_wg_tiles = (a.n_tiles + WN - 1) / WN, m_wg_tiles = (a.M + BM - 1) / BM;
+    const int n_wg_tiles = RN == 4 ? (a.n_tiles + WN - 1) / WN : (a.N + BW - 1) / BW, m_wg_tiles = (a.M + BM - 1) / BM;
     int mtw, ntw;
     if (!xcd_tile(a, n_wg_tiles, m_wg_tiles, mtw, ntw)) return;
     const int m0 = mtw * BM;
@@ -66,6 +170,12 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_wide_kernel(GemmArgs a) {
         if (l < VA) {
             base[l] = (const unsigned char*)a.A + (long)m0 * a.K * 2;
             off[l] = (uint32_t)(min((l * NW + wave) * 8 + lrow, a.M - 1 - m0) * a.K * 2 + koff);
+        } else if constexpr (RN < 4) {
+            // a wavefront's blocks 0 and 1 are its columns 8 q .. 8 q + 7, block 2 is 32 + 4 q .. 32 + 4 q + 3
+            const int s = ((l - VA) * NW + wave) * 8 + lrow, j = (s % CW) >> 4, cc = s & 15, b = ntw * BW;
+            const int col = s / CW * CW + (j == 2 ? 32 + cc : 8 * (cc >> 2) + 4 * j + (cc & 3));
+            base[l] = (const unsigned char*)a.W + (long)b * a.K * 2;
+            off[l] = (uint32_t)(min(col, a.N - 1 - b) * a.K * 2 + koff);
         } else {
             const int slab = (l - VA) * NW + wave, s = (slab & 7) * 8 + lrow, cc = s & 15;
             const TileCols t = tile_cols<kEpi>(a, ntw * WN + (slab >> 3));
@@ -98,7 +208,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_wide_kernel(GemmArgs a) {
     // the WN wavefronts that read the same rows take every WN-th row block each.
     float ssq[SB][4] = {}, ssum[SB][4] = {};
 
-    const int fa = (wm * RM * 16 + c) * KB, fw = (BM + wn * 64 + c) * KB, fsw = (c >> 1) & 7;
+    const int fa = (wm * RM * 16 + c) * KB, fw = (BM + wn * CW + c) * KB, fsw = (c >> 1) & 7;
     typedef u32x4_t FragA[RM];
     typedef u32x4_t FragW[RN];
     FragA a0, a1;
@@ -187,6 +297,10 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_wide_kernel(GemmArgs a) {
         st = sn;
     }
 
+    if constexpr (RN < 4) {
+        plain_rows<RM, RN>(a, acc, m0 + wm * RM * 16 + c, ntw * BW + wn * CW, q);
+        return;
+    } else {
     // Epilogue: this lane's rows m0 + 16 (wm RM + i) + c, columns 8 q .. + 7 of both halves of sub-tile nt.
     const int nt = ntw * WN + wn, jg = q * 8;
     float* row_f = reinterpret_cast<float*>(lds);  // (rstd, mean rstd) of the tile's rows
@@ -302,27 +416,28 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_wide_kernel(GemmArgs a) {
             }
         }
     }
+    }
 }
 
-template <int kEpi, int RM, int WM, int WN, int NS>
+template <int kEpi, int RM, int WM, int WN, int NS, int RN = 4>
 bool launch_tile(GemmArgs a, hipStream_t st) {
-    const unsigned grid = xcd_split(a, (a.M + 16 * RM * WM - 1) / (16 * RM * WM), (a.n_tiles + WN - 1) / WN, 2.0, 64 * WN, 2.0);
+    const unsigned grid = xcd_split(a, (a.M + 16 * RM * WM - 1) / (16 * RM * WM), RN == 4 ? (a.n_tiles + WN - 1) / WN : (a.N + 16 * RN * WN - 1) / (16 * RN * WN), 2.0, 16 * RN * WN, 2.0);
     if (!grid) return false;  // more workgroups than the tile walk can count
     constexpr int T = 64 * WM * WN;
     if (kEpi == EPI_QKV) a.div_s = make_divc(a.S, a.M);
     if constexpr (kEpi == EPI_QKV) {
         if (a.norm_eps >= 0.f && a.colsum) {
-            gemm_wide_kernel<kEpi, NORM_LAYER, RM, WM, WN, NS><<<grid, T, 0, st>>>(a);
+            gemm_wide_kernel<kEpi, NORM_LAYER, RM, RN, WM, WN, NS><<<grid, T, 0, st>>>(a);
             return true;
         }
     }
     if constexpr (kEpi == EPI_QKV || kEpi == EPI_GLU) {
         if (a.norm_eps >= 0.f) {
-            gemm_wide_kernel<kEpi, NORM_RMS, RM, WM, WN, NS><<<grid, T, 0, st>>>(a);
+            gemm_wide_kernel<kEpi, NORM_RMS, RM, RN, WM, WN, NS><<<grid, T, 0, st>>>(a);
             return true;
         }
     }
-    gemm_wide_kernel<kEpi, NORM_NONE, RM, WM, WN, NS><<<grid, T, 0, st>>>(a);
+    gemm_wide_kernel<kEpi, NORM_NONE, RM, RN, WM, WN, NS><<<grid, T, 0, st>>>(a);
     return true;
 }
 
@@ -332,6 +447,14 @@ namespace vk {
 
 template <int kEpi>
 bool launch_wide(const GemmArgs& a, int tile, hipStream_t st) {
+    if constexpr (kEpi == EPI_PLAIN) {
+        switch (tile) {
+            case vla_rules::PLAIN_96X96_PAIRS: return launch_tile<kEpi, 3, 2, 2, 3, 3>(a, st);
+            case vla_rules::PLAIN_128X96: return launch_tile<kEpi, 4, 2, 2, 5, 3>(a, st);
+            case vla_rules::PLAIN_96X64_PAIRS: return launch_tile<kEpi, 3, 2, 2, 4, 2>(a, st);
+            default: break;
+        }
+    }
     switch (tile) {
         case vla_rules::WIDE_256X256: return launch_tile<kEpi, 8, 2, 4, 2>(a, st);
         case vla_rules::WIDE_192X192: return launch_tile<kEpi, 3, 4, 3, 3>(a, st);

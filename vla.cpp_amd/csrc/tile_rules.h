@@ -2,6 +2,8 @@
 // checked over its whole range on any host.
 #pragma once
 
+#include <cmath>
+
 namespace vla_rules {
 
 // Row blocks (16 rows) and column tiles (16 columns) per workgroup of the narrow-tile projection kernel.
@@ -142,8 +144,9 @@ struct TileTime {
     }
 };
 
-// Tile of the wide-tile kernel: rows x columns, and whether two workgroups share a CU.
-enum { WIDE_256X256 = 0, WIDE_192X192, WIDE_256X128, WIDE_192X128, WIDE_128X128, WIDE_128X128_PAIRS, WIDE_TILES };
+// Tile of the wide-tile kernel: rows x columns, and whether two workgroups share a CU.  PLAIN_*: plain epilogue only.
+enum { WIDE_256X256 = 0, WIDE_192X192, WIDE_256X128, WIDE_192X128, WIDE_128X128, WIDE_128X128_PAIRS, WIDE_TILES,
+       PLAIN_96X96_PAIRS = WIDE_TILES, PLAIN_128X96, PLAIN_96X64_PAIRS, PLAIN_TILES };
 
 // The wide tile with the least predicted time, or -1 where the direct-to-LDS kernel's tile is not predicted 6 % slower.  kind:
 // 0 plain or gated, 1 QKV, 2 QKV with a LayerNorm inside.  On the fitted shapes the wide tile is taken on 60 %, where it needs
@@ -151,7 +154,7 @@ enum { WIDE_256X256 = 0, WIDE_192X192, WIDE_256X128, WIDE_192X128, WIDE_128X128,
 // slower, one 15 % (576 x 2752 x 5552 gated, 71.6 -> 82.0 us).  1323 x 6144 x 1536 46.3 -> 28.3 us (192 x 192: 224 workgroups, one
 // round, where 528 of 128 x 128 left 16 for a second one), 816 x 8192 x 1024 gated 21.4 -> 19.6, 13824 x 3072 x 2048 186 -> 144
 // (256 x 256), 4096 x 4096 x 4096 147 -> 102 (weights not in the caches).
-inline int wide_tile(int M, int N, int K, int kind) {
+inline int wide_tile(int M, int N, int K, int kind, double* predicted = nullptr) {
     static const TileTime wide[WIDE_TILES] = {
         {256, 256, false, 0.18, 11.50, 1.234, 0.314, 0, 0, 1.57, 3.50}, {192, 192, false, 1.05, 7.02, 0.703, 0.225, 0, 0, 2.04, 3.15},
         {256, 128, false, 1.05, 6.86, 0.676, 0.188, 0, 0, 1.31, 2.89},  {192, 128, false, 1.38, 5.32, 0.565, 0.152, 0, 0, 1.51, 2.93},
@@ -161,7 +164,8 @@ inline int wide_tile(int M, int N, int K, int kind) {
         {128, 64, true, 3.53, 1.36, 0.335, 0.063, 2.32, 0.662, 0.13, 0.81},   {128, 64, true, 3.53, 1.36, 0.335, 0.063, 2.32, 0.662, 0.13, 0.81},
         {64, 64, true, 4.86, 1.00, 0.300, 0.300, 0.00, 0.378, -0.42, 0.31},   {128, 192, false, 6.38, 2.96, 0.637, 0.119, 0, 0, 0.21, 0.71}};
     const int cfg = dl_tile(M, (N + 63) / 64);
-    double least = 0.94 * dl[cfg].us(M, N, K, kind);
+    const double dl_us = dl[cfg].us(M, N, K, kind);
+    double least = 0.94 * dl_us;
     int best = -1;
     for (int t = 0; t < WIDE_TILES; ++t) {
         // one 128 x 128 tile per CU, where 128 x 64 tiles cover the chip: up to 18 % slower than those
@@ -170,6 +174,34 @@ inline int wide_tile(int M, int N, int K, int kind) {
         if (us < least) {
             least = us;
             best = t;
+        }
+    }
+    if (predicted) *predicted = best < 0 ? dl_us : least;
+    return best;
+}
+
+// The same for a plain product, whose epilogue also comes with 32- and 48-column wavefronts: one of those tiles where it is predicted 6 %
+// faster than what wide_tile takes.  Their step per 64 k is the root of the squares of what a CU needs for itself and what its share of the
+// L2s' rate allows (load, times the share of the CUs that are busy): 1323 x 1536 x 6144 takes 46.1 us on 224 tiles of 96 x 96, 42.6 on 176 of
+// 128 x 96.  On 948 shapes (200 to 4000 rows, N 256 to 8192, K 128 to 8192, weights from memory) taken on 253, where it needs 0.88 of the time
+// (geometric mean); six of them are 1 to 6 % slower.  Long rows that do not start on a cache line are left out: predicted as well on the mean,
+// but 672 x 1536 x 4432 and 1042 x 1152 x 5008 take 1.22 times as long.  1323 x 1536 x 6144 55.2 -> 42.6 us, 2000 x 1536 x 6144 59.1 -> 48.4, 1600 x 720 x 2048
+// 13.8 -> 12.0; 408 x 1536 x 6144 stays: 24.4, here 29.4.
+inline int plain_tile(int M, int N, int K) {
+    static const struct { int rows, cols; bool pairs; double fixed, round, step, load, round2, step2; } t[PLAIN_TILES - WIDE_TILES] = {
+        {96, 96, true, 1.08, 3.64, 0.357, 0.329, 4.44, 0.708}, {128, 96, false, 1.33, 4.80, 0.410, 0.285, 0, 0}, {96, 64, true, 1.94, 1.93, 0.287, 0.200, 2.31, 0.609}};
+    double least;
+    int best = wide_tile(M, N, K, 0, &least);
+    if (K % 64 != 0 && K > 1024) return best;
+    least *= 0.94;
+    for (int i = 0; i < PLAIN_TILES - WIDE_TILES; ++i) {
+        const XcdGrid g = xcd_grid(M, N, K, (M + t[i].rows - 1) / t[i].rows, (N + t[i].cols - 1) / t[i].cols, 2.0, t[i].cols, 2.0, 0);
+        const long n = (g.wgs + 31) / 32, n2 = t[i].pairs ? n / 2 : 0, n1 = n - 2 * n2;
+        const double load = t[i].load * (g.wgs < 32 ? g.wgs / 32.0 : 1.0), kt = (K + 63) / 64;
+        const double us = t[i].fixed + n2 * (t[i].round2 + kt * t[i].step2) + n1 * (t[i].round + kt * std::sqrt(t[i].step * t[i].step + load * load));
+        if (us < least) {
+            least = us;
+            best = WIDE_TILES + i;
         }
     }
     return best;
