@@ -62,7 +62,7 @@ struct AttnArgs {
     int mask_kind, n_prefix, pad_start, pad_end;
     const float* mask;
     int n_groups, n_split, tiles_per_split, r_pad, p2;
-    int n_rblocks;  // direct kernel: 32-row blocks per (batch, kv head)
+    int n_rblocks;  // direct kernel: 32-row blocks per (batch, kv head); LDS kernel, 128-wide heads: workgroups of an XCD
     int n_slices;   // LDS kernel, direct-to-LDS variant: key slices (wavefronts) per row tile
     float* part_o;   // [pair][split][r_pad][D] fp32 unnormalised, or fp16 normalised (part_half); merged in the launch: [pair][r_pad][split][D]
     float* part_ml;  // [pair][split][r_pad][2]; merged in the launch: [pair][r_pad][split][2]
@@ -214,7 +214,7 @@ template <> struct AT<float> {
 constexpr int WIDE_FB = 4;  // LDS fragments read ahead of their MFMAs, 256-wide heads (8 spills registers)
 
 template <typename T, int D, int NW, bool P2, int NL, int NSL = 0, int RS = 1>
-__global__ void __launch_bounds__((NW * (NSL > 0 ? NSL : 1) + NL) * 64, (D * sizeof(T) <= 128) ? 2 : 1) attn_kernel(AttnArgs a) {
+__global__ void __launch_bounds__((NW * (NSL > 0 ? NSL : 1) + NL) * 64, (D * sizeof(T) <= 128 || NSL > 0) ? 2 : 1) attn_kernel(AttnArgs a) {
     typedef AT<T> A;
     constexpr int EB = A::EB, CE = A::CE;
     constexpr bool DLOAD = NSL > 0;
@@ -252,9 +252,12 @@ __global__ void __launch_bounds__((NW * (NSL > 0 ? NSL : 1) + NL) * 64, (D * siz
     // ---- XCD-aware decode of the linear workgroup id
     const int GS = a.n_groups * a.n_split;
     const int id = blockIdx.x;
-    const int pair = (int)div_c(id, a.d8GS) * 8 + (id & 7);
+    // Pairs are dealt out over the XCDs; of 128-wide heads (BitVLA's five kv heads an observation) an XCD has n_rblocks consecutive
+    // workgroups: ten pairs were two on each of two XCDs and one on the others, 515 rows, two observations 40.5 -> 23.4 us, twelve 102 -> 86.2.
+    const int flat = D == 128 ? (id & 7) * a.n_rblocks + (id >> 3) : 0;
+    const int pair = D == 128 ? (int)div_c(flat, a.dGS) : (int)div_c(id, a.d8GS) * 8 + (id & 7);
     if (pair >= a.batch * a.Hkv) return;
-    const int t_idx = (id >> 3) - (int)div_c(id >> 3, a.dGS) * GS;
+    const int t_idx = D == 128 ? flat - pair * GS : (id >> 3) - (int)div_c(id >> 3, a.dGS) * GS;
     const int group = (int)div_c(t_idx, a.dns), split = t_idx - group * a.n_split;
     const int b = (int)div_c(pair, a.dHkv), hk = pair - b * a.Hkv;
 
@@ -2676,8 +2679,19 @@ int launch_merge(AttnArgs& a, hipStream_t st) {
 template <typename T, int D, int NW>
 int launch_nw(AttnArgs& a, hipStream_t st) {
     const int n_pairs = a.batch * a.Hkv;
-    const int grid = (n_pairs + 7) / 8 * 8 * a.n_groups * a.n_split;
+    const int wgs = n_pairs * a.n_groups * a.n_split, grid = D == 128 ? (wgs + 7) / 8 * 8 : (n_pairs + 7) / 8 * 8 * a.n_groups * a.n_split;
+    if (D == 128) a.n_rblocks = grid / 8;
     set_divisors(a, grid);
+    if constexpr (sizeof(T) == 2 && D == 128 && NW >= 3) {
+        // More workgroups than CUs: tiles straight into LDS and few enough registers for two workgroups a CU (the same bits), so that one's
+        // products run beside the other's softmax.  515 rows of 20 heads on 5 kv heads, two-term probabilities: 3 observations (255
+        // workgroups) 24.8 us, here 28.4; 4, 8, 12 (340, 680, 1020) 42.9, 64.8, 86.2, here 37.6, 59.1, 72.3; 16 of 100 rows 18.5, here 14.8.
+        if (wgs > 256 && (((uintptr_t)a.k_cache | (uintptr_t)a.vt_cache) & 15) == 0) {
+            if (a.p2) attn_kernel<T, D, NW, true, 0, 1, 2><<<grid, NW * 64, 0, st>>>(a);
+            else attn_kernel<T, D, NW, false, 0, 1, 2><<<grid, NW * 64, 0, st>>>(a);
+            return hipGetLastError() == hipSuccess ? launch_merge<T, D>(a, st) : VLA_K_ERR_LAUNCH;
+        }
+    }
     if constexpr (sizeof(T) == 2 && D == 64) {
         // 64-wide bf16 heads: tiles go straight into a swizzled LDS ring (the tuning override
         // attn_dl = 0 pins the register-staged path), and with three or more key tiles they
