@@ -1524,7 +1524,7 @@ __global__ void __launch_bounds__(64) attn_decode16_kernel(AttnArgs a) {
 // (row >> 1) & 7: the loading lane picks the global piece that belongs in its slot.  The
 // arithmetic per block is the direct kernel's, in the same order: the two give the same bits.
 __device__ __forceinline__ void dma16(uint32_t voff, const void* sbase, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voff), "s"(sbase) : "memory");
+    load_to_lds16_at(sbase, voff, lds_base);
 }
 // A wavefront-uniform pointer the compiler may hold in vector registers, moved to scalar ones (the address operand above).
 __device__ __forceinline__ const unsigned char* uniform_ptr(const unsigned char* p) {

@@ -362,20 +362,22 @@ __device__ __forceinline__ unsigned div_c(unsigned x, DivC c) { return c.mg ? __
 // lane i's bytes land at lds_base + 16 i (lds_base wavefront-uniform, held in M0); the
 // per-lane global address is free.  Completion is tracked by vmcnt like any vector load.
 // Issued from inline assembly so that the wait counts stay under this file's control.
+// The ISA asks for one wait state between a scalar write of M0 and the LDS load that reads it; the compiler puts none inside
+// an asm statement, hence the s_nop in each of these.
 __device__ __forceinline__ void load_to_lds16(const void* gptr, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(gptr) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(gptr) : "memory");
 }
 // One 16-byte load per lane from uniform base + 32-bit lane offset straight into LDS (see load_to_lds16).
 __device__ __forceinline__ void load_to_lds16_at(const void* base, uint32_t off, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(off), "s"(base) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(off), "s"(base) : "memory");
 }
 // The same to lds_base + plus (a constant): no scalar register per destination.
 __device__ __forceinline__ void load_to_lds16_plus(const void* base, uint32_t off, uint32_t lds_base, int plus) {
-    asm volatile("s_add_u32 m0, %0, %3\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(off), "s"(base), "i"(plus) : "memory", "scc");
+    asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(off), "s"(base), "i"(plus) : "memory", "scc");
 }
 // The same if c (uniform), without a branch that the compiler sees.
 __device__ __forceinline__ void load_to_lds16_plus_if(bool c, const void* base, uint32_t off, uint32_t lds_base, int plus) {
-    asm volatile("s_cmp_eq_u32 %4, 0\n\ts_cbranch_scc1 skip%=\n\ts_add_u32 m0, %0, %3\n\tglobal_load_lds_dwordx4 %1, %2\nskip%=:" ::"s"(lds_base), "v"(off), "s"(base), "i"(plus), "s"(__builtin_amdgcn_readfirstlane(c ? 1 : 0)) : "memory", "scc");
+    asm volatile("s_cmp_eq_u32 %4, 0\n\ts_cbranch_scc1 skip%=\n\ts_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\nskip%=:" ::"s"(lds_base), "v"(off), "s"(base), "i"(plus), "s"(__builtin_amdgcn_readfirstlane(c ? 1 : 0)) : "memory", "scc");
 }
 
 }  // namespace vk

@@ -1132,7 +1132,7 @@ __device__ __forceinline__ void tern_wload_i(u32x2_t& dst, uint32_t voff, const 
     asm volatile("global_load_dwordx2 %0, %1, %2 offset:%3" : "+v"(dst) : "v"(voff), "s"(sbase), "n"(IMM) : "memory");
 }
 __device__ __forceinline__ void tern_aload_lds(uint32_t voff, const void* sbase, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(voff), "s"(sbase) : "memory");
+    load_to_lds16_at(sbase, voff, lds_base);
 }
 __device__ __forceinline__ void tern_gload(uint32_t& dst, const void* p) {
     asm volatile("global_load_dword %0, %1, off" : "=v"(dst) : "v"(p) : "memory");
