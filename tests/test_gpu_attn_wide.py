@@ -77,3 +77,22 @@ def test_attention_of_256_wide_heads(tune, B, S, Hq, Hkv, n_keys, t_max, forced,
         return
     assert error(new, want) <= 1.1 * error(tiled, want) + 1e-4
     assert error(new, want) < 2 ** -8
+
+
+@pytest.mark.parametrize("B,n_keys", [(1, 955), (5, 842), (8, 955), (16, 842)])  # four key slices, none, none, workgroups of 32 rows
+@pytest.mark.parametrize("size", [0.25, 4.0])  # rows of many alike and of few dominating probabilities
+def test_error_is_no_larger_than_the_tiled_kernels(tune, B, n_keys, size):
+    """Over 100,000 rounded outputs and more the ratio of the two errors is known to 2 / sqrt(100,000), about half a per cent."""
+    S, Hq = 50, 8
+    g = torch.Generator().manual_seed(B + n_keys)
+    rnd = lambda *shape: torch.randn(*shape, generator=g).to(torch.bfloat16).cuda()
+    k, vt, q = rnd(B, 1, 960, D), rnd(B, 1, D, 960), rnd(B, S, Hq, D) * size
+    want = reference(q, k, vt, n_keys, pkg.VLA_MASK_NONE, 0, (0, 0), None)
+    out = []
+    for rows in ("0", "-1"):
+        tune.set("VLA_ATTN_ROWS", rows)
+        out.append(torch.empty_like(q))
+        pkg.call("vla_attn_prefix_suffix", q, k, vt, out[-1], BF16, B, S, Hq, 1, D, 960, n_keys, D ** -0.5, pkg.VLA_MASK_NONE, 0, 0, 0, None)
+    tiled, new = out
+    assert not torch.equal(tiled, new)  # two kernels
+    assert error(new, want) <= 1.006 * error(tiled, want)

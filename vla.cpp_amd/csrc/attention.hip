@@ -2379,11 +2379,12 @@ __global__ void __launch_bounds__(W * 64, 1) attn_wide_kernel(AttnArgs a) {
     constexpr float LOG2E = 1.4426950408889634f;
     const float c2 = a.scale * LOG2E;
     f32x4_t o[RB][NDB];
-    float m_run[RB], l_run[RB];
+    float m_run[RB];
+    f32x4_t l_run[RB];  // the row sum, four times
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
         m_run[rb] = -INFINITY;
-        l_run[rb] = 0.f;
+        l_run[rb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int db = 0; db < NDB; ++db) o[rb][db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
@@ -2476,7 +2477,8 @@ __global__ void __launch_bounds__(W * 64, 1) attn_wide_kernel(AttnArgs a) {
             for (int rb = 0; rb < RB; ++rb) {
                 const float m_new = fmaxf(m_run[rb], m_tile[rb]);
                 const float alpha = __builtin_amdgcn_exp2f(m_run[rb] - (m_new == -INFINITY ? 0.f : m_new));
-                l_run[rb] *= alpha;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) l_run[rb][e] *= alpha;
                 m_run[rb] = m_new;
                 if (n) {  // uniform; before that the sums are zero
 #pragma unroll
@@ -2489,19 +2491,23 @@ __global__ void __launch_bounds__(W * 64, 1) attn_wide_kernel(AttnArgs a) {
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb) {
             const float m_use = m_run[rb] == -INFINITY ? 0.f : m_run[rb];
-            float psum[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 // (a mask value is added before the reference is taken off: beside a very low one the score has to vanish)
                 const float x = GIVEN && add[rb][i] != 0.f ? fmaf(p[rb][i], c2, add[rb][i]) - m_use : fmaf(p[rb][i], c2, -m_use);
                 p[rb][i] = __builtin_amdgcn_exp2f(x);
-                psum[i & 3] += p[rb][i];
             }
-            l_run[rb] += rows_sum((psum[0] + psum[1]) + (psum[2] + psum[3]));
+            // The row sum is one more product, with ones, of the probabilities as rounded to bf16: the rounding of a weight that dominates its row
+            // then cancels in o / l.  Summed up unrounded, 5 to 9 observations of 842 and 955 keys with scores of standard deviation 4 were up to
+            // 1.05 times as far from float64 as on the tiled kernel, whose key slices have a probability of 1 each; now 0.94 times (geometric mean
+            // over 192 shapes, at most 1.002), in the same time.
 #pragma unroll
-            for (int hh = 0; hh < 2; ++hh)
+            for (int hh = 0; hh < 2; ++hh) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) pf[rb][hh][e] = pack_bf2(p[rb][8 * hh + 2 * e], p[rb][8 * hh + 2 * e + 1]);
+                const u32x4_t ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};  // bf16
+                l_run[rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, ones), __builtin_bit_cast(bf16x8_t, pf[rb][hh]), l_run[rb], 0, 0, 0);
+            }
         }
         step(std::integral_constant<int, 4>{});
         step(std::integral_constant<int, 5>{});
@@ -2516,7 +2522,7 @@ __global__ void __launch_bounds__(W * 64, 1) attn_wide_kernel(AttnArgs a) {
     for (int rb = 0; rb < RB; ++rb) {
 #pragma unroll
         for (int db = 0; db < NDB; ++db) *reinterpret_cast<f32x4_t*>(ring + (rb * 16 + c) * 1024 + (((db * 4 + q) ^ c) * 16)) = o[rb][db];
-        if (q == 0) row_ml[wave][rb * 16 + c] = f32x2_t{m_run[rb], l_run[rb]};
+        if (q == 0) row_ml[wave][rb * 16 + c] = f32x2_t{m_run[rb], l_run[rb][0]};
     }
     __syncthreads();
 #pragma unroll
