@@ -2,6 +2,7 @@
 import concurrent.futures
 import glob
 import os
+import re
 import subprocess
 import sys
 
@@ -28,17 +29,23 @@ def sources():
 # not spill: a spilled in-flight register is stored before its data arrives and reused while
 # the load is still due.  Kernels that count their vector-memory waits by hand must not either: spills add operations
 # to the count, and the waits no longer leave in flight what they were meant to.  Their scratch size is read from the
-# compiler's resource remarks.
-NO_SPILL_KERNELS = {"gemm.hip": ["ternary_gemm_x16_kernel"], "dit_self.hip": ["dit_self_block_kernel"], "gemm_wide.hip": ["gemm_wide_kernel"],
-                    "gemm_f32.hip": ["gemm_narrow_f32_kernel"], "attention.hip": ["attn_tiles_kernel", "attn_rows_kernel", "attn_wide_kernel"]}
+# compiler's resource remarks.  Name -> pattern of the mangled names (attn_kernel: its direct-to-LDS forms, NL = 0 and NSL > 0).
+NO_SPILL_KERNELS = {
+    "gemm.hip": {k: k for k in ("ternary_gemm_x16_kernel", "ternary_gemm_ring_kernel", "gemm_dl_kernel", "gemm_narrow_kernel")},
+    "dit_self.hip": {"dit_self_block_kernel": "dit_self_block_kernel"},
+    "gemm_wide.hip": {"gemm_wide_kernel": "gemm_wide_kernel"},
+    "gemm_f32.hip": {"gemm_narrow_f32_kernel": "gemm_narrow_f32_kernel"},
+    "attention.hip": dict({k: k for k in ("attn_stream_kernel", "attn_tiles_kernel", "attn_rows_kernel", "attn_wide_kernel")},
+                          attn_kernel=r"attn_kernelI\w+?ELi0ELi[1-9]ELi\d+EE"),
+}
 
 
 def _check_no_spill(src, remarks):
-    for kernel in NO_SPILL_KERNELS.get(os.path.basename(src), []):
+    for kernel, pattern in NO_SPILL_KERNELS.get(os.path.basename(src), {}).items():
         lines = remarks.splitlines()
         seen = False
         for i, l in enumerate(lines):
-            if "Function Name:" in l and kernel in l:
+            if "Function Name:" in l and re.search(pattern, l):
                 for m in lines[i:i + 40]:
                     if "ScratchSize [bytes/lane]:" in m:
                         seen = True
