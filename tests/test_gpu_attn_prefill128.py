@@ -16,7 +16,7 @@ D = 128
                                                      (7, 301, 20, 5, 583, 584)])
 @pytest.mark.parametrize("mask", ["none", "causal", "padded", "given"])
 @pytest.mark.parametrize("dtype", [pkg.VLA_DT_BF16, pkg.VLA_DT_BF16_P2])
-def test_many_workgroups(B, S, Hq, Hkv, n_keys, t_max, mask, dtype):
+def test_many_workgroups(tune, B, S, Hq, Hkv, n_keys, t_max, mask, dtype):
     g = torch.Generator().manual_seed(1000 * n_keys + S)
     rnd = lambda *shape: torch.randn(*shape, generator=g).to(torch.bfloat16).cuda()
     k = torch.full((B, Hkv, t_max, D), float("nan"), dtype=torch.bfloat16, device="cuda")  # stale cache contents
@@ -48,3 +48,5 @@ def test_many_workgroups(B, S, Hq, Hkv, n_keys, t_max, mask, dtype):
     for b in (0, B // 2, B - 1):
         assert torch.equal(run(b, b + 1)[0], every[b])
     assert torch.equal(run(0, B, 4), every)  # eight bytes off
+    tune.set("VLA_ATTN_DL", 0)  # the kernel that stages tiles in registers, on the same launch
+    assert torch.equal(run(0, B), every)

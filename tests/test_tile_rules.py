@@ -19,6 +19,7 @@ extern "C" int plan_f32(int M, int N, int gated) { return vla_rules::narrow_plan
 extern "C" int rows_kernel(int grid, int blocks, int sliced) { return vla_rules::attn_rows(grid, blocks, sliced); }
 extern "C" int tiles_kernel(int grid, int tiles) { return vla_rules::attn_tiles(grid, tiles); }
 extern "C" int f32_tile(int M, int n_tiles) { return vla_rules::f32_tile(M, n_tiles); }
+extern "C" int ring128(int wgs, int aligned, int dl) { return vla_rules::attn_ring128(wgs, aligned, dl); }
 extern "C" int wide(int M, int N, int K, int kind) { return vla_rules::wide_tile(M, N, K, kind); }
 extern "C" int plain(int M, int N, int K) { return vla_rules::plain_tile(M, N, K); }
 extern "C" int ternary(int M, int N, int K) { return vla_rules::ternary_tile(M, N, K); }
@@ -220,3 +221,9 @@ def test_a_plain_tile_is_named_for_every_size(rules):
                 assert -1 <= t < 9
                 if t < 6:
                     assert t == rules.wide(M, N, K, 0)
+
+
+def test_128_wide_heads_leave_the_staged_tiles_beyond_one_workgroup_a_cu(rules):
+    """... unless the caches are unaligned or the override pins the staged tiles."""
+    assert [rules.ring128(w, 1, -1) for w in (1, 255, 256, 257, 1020)] == [0, 0, 0, 1, 1]
+    assert not rules.ring128(1020, 0, -1) and not rules.ring128(1020, 1, 0) and rules.ring128(1020, 1, 1)

@@ -2689,12 +2689,10 @@ int launch_nw(AttnArgs& a, hipStream_t st) {
     if (D == 128) a.n_rblocks = grid / 8;
     set_divisors(a, grid);
     if constexpr (sizeof(T) == 2 && D == 128 && NW >= 3) {
-        // More workgroups than CUs: tiles straight into LDS and few enough registers for two workgroups a CU (the same bits), so that one's
-        // products run beside the other's softmax.  515 rows of 20 heads on 5 kv heads, two-term probabilities: 3 observations (255
-        // workgroups) 24.8 us, here 28.4; 4, 8, 12 (340, 680, 1020) 42.9, 64.8, 86.2, here 37.6, 59.1, 72.3; 16 of 100 rows 18.5, here 14.8.
+        // Tiles straight into LDS and few enough registers for two workgroups a CU (the same bits), so that one's products run beside the other's softmax.
         // Groups of three row tiles take the four-wavefront form too, whose last one then only loads: 53 observations of 20 rows 14.1 us staged,
         // 11.7 with three wavefronts (which did not fit 256 registers: 12 bytes a lane in scratch), 11.4 with four; 40 of 72 rows 30.4, 26.2, 25.6.
-        if (wgs > 256 && (((uintptr_t)a.k_cache | (uintptr_t)a.vt_cache) & 15) == 0) {
+        if (vla_rules::attn_ring128(wgs, (((uintptr_t)a.k_cache | (uintptr_t)a.vt_cache) & 15) == 0, tuning().attn_dl)) {
             if (a.p2) attn_kernel<T, D, 4, true, 0, 1, 2><<<grid, 256, 0, st>>>(a);
             else attn_kernel<T, D, 4, false, 0, 1, 2><<<grid, 256, 0, st>>>(a);
             return hipGetLastError() == hipSuccess ? launch_merge<T, D>(a, st) : VLA_K_ERR_LAUNCH;
@@ -2703,8 +2701,7 @@ int launch_nw(AttnArgs& a, hipStream_t st) {
     if constexpr (sizeof(T) == 2 && D == 64) {
         // 64-wide bf16 heads: tiles go straight into a swizzled LDS ring (the tuning override
         // attn_dl = 0 pins the register-staged path), and with three or more key tiles they
-        // are split over two wavefronts per row tile (attn_slices = 1 | 2 overrides).  The
-        // kernel also builds for 128-wide heads, where its register use makes it the slower choice.
+        // are split over two wavefronts per row tile (attn_slices = 1 | 2 overrides).
         if (tuning().attn_dl != 0) {
             const int nsl = a.n_slices;
             if constexpr (D == 64 && NW <= 2) {

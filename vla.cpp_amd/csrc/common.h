@@ -18,7 +18,7 @@ namespace vk {
 // environment once (vla_kernels_init, or the first launch that asks) and again only by
 // vla_kernels_reload_env: no launch path calls getenv.
 struct Tuning {
-    int attn_dl = -1;           // VLA_ATTN_DL: 0 pins the register-staged LDS kernel for 64-wide bf16 heads
+    int attn_dl = -1;           // VLA_ATTN_DL: 0 pins the register-staged LDS kernel for 64- and 128-wide bf16 heads
     int attn_slices = 0;        // VLA_ATTN_SLICES: 1 | 2 key slices per row tile in the direct-to-LDS kernel
     int attn_split = -1;        // VLA_ATTN_SPLIT: key slices across workgroups (<= 0 pins one)
     bool attn_split_set = false;

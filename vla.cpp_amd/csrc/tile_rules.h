@@ -251,6 +251,12 @@ inline bool attn_tiles(long grid, int blocks) {
 // it: 16 rows x 16 heads on 4, 1000 keys 14.8 us, here 16.0 (one slice only: 50 x 15 on 5, two observations 87.9, here 17.1).
 inline bool attn_rows(long grid, int blocks, bool sliced) { return grid <= 512 && (blocks <= 20 || !sliced); }
 
+// Whether a bf16 attention launch of 128-wide heads with three or four row tiles a workgroup takes the tiled kernel's direct-to-LDS form rather than
+// the register-staged one: more workgroups than CUs, so that a CU has two.  515 rows of 20 heads on 5 kv heads, two-term probabilities: 3 observations
+// (255 workgroups) 24.8 us, direct 28.4; 4, 8, 12 (340, 680, 1020) 42.9, 64.8, 86.2, direct 37.6, 59.1, 72.3; 16 of 100 rows 18.5, direct
+// 14.8.  dl: the tuning override VLA_ATTN_DL, 0 pins the register-staged form.
+inline bool attn_ring128(long wgs, bool aligned, int dl) { return dl != 0 && aligned && wgs > 256; }
+
 // Row blocks (of 16) per workgroup and key slices of a bf16 attention launch of 256-wide heads on attn_wide_kernel, or rb = 0 for the tiled
 // kernel.  pairs: (observation, kv head); units: 64-key units, four of which a workgroup walks at a time; part_rows: rows of partials
 // that the call's scratch holds (what the tiled kernel asks for, so that no call needs more than it did).  A workgroup fills a CU, so only splits whose
