@@ -96,3 +96,24 @@ def test_error_is_no_larger_than_the_tiled_kernels(tune, B, n_keys, size):
     tiled, new = out
     assert not torch.equal(tiled, new)  # two kernels
     assert error(new, want) <= 1.006 * error(tiled, want)
+
+
+def test_fp32_partials_pin_the_tiled_kernel(tune):
+    """VLA_ATTN_PART_F32 says in what format the tiled kernel's key slices travel: alone it gives the bits that it gives with that kernel
+    pinned, and they are those neither of fp16 partials nor of the kernel that this launch takes by itself."""
+    B, S, Hq, n_keys = 1, 51, 8, 867
+    g = torch.Generator().manual_seed(9)
+    rnd = lambda *shape: torch.randn(*shape, generator=g).to(torch.bfloat16).cuda()
+    q, k, vt = rnd(B, S, Hq, D), rnd(B, 1, 896, D), rnd(B, 1, D, 896)
+
+    def run(**env):
+        tune.clear("VLA_ATTN_PART_F32", "VLA_ATTN_ROWS")
+        for key, value in env.items():
+            tune.set("VLA_ATTN_" + key, value)
+        o = torch.empty_like(q)
+        pkg.call("vla_attn_prefix_suffix", q, k, vt, o, BF16, B, S, Hq, 1, D, 896, n_keys, D ** -0.5, pkg.VLA_MASK_NONE, 0, 0, 0, None)
+        return o
+
+    f32 = run(PART_F32=1)
+    assert torch.equal(f32, run(PART_F32=1, ROWS=0))
+    assert not torch.equal(f32, run(ROWS=0)) and not torch.equal(f32, run())

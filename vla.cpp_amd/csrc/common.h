@@ -22,16 +22,16 @@ struct Tuning {
     int attn_slices = 0;        // VLA_ATTN_SLICES: 1 | 2 key slices per row tile in the direct-to-LDS kernel
     int attn_split = -1;        // VLA_ATTN_SPLIT: key slices across workgroups (<= 0 pins one)
     bool attn_split_set = false;
-    bool attn_part_f32 = false;  // VLA_ATTN_PART_F32: fp32 partials where fp16 would be used
+    bool attn_part_f32 = false;  // VLA_ATTN_PART_F32: the tiled kernel, with fp32 partials where fp16 would be used
     bool attn_no_arrive = false; // VLA_ATTN_NO_ARRIVE: no in-launch merge by the last slice to arrive
     bool attn_no_direct = false; // VLA_ATTN_NO_DIRECT: never the register-direct kernel
     bool attn_no_stream = false; // VLA_ATTN_NO_STREAM: never the streaming (LDS-ring) form of the register-direct kernel
     int gemm_rows_max = 512;     // VLA_GEMM_ROWS_MAX: projections of at most this many rows may take the narrow-tile kernels, 0 = never
     int gemm_rows_plan = 0;      // VLA_GEMM_ROWS_PLAN: 1..4 pins those kernels' rows x columns per workgroup (16x16, 32x16, 64x16, 64x32; fp32: 1 and 3), 0 = by shape
     bool attn_no_small = false;  // VLA_ATTN_NO_SMALL: fp32 launches with few row tiles do not split their keys beyond the usual rule
-    int attn_rows = -1;          // VLA_ATTN_ROWS: 0 never, 1 always (as far as they serve the shape) the kernels of a wavefront per key block for 48- and 64-wide heads; unset = by shape
+    int attn_rows = -1;          // VLA_ATTN_ROWS: 0 never, 1 always (as far as they serve the shape) the kernels of a wavefront per key block for 48- and 64-wide heads and per 64-key unit for 256-wide bf16 ones; unset = by shape
     int attn_direct_rows = 32;   // VLA_ATTN_DIRECT_ROWS: row limit of the register-direct kernel
-    int gemm_tile = -1;          // VLA_GEMM_TILE: 0..5, wide tiles 16..24
+    int gemm_tile = -1;          // VLA_GEMM_TILE: 0..5, wide tiles 16..21, plain products also 22..24
     int gemm_panel = 0;          // VLA_GEMM_PANEL: N tiles per panel of an XCD's walk over its tiles; 0 = by size
     int gemm_dl = -1;            // VLA_GEMM_DL: 0 pins the register-staged GEMM
     int gemm_stages = 0;         // VLA_GEMM_STAGES: ring depth of the direct-to-LDS GEMM

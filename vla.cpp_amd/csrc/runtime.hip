@@ -37,7 +37,7 @@ void load_locked() {
     t.gemm_rows_max = env_int("VLA_GEMM_ROWS_MAX", 512);
     t.gemm_rows_plan = env_int("VLA_GEMM_ROWS_PLAN", 0);
     t.attn_no_small = getenv("VLA_ATTN_NO_SMALL") != nullptr;
-    t.attn_rows = env_int("VLA_ATTN_ROWS", t.attn_dl >= 0 || t.attn_slices || t.attn_split_set || t.attn_no_small ? 0 : -1);  // those pin forms of the tiled kernel
+    t.attn_rows = env_int("VLA_ATTN_ROWS", t.attn_dl >= 0 || t.attn_slices || t.attn_split_set || t.attn_no_small || t.attn_part_f32 ? 0 : -1);  // those pin forms of the tiled kernel
     t.attn_direct_rows = env_int("VLA_ATTN_DIRECT_ROWS", 32);
     t.gemm_tile = env_int("VLA_GEMM_TILE", -1);
     t.gemm_panel = env_int("VLA_GEMM_PANEL", 0);
