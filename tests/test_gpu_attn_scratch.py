@@ -26,9 +26,11 @@ BF16 = pkg.VLA_DT_BF16
 SLICED = [
     ("decode-arrive", 8, 1, 20, 5, 128, 519, pkg.VLA_DT_BF16_P2, pkg.VLA_MASK_NONE),
     ("decode-merge-kernel", 2, 5, 6, 2, 64, 2100, BF16, pkg.VLA_MASK_NONE),
-    ("pi0-wide-fp16-partials", 1, 51, 8, 1, 256, 867, BF16, pkg.VLA_MASK_PI0_STATE),
+    ("pi0-wide-fp32-partials", 1, 51, 8, 1, 256, 867, BF16, pkg.VLA_MASK_PI0_STATE),
     # (more keys than the kernel that merges its key blocks in LDS takes when the tiled one would slice them)
     ("fp32-lds-split", 2, 5, 6, 2, 64, 1000, pkg.VLA_DT_F32, pkg.VLA_MASK_CAUSAL_SUFFIX),
+    # (more row tiles than one round of the 256-wide kernel's workgroups: the tiled kernel and its fp16 partials)
+    ("pi0-tiled-fp16-partials", 20, 51, 8, 1, 256, 867, BF16, pkg.VLA_MASK_PI0_STATE),
 ]
 
 
@@ -62,6 +64,24 @@ def run(entry, case, q, kc, vc, t_max, extra=()):
             None, *extra, pkg.stream())
     torch.cuda.synchronize()
     return rc, out.cpu().numpy()
+
+
+def test_fp16_partials_take_half_the_room_of_fp32_ones(tune):
+    """Bytes that the tiled kernel leaves in its scratch by default, and with the switch that keeps its partials in fp32: a launch
+    that another kernel served, or in another format, would leave as many both times (a byte is zero by chance once in a few hundred)."""
+    case = SLICED[-1]
+    name, B, S, Hq, Hkv, D, T, dt, mk = case
+    need = pkg.lib().vla_attn_workspace_bytes(dt, B, S, Hq, Hkv, D, T)
+    q, kc, vc, t_max = setup_case(case)
+    used = {}
+    for f32 in (0, 1):
+        if f32:
+            tune.set("VLA_ATTN_PART_F32", 1)
+        ws = torch.zeros(need, dtype=torch.uint8, device="cuda")
+        rc, _ = run("vla_attn_prefix_suffix_ws", case, q, kc, vc, t_max, (ws.data_ptr(), need))
+        assert rc == pkg.VLA_K_OK
+        used[f32] = int((ws != 0).sum())
+    assert 1.8 < used[1] / used[0] < 2.2
 
 
 @pytest.mark.parametrize("case", SLICED, ids=[c[0] for c in SLICED])
@@ -156,7 +176,7 @@ def _obs(cfg, r, n_views):
 
 
 def test_two_handles_with_different_scratch_needs_do_not_disturb_each_other(tmp_path):
-    # pi0 at batch 1 (seven key slices) and a second handle at batch 4 whose partial rows need
+    # pi0 at batch 1 (four key slices) and a second handle at batch 4 whose partial rows need
     # a larger block: each handle replays its captured chunk; alternating them three times
     # gives, every time, the bits each gives alone.
     cfg = ckpt.pi0_config(n_layers=3)

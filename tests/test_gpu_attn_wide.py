@@ -75,6 +75,7 @@ def test_attention_of_256_wide_heads(tune, B, S, Hq, Hkv, n_keys, t_max, forced,
     if want.norm() == 0:
         assert torch.equal(new, torch.zeros_like(new))
         return
+    assert error(tiled, want) < 2 ** -8
     assert error(new, want) <= 1.1 * error(tiled, want) + 1e-4
     assert error(new, want) < 2 ** -8
 

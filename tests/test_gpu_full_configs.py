@@ -65,7 +65,7 @@ def test_config2_pi0_18_layers_batch_16(tmp_path):
     got = m.predict_batch(obs).reshape(16, 50, 32)
     _check_first_and_last(cfg, w, obs, got)
     assert np.array_equal(m.predict_batch(obs).reshape(16, 50, 32), got)
-    # batch 1: seven key slices instead of four -- the other dispatch the bench line reports
+    # batch 1: 16-row workgroups and four key slices instead of 32-row ones without -- the other dispatch the bench line reports
     solo = m.predict(obs[0]).reshape(50, 32)
     want = orc_chunk.flow_expert_chunk(cfg, w, obs[0], emulate_bf16=False)
     assert bf16_close(solo, want), np.abs(solo - want).max()

@@ -904,10 +904,10 @@ def test_attention_cache_rows_of_any_multiple_of_8(dtype, case):
 
 
 @pytest.mark.parametrize("dtype", [F32, BF16], ids=["f32", "bf16"])
-@pytest.mark.parametrize("case", [c for c in CASES if c[5] in (48, 64)], ids=[c[0] for c in CASES if c[5] in (48, 64)])
+@pytest.mark.parametrize("case", [c for c in CASES if c[5] in (48, 64, 256)], ids=[c[0] for c in CASES if c[5] in (48, 64, 256)])
 def test_tiled_attention_where_few_workgroups_take_another_kernel(tune, dtype, case):
-    """48- and 64-wide heads: launches of the size of CASES take the kernels with a wavefront per key block.  The tiled kernel that
-    larger launches take (in fp32 with its key slices and the merge launch) on the same cases."""
+    """48-, 64- and 256-wide heads: launches of the size of CASES take the kernels with a wavefront per key block or unit.  The tiled kernel
+    that larger launches take (in fp32 with its key slices and the merge launch, 256-wide bf16 heads with fp16 partials) on the same cases."""
     tune.set("VLA_ATTN_ROWS", 0)
     test_attention_against_oracle(tune, dtype, "auto", case)
     test_attention_cache_rows_of_any_multiple_of_8(dtype, case)
@@ -997,9 +997,10 @@ def test_attention_decode_slices_merged_by_the_last_to_arrive(tune, B, S, Hq, Hk
 
 @pytest.mark.parametrize("B", [1, 4])
 def test_attention_wide_heads_key_slices_and_partial_formats(tune, B):
-    # pi0's 256-wide MQA heads: with few workgroups the keys are walked in slices whose partial
-    # outputs travel as fp16 (normalised per slice) to a merge launch.  Unsliced, fp32 partials
-    # and fp16 partials all meet the oracle; the fp16 partials cost less than the output rounding.
+    # pi0's 256-wide MQA heads on the tiled kernel, which serves what does not fit one round of the other one's
+    # workgroups: with few workgroups the keys are walked in slices whose partial outputs travel as fp16 (normalised
+    # per slice) to a merge launch.  Unsliced, fp32 partials and fp16 partials all meet the oracle; the fp16 partials cost
+    # less than the output rounding.  Three launches of the tiled kernel that differ: no two have the same bits.
     r = np.random.default_rng(130 + B)
     S, Hq, Hkv, D, P = 51, 8, 1, 256, 816
     T, t_max = P + S, 896
@@ -1012,6 +1013,7 @@ def test_attention_wide_heads_key_slices_and_partial_formats(tune, B):
     mask = orc.mask_pi0_full(P, S)
     want = np.stack([orc.attention(Q[b], K[b], V[b], mask, 1.0 / 16) for b in range(B)])
     got = {}
+    tune.set("VLA_ATTN_ROWS", 0)
     for name, env in (("sliced-fp16", {}), ("sliced-fp32", {"VLA_ATTN_PART_F32": "1"}), ("unsliced", {"VLA_ATTN_SPLIT": "1"})):
         for k in ("VLA_ATTN_PART_F32", "VLA_ATTN_SPLIT"):
             tune.clear(k)
@@ -1025,6 +1027,7 @@ def test_attention_wide_heads_key_slices_and_partial_formats(tune, B):
         assert np.isfinite(got[name]).all() and bf16_close(got[name], want) and rel_err(got[name], want) < 1e-2, name
     assert rel_err(got["sliced-fp16"], want) <= rel_err(got["unsliced"], want) * 1.25 + 1e-4
     assert rel_err(got["sliced-fp16"], got["sliced-fp32"]) < 1e-2
+    assert not any(np.array_equal(got[a], got[b]) for a, b in (("sliced-fp16", "sliced-fp32"), ("sliced-fp16", "unsliced"), ("sliced-fp32", "unsliced")))
 
 
 def test_attention_special_cases_fp32():
