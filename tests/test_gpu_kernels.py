@@ -1230,7 +1230,9 @@ def test_ternary_gemm_add_matches_gemm_then_add(tune, M, N, K, tile):
     assert np.array_equal(host(fused), host(want))
 
 
-@pytest.mark.parametrize("M,K", [(8, 2560), (37, 720), (4, 4096), (300, 2560), (129, 720), (70, 4096), (9, 6912), (3, 16384)])
+# (2056, 2304, 2552: rows that end inside the fifth vector of a lane, in its first and in its last one; 4104: the first row too long for a wavefront)
+@pytest.mark.parametrize("M,K", [(8, 2560), (37, 720), (4, 4096), (300, 2560), (129, 720), (70, 4096), (9, 6912), (3, 16384),
+                                 (5, 2048), (5, 2056), (6, 2304), (7, 2552), (5, 2568), (1, 8), (2, 4104)])
 def test_rmsnorm_act_quant_fused_is_the_pair(M, K):
     r = np.random.default_rng(K + M)
     x = orc.to_bf16((r.standard_normal((M, K)) * 3).astype(np.float32))
@@ -1261,7 +1263,7 @@ def test_rmsnorm_act_quant_fused_is_the_pair(M, K):
 
 
 @pytest.mark.parametrize("M,N,K,ws_num", [(1, 3840, 2560, 3), (8, 3840, 2560, 3), (8, 2560, 2560, 1), (3, 48, 128, 3),
-                                          (5, 640, 4096, 1), (7, 100, 1024, 1)])
+                                          (5, 640, 4096, 1), (7, 100, 1024, 1), (8, 96, 2176, 3), (3, 100, 2304, 1), (1, 64, 2688, 1)])
 def test_rmsnorm_ternary_gemv_one_launch_is_the_chain(M, N, K, ws_num):
     # Decode rows: norm + quantisation inside the GEMV launch gives the bits of
     # vla_rmsnorm_act_quant_bf16 -> vla_ternary_gemm_add, with and without the residual
@@ -1284,8 +1286,12 @@ def test_rmsnorm_ternary_gemv_one_launch_is_the_chain(M, N, K, ws_num):
         got, got_res = torch.zeros_like(want), dev(res)
         pkg.call("vla_rmsnorm_ternary_gemv", dev(x), dw, 1e-5, dW, got, None, dws, ws_num, M, N, K)
         pkg.call("vla_rmsnorm_ternary_gemv", dev(x), dw, 1e-5, dW, got_res, got_res, dws, ws_num, M, N, K)
+        got_w = torch.zeros_like(want)  # a norm weight that is not 16-byte aligned takes element loads: same bits
+        wpad = torch.zeros(K + 8, dtype=torch.int16, device="cuda")
+        wpad[1:K + 1] = dw
+        pkg.call("vla_rmsnorm_ternary_gemv", dev(x), wpad[1:K + 1], 1e-5, dW, got_w, None, dws, ws_num, M, N, K)
         sync()
-        assert torch.equal(got, want) and torch.equal(got_res, want_res)
+        assert torch.equal(got, want) and torch.equal(got_res, want_res) and torch.equal(got_w, want)
     # and the chain follows the oracle: norm -> bf16 -> quantise -> int32 GEMM -> epilogue
     n = orc.round_bf16(orc.rms_norm(orc.from_bf16(x), orc.from_bf16(w), 1e-5))
     qo, so = orc.act_quant(n)

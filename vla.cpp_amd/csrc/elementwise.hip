@@ -404,15 +404,18 @@ bool launch_row_norm(const void* x, const void* w, const float* sc, const float*
     const int nvec = K / EPV, blocks = (M + 3) / 4;
 #define VLA_ROW_NORM(NV) \
     row_norm_kernel<T, NV, MODE, GLU><<<blocks, 256, 0, st>>>((const T*)x, (const T*)w, sc, sh, (T*)y, q, scales, rowsum, M, K, eps)
-    if (nvec <= 64 * 2) VLA_ROW_NORM(2);
-    else if (nvec <= 64 * 4) VLA_ROW_NORM(4);
-    else if (MODE == NORM_RMS_AQ && sizeof(T) == 2 && nvec <= 64 * 5) VLA_ROW_NORM(5);  // the 2560-wide model
-    else if (nvec <= 64 * 8) VLA_ROW_NORM(8);
-    else if constexpr (MODE == NORM_RMS_AQ && sizeof(T) == 2) {  // the 6912-wide BitNet FFN rows
+    if constexpr (MODE == NORM_RMS_AQ && sizeof(T) == 2) {
         if (nvec > 64 * 16) return false;
-        row_norm_wide_kernel<GLU><<<M, 256, 0, st>>>((const bf16_t*)x, (const bf16_t*)w, q, scales, rowsum, K, eps);
+        if (nvec > 64 * 8) row_norm_wide_kernel<GLU><<<M, 256, 0, st>>>((const bf16_t*)x, (const bf16_t*)w, q, scales, rowsum, K, eps);  // the 6912-wide BitNet FFN rows
+        else if (nvec > 64 * 5) VLA_ROW_NORM(8);
+        else if (nvec > 64 * 4) VLA_ROW_NORM(5);  // the 2560-wide model
+        else if (nvec > 64 * 2) VLA_ROW_NORM(4);
+        else VLA_ROW_NORM(2);
     } else {
-        return false;
+        if (nvec > 64 * 8) return false;
+        if (nvec > 64 * 4) VLA_ROW_NORM(8);
+        else if (nvec > 64 * 2) VLA_ROW_NORM(4);
+        else VLA_ROW_NORM(2);
     }
 #undef VLA_ROW_NORM
     return true;

@@ -2044,8 +2044,7 @@ int launch_gemv_norm(const GemmArgs& a, vla_stream_t stream) {
     if (groups <= 10) {
         if (nvec <= 128) VLA_GEMV_NORM(10, 2);
         else if (nvec <= 256) VLA_GEMV_NORM(10, 4);
-        else if (nvec <= 320) VLA_GEMV_NORM(10, 5);  // the 2560-wide model: three vectors of eight would be padding
-        else VLA_GEMV_NORM(10, 8);
+        else VLA_GEMV_NORM(10, 5);  // up to 2560 wide, the model's rows: three vectors of eight would be padding
     } else if (groups <= 16) {
         VLA_GEMV_NORM(16, 8);
     } else {
