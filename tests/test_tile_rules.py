@@ -227,3 +227,19 @@ def test_128_wide_heads_leave_the_staged_tiles_beyond_one_workgroup_a_cu(rules):
     """... unless the caches are unaligned or the override pins the staged tiles."""
     assert [rules.ring128(w, 1, -1) for w in (1, 255, 256, 257, 1020)] == [0, 0, 0, 1, 1]
     assert not rules.ring128(1020, 0, -1) and not rules.ring128(1020, 1, 0) and rules.ring128(1020, 1, 1)
+
+
+# (observation, kv head) pairs, query rows, keys -> measured us of the tiled kernel with its merge launch and of the 256-wide kernel
+HEADS_US = [((1, 400, 955), 16.6, 10.8), ((8, 400, 955), 21.9, 16.2), ((16, 400, 955), 27.8, 21.9),
+            ((1, 8, 523), 8.8, 9.8), ((1, 16, 523), 9.6, 10.3), ((2, 8, 700), 10.9, 11.6), ((1, 32, 400), 9.7, 10.1), ((6, 32, 400), 11.8, 12.3), ((16, 8, 955), 14.5, 12.6),
+            ((32, 128, 1990), 31.1, 72.7), ((64, 64, 1990), 38.0, 78.4), ((24, 256, 1990), 32.6, 53.2), ((48, 64, 955), 21.1, 25.6), ((24, 128, 1990), 26.5, 36.9),
+            ((16, 256, 3000), 32.1, 47.1), ((12, 400, 3000), 53.1, 57.5), ((8, 400, 3000), 27.1, 32.5), ((6, 400, 1990), 22.4, 26.2), ((1, 400, 1990), 50.2, 17.6),
+            ((64, 8, 1990), 37.9, 30.6)]
+
+
+@pytest.mark.parametrize("shape,tiled,wide", HEADS_US)
+def test_256_wide_heads_take_the_faster_kernel(rules, shape, tiled, wide):
+    """... also where an XCD's L2 does not hold the K and V^T that its row tiles share, and where few rows leave the wavefronts idle."""
+    pairs, rows, keys = shape
+    took = wide if rules.heads256(pairs, rows, -(-keys // 64), 1 << 20, 0) >= 100 else tiled
+    assert took <= 1.04 * min(tiled, wide)

@@ -264,15 +264,23 @@ inline bool attn_ring128(long wgs, bool aligned, int dl) { return dl != 0 && ali
 // V^T once per 128 rows (50 positions x 8 heads on 955 keys, 20 observations, 260 workgroups: tiled 40.5 us, here 41.7; 32: 34.6, 46.8).  Of
 // these the least predicted time (us): start and end 5.5, a round of units 2.5 (16 rows) or 3.3 (32), the merge launch 1.8 and 0.75 per
 // 1000 partial rows.  Against the tiled kernel and its merge, 50 positions, 955 keys from memory: 1, 2, 4, 8, 12, 16 observations 16.6, 18.3, 19.1,
-// 22.0, 31.2, 27.8 us, here 10.8, 13.1, 15.6, 16.2, 21.2, 21.9; 60 to 330 keys at 1 to 16 observations 0.59 to 0.95 of its time.  16 rows or
-// fewer on 5 to 8 units: two rounds for what one wavefront row of the tiled kernel's slices does as fast (8 rows, 281 keys 9.1 us,
-// here 9.8): left to it.
+// 22.0, 31.2, 27.8 us, here 10.8, 13.1, 15.6, 16.2, 21.2, 21.9; 60 to 330 keys at 1 to 16 observations 0.59 to 0.95 of its time.  Left to the
+// tiled kernel (of 1067 launches of 8 to 800 rows on 60 to 3000 keys, 1 to 64 observations, 932 are taken, in 0.70 of its time (geometric mean, 1.06 at most)):
+//  - 16 rows or fewer on 5 to 8 units, on up to 11 of up to four pairs; up to 32 rows on 5 to 8 of up to six: two rounds for what one wavefront row of the
+//    tiled kernel's slices does as fast (8 rows, 281 keys 9.1 us, here 9.8; 8 rows, 523 keys 8.8, 9.8; 16 rows, 523 keys 9.6, 10.3);
+//  - more than 5 MiB of K and V^T for an XCD's 4 MiB L2 and more than 32 rows: its row tiles start at different units, and what one has
+//    read is gone before the next one comes (128 rows, 1990 keys: 32 pairs 31.1 us, here 72.7; 24 pairs 26.5, 36.9; 20 pairs 34.0, 27.1);
+//  - more than 256 rows on more than 24 units of five to eight pairs: level on the mean, 0.79 to 1.20 of its time (400 rows, eight pairs, 3000 keys 27.1, 32.5).
 struct WideHeads {
     int rb, slices;
 };
 inline WideHeads wide_heads(long pairs, int rows, int units, long part_rows, bool forced) {
     WideHeads best = {0, 1};
-    if (rows <= 16 && units > 4 && units <= 8 && !forced) return best;
+    if (!forced) {
+        if (rows <= 16 ? units > 4 && (units <= 8 || (units <= 11 && pairs <= 4)) : rows <= 32 && units > 4 && units <= 8 && pairs <= 6) return best;
+        if (rows > 32 && (pairs + 7) / 8 * units > 80) return best;  // a unit of a pair is 64 KiB
+        if (rows > 256 && pairs > 4 && pairs <= 8 && units > 24) return best;
+    }
     double least = 1e30;
     for (int rb = 1; rb <= 2; ++rb) {
         const long tiles = (rows + 16 * rb - 1) / (16 * rb);
