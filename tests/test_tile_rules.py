@@ -203,6 +203,9 @@ PLAIN_US = [
     ((408, 1536, 6144), 24.4, (42.5, 39.5, 29.4)),
     ((816, 1024, 4096), 15.6, (23.5, 26.7, 18.5)),
     ((1323, 6144, 1536), 29.7, (42.8, 50.5, 43.8)),
+    ((6301, 8, 112), 3.5, (9.9, 9.9, 3.8)),  # (of these three 96 x 64 alone was timed)
+    ((7527, 32, 96), 3.6, (9.9, 9.9, 3.9)),
+    ((1330, 32, 128), 3.6, (9.9, 9.9, 3.8)),
 ]
 
 

@@ -183,16 +183,17 @@ inline int wide_tile(int M, int N, int K, int kind, double* predicted = nullptr)
 // The same for a plain product, whose epilogue also comes with 32- and 48-column wavefronts: one of those tiles where it is predicted 6 %
 // faster than what wide_tile takes.  Their step per 64 k is the root of the squares of what a CU needs for itself and what its share of the
 // L2s' rate allows (load, times the share of the CUs that are busy): 1323 x 1536 x 6144 takes 46.1 us on 224 tiles of 96 x 96, 42.6 on 176 of
-// 128 x 96.  On 948 shapes (200 to 4000 rows, N 256 to 8192, K 128 to 8192, weights from memory) taken on 253, where it needs 0.88 of the time
-// (geometric mean); six of them are 1 to 6 % slower.  Long rows that do not start on a cache line are left out: predicted as well on the mean,
+// 128 x 96.  On 947 shapes (200 to 4000 rows, N 256 to 8192, K 128 to 8192, weights from memory) taken on 253, where it needs 0.88 of the time
+// (geometric mean); five of them are up to 6 % slower.  Long rows that do not start on a cache line are left out: predicted as well on the mean,
 // but 672 x 1536 x 4432 and 1042 x 1152 x 5008 take 1.22 times as long.  1323 x 1536 x 6144 55.2 -> 42.6 us, 2000 x 1536 x 6144 59.1 -> 48.4, 1600 x 720 x 2048
-// 13.8 -> 12.0; 408 x 1536 x 6144 stays: 24.4, here 29.4.
+// 13.8 -> 12.0; 408 x 1536 x 6144 stays: 24.4, here 29.4.  Outside of those limits (16 to 20000 rows, N 8 to 40000, K 16 to 20000; 406 shapes for which it names a
+// tile) it needs 0.89 of the time, at most 1.03, but for two k tiles of up to 32 columns, which stay: 6301 x 8 x 112 3.5 us, here 3.8; 7527 x 32 x 96 3.6, 3.9.
 inline int plain_tile(int M, int N, int K) {
     static const struct { int rows, cols; bool pairs; double fixed, round, step, load, round2, step2; } t[PLAIN_TILES - WIDE_TILES] = {
         {96, 96, true, 1.08, 3.64, 0.357, 0.329, 4.44, 0.708}, {128, 96, false, 1.33, 4.80, 0.410, 0.285, 0, 0}, {96, 64, true, 1.94, 1.93, 0.287, 0.200, 2.31, 0.609}};
     double least;
     int best = wide_tile(M, N, K, 0, &least);
-    if (K % 64 != 0 && K > 1024) return best;
+    if ((K % 64 != 0 && K > 1024) || (N <= 32 && K > 64 && K <= 128)) return best;
     least *= 0.94;
     for (int i = 0; i < PLAIN_TILES - WIDE_TILES; ++i) {
         const XcdGrid g = xcd_grid(M, N, K, (M + t[i].rows - 1) / t[i].rows, (N + t[i].cols - 1) / t[i].cols, 2.0, t[i].cols, 2.0, 0);
