@@ -2253,11 +2253,11 @@ bool launch_rows(AttnArgs& a, hipStream_t st) {
 // against query row c: already the right operand of O^T += V^T P^T.  LDS pieces (16 bytes) are XOR-swizzled, K and Q by the row, V^T by
 // row / 2: the fragment reads, sixteen lanes at a time, are free of bank conflicts.
 //
-// What bounds it: 8 KiB a part is 512 clocks of a CU's 64 bytes a clock from the L2 for four wavefronts, and a wavefront whose request has to wait its
-// turn cannot go on with its products either: of some 7000 clocks that a unit takes (32 rows, 2.1 GHz), 4096 are that, 2048 products and 1900
-// the softmax.  Hence requests, fragment reads and products take turns; one wavefront a SIMD, since 32 rows x 256 of output and the query
+// What bounds it: 8 KiB a part for each of four wavefronts is 512 clocks of a CU's 64 bytes a clock from the L2, 4096 a unit of eight parts; products (2048 clocks
+// at 32 rows) and softmax hide behind that in part, since a wavefront whose request has to wait its turn cannot go on with its products
+// either.  Hence requests, fragment reads and products take turns; one wavefront a SIMD, since 32 rows x 256 of output and the query
 // fragments are 192 registers.  50 positions x 8 heads, 955 keys, keys from memory: 16 observations 27.8 -> 21.9 us, 8 21.9 -> 16.2 (16 rows a
-// workgroup), one 16.6 -> 10.8 (four slices, merged by a launch).  Tried: K through registers (the compiler's waits drain V^T's
+// workgroup), one 16.6 -> 10.8 (four slices, merged by a launch), launches alone.  Tried: K through registers (the compiler's waits drain V^T's
 // requests with them), two wavefronts a workgroup and twice the slices (level at one observation), fragments in two sets
 // (registers moved about: 21.3 us with the keys in the caches, now 20.2).
 // RB: 16-row blocks; W: wavefronts; GIVEN: the mask is data (added to the scaled scores; zeros and -inf give the generated masks' bits).

@@ -259,8 +259,9 @@ void BitvlaLm::prefill(const Inputs* in, int batch) {
         }
     };
     run_staged(
-        // One thread at every batch.  2.6 MB of features and 256 rows of text an observation: with eight threads eight observations
-        // take 23.7 ms a call where they take 25.8, twelve 31.0 and 34.1; the caller's refill of its buffers takes 0.6 and 1.1 ms with either.
+        // One thread at every batch: nothing speaks against more of them for large ones, they are not taken up yet.  2.6 MB of features and 256 rows of
+        // text an observation: eight threads take eight observations from 25.8 to 23.7 ms a call and twelve from 34.1 to 31.0; the caller's
+        // refill of its buffers takes 0.6 and 1.1 ms with either.
         first, 1,
         [&](int t) {
             const int b = t / per_obs, piece = t % per_obs - 1;
@@ -359,9 +360,9 @@ bool BitvlaLm::run_layers(Ctx& C, int M, int S, int tok_offset, int n_keys, uint
             prof_mark("sqrelu_norm_quant_down_gemv_add");
             continue;
         }
-        // Longer rows (the model's 6912): every 32-column workgroup of the one-launch form would
-        // repeat the rows' activation and norm, which costs more than a launch; the activation
-        // still stays on chip, inside the norm + quantisation launch.
+        // Longer rows (the model's 6912): every 32-column workgroup of the one-launch form would repeat the
+        // rows' activation and norm, which by a wavefront a row (its form there) costs more than a launch; the
+        // activation still stays on chip, inside the norm + quantisation launch.
         const int rc = vla_sqrelu_rmsnorm_act_quant_bf16(gu_.as<uint16_t>(), w.ffn_sub_norm.as<uint16_t>(), q8_.as<int8_t>(),
                                                          s_.as<float>(), rowsum_.as<int32_t>(), eps_, M, F_, C.stream);
         if (rc != VLA_K_ERR_SHAPE) VLA_K(rc);
